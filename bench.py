@@ -5,8 +5,10 @@ metagenome (1,000 order-3 Markov genomes, log-normal lengths median 8 kb,
 sigma 1.0, clipped to [1.5 kb, 500 kb], 0.5% N): the thresholded, per-row
 capped edge list (cutoff 0.95, maxEdges 200) of all n(n-1)/2 pairs, from
 HBM-resident FP32 TNF rows and FP64 log sizes.  The timed mode is the BF16
-MFMA Gram prefilter + FP32 refinement; the exact FP32 mode and the FP16 mode
-run in the same process, and their edge lists must be identical.
+mode: an MFMA scan bounds every pair's distance from below in 28 projected
+dimensions, the tiles it cannot rule out go through the BF16 Gram and the FP32
+refinement; the exact FP32 mode and the FP16 mode run in the same process, and
+their edge lists must be identical.
 
 value = n(n-1)/2 / (seconds per step): effective pair evaluations per second.
 
@@ -42,15 +44,8 @@ from mdet_amd import workload as W  # noqa: E402
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense BF16/FP16 MFMA
 PEAK_FP32_TFLOPS = 157.3   # MI355X FP32
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
-FLOPS_PER_PAIR = 2 * 136   # algorithmic: one K=136 dot product per unordered pair
+SCAN_FLOPS_PER_PAIR = 2 * 28  # the scan's dot product of two projected rows per unordered pair
 CUTOFF, MAX_EDGES = 0.95, 200
-# Memory-side bytes per launch of the BF16 prefilter at the 200,000-contig
-# workload, from rocprofv3 FETCH_SIZE / WRITE_SIZE (KiB per dispatch) scaled by
-# the same counters on a plain 1 GiB copy (x2.0 fetch, x1.0 write); summary and
-# commands in profiles/pairs_200k_pmc_traffic.md.  Counters cannot be read in
-# the timed run, so the figure is carried here for the workload it was taken on.
-PMC_TRAFFIC = {"c3_200k": {"fetch_kib": 1497722.6, "write_kib": 165978.5, "fetch_scale": 2.0, "write_scale": 1.0}}
-
 
 def log(msg):
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
@@ -437,7 +432,7 @@ def main():
         ctx.close()
         return
 
-    # headline: BF16 MFMA prefilter + FP32 refine, at the launch shape the autotuner picks for this input
+    # headline: the BF16 mode, at the launch shape the autotuner picks for this input
     if args.no_autotune:
         tune = ctx.tune_get(M.BF16_REFINE)
     else:
@@ -491,15 +486,10 @@ def main():
         ec["speedup_vs_bf16_refine"] = modes["bf16_refine"]["ms_per_step"] / ec["ms_per_step"]
         modes["learned"] = lm
 
-    achieved = FLOPS_PER_PAIR * P / (pf_ms * 1e-3) / 1e12
-    traffic = None
-    pm = PMC_TRAFFIC.get(args.workload) if args.n is None else None
-    if pm:
-        traffic = 1024 * (pm["fetch_kib"] * pm["fetch_scale"] + pm["write_kib"] * pm["write_scale"])
-    roofline = {"bound": "mfma", "kernel": "k_prefilter_mfma<bf16>", "achieved": achieved, "peak": PEAK_BF16_TFLOPS,
-                "unit": "TFLOP/s", "frac": achieved / PEAK_BF16_TFLOPS, "traffic": traffic,
-                "traffic_unit": "bytes per launch (memory side, rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated)",
-                "flops_per_launch": FLOPS_PER_PAIR * P, "avg_launch_ms": pf_ms,
+    achieved = SCAN_FLOPS_PER_PAIR * P / (pf_ms * 1e-3) / 1e12
+    roofline = {"bound": "mfma", "kernel": "k_tile_scan (projected rows, FP16)", "achieved": achieved,
+                "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_BF16_TFLOPS,
+                "flops_per_launch": SCAN_FLOPS_PER_PAIR * P, "avg_launch_ms": pf_ms,
                 "timing": "HIP events recorded on the context stream around the launch, mean of the timed steps"}
 
     cpu = None

@@ -171,9 +171,10 @@ int mdet_tnf_count_ascii(mdet_ctx *ctx, const char *seqs_dev, const uint64_t *in
 /* ---------------------------------------------------------------- pairs -- */
 /* Precision of the all-pairs distance stage; every mode yields the same edge
  * set (see mdet_tnf_edges). */
-#define MDET_EXACT_F32 0   /* FP32 sum of squared differences for every pair */
-#define MDET_BF16_REFINE 1 /* BF16 MFMA Gram prefilter + FP32 refinement */
-#define MDET_F16_REFINE 2  /* FP16 MFMA Gram prefilter + FP32 refinement */
+#define MDET_EXACT_F32 0   /* FP32 sum of squared differences for every pair that a lower
+                            * bound of its distance does not rule out */
+#define MDET_BF16_REFINE 1 /* the same with a BF16 MFMA Gram ahead of the FP32 refinement */
+#define MDET_F16_REFINE 2  /* the same with an FP16 MFMA Gram */
 #define MDET_LEARNED 3     /* learned embedding proposals + FP32 refinement
                             * (mdet_tnf_edges_learned; recall measured, full rows exact) */
 
@@ -189,7 +190,8 @@ typedef struct mdet_edges {
 
 typedef struct mdet_pair_stats {
     uint64_t pairs_total;      /* n(n-1)/2 */
-    uint64_t pairs_evaluated;  /* pairs whose distance was computed (all modes: pairs_total) */
+    uint64_t pairs_evaluated;  /* pairs decided (exhaustive modes: pairs_total, most of them by a
+                                * lower bound of their distance) */
     uint64_t survivors;        /* pairs passed from the prefilter to FP32 evaluation */
     uint64_t candidates;       /* pairs with FP32 preProb above threshold - band */
     uint64_t adjudicated;      /* pairs decided by the FP64 tie-breaker */

@@ -26,7 +26,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 HOST_SRCS = ["host_ingest.cpp", "host_gen.cpp", "model_host.cpp", "host_binning.cpp", "host_fit.cpp"]
-HIP_SRCS = ["capi_ctx.hip", "tnf_count.hip", "tnf_ingest.hip", "tnf_pairs.hip", "tnf_ivf.hip", "tnf_mlp.hip", "tnf_fit.hip", "tnf_bin.hip"]
+HIP_SRCS = ["capi_ctx.hip", "tnf_count.hip", "tnf_ingest.hip", "tnf_order.hip", "tnf_pairs.hip", "tnf_ivf.hip", "tnf_mlp.hip", "tnf_fit.hip", "tnf_bin.hip"]
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-Wall"]
 HIP_FLAGS = COMMON + [

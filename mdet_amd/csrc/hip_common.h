@@ -45,8 +45,9 @@ struct mdet_ctx {
     double radius_key[3] = {0, 0, 0};
     double radius = 0;
     bool radius_valid = false;
-    // cached MFMA work items for a padded row count and column span
-    uint32_t items_npad = 0;
+    // cached scan items for a row count, rows per block and column span
+    uint32_t items_n = 0;
+    uint32_t items_rows = 0;
     uint32_t items_seg = 0;
     uint32_t items_order = 0;
     uint32_t nitems = 0;

@@ -3,32 +3,35 @@
 // cal_tnf_pre_dist_d (cuda/Cuda2.cu:192-241).
 //
 // Pipeline (one mdet_tnf_edges call):
-//   prep     per-contig: log-size -> Chebyshev coordinate, range check; for the
-//            MFMA modes the TNF rows in BF16/FP16, K padded 136 -> 144, stored
-//            in MFMA fragment order, and their FP32 squared norms.
-//   prefilter over the upper triangle of contig pairs, keep (i, j) whose
-//            distance can be below R = max over the length range of the edge
-//            distance threshold (+ the rounding error of the mode):
-//              EXACT_F32   FP32 sum of squared differences, VALU tiles
+//   prep     per-contig: log-size -> Chebyshev coordinate, range check; the
+//            row order and the rows' projection on 28 directions (tnf_order.hip);
+//            for the Gram modes the TNF rows in BF16/FP16, K padded 136 -> 144,
+//            in MFMA fragment order.  R = max over the length range of the edge
+//            distance threshold.
+//   scan     (k_tile_scan) which 32 x 32 tiles of the upper triangle can hold a
+//            pair within R: MFMA products of the projected rows, a lower bound
+//            of every pair's distance, with the threshold folded into K; small
+//            inputs skip it and take every tile.
+//            LEARNED: the same kernel on the TNF rows over the pairs of cluster
+//            pairs chosen by the learned embeddings (tnf_ivf.hip).
+//   select survivors of the listed tiles
+//              EXACT_F32   FP32 sum of squared differences of every pair
+//                          (k_tile_f32), d < R
 //              *_REFINE    Gram d^2 = |a|^2 + |b|^2 - 2 a.b on MFMA
-//                          (v_mfma_f32_32x32x16_{bf16,f16}), FP32 accumulate,
-//                          over (256-row block, column segment) items taken
-//                          by persistent blocks from per-XCD queues; the
-//                          survivors leave in tagged chunks, sorted into a
-//                          tile-by-tile list
-//              LEARNED     the same kernel over the pairs of cluster pairs
-//                          chosen by the learned embeddings (tnf_ivf.hip)
-//   refine   per survivor: FP32 sum of squared differences, FP32 model via
-//            the Chebyshev form; a pair whose FP32 preProb lies within EPS of
-//            the threshold (or whose model-1 value lies within EPS of ln 9,
-//            where the model switches) is decided by the FP64 tie-breaker,
-//            which repeats the reference's device arithmetic operation by
-//            operation.  Output: candidates (i, j, preProb).
+//                          (v_mfma_f32_32x32x16_{bf16,f16}), FP32 accumulate
+//                          (k_tile_gram), d < R + the rounding of the rows
+//   refine   (k_tile_refine) per survivor: FP32 sum of squared differences,
+//            FP32 model via the Chebyshev form; a pair whose FP32 preProb lies
+//            within EPS of the threshold (or whose model-1 value lies within EPS
+//            of ln 9, where the model switches) is decided by the FP64
+//            tie-breaker, which repeats the reference's device arithmetic
+//            operation by operation.  Output: candidates (i, j, preProb).
 //   select   candidates -> per-row lists (both endpoints) -> per row the
 //            max_edges largest preProb (ties of FP32 values within 2*EPS of
 //            the cut are re-ranked in FP64) -> edges i < j, sorted.
-// The prefilter only has to be a superset, so every mode returns the same
-// edge set; the modes differ only in how much distance arithmetic is spent.
+// Every pass before the refinement only has to keep a superset, so every mode
+// returns the same edge set; the modes differ in the arithmetic of the pairs
+// that the scan's bound does not rule out.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -38,6 +41,7 @@
 #include "hip_common.h"
 #include "ivf.h"
 #include "model_tables.h"
+#include "order.h"
 #include "tnf_tables.h"
 
 namespace {
@@ -65,6 +69,7 @@ __constant__ double c_c2[19] = {E17(mdet::kC2), mdet::kC2[17], mdet::kC2[18]};
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 struct Cand {
     uint32_t i, j;
@@ -208,21 +213,6 @@ __device__ inline double ord2d(unsigned long long u) {
 // ------------------------------------------------------- wave utilities --
 __device__ inline uint32_t lane_id() { return __lane_id(); }
 
-// Survivor output without a hot counter: every wave appends to one of
-// NSHARD sub-buffers (wave id modulo NSHARD), each with its own counter on
-// its own 128-byte line, so the appends of ~10^6 waves never serialise on
-// one address.  A shard's counter keeps counting past its capacity so the
-// host learns the size needed; k_shard_scan/k_compact then pack the shards
-// into one dense list.
-constexpr int NSHARD = 2048;
-constexpr int SHARD_STRIDE = 16;  // counters 16 x 8 B = 128 B apart
-
-struct SurvOut {
-    uint2* buf;                // NSHARD * cap entries
-    unsigned long long* cnt;   // NSHARD * SHARD_STRIDE
-    unsigned long long cap;    // entries per shard
-};
-
 // Inclusive prefix sum over the 64 lanes with DPP moves (no LDS round
 // trips): row_shr 1, 2, 4, 8 within each 16-lane row, then row_bcast 15 and
 // row_bcast 31 carry the row totals across rows.  All 64 lanes must be active.
@@ -236,12 +226,8 @@ __device__ inline uint32_t wave_incl_sum_dpp(uint32_t x) {
     return x;
 }
 
-__device__ inline uint32_t wave_shard() {
-    return ((blockIdx.x * (blockDim.x >> 6)) + (threadIdx.x >> 6)) & (NSHARD - 1);
-}
-
 // Rows of the select stage are grouped in buckets of S_BUCKET consecutive
-// positions of the prefilter's row order (a multiple of 64; at 200k contigs 64
+// positions of the scan's row order (a multiple of 64; at 200k contigs 64
 // rows selected 5-9% faster than 128 and 256 rows 28% slower: more, shorter
 // blocks balance better, for slightly more bucket counting in the refinement;
 // at 1M contigs the BF16 step's selection took 4.4 ms with 64 against 3.9).
@@ -284,127 +270,46 @@ __device__ inline void wave_aggregated_count(uint32_t* counter, uint32_t key, bo
     }
 }
 
-// All 64 lanes call; lane l gets the shard-local slot of its first item.
-__device__ inline unsigned long long wave_reserve_shard(uint32_t cnt, const SurvOut& o, uint32_t shard) {
-    const uint32_t lane = lane_id();
-    uint32_t x = cnt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= (uint32_t)off) x += y;
-    }
-    const uint32_t total = __shfl(x, 63, 64);
-    unsigned long long base = 0;
-    if (lane == 63 && total) base = atomicAdd(&o.cnt[(size_t)shard * SHARD_STRIDE], (unsigned long long)total);
-    base = __shfl(base, 63, 64);
-    return base + (x - cnt);
-}
-
-__device__ inline void shard_put(const SurvOut& o, uint32_t shard, unsigned long long slot, uint32_t i, uint32_t j) {
-    if (slot < o.cap) o.buf[(size_t)shard * o.cap + slot] = make_uint2(i, j);
-}
-
-// offsets[s] = sum of min(cnt, cap) of shards < s; offsets[NSHARD] = total;
-// stat[0] = total, stat[1] = largest raw count (overflow check).  One block:
-// thread t owns shards 2t and 2t + 1; wave scans, then a scan of the 16 wave
-// totals (integer sums, so the result is the serial prefix sum).
-static_assert(NSHARD == 2 * 1024, "k_shard_scan gives each of its 1024 threads two shards");
-__global__ __launch_bounds__(1024) void k_shard_scan(const unsigned long long* __restrict__ cnt,
-                                                     unsigned long long cap, unsigned long long* __restrict__ offsets,
-                                                     unsigned long long* __restrict__ stat) {
-    __shared__ unsigned long long wsum[16], wmax[16];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const unsigned long long c0 = cnt[(size_t)(2 * t) * SHARD_STRIDE], c1 = cnt[(size_t)(2 * t + 1) * SHARD_STRIDE];
-    const unsigned long long v0 = c0 < cap ? c0 : cap, v1 = c1 < cap ? c1 : cap;
-    unsigned long long x = v0 + v1, m = c0 > c1 ? c0 : c1;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned long long y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-        const unsigned long long z = __shfl_xor(m, off, 64);
-        m = z > m ? z : m;
-    }
-    if (lane == 63) wsum[w] = x;
-    if (lane == 0) wmax[w] = m;
-    __syncthreads();
-    if (w == 0) {
-        const unsigned long long own = lane < 16 ? wsum[lane] : 0ull;
-        unsigned long long sc = own, mm = lane < 16 ? wmax[lane] : 0ull;
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            const unsigned long long y = __shfl_up(sc, off, 64);
-            if (lane >= off) sc += y;
-            const unsigned long long z = __shfl_xor(mm, off, 64);
-            mm = z > mm ? z : mm;
-        }
-        if (lane < 16) wsum[lane] = sc - own;  // exclusive prefix of wave `lane`
-        if (lane == 15) {
-            offsets[NSHARD] = sc;
-            stat[0] = sc;
-        }
-        if (lane == 0) stat[1] = mm;
-    }
-    __syncthreads();
-    const unsigned long long base = wsum[w] + (x - (v0 + v1));
-    offsets[2 * t] = base;
-    offsets[2 * t + 1] = base + v0;
-}
-
-__global__ __launch_bounds__(256) void k_compact(const uint2* __restrict__ sbuf, unsigned long long cap,
-                                                 const unsigned long long* __restrict__ offsets,
-                                                 uint2* __restrict__ dense) {
-    const uint32_t s = blockIdx.x;
-    const unsigned long long b = offsets[s], c = offsets[s + 1] - b;
-    for (unsigned long long k = threadIdx.x; k < c; k += blockDim.x) dense[b + k] = sbuf[(size_t)s * cap + k];
-}
-
 // --------------------------------------------------------------- prep ----
-// Chebyshev coordinate of each log size, domain check, min/max.
+// Chebyshev coordinate of each log size, domain check, min/max.  mm (zero
+// before): [0] complement of the smallest log size's bits, [1] largest log
+// size's bits, [2] count outside the domain.
 __global__ void k_prep_rows(const double* __restrict__ ls, uint32_t n, float* __restrict__ tvec,
-                            unsigned long long* __restrict__ mm, unsigned int* __restrict__ bad) {
-    __shared__ unsigned long long smin[256], smax[256];
+                            unsigned long long* __restrict__ mm) {
+    __shared__ unsigned long long smin[4], smax[4];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long lo = ~0ull, hi = 0ull;
+    unsigned long long lo = 0ull, hi = 0ull;
+    bool bad = false;
     if (i < n) {
         const double v = ls[i];
         // domain: [log10 1500, log10 500000] up to rounding of the caller's log10
-        if (!(v >= MODEL_XLO - 1e-12 && v <= MODEL_XHI + 1e-12)) atomicAdd(bad, 1u);
+        bad = !(v >= MODEL_XLO - 1e-12 && v <= MODEL_XHI + 1e-12);
         tvec[i] = (float)((2.0 * v - (MODEL_XLO + MODEL_XHI)) / (MODEL_XHI - MODEL_XLO));
         if (v > 0) {
-            unsigned long long u = (unsigned long long)__double_as_longlong(v);
-            lo = u;
-            hi = u;
+            hi = (unsigned long long)__double_as_longlong(v);
+            lo = ~hi;
         }
     }
-    smin[threadIdx.x] = lo;
-    smax[threadIdx.x] = hi;
+    const uint64_t nbad = __ballot(bad);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        lo = max(lo, (unsigned long long)__shfl_xor(lo, off, 64));
+        hi = max(hi, (unsigned long long)__shfl_xor(hi, off, 64));
+    }
+    const uint32_t w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        smin[w] = lo;
+        smax[w] = hi;
+        if (nbad) atomicAdd(&mm[2], (unsigned long long)__popcll(nbad));
+    }
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < (unsigned)s) {
-            smin[threadIdx.x] = min(smin[threadIdx.x], smin[threadIdx.x + s]);
-            smax[threadIdx.x] = max(smax[threadIdx.x], smax[threadIdx.x + s]);
-        }
-        __syncthreads();
-    }
     if (threadIdx.x == 0) {
-        atomicMin(&mm[0], smin[0]);
-        atomicMax(&mm[1], smax[0]);
-    }
-}
-
-// TNF transposed to K-major [136][n_pad] (zero padding) for the FP32 tiles.
-__global__ __launch_bounds__(256) void k_prep_f32t(const float* __restrict__ tnf, uint32_t n, uint32_t n_pad,
-                                                   float* __restrict__ tnft) {
-    __shared__ float tile[64][NT + 1];
-    const uint32_t r0 = blockIdx.x * 64;
-    for (int e = threadIdx.x; e < 64 * NT; e += 256) {
-        int r = e / NT, k = e - r * NT;
-        tile[r][k] = (r0 + r < n) ? tnf[(size_t)(r0 + r) * NT + k] : 0.f;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < 64 * NT; e += 256) {
-        int k = e / 64, r = e - k * 64;
-        tnft[(size_t)k * n_pad + r0 + r] = tile[r][k];
+        for (uint32_t k = 1; k < blockDim.x / 64; ++k) {
+            lo = max(lo, smin[k]);
+            hi = max(hi, smax[k]);
+        }
+        atomicMax(&mm[0], lo);
+        atomicMax(&mm[1], hi);
     }
 }
 
@@ -416,58 +321,10 @@ __device__ inline uint16_t to_bf16_rne(float f) {
 }
 __device__ inline float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-// Locality order for the MFMA prefilter.  Contigs are visited in order of a
-// composition key (the GC content implied by the TNF row: sum over columns of
-// the column's G+C fraction times its frequency), so that contigs of one
-// genome sit close together: survivors then fall into a band around the
-// diagonal, most 32x32 tiles have none (fast path only), and the tiles that
-// have survivors are dense.  Every pair is still evaluated; results are
-// mapped back through the permutation.
-struct GcWeights {
-    float w[NT];
-};
-constexpr GcWeights make_gc_weights() {
-    GcWeights g{};
-    for (int c = 0; c < NT; ++c) {
-        int gcn = 0;
-        for (int k = 0; k < 4; ++k) {
-            const char ch = mdet::kTnColumnsCx[4 * c + k];
-            gcn += (ch == 'G' || ch == 'C') ? 1 : 0;
-        }
-        g.w[c] = 0.25f * (float)gcn;
-    }
-    return g;
-}
-constexpr GcWeights kGc = make_gc_weights();
-#define W8(i) kGc.w[i], kGc.w[i + 1], kGc.w[i + 2], kGc.w[i + 3], kGc.w[i + 4], kGc.w[i + 5], kGc.w[i + 6], kGc.w[i + 7]
-__constant__ float c_gcw[NT] = {W8(0),  W8(8),  W8(16), W8(24), W8(32),  W8(40),  W8(48),  W8(56), W8(64),
-                                W8(72), W8(80), W8(88), W8(96), W8(104), W8(112), W8(120), W8(128)};
-#undef W8
-
-// One wavefront per row: key = sum_c gcw[c] * tnf[c]; idx = row.  Rows whose
-// key is NaN (no valid window) sort last.
-__global__ __launch_bounds__(256) void k_sort_key(const float* __restrict__ tnf, uint32_t n, float* __restrict__ key,
-                                                  uint32_t* __restrict__ idx) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= n) return;
-    const float* t = tnf + (size_t)r * NT;
-    float v = c_gcw[lane] * t[lane] + c_gcw[lane + 64] * t[lane + 64];
-    if (lane < 8) v += c_gcw[lane + 128] * t[lane + 128];
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) {
-        key[r] = (v == v) ? v : __builtin_inff();
-        idx[r] = r;
-    }
-}
-
-// FP32 rows and Chebyshev coordinates in sorted order (sorted position s holds
-// contig perm[s]; zero rows past n), so that refinement reads the rows of a
-// 64-row group of the prefilter as one contiguous range.  One wave per row.
-__global__ __launch_bounds__(256) void k_sort_rows(const float* __restrict__ tnf, const float* __restrict__ tvec,
-                                                   const uint32_t* __restrict__ perm, uint32_t n, uint32_t n_pad,
-                                                   float* __restrict__ tnfs, float* __restrict__ tvs) {
+// FP32 rows in cluster order for the exact cover (position s holds contig
+// perm[s]; zero rows past n).  One wave per row.
+__global__ __launch_bounds__(256) void k_sort_rows(const float* __restrict__ tnf, const uint32_t* __restrict__ perm,
+                                                   uint32_t n, uint32_t n_pad, float* __restrict__ tnfs) {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t s = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (s >= n_pad) return;
@@ -475,7 +332,6 @@ __global__ __launch_bounds__(256) void k_sort_rows(const float* __restrict__ tnf
     const size_t src = real ? (size_t)perm[s] * NT : 0;
     float* dst = tnfs + (size_t)s * NT;
     for (uint32_t c = lane; c < (uint32_t)NT; c += 64) dst[c] = real ? tnf[src + c] : 0.f;
-    if (lane == 0) tvs[s] = real ? tvec[perm[s]] : 0.f;
 }
 
 // Low-precision rows in MFMA fragment order.  For the 32-row tile t, k-step
@@ -512,197 +368,120 @@ __device__ inline uint4 pack8(const uint16_t* h) {
 }
 
 // Rows of D values (D = 136 TNF columns, or 32 embedding dimensions) padded
-// to KSX k-steps of 16; the threshold slots are k = D .. D+5.
-// ROW_MARGIN = false: R2 already holds the low-precision margin (unit TNF
-// rows), h = |x~|^2/2 - R2/4 for every row.  ROW_MARGIN = true (rows of any
-// norm, the learned embeddings): every pair with |a - b|^2 < R2 in FP32 must
-// pass, and |a~ - b~| <= |a - b| + u(|a| + |b|) (u = unit roundoff of the
-// format), so each row carries its own share s = 2 (sqrt(R2)/2 + u|x|)^2 (+ a
-// slack for the FP32 accumulation): s_i + s_j >= (sqrt(R2) + u|a| + u|b|)^2,
-// h = |x~|^2/2 - s/2, and acc > 0 iff |a~ - b~|^2 < s_i + s_j.
-template <bool BF16, int D, int KSX, bool ROW_MARGIN = false>
+// to KSX k-steps of 16; the threshold slots are k = D .. D+5.  Every pair with
+// |a - b| < R must pass, and |a~ - b~| <= |a - b| + e_a + e_b with e = |x - x~|,
+// so each row carries its own share s = 2 (R/2 + e)^2 (+ a slack for the FP32
+// accumulation, below 3e-5 for unit rows): s_a + s_b >= (R + e_a + e_b)^2,
+// h = |x~|^2/2 - s/2, and acc > 0 iff |a~ - b~|^2 < s_a + s_b.
+// TNF rows (EMB = false): e as the row's rounding gives it (~0.3 of the unit
+// roundoff u times the norm: with u|x| for every row 0.7% more survivors, and
+// twice the tiles the scan has to list for them).  Embeddings (EMB): e = u|x|.
+// One block per 32-row tile: the rows (perm: position -> row; null: itself)
+// pass through LDS once, so reads and the 16-byte fragment writes are both
+// whole lines.
+constexpr float GRAM_SLACK = 5e-5f;
+
+template <bool BF16, int D, int KSX, bool EMB = false>
 __global__ __launch_bounds__(256) void k_prep_lowp(const float* __restrict__ x, const uint32_t* __restrict__ perm,
-                                                   uint32_t n, uint32_t n_pad, float R2, uint4* __restrict__ frag,
+                                                   uint32_t n, float R, uint4* __restrict__ frag,
                                                    uint4* __restrict__ frag_a) {
-    static_assert(D + 6 <= 16 * KSX, "no room for the threshold slots");
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= n_pad) return;
-    const uint32_t t = r >> 5;
-    const size_t src = (r < n) ? (size_t)perm[r] : 0;  // sorted position r holds row perm[r]
-    const int k0 = 8 * (int)lane;
-    float vals[8];
-    float part = 0.f, norm2 = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int k = k0 + e;
-        const float v = (r < n && k < D && lane < 2 * KSX) ? x[src * D + k] : 0.f;
-        const float back = from_low<BF16>(to_low<BF16>(v));
-        vals[e] = v;
-        part = fmaf(back, back, part);
-        norm2 = fmaf(v, v, norm2);
+    static_assert(D + 6 <= 16 * KSX && D % 8 == 0, "no room for the threshold slots");
+    constexpr int STR = D + 4;
+    __shared__ __align__(16) float X[32][STR];
+    __shared__ uint32_t H[32][3];  // the pieces of each row's h
+    const uint32_t tid = threadIdx.x, t = blockIdx.x;
+    for (uint32_t e = tid; e < 32 * (D / 4); e += 256) {
+        const uint32_t r = e / (D / 4), q = e % (D / 4), pos = t * 32 + r;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (pos < n) v = reinterpret_cast<const float4*>(x + (size_t)(perm ? perm[pos] : pos) * D)[q];
+        *reinterpret_cast<float4*>(&X[r][4 * q]) = v;
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        part += __shfl_xor(part, off, 64);
-        norm2 += __shfl_xor(norm2, off, 64);
-    }
-    if (lane >= 2 * KSX) return;
-    // padding rows get a large finite h (the split of +inf would be NaN)
-    const float big = BF16 ? 1e30f : 6.0e4f;
-    float share = 0.5f * R2;  // this row's part of the squared radius
-    if (ROW_MARGIN) {
-        const float u = BF16 ? 1.0f / 256.0f : 1.0f / 2048.0f;
-        const float half_r = 0.5f * sqrtf(R2) + u * 1.0001f * sqrtf(norm2);
-        share = 2.0f * half_r * half_r + 1e-5f * (norm2 + 1.0f);
-    }
-    const float hv = (r < n) ? fmaf(0.5f, part, -0.5f * share) : big;
-    uint16_t hp[3];
-    float rem = hv;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        hp[q] = to_low<BF16>(rem);
-        rem = rem - from_low<BF16>(hp[q]);
-    }
-    const uint16_t one = to_low<BF16>(1.f);
-    uint16_t hb[8], ha[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int k = k0 + e;
-        uint16_t v = (k < D) ? to_low<BF16>(vals[e]) : (uint16_t)0;
-        uint16_t va = v;
-        if (k >= D && k < D + 3) {  // column role: 1, row role: -h pieces
-            v = one;
-            va = hp[k - D] ^ 0x8000u;
-        } else if (k >= D + 3 && k < D + 6) {  // column role: -h pieces, row role: 1
-            v = hp[k - D - 3] ^ 0x8000u;
-            va = one;
-        }
-        hb[e] = v;
-        ha[e] = va;
-    }
-    const uint32_t ks = lane >> 1, half = lane & 1;
-    frag[((size_t)t * KSX + ks) * 64 + (r & 31) + 32 * half] = pack8(hb);
-    if (ks == KSX - 1) frag_a[(size_t)t * 64 + (r & 31) + 32 * half] = pack8(ha);
-}
-
-// ------------------------------------------------------ FP32 prefilter ----
-// Upper-triangle 128x128 tiles; thread (ty, tx) owns rows ty+16a, columns
-// tx+16b (a, b < 8).  K streamed through LDS in chunks of 8 from the K-major
-// copy, so every global load is a contiguous 512-byte row segment.
-constexpr int F_T = 128, F_KC = 8;
-
-__device__ __forceinline__ void prefilter_f32_tile(const float* __restrict__ tnft, uint32_t n, uint32_t n_pad,
-                                                   uint32_t ntiles, uint64_t lin, float R2, const SurvOut& out,
-                                                   float (*As)[F_T], float (*Bs)[F_T]) {
-    // linear index -> (bi, bj), bi <= bj, rows of the triangle of length ntiles - bi
-    const double T = ntiles;
-    double disc = (2.0 * T + 1.0) * (2.0 * T + 1.0) - 8.0 * (double)lin;
-    int64_t bi = (int64_t)floor(((2.0 * T + 1.0) - sqrt(disc)) * 0.5);
-    auto start = [&](int64_t b) { return (uint64_t)(b * (int64_t)ntiles - b * (b - 1) / 2); };
-    while (bi > 0 && start(bi) > lin) --bi;
-    while (start(bi + 1) <= lin) ++bi;
-    const uint32_t bj = (uint32_t)(bi + (int64_t)(lin - start(bi)));
-    const uint32_t rb = (uint32_t)bi * F_T, cb = bj * F_T;
-
-    const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-    const int lk = tid >> 5, lc = (tid & 31) * 4;
-    float acc[8][8];
-#pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = 0; b < 8; ++b) acc[a][b] = 0.f;
-
-    float4 pa = *reinterpret_cast<const float4*>(tnft + (size_t)lk * n_pad + rb + lc);
-    float4 pb = *reinterpret_cast<const float4*>(tnft + (size_t)lk * n_pad + cb + lc);
-    for (int k0 = 0; k0 < NT; k0 += F_KC) {
-        *reinterpret_cast<float4*>(&As[lk][lc]) = pa;
-        *reinterpret_cast<float4*>(&Bs[lk][lc]) = pb;
-        __syncthreads();
-        if (k0 + F_KC < NT) {
-            pa = *reinterpret_cast<const float4*>(tnft + (size_t)(k0 + F_KC + lk) * n_pad + rb + lc);
-            pb = *reinterpret_cast<const float4*>(tnft + (size_t)(k0 + F_KC + lk) * n_pad + cb + lc);
+    __syncthreads();
+    {  // eight lanes a row: squared norms of the rounded and the given values
+        const uint32_t r = tid >> 3, s = tid & 7, pos = t * 32 + r;
+        float part = 0.f, norm2 = 0.f, err2 = 0.f;
+        for (uint32_t k = s; k < (uint32_t)D; k += 8) {
+            const float v = X[r][k], back = from_low<BF16>(to_low<BF16>(v));
+            part = fmaf(back, back, part);
+            norm2 = fmaf(v, v, norm2);
+            err2 = fmaf(v - back, v - back, err2);
         }
 #pragma unroll
-        for (int kk = 0; kk < F_KC; ++kk) {
-            float av[8], bv[8];
-#pragma unroll
-            for (int a = 0; a < 8; ++a) av[a] = As[kk][ty + 16 * a];
-#pragma unroll
-            for (int b = 0; b < 8; ++b) bv[b] = Bs[kk][tx + 16 * b];
-#pragma unroll
-            for (int a = 0; a < 8; ++a)
-#pragma unroll
-                for (int b = 0; b < 8; ++b) {
-                    const float df = av[a] - bv[b];
-                    acc[a][b] = fmaf(df, df, acc[a][b]);
-                }
+        for (int off = 4; off >= 1; off >>= 1) {
+            part += __shfl_xor(part, off, 64);
+            norm2 += __shfl_xor(norm2, off, 64);
+            err2 += __shfl_xor(err2, off, 64);
         }
-        __syncthreads();
-    }
-    uint32_t cnt = 0;
+        if (s == 0) {
+            // padding rows get a large finite h (the split of +inf would be NaN)
+            const float big = BF16 ? 1e30f : 6.0e4f;
+            const float u = BF16 ? 1.0f / 256.0f : 1.0f / 2048.0f;
+            const float half_r = 0.5f * R + (EMB ? u * 1.0001f * sqrtf(norm2) : 1.001f * sqrtf(err2) + 1e-6f);
+            const float share = 2.0f * half_r * half_r + (EMB ? 1e-5f : GRAM_SLACK) * (norm2 + 1.0f);
+            float rem = (pos < n) ? fmaf(0.5f, part, -0.5f * share) : big;
 #pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const uint32_t i = rb + ty + 16 * a, j = cb + tx + 16 * b;
-            cnt += (acc[a][b] < R2 && i < j && j < n) ? 1u : 0u;
-        }
-    if (__any(cnt != 0)) {
-        const uint32_t shard = wave_shard();
-        unsigned long long pos = wave_reserve_shard(cnt, out, shard);
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const uint32_t i = rb + ty + 16 * a, j = cb + tx + 16 * b;
-                if (acc[a][b] < R2 && i < j && j < n) shard_put(out, shard, pos++, i, j);
+            for (int q = 0; q < 3; ++q) {
+                const uint16_t p = to_low<BF16>(rem);
+                H[r][q] = p;
+                rem = rem - from_low<BF16>(p);
             }
+        }
+    }
+    __syncthreads();
+    const uint16_t one = to_low<BF16>(1.f);
+    for (uint32_t e = tid; e < (uint32_t)KSX * 64; e += 256) {
+        const uint32_t ks = e >> 6, l = e & 63, r = l & 31, k0 = 16 * ks + 8 * (l >> 5);
+        uint16_t hb[8], ha[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) {
+            uint16_t v = 0, va = 0;
+            if (k0 < (uint32_t)D) {  // whole octets of values (D is a multiple of 8)
+                v = va = to_low<BF16>(X[r][k0 + i]);
+            } else if (k0 == (uint32_t)D) {
+                if (i < 3) {  // column role: 1, row role: -h pieces
+                    v = one;
+                    va = (uint16_t)H[r][i] ^ 0x8000u;
+                } else if (i < 6) {  // column role: -h pieces, row role: 1
+                    v = (uint16_t)H[r][i - 3] ^ 0x8000u;
+                    va = one;
+                }
+            }
+            hb[i] = v;
+            ha[i] = va;
+        }
+        frag[((size_t)t * KSX + ks) * 64 + l] = pack8(hb);
+        if (ks == KSX - 1) frag_a[(size_t)t * 64 + l] = pack8(ha);
     }
 }
 
-// Blocks stride over the ntri triangle tiles: a launch covers at most
-// 2^32 - 1 work-items per grid dimension (the dispatch packet's grid size is
-// 32 bits), and at 1M contigs the triangle has 3.05e7 tiles of 256 threads.
-__global__ __launch_bounds__(256) void k_prefilter_f32(const float* __restrict__ tnft, uint32_t n, uint32_t n_pad,
-                                                       uint32_t ntiles, uint64_t ntri, float R2, SurvOut out) {
-    __shared__ float As[F_KC][F_T], Bs[F_KC][F_T];
-    for (uint64_t lin = blockIdx.x; lin < ntri; lin += gridDim.x) {
-        __syncthreads();  // the previous tile's LDS reads are done
-        prefilter_f32_tile(tnft, n, n_pad, ntiles, lin, R2, out, As, Bs);
-    }
-}
-
-// ------------------------------------------------------- MFMA prefilter ---
-// Block = 4 waves = 256 rows (64 per wave: two 32-row MFMA tiles held in
-// registers for the whole column sweep); columns stream through LDS in
-// steps of 128 (four 32-column tiles, 36 KiB in fragment order), double
-// buffered and filled by global_load_lds_dwordx4 (no register staging).  Per
-// step a wave issues 2 x 4 x 9 v_mfma_f32_32x32x16, as two 64-column halves
-// of 4 independent accumulator chains each; with the threshold folded into K, the test of a pair is
-// "acc > 0".  Only 32x32 tiles with a survivor enter the extraction: each
-// lane's 16 compares form a bit mask without branches (the diagonal and
-// range conditions are a second mask, applied only in the steps that meet
-// them), a DPP prefix sum of the masks' counts gives each lane its stage
-// offset, and the lanes write their pairs.  Measured at 200k contigs: the
-// prefilter without extraction 3.87 ms, with it 6.30 ms using per-element
-// short-circuit conditions (compiled into a branch per accumulator) and a
-// shuffle (ds_bpermute) scan; 5.78 ms with the DPP scan; 5.25 ms with the
-// branch-free masks.  Writing the stage one accumulator index at a time
-// (a ballot and mbcnt per index, no per-lane loop) ran slower (6.6 ms): 16
-// ballots per tile and twice the code.
-// Column span per item (mdet_tune.seg_cols, default 1024, chosen per input by
-// the autotuner): at 200k contigs 1024 columns ran the step 3% faster than
-// 2048 (finer scheduling of the survivor-heavy diagonal items) with shorter
-// survivor runs for refinement; 512 and 768 were no faster overall.
-constexpr int M_GRAM_WAVES = 4;  // waves (64 rows each) per prefilter block of the Gram modes
-constexpr int M_ROWS = 64 * M_GRAM_WAVES, M_STEP = 128;
-// the registers are sized for 2 waves per SIMD: 8 resident waves per CU
-// Prefilter item: (r_lo, r_hi, c_lo, c_hi | ITEM_TRI) = pairs of row positions
+// ------------------------------------------------------------- tile scan --
+// The first pass over the pairs: which 32 x 32 tiles hold a pair within the
+// radius at all.  Block = 4 waves of RT row tiles each (held in registers for
+// the whole column sweep of an item); columns stream through LDS CT tiles a
+// step in fragment order, double buffered and filled by
+// global_load_lds_dwordx4 (no register staging).  With the threshold folded
+// into K the test of a pair is "acc > 0"; a tile with one goes to the list,
+// which the second pass works off.  Nothing else leaves the kernel, so its cost
+// is the MFMAs and the maximum tree.
+//   KSX = 2, RT = 4, CT = 8: the exhaustive modes, on the projected rows
+//     (order.h): a lower bound of the distance in 28 dimensions drops ~99% of
+//     the tiles.  Bound by the MFMAs (2 per tile, 64 cycles) and the maximum
+//     tree beside them.
+//   KSX = 9, RT = 2, CT = 4: cluster pairs and full rows of the learned
+//     filter, on the TNF rows themselves.
+//   KSX = 3, RT = 2, CT = 4: the embedding radius of the learned filter.
+// Measured and dropped in the full Gram form of this kernel (KSX = 9 over all
+// pairs): B reads ahead by hand, ping-pong accumulators (one wave per SIMD),
+// 8-wave blocks, s_setprio around the chains, two distinct LDS arrays.
+constexpr uint32_t SCAN_WAVES = 4;
+constexpr uint32_t scan_rows(int rt) { return 32u * rt * SCAN_WAVES; }  // rows per item of row blocks
+constexpr int PROJ_RT = 4, PROJ_CT = 8;
+constexpr int GRAM_RT = 2, GRAM_CT = 4;
+static_assert(scan_rows(GRAM_RT) == mdet::ITEM_ROWS, "cluster items hold one block's rows");
+// Scan item: (r_lo, r_hi, c_lo, c_hi | ITEM_TRI) = pairs of row positions
 // [r_lo, r_hi) and column positions [c_lo, c_hi), only i < j if ITEM_TRI;
-// r_hi - (r_lo & ~31) <= M_ROWS.  The fragment arrays must hold whole 128-
-// column steps from (c_lo & ~31) up to c_hi.
-static_assert(M_STEP % 64 == 0, "steps are whole 64-column halves");
+// r_hi - (r_lo & ~31) <= the block's rows.  The fragment arrays must hold
+// whole column steps from (c_lo & ~31) up to c_hi.
 
 template <bool BF16>
 __device__ inline f32x16_t mfma32(uint4 a, uint4 b, f32x16_t c) {
@@ -713,11 +492,12 @@ __device__ inline f32x16_t mfma32(uint4 a, uint4 b, f32x16_t c) {
                                                   0, 0);
 }
 
-// One step's column fragments (M_STEP / 32 tiles x KSX k-steps x 64 lanes of
-// 16 bytes) into LDS: each wave copies 1 KiB chunks, chunk m*4 + wave.
-template <int KSX, int THREADS>
+// One step's column fragments (CT tiles x KSX k-steps x 64 lanes of 16 bytes)
+// into LDS: each wave copies 1 KiB chunks, chunk m * 4 + wave.
+template <int KSX, int CT>
 __device__ inline void issue_btile(const uint4* __restrict__ frag, uint32_t c0, uint4* lds, int tid, int wave) {
-    constexpr int STEP_U4 = M_STEP / 32 * KSX * 64;
+    constexpr int STEP_U4 = CT * KSX * 64, THREADS = 64 * SCAN_WAVES;
+    static_assert(STEP_U4 % 64 == 0, "whole 1 KiB chunks");
     const uint4* src = frag + (size_t)(c0 / 32) * KSX * 64;
 #pragma unroll
     for (int m = 0; m < (STEP_U4 + THREADS - 1) / THREADS; ++m)
@@ -727,236 +507,145 @@ __device__ inline void issue_btile(const uint4* __restrict__ frag, uint32_t c0, 
                                              16, 0, 0);
 }
 
-// Per-wave survivor staging in LDS: survivors of a step are appended to a
-// 128-entry wave-private buffer and written out (one shard atomic + one
-// coalesced copy) only when it fills or the item ends, so most steps issue
-// neither an atomic nor a global store.
-constexpr int M_STAGE = 128;
+// Orders the LDS writes of a wave before its following LDS reads (the lanes
+// of one wave execute each LDS instruction together and in program order; the
+// fences keep the compiler from moving accesses across).
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
-// Chunked survivor output: a flush puts the staged survivors (all of one
-// item) into the next chunk slot of M_STAGE entries of the wave's shard and
-// (item, count) into the slot's meta entry, so sorting the chunks by item
-// lists the survivors item by item (k_chunk_list / k_chunk_compact).  A
-// shard's counter counts chunks and keeps counting past its capacity so the
-// host learns the size needed.
-struct ChunkOut {
-    uint2* buf;               // NSHARD * cap chunks of M_STAGE entries
-    uint2* meta;              // NSHARD * cap (item, count)
-    unsigned long long* cnt;  // NSHARD * SHARD_STRIDE
-    unsigned long long cap;   // chunk slots per shard
+// Tile list: entries (row tile, column tile, item, 0); the counter keeps
+// counting past the capacity so that the host learns the size needed.  A wave
+// stages its tiles in LDS over all its items and appends 64 at a time: a
+// returning atomic on one address costs ~15 ns of the whole chip's time, so a
+// flush per item (240k items at 1M contigs) bound the scan: 24.6 ms.
+struct TileList {
+    uint4* buf;
+    unsigned long long* cnt;
+    unsigned long long cap;
 };
+constexpr uint32_t TILE_STAGE = 64;
 
-__device__ inline void stage_flush(const ChunkOut& o, uint32_t shard, uint32_t item, uint2* stage, uint32_t& n,
-                                   int lane) {
+__device__ inline unsigned long long lane0_u64(unsigned long long v) {
+    return ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), 0) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 0);
+}
+
+__device__ inline void tiles_flush(const TileList& o, const uint4* stage, uint32_t& n, int lane) {
     if (n == 0) return;
     unsigned long long k = 0;
-    if (lane == 0) k = atomicAdd(&o.cnt[(size_t)shard * SHARD_STRIDE], 1ull);
-    k = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(k >> 32), 0) << 32) |
-        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, 0);
-    if (k < o.cap) {
-        const size_t slot = (size_t)shard * o.cap + k;
-        for (uint32_t e = lane; e < n; e += 64) o.buf[slot * M_STAGE + e] = stage[e];
-        if (lane == 0) o.meta[slot] = make_uint2(item, n);
-    }
+    if (lane == 0) k = atomicAdd(o.cnt, (unsigned long long)n);
+    k = lane0_u64(k);
+    wave_sync();
+    if ((uint32_t)lane < n && k + lane < o.cap) o.buf[k + lane] = stage[lane];
+    wave_sync();
     n = 0;
 }
 
-// Chunks of shard s (offsets from k_shard_scan over the chunk counters) ->
-// (item, chunk slot) pairs for the sort; survivor total into *total.
-// Sort key of a chunk: its item index, or with items != nullptr the
-// 1024 x 1024 tile of the item's first row and column, (r_lo / 1024) << 16 |
-// c_lo / 1024, so that the refinement walks the survivors tile by tile and
-// the rows in flight on an XCD stay few (row-block items span up to 4096
-// columns; cluster items are compact already).
-__global__ __launch_bounds__(256) void k_chunk_list(const uint2* __restrict__ meta, unsigned long long cap,
-                                                    const unsigned long long* __restrict__ offsets,
-                                                    const uint4* __restrict__ items, uint32_t* __restrict__ key,
-                                                    uint32_t* __restrict__ slot,
-                                                    unsigned long long* __restrict__ total) {
-    __shared__ unsigned int bsum;
-    if (threadIdx.x == 0) bsum = 0;
-    __syncthreads();
-    const uint32_t s = blockIdx.x;
-    const unsigned long long b = offsets[s], c = offsets[s + 1] - b;
-    unsigned int sum = 0;
-    for (unsigned long long k = threadIdx.x; k < c; k += blockDim.x) {
-        const uint2 m = meta[(size_t)s * cap + k];
-        if (items) {
-            const uint4 it = items[m.x];
-            key[b + k] = ((it.x >> 10) << 16) | (it.z >> 10);
-        } else {
-            key[b + k] = m.x;
-        }
-        slot[b + k] = (uint32_t)((size_t)s * cap + k);
-        sum += m.y;
-    }
-    if (sum) atomicAdd(&bsum, sum);
-    __syncthreads();
-    if (threadIdx.x == 0 && bsum) atomicAdd(total, (unsigned long long)bsum);
-}
-
-__global__ __launch_bounds__(256) void k_chunk_counts(const uint2* __restrict__ meta, const uint32_t* __restrict__ slot,
-                                                      uint32_t nchunks, uint32_t* __restrict__ count) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nchunks) count[i] = meta[slot[i]].y;
-}
-
-// One wave per chunk (in item order): its entries to their dense offset.
-__global__ __launch_bounds__(256) void k_chunk_compact(const uint2* __restrict__ buf, const uint32_t* __restrict__ slot,
-                                                       const uint32_t* __restrict__ count,
-                                                       const uint64_t* __restrict__ off, uint32_t nchunks,
-                                                       uint2* __restrict__ dense) {
-    const uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= nchunks) return;
-    const uint2* src = buf + (size_t)slot[i] * M_STAGE;
-    const uint32_t c = count[i];
-    const uint64_t d = off[i];
-    for (uint32_t e = lane; e < c; e += 64) dense[d + e] = src[e];
-}
-
-template <bool BF16, int KSX, int WAVES>
-__device__ __forceinline__ void prefilter_item(const uint4* __restrict__ frag, const uint4* __restrict__ frag_a8,
-                                               const uint4 it, const uint32_t item,
-                                               uint4 (*Bl)[M_STEP / 32 * KSX * 64], uint2 (*stage_all)[M_STAGE],
-                                               const ChunkOut& out) {
+template <bool BF16, int KSX, int RT, int CT>
+__device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const uint4* __restrict__ frag_a,
+                                          const uint4 it, const uint32_t item, uint4 (*Bl)[CT * KSX * 64],
+                                          uint4* stage, uint32_t& nstage, const TileList& out) {
+    constexpr int CG = 4 / RT;  // column tiles a pass: 4 independent accumulator chains
+    constexpr uint32_t STEP = 32 * CT;
+    static_assert(CG >= 1 && CT % CG == 0, "whole passes");
     const uint32_t r_lo = it.x, r_hi = it.y, c_lo = it.z, c_hi = it.w & ~ITEM_TRI;
     const bool tri = (it.w & ITEM_TRI) != 0;
     const uint32_t c_begin = c_lo & ~31u;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const uint32_t row0 = (r_lo & ~31u) + wave * 64;  // this wave's 64 rows
+    const uint32_t row0 = (r_lo & ~31u) + wave * (32 * RT);  // this wave's rows
     // a wave with no row of the item still takes its share of the column loads
-    const bool active = row0 < r_hi && row0 + 64 > r_lo;
-    const bool rows_edge = row0 < r_lo || row0 + 64 > r_hi;
+    const bool active = row0 < r_hi;
     const uint32_t t0 = row0 >> 5;
-    uint2* stage = stage_all[wave];
-    uint32_t nstage = 0;
-
-    issue_btile<KSX, 64 * WAVES>(frag, c_begin, Bl[0], tid, wave);
-    uint4 a[2][KSX];
+    issue_btile<KSX, CT>(frag, c_begin, Bl[0], tid, wave);
+    uint4 a[RT][KSX];
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
+    for (int rt = 0; rt < RT; ++rt) {
+        // row tiles past the item's rows are not in the arrays: the last one stands in (never listed)
+        const uint32_t t = min(t0 + rt, (r_hi - 1) >> 5);
 #pragma unroll
         for (int ks = 0; ks < KSX - 1; ++ks)
-            a[rt][ks] = active ? frag[((size_t)(t0 + rt) * KSX + ks) * 64 + lane] : make_uint4(0, 0, 0, 0);
-        a[rt][KSX - 1] = active ? frag_a8[(size_t)(t0 + rt) * 64 + lane] : make_uint4(0, 0, 0, 0);
+            a[rt][ks] = active ? frag[((size_t)t * KSX + ks) * 64 + lane] : make_uint4(0, 0, 0, 0);
+        a[rt][KSX - 1] = active ? frag_a[(size_t)t * 64 + lane] : make_uint4(0, 0, 0, 0);
     }
-    // accumulator r of row tile rt holds row row0 + 32*rt + rbase + r%4 + 8*(r/4)
-    const uint32_t rbase = 4 * (lane >> 5);
-    const uint32_t shard = wave_shard();
 
     int buf = 0;
-    for (uint32_t c0 = c_begin; c0 < c_hi; c0 += M_STEP, buf ^= 1) {
+    for (uint32_t c0 = c_begin; c0 < c_hi; c0 += STEP, buf ^= 1) {
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        // The next step's fill is issued after the first half-step's B reads
+        // The next step's fill is issued after the first pass's B reads
         // (below): the compiler cannot tell Bl[buf ^ 1] from Bl[buf] and waits
-        // for the fill before the second half's first read, so the first
-        // half's MFMA drain and survivor test cover part of it, and the CU's
-        // second block the rest (issued at the step's top: 0.8% slower at
-        // 200k contigs, 0.4% at 1M; two distinct arrays with the loop unrolled
-        // by two drop the wait but double the code and ran 7% slower).  The
-        // barrier above keeps the fill after every wave's reads of that buffer
-        // in the previous step; the wait and barrier at the next step's top
-        // keep the next reads after every wave's fill.
-        const bool more = c0 + M_STEP < c_hi;
-        if (!active) {
-            if (more) issue_btile<KSX, 64 * WAVES>(frag, c0 + M_STEP, Bl[buf ^ 1], tid, wave);
+        // for the fill before the next pass's first read, so the first pass's
+        // MFMA drain and maximum tree cover part of it, and the CU's other
+        // blocks the rest.  The barrier above keeps the fill after every
+        // wave's reads of that buffer in the previous step; the wait and
+        // barrier at the next step's top keep the next reads after every
+        // wave's fill.
+        const bool more = c0 + STEP < c_hi;
+        // steps wholly left of the wave's rows hold no pair i < j
+        if (!active || (tri && c0 + STEP <= row0)) {
+            if (more) issue_btile<KSX, CT>(frag, c0 + STEP, Bl[buf ^ 1], tid, wave);
             continue;
         }
         const uint4* B = Bl[buf];
-        // pairs with j <= i exist only where the step meets the diagonal
-        const bool diag = tri && c0 < row0 + 64;
-        // pairs outside the item's row or column range only where the wave
-        // or the step crosses the range's edge
-        const bool edge = rows_edge || c0 < c_lo || c0 + M_STEP > c_hi;
+#pragma unroll KSX == 9 ? CT / CG : 1
+        for (int p = 0; p < CT / CG; ++p) {
+            f32x16_t acc[RT][CG];
 #pragma unroll
-        for (int hc = 0; hc < M_STEP / 64; ++hc) {  // 64-column halves of the step
-            f32x16_t acc[2][2];
+            for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-                for (int ct = 0; ct < 2; ++ct) acc[rt][ct] = f32x16_t{};
+                for (int c = 0; c < CG; ++c) acc[rt][c] = f32x16_t{};
             // let the scheduler interleave the B-fragment LDS reads with the
-            // MFMA chains (measured 2% faster at 200k contigs)
-            __builtin_amdgcn_iglp_opt(0);
+            // MFMA chains (measured 2% faster with KSX = 9)
+            if (KSX == 9) __builtin_amdgcn_iglp_opt(0);
 #pragma unroll
             for (int ks = 0; ks < KSX; ++ks) {
-                uint4 b[2];
+                uint4 b[CG];
 #pragma unroll
-                for (int ct = 0; ct < 2; ++ct) b[ct] = B[((2 * hc + ct) * KSX + ks) * 64 + lane];
+                for (int c = 0; c < CG; ++c) b[c] = B[((CG * p + c) * KSX + ks) * 64 + lane];
 #pragma unroll
-                for (int rt = 0; rt < 2; ++rt)
+                for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int ct = 0; ct < 2; ++ct) acc[rt][ct] = mfma32<BF16>(a[rt][ks], b[ct], acc[rt][ct]);
+                    for (int c = 0; c < CG; ++c) acc[rt][c] = mfma32<BF16>(a[rt][ks], b[c], acc[rt][c]);
             }
-            if (hc == 0 && more) issue_btile<KSX, 64 * WAVES>(frag, c0 + M_STEP, Bl[buf ^ 1], tid, wave);
-            // fast path: per-lane maxima of each 32x32 tile.  acc > 0.0f
-            // exactly when its bits, read as a signed int, are > 0, so the
-            // maxima are integer max3 trees (no NaN canonicalisation).
-            int tmax[2][2];
+            if (p == 0 && more) issue_btile<KSX, CT>(frag, c0 + STEP, Bl[buf ^ 1], tid, wave);
+            // per-lane maxima of each 32 x 32 tile.  acc > 0.0f exactly when
+            // its bits, read as a signed int, are > 0, so the maxima are
+            // integer max3 trees (a NaN may list its tile, never a pair).
+            int tmax[RT][CG];
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
+            for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int ct = 0; ct < 2; ++ct) {
-                    const f32x16_t v = acc[rt][ct];
+                for (int c = 0; c < CG; ++c) {
+                    const f32x16_t v = acc[rt][c];
                     int b[16];
 #pragma unroll
                     for (int r = 0; r < 16; ++r) b[r] = __float_as_int(v[r]);
                     const int m0 = max(max(b[0], b[1]), b[2]), m1 = max(max(b[3], b[4]), b[5]);
                     const int m2 = max(max(b[6], b[7]), b[8]), m3 = max(max(b[9], b[10]), b[11]);
                     const int m4 = max(max(b[12], b[13]), b[14]);
-                    tmax[rt][ct] = max(max(max(m0, m1), m2), max(max(m3, m4), b[15]));
+                    tmax[rt][c] = max(max(max(m0, m1), m2), max(max(m3, m4), b[15]));
                 }
-            const int hmax = max(max(tmax[0][0], tmax[0][1]), max(tmax[1][0], tmax[1][1]));
+            int hmax = 0;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int c = 0; c < CG; ++c) hmax = max(hmax, tmax[rt][c]);
             if (!__any(hmax > 0)) continue;
-            const uint32_t jl = c0 + 64 * hc + (lane & 31);
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
+            for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int ct = 0; ct < 2; ++ct) {
-                    if (!__any(tmax[rt][ct] > 0)) continue;
-                    const uint32_t j = jl + 32 * ct;
-                    const uint32_t ib = row0 + 32 * rt + rbase;  // row of accumulator r: ib + (r & 3) + 8 (r >> 2)
-                    // bit r: accumulator r of this lane is a survivor
-                    uint32_t bits = 0;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) bits |= (acc[rt][ct][r] > 0.f ? 1u : 0u) << r;
-                    if (diag || edge) {
-                        // the pairs outside the item (diagonal tiles, range edges)
-                        uint32_t keep = 0;
-                        const bool j_in = !edge || (j >= c_lo && j < c_hi);
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const uint32_t i = ib + (r & 3) + 8 * (r >> 2);
-                            const bool ok = (!diag | (i < j)) & (!edge | (j_in & (i >= r_lo) & (i < r_hi)));
-                            keep |= (ok ? 1u : 0u) << r;
-                        }
-                        bits &= keep;
-                    }
-                    // each lane writes its own survivors at its offset in the wave
-                    const uint32_t cnt = (uint32_t)__popc(bits);
-                    const uint32_t incl = wave_incl_sum_dpp(cnt);
-                    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-                    // the tile's survivors take offsets [0, total) in lane order; each
-                    // round stages the ones that fit and flushes a full stage
-                    uint32_t o = incl - cnt, done = 0;
-                    while (done < total) {
-                        const uint32_t room = M_STAGE - nstage;
-                        while (bits && o < done + room) {
-                            const int r = __builtin_ctz(bits);
-                            bits &= bits - 1;
-                            stage[nstage + (o - done)] = make_uint2(ib + (r & 3) + 8 * (r >> 2), j);
-                            ++o;
-                        }
-                        const uint32_t took = total - done < room ? total - done : room;
-                        nstage += took;
-                        done += took;
-                        if (nstage == M_STAGE) stage_flush(out, shard, item, stage, nstage, lane);
-                    }
+                for (int c = 0; c < CG; ++c) {
+                    if (!__any(tmax[rt][c] > 0)) continue;
+                    const uint32_t tr = t0 + rt, tc = c0 / 32 + CG * p + c;
+                    if ((tri && tc < tr) || 32 * tr >= r_hi || 32 * tc >= c_hi) continue;
+                    if (lane == 0) stage[nstage] = make_uint4(tr, tc, item, 0u);
+                    if (++nstage == TILE_STAGE) tiles_flush(out, stage, nstage, lane);
                 }
         }
     }
-    stage_flush(out, shard, item, stage, nstage, lane);
 }
 
 // One block per item (item_ctr == nullptr: item = blockIdx.x), or persistent
@@ -967,15 +656,15 @@ __device__ __forceinline__ void prefilter_item(const uint4* __restrict__ frag, c
 constexpr int PF_QUEUES = 8;
 constexpr int PF_CTR_STRIDE = 16;  // counters 64 bytes apart
 
-template <bool BF16, int KSX, int WAVES = 4>
-__global__ __launch_bounds__(64 * WAVES, 2) void k_prefilter_mfma(const uint4* __restrict__ frag,
-                                                           const uint4* __restrict__ frag_a8,
-                                                           const uint4* __restrict__ items, uint32_t nitems,
-                                                           uint32_t* __restrict__ item_ctr,
-                                                           const uint32_t* __restrict__ qbounds, ChunkOut out) {
-    constexpr int STEP_U4 = M_STEP / 32 * KSX * 64;  // uint4 per B step
-    __shared__ uint4 Bl[2][STEP_U4];
-    __shared__ uint2 stage_all[WAVES][M_STAGE];
+template <bool BF16, int KSX, int RT, int CT, int WPE>
+__global__ __launch_bounds__(64 * SCAN_WAVES, WPE) void k_tile_scan(const uint4* __restrict__ frag,
+                                                                    const uint4* __restrict__ frag_a,
+                                                                    const uint4* __restrict__ items, uint32_t nitems,
+                                                                    uint32_t* __restrict__ item_ctr,
+                                                                    const uint32_t* __restrict__ qbounds,
+                                                                    TileList out) {
+    __shared__ uint4 Bl[2][CT * KSX * 64];
+    __shared__ uint4 stage_all[SCAN_WAVES][TILE_STAGE];
     __shared__ uint32_t s_item;
     uint32_t item = blockIdx.x, q_end = nitems, q_base = 0;
     uint32_t* ctr = item_ctr;
@@ -990,36 +679,520 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_prefilter_mfma(const uint4* _
         __syncthreads();
         item = s_item;
     }
+    uint4* stage = stage_all[threadIdx.x >> 6];
+    uint32_t nstage = 0;
     while (item < q_end) {
-        prefilter_item<BF16, KSX, WAVES>(frag, frag_a8, items[item], item, Bl, stage_all, out);
+        scan_item<BF16, KSX, RT, CT>(frag, frag_a, items[item], item, Bl, stage, nstage, out);
         if (!item_ctr) break;
         __syncthreads();  // every wave is done with Bl and s_item
         if (threadIdx.x == 0) s_item = q_base + atomicAdd(ctr, 1u);
         __syncthreads();
         item = s_item;
     }
+    tiles_flush(out, stage, nstage, threadIdx.x & 63);
 }
 
-// ---------------------------------------------------------------- refine --
-// Four lanes per survivor: each lane streams 1/4 of the two FP32 rows
-// (float4 q = lane%4 + 4m), two shuffles complete d^2, the quad's first lane
-// evaluates the model.  16 survivors per wave in flight, 64-byte contiguous
-// segments per row per load instruction.
-//
-// Survivors are (row, column) indices into `rows`/`tv`: contig ids for the
-// FP32 prefilter (perm == nullptr), sorted positions for the MFMA ones (rows
-// and tv in sorted order, perm maps back to contig ids).  The survivor list
-// holds runs of one wave's 64-row group against one column segment, so each
-// XCD takes one contiguous eighth of it (block b runs on XCD b % 8) and its
-// blocks walk that eighth together: the rows in flight on an XCD stay few
-// enough for its L2.  gridDim.x is a multiple of 8.
-// Edge rule of the refinement: RULE_PRE (gen_tnf_graph, cuda/Cuda2.cu:884:
-// preProb > T) or RULE_PROB (the MetaBAT1 variant's TNF-only graph,
-// cuda/Cuda.cu:1750-1753: 1 - prob >= required_min_p with prob as
-// cal_tnf_dist_d forms it, cuda/Cuda.cu:152-162).  Both are pre ~ T with
-// T = log(1/(1 - p) - 1) away from the tie band; inside it the FP64 value
-// decides with the rule's own arithmetic.
+// ------------------------------------------------------------ tile pairs --
+// The second pass: the pairs of the listed tiles, decided in FP32.
+//   k_tile_gram    the low-precision Gram (9 k-steps, or 3 on embeddings) of
+//                  each listed tile: its survivor mask, and a second list of
+//                  the tiles that have any.  One wave a tile, fragments
+//                  straight from L2; bound by that traffic (18 KiB a tile).
+//                  FULL: the learned filter's full rows (below): row positions
+//                  past the appended rows' base map through full_pos, and only
+//                  pairs that phase one did not decide are taken.
+//   k_tile_f32     the same mask from FP32 differences of every pair of a
+//                  listed tile (EXACT_F32).
+//   k_tile_refine  the survivors' FP32 distances and model.
+// Edge rule: RULE_PRE (gen_tnf_graph, cuda/Cuda2.cu:884: preProb > T) or
+// RULE_PROB (the MetaBAT1 variant's TNF-only graph, cuda/Cuda.cu:1750-1753:
+// 1 - prob >= required_min_p with prob as cal_tnf_dist_d forms it,
+// cuda/Cuda.cu:152-162).  Both are pre ~ T with T = log(1/(1 - p) - 1) away
+// from the tie band; inside it the FP64 value decides with the rule's own
+// arithmetic: those candidates are listed (amb, count *amb_cnt) with their
+// FP32 value and decided by k_adjudicate (inlined, the FP64 evaluator costs a
+// third of the waves).
 constexpr int RULE_PRE = 0, RULE_PROB = 1;
+constexpr uint32_t TILE_CHUNK = 16;  // consecutive list entries that stay on one XCD
+
+// Entry of step k of worker w (of W, a multiple of 8; worker w runs on XCD
+// w % 8): the workers of an XCD take its chunks of TILE_CHUNK entries in
+// order, so neighbouring tiles of one scan wave, which share rows, meet in one
+// L2.  Increasing in k.
+__device__ inline uint64_t chunk_entry(uint32_t w, uint32_t W, uint64_t k) {
+    const uint64_t l = (w >> 3) + k * (W >> 3);
+    return ((l / TILE_CHUNK) * 8 + (w & 7)) * TILE_CHUNK + l % TILE_CHUNK;
+}
+
+// Tiles with survivors: (row tile, column tile, first candidate record's low 32
+// bits, survivors | its high bits << 11) and the 64 lanes' masks.  The tiles'
+// slots and their candidate records are reserved TILE_BATCH tiles at a time
+// (one returning atomic each costs ~15-25 ns of the whole chip's time: reserved
+// tile by tile they bound the second pass, 1.9 ms at 200k contigs).
+struct SurvTiles {
+    uint4* buf;
+    uint16_t* mask;
+    unsigned long long* cnt;     // counts past the capacity
+    unsigned long long cap;
+    unsigned long long* n_cand;  // candidate records reserved
+};
+constexpr uint32_t TILE_BATCH = 32;
+
+struct TileStage {
+    uint16_t mask[TILE_BATCH][64];
+    uint2 tile[TILE_BATCH];
+    uint32_t count[TILE_BATCH];
+};
+
+// A wave's n staged tiles to the list from slot on, their records from base on.
+__device__ inline void stage_write(const SurvTiles& o, const TileStage& st, uint32_t n, uint32_t lane,
+                                   unsigned long long slot, unsigned long long base) {
+    const uint32_t c = lane < n ? st.count[lane] : 0u;
+    base += wave_incl_sum_dpp(c) - c;
+    if (lane < n && slot + lane < o.cap)
+        o.buf[slot + lane] = make_uint4(st.tile[lane].x, st.tile[lane].y, (uint32_t)base,
+                                        c | (uint32_t)(base >> 32) << 11);
+    for (uint32_t t = 0; t < n; ++t)
+        if (slot + t < o.cap) o.mask[(slot + t) * 64 + lane] = st.mask[t][lane];
+}
+
+// Reserves and writes a wave's n staged tiles (n > 0).
+__device__ inline void stage_flush(const SurvTiles& o, const TileStage& st, uint32_t n, uint32_t lane) {
+    wave_sync();
+    const uint32_t c = lane < n ? st.count[lane] : 0u;
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_sum_dpp(c), 63);
+    unsigned long long slot = 0, base = 0;
+    if (lane == 0) {
+        slot = atomicAdd(o.cnt, (unsigned long long)n);
+        base = atomicAdd(o.n_cand, (unsigned long long)total);
+    }
+    stage_write(o, st, n, lane, lane0_u64(slot), lane0_u64(base));
+    wave_sync();
+}
+
+struct GramArgs {
+    const uint4 *frag, *frag_a;
+    const uint4* items;  // null: `whole`
+    uint4 whole;
+    const uint4* list;  // null: every tile (tr <= tc < ntiles) of the triangle
+    const unsigned long long* n_list;
+    unsigned long long list_cap;
+    uint32_t ntiles;
+    SurvTiles out;
+    // FULL
+    const uint32_t* full_pos;
+    uint32_t full_base;
+    const uint8_t* full;
+    const uint32_t *cl, *bits;
+    uint32_t k;
+};
+
+// Tile e of the triangle's tiles, column by column: column tc's tiles tr = 0 ..
+// tc follow tc (tc + 1) / 2 others.
+__device__ inline uint4 triangle_tile(uint64_t e) {
+    uint32_t tc = (uint32_t)((sqrt(8.0 * (double)e + 1.0) - 1.0) * 0.5);
+    while ((uint64_t)tc * (tc + 1) / 2 > e) --tc;
+    while ((uint64_t)(tc + 1) * (tc + 2) / 2 <= e) ++tc;
+    return make_uint4((uint32_t)(e - (uint64_t)tc * (tc + 1) / 2), tc, 0u, 0u);
+}
+
+template <bool BF16, int KSX, bool FULL>
+__global__ __launch_bounds__(256) void k_tile_gram(const GramArgs A) {
+    __shared__ TileStage stages[4];
+    __shared__ uint32_t fin_n[4], fin_c[4];
+    __shared__ unsigned long long s_slot, s_base;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    TileStage& st = stages[wave];
+    uint32_t nst = 0;
+    const unsigned long long n_ent =
+        A.list ? min(*A.n_list, A.list_cap) : (unsigned long long)A.ntiles * (A.ntiles + 1) / 2;
+    // the block's four waves take four neighbouring entries
+    for (uint64_t step = 0;; ++step) {
+        const uint64_t b = chunk_entry(blockIdx.x, gridDim.x, step);
+        if (4 * b >= n_ent) break;
+        const uint64_t e = 4 * b + wave;
+        if (e >= n_ent) continue;
+        const uint4 en = A.list ? A.list[e] : triangle_tile(e);
+        const uint4 it = A.items ? A.items[en.z] : A.whole;
+        const uint32_t r_lo = it.x, r_hi = it.y, c_lo = it.z, c_hi = it.w & ~ITEM_TRI;
+        const bool tri = (it.w & ITEM_TRI) != 0;
+        f32x16_t acc = f32x16_t{};
+#pragma unroll
+        for (int ks = 0; ks < KSX; ++ks) {
+            const uint4 a = ks == KSX - 1 ? A.frag_a[(size_t)en.x * 64 + lane]
+                                          : A.frag[((size_t)en.x * KSX + ks) * 64 + lane];
+            acc = mfma32<BF16>(a, A.frag[((size_t)en.y * KSX + ks) * 64 + lane], acc);
+        }
+        // bit r: accumulator r of this lane is a survivor (row
+        // 4 (l / 32) + r % 4 + 8 (r / 4), column l % 32)
+        uint32_t bits = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bits |= (acc[r] > 0.f ? 1u : 0u) << r;
+        const uint32_t i0 = 32 * en.x + 4 * (lane >> 5), j = 32 * en.y + (lane & 31);
+        if ((tri && en.x == en.y) || 32 * en.x < r_lo || 32 * en.x + 32 > r_hi || 32 * en.y < c_lo ||
+            32 * en.y + 32 > c_hi) {  // the diagonal or an edge of the item
+            uint32_t keep = 0;
+            const bool j_in = j >= c_lo && j < c_hi;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t i = i0 + (r & 3) + 8 * (r >> 2);
+                const bool ok = j_in & (i >= r_lo) & (i < r_hi) & (!tri | (i < j));
+                keep |= (ok ? 1u : 0u) << r;
+            }
+            bits &= keep;
+        }
+        if (FULL && bits) {
+            // not the row itself, not a probed cluster pair, and of two full
+            // rows only from the smaller position
+            const uint32_t cj = A.cl[j];
+            const bool fj = A.full[j] != 0;
+            for (uint32_t left = bits; left; left &= left - 1) {
+                const int r = __builtin_ctz(left);
+                const uint32_t pi = A.full_pos[i0 + (r & 3) + 8 * (r >> 2) - A.full_base];
+                const uint64_t ab = (uint64_t)A.cl[pi] * A.k + cj;
+                if (j == pi || ((A.bits[ab >> 5] >> (ab & 31)) & 1u) || (fj && j < pi)) bits &= ~(1u << r);
+            }
+        }
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_sum_dpp((uint32_t)__popc(bits)), 63);
+        if (total == 0) continue;
+        st.mask[nst][lane] = (uint16_t)bits;
+        if (lane == 0) {
+            st.tile[nst] = make_uint2(en.x, en.y);
+            st.count[nst] = total;
+        }
+        if (++nst == TILE_BATCH) {
+            stage_flush(A.out, st, nst, lane);
+            nst = 0;
+        }
+    }
+    // what is left of the block's four waves in one reservation
+    wave_sync();
+    const uint32_t left = (uint32_t)__builtin_amdgcn_readlane(
+        (int)wave_incl_sum_dpp(lane < nst ? st.count[lane] : 0u), 63);
+    if (lane == 0) {
+        fin_n[wave] = nst;
+        fin_c[wave] = left;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t n = fin_n[0] + fin_n[1] + fin_n[2] + fin_n[3], c = fin_c[0] + fin_c[1] + fin_c[2] + fin_c[3];
+        s_slot = n ? atomicAdd(A.out.cnt, (unsigned long long)n) : 0ull;
+        s_base = n ? atomicAdd(A.out.n_cand, (unsigned long long)c) : 0ull;
+    }
+    __syncthreads();
+    if (nst) {
+        unsigned long long slot = s_slot, base = s_base;
+        for (uint32_t w = 0; w < wave; ++w) {
+            slot += fin_n[w];
+            base += fin_c[w];
+        }
+        stage_write(A.out, st, nst, lane, slot, base);
+    }
+}
+
+struct RowArgs {
+    const float* tnf;
+    const float* tvec;     // Chebyshev coordinates, by contig
+    const uint32_t* perm;  // position -> contig (null: itself)
+    uint32_t n;
+    const uint32_t* full_pos;  // appended full rows: positions of rows full_base + t (null: none)
+    uint32_t full_base;
+};
+
+// Contig of lane l of a tile: its row l for l < 32, its column l - 32 for the
+// others; contig 0 past the rows, and for no tile (valid = false).
+__device__ inline uint32_t tile_contig(const RowArgs& A, uint32_t tr, uint32_t tc, bool valid, uint32_t lane) {
+    if (!valid) return 0u;
+    uint32_t p = lane < 32 ? 32 * tr + lane : 32 * tc + (lane - 32);
+    if (A.full_pos && lane < 32) p = p - A.full_base < A.n ? A.full_pos[p - A.full_base] : A.n;
+    return p < A.n ? (A.perm ? A.perm[p] : p) : 0u;
+}
+
+// The 64 FP32 rows of a tile (32 of its rows, then 32 of its columns) pass
+// through registers into LDS: 544-byte contiguous reads by contig, no sorted
+// copy of the rows.  Four lanes a row, pieces lane % 4 + 4 m and piece 32 or 33
+// (two lanes each).  The row stride of 35 float4 puts 16 different rows in
+// different banks.
+constexpr int TQ = NT / 4, TSTR = TQ + 1, TLOADS = 9;
+static_assert(TQ == 34, "four lanes load a row in eight pieces each and two more");
+struct TileRows {
+    f32x4_t v[TLOADS];
+    __device__ inline void load(const float* tnf, uint32_t contig, uint32_t tid) {
+        const f32x4_t* src = reinterpret_cast<const f32x4_t*>(tnf + (size_t)contig * NT);
+        const uint32_t q = tid & 3;
+#pragma unroll
+        for (int m = 0; m < TLOADS - 1; ++m) v[m] = src[q + 4 * m];
+        v[TLOADS - 1] = src[32 + (q & 1)];
+    }
+    __device__ inline void store(f32x4_t (*rows)[TSTR], uint32_t tid) const {
+        const uint32_t r = tid >> 2, q = tid & 3;
+#pragma unroll
+        for (int m = 0; m < TLOADS - 1; ++m) rows[r][q + 4 * m] = v[m];
+        rows[r][32 + (q & 1)] = v[TLOADS - 1];
+    }
+};
+
+// Squared FP32 distance of two LDS rows; every mode's similarity comes from
+// this sum (eight accumulators, the same order everywhere).
+__device__ inline float tile_dist2(const f32x4_t* x4, const f32x4_t* y4) {
+    float s[8] = {};
+#pragma unroll 1
+    for (int q = 0; q < TQ; q += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const f32x4_t x = x4[q + h], y = y4[q + h];
+            const float d0 = x.x - y.x, d1 = x.y - y.y, d2 = x.z - y.z, d3 = x.w - y.w;
+            s[4 * h] = fmaf(d0, d0, s[4 * h]);
+            s[4 * h + 1] = fmaf(d1, d1, s[4 * h + 1]);
+            s[4 * h + 2] = fmaf(d2, d2, s[4 * h + 2]);
+            s[4 * h + 3] = fmaf(d3, d3, s[4 * h + 3]);
+        }
+    }
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
+struct F32Args {
+    RowArgs rows;
+    const uint4* list;  // null: every tile of the triangle
+    const unsigned long long* n_list;
+    unsigned long long list_cap;
+    uint32_t ntiles;
+    float R2;
+    SurvTiles out;
+};
+
+// EXACT_F32's form of the survivor mask: FP32 differences of every pair of a
+// listed tile, d^2 < R2.  One block a tile, 2 x 2 pairs a thread; the next
+// tile's rows are in registers meanwhile.
+__global__ __launch_bounds__(256, 3) void k_tile_f32(const F32Args A) {
+    __shared__ __align__(16) f32x4_t rows[64][TSTR];
+    __shared__ uint32_t id[2][64], smask[64];
+    __shared__ TileStage st;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const unsigned long long n_ent =
+        A.list ? min(*A.n_list, A.list_cap) : (unsigned long long)A.ntiles * (A.ntiles + 1) / 2;
+    auto entry = [&](uint64_t e) {
+        return e < n_ent ? (A.list ? A.list[e] : triangle_tile(e)) : make_uint4(0, 0, 0, 0);
+    };
+    uint64_t step = 0, e0 = chunk_entry(blockIdx.x, gridDim.x, 0);
+    if (e0 >= n_ent) return;
+    uint64_t e1 = chunk_entry(blockIdx.x, gridDim.x, 1);
+    uint4 en = entry(e0), en1 = entry(e1);
+    uint32_t next_id = 0, nst = 0;
+    if (wave == 0) {
+        id[0][lane] = tile_contig(A.rows, en.x, en.y, true, lane);
+        next_id = tile_contig(A.rows, en1.x, en1.y, e1 < n_ent, lane);
+    }
+    __syncthreads();
+    TileRows pre;
+    pre.load(A.rows.tnf, id[0][tid >> 2], tid);
+    for (int buf = 0;; buf ^= 1) {
+        pre.store(rows, tid);
+        if (wave == 0) {
+            id[buf ^ 1][lane] = next_id;
+            smask[lane] = 0;
+        }
+        __syncthreads();
+        const bool more = e1 < n_ent;
+        const uint64_t e2 = chunk_entry(blockIdx.x, gridDim.x, step + 2);
+        const uint4 en2 = entry(e2);
+        pre.load(A.rows.tnf, id[buf ^ 1][tid >> 2], tid);  // past the last tile: rows of no use
+        if (wave == 0) next_id = tile_contig(A.rows, en2.x, en2.y, e2 < n_ent, lane);
+        const uint32_t ty = tid >> 4, tx = tid & 15;
+        float s[2][2][8] = {};
+#pragma unroll 1
+        for (int q = 0; q < TQ; q += 2)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                f32x4_t x[2], y[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    x[u] = rows[ty + 16 * u][q + h];
+                    y[u] = rows[32 + tx + 16 * u][q + h];
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const float d0 = x[u].x - y[v].x, d1 = x[u].y - y[v].y, d2 = x[u].z - y[v].z,
+                                    d3 = x[u].w - y[v].w;
+                        float* t = s[u][v] + 4 * h;
+                        t[0] = fmaf(d0, d0, t[0]);
+                        t[1] = fmaf(d1, d1, t[1]);
+                        t[2] = fmaf(d2, d2, t[2]);
+                        t[3] = fmaf(d3, d3, t[3]);
+                    }
+            }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                const float* t = s[u][v];
+                const float d2 = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+                const uint32_t r = ty + 16 * u, c = tx + 16 * v, i = 32 * en.x + r, j = 32 * en.y + c;
+                // the mask's layout: lane 32 (r / 4 % 2) + c, bit r % 4 + 4 (r / 8)
+                if (d2 < A.R2 && i < j && j < A.rows.n)
+                    atomicOr(&smask[32 * ((r >> 2) & 1) + c], 1u << ((r & 3) + 4 * (r >> 3)));
+            }
+        __syncthreads();  // the mask is complete; rows and id[buf] are free again
+        if (wave == 0) {
+            const uint32_t bits = smask[lane];
+            const uint32_t total =
+                (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_sum_dpp((uint32_t)__popc(bits)), 63);
+            if (total) {
+                st.mask[nst][lane] = (uint16_t)bits;
+                if (lane == 0) {
+                    st.tile[nst] = make_uint2(en.x, en.y);
+                    st.count[nst] = total;
+                }
+                if (++nst == TILE_BATCH) {
+                    stage_flush(A.out, st, nst, lane);
+                    nst = 0;
+                }
+            }
+        }
+        if (!more) break;
+        ++step;
+        e1 = e2;
+        en = en1;
+        en1 = en2;
+    }
+    if (wave == 0 && nst) stage_flush(A.out, st, nst, lane);
+}
+
+struct RefineArgs {
+    RowArgs rows;
+    SurvTiles in;
+    float T32;
+    Cand* cand;
+    unsigned long long cand_cap;
+    unsigned long long* kept;
+    uint32_t* bcnt;  // kept endpoints per select bucket
+    uint64_t* amb;
+    unsigned long long* amb_cnt;
+};
+
+// One block a tile: the rows in LDS, one survivor a thread: 68 16-byte LDS
+// reads, 136 differences, the FP32 Chebyshev model.  The next tile's rows are
+// in registers while this tile is worked off (its contigs known one tile
+// ahead), so the loads' latency is covered by this and the CU's other blocks.
+// Survivors become candidate records {i, j, preProb, flags} in place: there is
+// no survivor list to sort and pack, and a tile's kept pairs share one row and
+// one column bucket of the selection, so two atomics a tile count them.
+// Tie-band candidates are staged in LDS over the tiles.
+// Before (four lanes a survivor streaming both rows from L2, 19.4M survivors at
+// 200k contigs): 1.54 ms, and 0.3 ms to sort and pack the survivor list.
+constexpr uint32_t AMB_STAGE = 192;
+
+__global__ __launch_bounds__(256, 4) void k_tile_refine(const RefineArgs A) {
+    __shared__ __align__(16) f32x4_t rows[64][TSTR];
+    __shared__ uint16_t pl[1024];  // survivors of the tile: row << 5 | column
+    __shared__ uint32_t id[2][64];
+    __shared__ float tv[2][64];
+    __shared__ uint64_t amb_at[AMB_STAGE];  // staged tie-band records
+    __shared__ uint32_t s_keep, s_amb;
+    __shared__ unsigned long long s_dst;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const unsigned long long n_ent = min(*A.in.cnt, A.in.cap);
+    const uint4 none = make_uint4(0, 0, 0, 0);
+    uint64_t step = 0, e0 = chunk_entry(blockIdx.x, gridDim.x, 0);
+    if (e0 >= n_ent) return;
+    uint64_t e1 = chunk_entry(blockIdx.x, gridDim.x, 1);
+    uint4 en = A.in.buf[e0], en1 = e1 < n_ent ? A.in.buf[e1] : none;
+    uint32_t next_id = 0, bits = 0;
+    if (wave == 0) {
+        const uint32_t c = tile_contig(A.rows, en.x, en.y, true, lane);
+        id[0][lane] = c;
+        tv[0][lane] = A.rows.tvec[c];
+        next_id = tile_contig(A.rows, en1.x, en1.y, e1 < n_ent, lane);
+    }
+    if (wave == 1) bits = A.in.mask[e0 * 64 + lane];
+    if (tid == 0) s_amb = 0;
+    __syncthreads();
+    TileRows pre;
+    pre.load(A.rows.tnf, id[0][tid >> 2], tid);
+    unsigned int nkeep = 0;
+    for (int buf = 0;; buf ^= 1) {
+        // this tile's rows and survivor list to LDS, the next tile's contigs beside them
+        pre.store(rows, tid);
+        if (wave == 0) id[buf ^ 1][lane] = next_id;
+        if (wave == 1) {
+            const uint32_t pc = (uint32_t)__popc(bits);
+            uint32_t o = wave_incl_sum_dpp(pc) - pc;
+            for (; bits; bits &= bits - 1) {
+                const int r = __builtin_ctz(bits);
+                pl[o++] = (uint16_t)((4 * (lane >> 5) + (r & 3) + 8 * (r >> 2)) << 5 | (lane & 31));
+            }
+        }
+        if (tid == 0) s_keep = 0;
+        __syncthreads();
+        // the next tile's loads, and the one after's contigs
+        const bool more = e1 < n_ent;
+        const uint64_t e2 = chunk_entry(blockIdx.x, gridDim.x, step + 2);
+        const uint4 en2 = e2 < n_ent ? A.in.buf[e2] : none;
+        float next_tv = 0.f;
+        pre.load(A.rows.tnf, id[buf ^ 1][tid >> 2], tid);  // past the last tile: rows of no use
+        if (wave == 0) {
+            next_tv = A.rows.tvec[next_id];
+            next_id = tile_contig(A.rows, en2.x, en2.y, e2 < n_ent, lane);
+        }
+        if (wave == 1 && more) bits = A.in.mask[e1 * 64 + lane];
+        // a tile past the capacity is left out (the host runs the pass again)
+        const uint32_t c = en.w & 2047u;
+        const unsigned long long base = (unsigned long long)(en.w >> 11) << 32 | en.z;
+        const bool fits = base + c <= A.cand_cap;
+        uint32_t kept_w = 0;
+        for (uint32_t t0 = 0; t0 < c && fits; t0 += 256) {
+            const uint32_t t = t0 + tid;
+            bool keep = false;
+            uint32_t r = 0;
+            if (t < c) {
+                r = pl[t] >> 5;
+                const uint32_t col = 32 + (pl[t] & 31);
+                const Pre32 m = model32(sqrtf(tile_dist2(rows[r], rows[col])), tv[buf][r], tv[buf][col]);
+                const bool amb = fabsf(m.pre - A.T32) <= EPS_PRE || fabsf(m.pre1 - FLOOR32) <= EPS_PRE;
+                keep = !amb && m.pre > A.T32;  // a tie-band pair is kept (or not) by k_adjudicate
+                Cand cd;
+                cd.i = id[buf][r];
+                cd.j = id[buf][col];
+                cd.pre = m.pre;
+                cd.flags = (amb ? 1u : 0u) | (keep ? 2u : 0u);
+                A.cand[base + t] = cd;
+                if (amb) {
+                    const uint32_t a = atomicAdd(&s_amb, 1u);
+                    if (a < AMB_STAGE)
+                        amb_at[a] = base + t;
+                    else  // more ties than the stage holds: one by one
+                        A.amb[atomicAdd(A.amb_cnt, 1ull)] = base + t;
+                }
+            }
+            kept_w += (uint32_t)__popcll(__ballot(keep));
+            if (A.rows.full_pos && keep)
+                atomicAdd(&A.bcnt[A.rows.full_pos[32 * en.x + r - A.rows.full_base] / S_BUCKET], 1u);
+        }
+        if (lane == 0 && kept_w) atomicAdd(&s_keep, kept_w);
+        if (more && wave == 0) tv[buf ^ 1][lane] = next_tv;
+        __syncthreads();  // rows, pl, id[buf] and tv[buf] are free again; s_keep and s_amb are complete
+        if (tid == 0 && s_keep) {
+            if (!A.rows.full_pos) atomicAdd(&A.bcnt[32 * en.x / S_BUCKET], s_keep);
+            atomicAdd(&A.bcnt[32 * en.y / S_BUCKET], s_keep);
+            nkeep += s_keep;
+        }
+        const uint32_t na = min(s_amb, AMB_STAGE);  // block-uniform
+        if (na && (!more || na >= AMB_STAGE / 2)) {
+            if (tid == 0) s_dst = atomicAdd(A.amb_cnt, (unsigned long long)na);
+            __syncthreads();
+            for (uint32_t a = tid; a < na; a += 256) A.amb[s_dst + a] = amb_at[a];
+            if (tid == 0) s_amb = 0;
+        }
+        if (!more) break;
+        ++step;
+        e1 = e2;
+        en = en1;
+        en1 = en2;
+    }
+    if (tid == 0 && nkeep) atomicAdd(A.kept, (unsigned long long)nkeep);
+}
 
 __device__ inline bool prob_rule_keeps(double pre64, double required_min_p) {
     // the FP64 tie-breaker returns exactly ln 9 where the variant's model 2
@@ -1028,98 +1201,16 @@ __device__ inline bool prob_rule_keeps(double pre64, double required_min_p) {
     return 1. - prob >= required_min_p;
 }
 
-// Candidates inside the tie band are listed (amb_list, count in *amb_ctr)
-// with their FP32 value and decided by k_adjudicate afterwards: inlined, the
-// FP64 evaluator took the kernel from 120 to 157 registers (3 waves per SIMD
-// instead of 4; 1.83 -> 1.58 ms at 200k contigs).  More waves than 4 (73
-// registers under amdgpu_waves_per_eu 5 or 8) ran slower: the rows in
-// flight then overflow the caches.
-__global__ __launch_bounds__(256) void k_refine(const uint2* __restrict__ surv, uint64_t ns,
-                                                const uint32_t* __restrict__ perm,
-                                                const float* __restrict__ rows,
-                                                const float* __restrict__ tv, double T,
-                                                Cand* __restrict__ cand, unsigned long long* __restrict__ counters,
-                                                uint32_t* __restrict__ bcnt, uint64_t* __restrict__ amb_list,
-                                                unsigned long long* __restrict__ amb_ctr) {
-    __shared__ unsigned int s_keep;
-    if (threadIdx.x == 0) s_keep = 0;
-    __syncthreads();
-    const float T32 = (float)T;
-    const uint32_t q = threadIdx.x & 3;
-    const uint32_t per_xcd_blocks = gridDim.x / 8;
-    const uint64_t per_xcd = (ns + 7) / 8;
-    const uint64_t lo = (uint64_t)(blockIdx.x % 8) * per_xcd;
-    const uint64_t hi = lo + per_xcd < ns ? lo + per_xcd : ns;
-    const uint64_t stride = (uint64_t)per_xcd_blocks * (blockDim.x / 4);
-    const uint64_t first = lo + (uint64_t)(blockIdx.x / 8) * (blockDim.x / 4);
-    unsigned int nkeep = 0;
-    for (uint64_t base = first; base < hi; base += stride) {
-        const uint64_t idx = base + (threadIdx.x >> 2);
-        uint2 p = make_uint2(0, 0);
-        float part = 0.f;
-        if (idx < hi) {
-            p = surv[idx];
-            const float4* a4 = reinterpret_cast<const float4*>(rows + (size_t)p.x * NT);
-            const float4* b4 = reinterpret_cast<const float4*>(rows + (size_t)p.y * NT);
-            float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-            for (int m = 0; m < 9; ++m) {
-                const uint32_t k = q + 4 * m;
-                if (k < NT / 4) {
-                    const float4 x = a4[k], y = b4[k];
-                    const float d0 = x.x - y.x, d1 = x.y - y.y, d2 = x.z - y.z, d3 = x.w - y.w;
-                    s0 = fmaf(d0, d0, s0);
-                    s1 = fmaf(d1, d1, s1);
-                    s0 = fmaf(d2, d2, s0);
-                    s1 = fmaf(d3, d3, s1);
-                }
-            }
-            part = s0 + s1;
-        }
-        part += __shfl_xor(part, 1, 64);
-        part += __shfl_xor(part, 2, 64);
-        bool kept = false, amb = false;
-        if (idx < hi && q == 0) {
-            const float d = sqrtf(part);
-            const Pre32 m = model32(d, tv[p.x], tv[p.y]);
-            amb = fabsf(m.pre - T32) <= EPS_PRE || fabsf(m.pre1 - FLOOR32) <= EPS_PRE;
-            const uint2 id = perm ? make_uint2(perm[p.x], perm[p.y]) : p;
-            // a tie-band pair is kept (or not) by k_adjudicate
-            const bool keep = !amb && m.pre > T32;
-            nkeep += keep ? 1u : 0u;
-            kept = keep;
-            Cand c;
-            c.i = id.x;
-            c.j = id.y;
-            c.pre = m.pre;
-            c.flags = (amb ? 1u : 0u) | (keep ? 2u : 0u);
-            cand[idx] = c;
-        }
-        // rows of the select buckets: p holds prefilter row positions
-        wave_aggregated_count(bcnt, p.x / S_BUCKET, kept);
-        wave_aggregated_count(bcnt, p.y / S_BUCKET, kept);
-        // tie-band candidates to the adjudication list, one atomic per wave
-        const uint64_t amask = __ballot(amb);
-        if (amask) {
-            const uint32_t lane = lane_id();
-            unsigned long long base = 0;
-            if (lane == 0) base = atomicAdd(amb_ctr, (unsigned long long)__popcll(amask));
-            base = __shfl(base, 0, 64);
-            if (amb) amb_list[base + __popcll(amask & ((1ull << lane) - 1ull))] = idx;
-        }
-    }
-    if (nkeep) atomicAdd(&s_keep, nkeep);
-    __syncthreads();
-    if (threadIdx.x == 0 && s_keep) atomicAdd(&counters[0], (unsigned long long)s_keep);
+__device__ inline uint32_t position_of(const uint32_t* __restrict__ iperm, uint32_t c) {
+    return iperm ? iperm[c] : c;
 }
 
 // The FP64 decision of each listed tie-band candidate (cuda/Cuda2.cu:192-241
 // arithmetic, model64): its preProb, kept flag, bucket counts and the kept /
 // adjudicated totals.  The list length is read on the device.
-__global__ __launch_bounds__(256) void k_adjudicate(const uint2* __restrict__ surv, const uint32_t* __restrict__ perm,
-                                                    const float* __restrict__ rows, const double* __restrict__ ls,
-                                                    double T, int rule, double min_p,
-                                                    const uint64_t* __restrict__ amb_list,
+__global__ __launch_bounds__(256) void k_adjudicate(const float* __restrict__ tnf, const double* __restrict__ ls,
+                                                    const uint32_t* __restrict__ iperm, double T, int rule,
+                                                    double min_p, const uint64_t* __restrict__ amb_list,
                                                     const unsigned long long* __restrict__ amb_ctr,
                                                     Cand* __restrict__ cand, unsigned long long* __restrict__ counters,
                                                     uint32_t* __restrict__ bcnt) {
@@ -1131,15 +1222,14 @@ __global__ __launch_bounds__(256) void k_adjudicate(const uint2* __restrict__ su
     for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n_amb;
          t += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t idx = amb_list[t];
-        const uint2 p = surv[idx];
-        const uint2 id = perm ? make_uint2(perm[p.x], perm[p.y]) : p;
-        const double p64 = model64(rows + (size_t)p.x * NT, rows + (size_t)p.y * NT, ls[id.x], ls[id.y]);
+        const uint32_t i = cand[idx].i, j = cand[idx].j;
+        const double p64 = model64(tnf + (size_t)i * NT, tnf + (size_t)j * NT, ls[i], ls[j]);
         const bool keep = rule == RULE_PROB ? prob_rule_keeps(p64, min_p) : p64 > T;
         cand[idx].pre = (float)p64;
         cand[idx].flags = 1u | (keep ? 2u : 0u);
         if (keep) {
-            atomicAdd(&bcnt[p.x / S_BUCKET], 1u);
-            atomicAdd(&bcnt[p.y / S_BUCKET], 1u);
+            atomicAdd(&bcnt[position_of(iperm, i) / S_BUCKET], 1u);
+            atomicAdd(&bcnt[position_of(iperm, j) / S_BUCKET], 1u);
             ++nkeep;
         }
     }
@@ -1155,7 +1245,7 @@ __global__ __launch_bounds__(256) void k_adjudicate(const uint2* __restrict__ su
 // The cluster index proposes pairs; a row whose proposals fill its max_edges
 // slots (a "full row") may have missed a better partner, which would leave a
 // wrong edge in its list.  Full rows are therefore evaluated again against
-// every column with the BF16 Gram prefilter (their fragments appended to the
+// every column with the BF16 Gram scan (their fragments appended to the
 // fragment array as extra rows), and the survivors outside the probed cluster
 // pairs (which phase one decided already) go through the same refinement and
 // selection.  A full row's kept set is then the exhaustive one.
@@ -1200,20 +1290,26 @@ __device__ inline void kept_count(uint32_t* __restrict__ h, uint32_t* __restrict
     }
 }
 
-__global__ __launch_bounds__(256) void k_row_kept(const uint2* __restrict__ surv, const Cand* __restrict__ cand,
-                                                  uint64_t nc, uint32_t* __restrict__ cnt) {
+__global__ __launch_bounds__(256) void k_row_kept(const Cand* __restrict__ cand,
+                                                  const unsigned long long* __restrict__ n_cand,
+                                                  unsigned long long cap, const uint32_t* __restrict__ iperm,
+                                                  uint32_t* __restrict__ cnt) {
     __shared__ uint32_t hist[4][2][KEPT_SPAN];
     const uint32_t w = threadIdx.x >> 6, lane = lane_id();
     for (uint32_t s = lane; s < KEPT_SPAN; s += 64) hist[w][0][s] = hist[w][1][s] = 0u;
     __builtin_amdgcn_s_waitcnt(0);
+    const uint64_t nc = min(*n_cand, cap);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < nc; base += stride) {
         const uint64_t k = base + lane;
         bool kept = false;
         uint2 p = make_uint2(0, 0);
-        if (k < nc && (cand[k].flags & 2u)) {
-            p = surv[k];
-            kept = true;
+        if (k < nc) {
+            const Cand c = cand[k];
+            if (c.flags & 2u) {
+                p = make_uint2(iperm[c.i], iperm[c.j]);
+                kept = true;
+            }
         }
         if (!__any(kept)) continue;
         kept_count(hist[w][0], cnt, p.x, kept, lane);
@@ -1247,48 +1343,10 @@ __global__ __launch_bounds__(256) void k_probed_bits(const uint32_t* __restrict_
     atomicOr(&bits[ba >> 5], 1u << (ba & 31));
 }
 
-// The fallback prefilter's chunks (rows base + t = full row t, columns =
-// positions) -> pairs of positions (p, j) that phase one did not evaluate:
-// j != p, j's cluster not probed with p's, and when both rows are full only
-// from the smaller position.  Appended to out (counted past cap).
-__global__ __launch_bounds__(256) void k_fb_collect(const ChunkOut co, const uint32_t* __restrict__ full_pos,
-                                                    uint32_t base, const uint8_t* __restrict__ full,
-                                                    const uint32_t* __restrict__ cl, const uint32_t* __restrict__ bits,
-                                                    uint32_t k, uint2* __restrict__ out, uint64_t cap,
-                                                    unsigned long long* __restrict__ ctr) {
-    const uint32_t s = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const unsigned long long nch = min(co.cnt[(size_t)s * SHARD_STRIDE], co.cap);
-    for (unsigned long long c = wave; c < nch; c += 4) {
-        const size_t slot = (size_t)s * co.cap + c;
-        const uint2 m = co.meta[slot];
-        for (uint32_t e0 = 0; e0 < m.y; e0 += 64) {
-            bool take = false;
-            uint2 pr = make_uint2(0, 0);
-            if (e0 + lane < m.y) {
-                const uint2 q = co.buf[slot * M_STAGE + e0 + lane];
-                const uint32_t p = full_pos[q.x - base], j = q.y;
-                const uint64_t ab = (uint64_t)cl[p] * k + cl[j];
-                const bool probed = (bits[ab >> 5] >> (ab & 31)) & 1u;
-                take = j != p && !probed && !(full[j] && j < p);
-                pr = make_uint2(p, j);
-            }
-            const uint64_t bal = __ballot(take);
-            const uint32_t cnt = (uint32_t)__popcll(bal);
-            if (!cnt) continue;
-            unsigned long long b0 = 0;
-            if (lane == 0) b0 = atomicAdd(ctr, (unsigned long long)cnt);
-            b0 = __shfl(b0, 0, 64);
-            const uint32_t rank = (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-            if (take && b0 + rank < cap) out[b0 + rank] = pr;
-        }
-    }
-}
-
 // ---------------------------------------------------------------- select --
 // Kept candidates -> per row the max_edges largest preProb -> edges i < j,
 // sorted by (i, j).  Rows are handled in buckets of S_BUCKET consecutive
-// positions of the prefilter's row order (the composition order of the MFMA
-// modes, contig order for the FP32 mode).  A refined survivor run shares one
+// positions of the scan's row order.  A refined survivor run shares one
 // row bucket and spans a few column buckets, so the bucket counts and slot
 // reservations are aggregated per wave (one device atomic per distinct bucket
 // among a wave's 64 candidates, instead of one per candidate endpoint) and a
@@ -1306,61 +1364,53 @@ struct Ent {
     uint32_t lrow;  // row within the bucket
 };
 
-__device__ inline uint32_t position_of(const uint32_t* __restrict__ iperm, uint32_t c) {
-    return iperm ? iperm[c] : c;
-}
-
 __global__ __launch_bounds__(256) void k_iperm(const uint32_t* __restrict__ perm, uint32_t n,
                                                uint32_t* __restrict__ iperm) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < n) iperm[perm[s]] = s;
 }
 
-// The candidate list runs item by item, so neighbouring candidates share row
+// The candidate list runs tile by tile, so neighbouring candidates share row
 // buckets: consecutive blocks take 256-candidate pieces FILL_SPREAD pieces
-// apart (piece = (block % FILL_SPREAD) * per + block / FILL_SPREAD), which
-// keeps the blocks in flight on different buckets' counters.
+// apart (piece = (b % FILL_SPREAD) * per + b / FILL_SPREAD), which keeps the
+// blocks in flight on different buckets' counters.  The list's length is read
+// on the device.
 constexpr uint32_t FILL_SPREAD = 2048;
 
-__global__ __launch_bounds__(256) void k_bucket_fill(const Cand* __restrict__ cand, uint64_t nc,
-                                                     const uint32_t* __restrict__ iperm,
+__global__ __launch_bounds__(256) void k_bucket_fill(const Cand* __restrict__ cand,
+                                                     const unsigned long long* __restrict__ n_cand,
+                                                     unsigned long long cap, const uint32_t* __restrict__ iperm,
                                                      const uint64_t* __restrict__ boff, uint32_t* __restrict__ bcur,
                                                      Ent* __restrict__ ent) {
+    const uint64_t nc = min(*n_cand, cap);
     const uint64_t pieces = (nc + 255) / 256, per = (pieces + FILL_SPREAD - 1) / FILL_SPREAD;
-    const uint64_t piece = (uint64_t)(blockIdx.x % FILL_SPREAD) * per + blockIdx.x / FILL_SPREAD;
-    if (piece >= pieces) return;  // whole block: the wave collectives below see all lanes
-    const uint64_t k = piece * 256 + threadIdx.x;
-    bool act = false;
-    Cand c{0, 0, 0.f, 0};
-    uint32_t si = 0, sj = 0;
-    if (k < nc) {
-        c = cand[k];
-        if (c.flags & 2u) {
-            act = true;
-            si = position_of(iperm, c.i);
-            sj = position_of(iperm, c.j);
+    for (uint64_t b = blockIdx.x; b < per * FILL_SPREAD; b += gridDim.x) {
+        const uint64_t piece = (b % FILL_SPREAD) * per + b / FILL_SPREAD;
+        if (piece >= pieces) continue;  // whole block: the wave collectives below see all lanes
+        const uint64_t k = piece * 256 + threadIdx.x;
+        bool act = false;
+        Cand c{0, 0, 0.f, 0};
+        uint32_t si = 0, sj = 0;
+        if (k < nc) {
+            c = cand[k];
+            if (c.flags & 2u) {
+                act = true;
+                si = position_of(iperm, c.i);
+                sj = position_of(iperm, c.j);
+            }
         }
-    }
-    const uint32_t s1 = wave_aggregated_add(bcur, si / S_BUCKET, act);
-    const uint32_t s2 = wave_aggregated_add(bcur, sj / S_BUCKET, act);
-    if (act) {
-        ent[boff[si / S_BUCKET] + s1] = Ent{c.j, c.pre, si % S_BUCKET};
-        ent[boff[sj / S_BUCKET] + s2] = Ent{c.i, c.pre, sj % S_BUCKET};
+        const uint32_t s1 = wave_aggregated_add(bcur, si / S_BUCKET, act);
+        const uint32_t s2 = wave_aggregated_add(bcur, sj / S_BUCKET, act);
+        if (act) {
+            ent[boff[si / S_BUCKET] + s1] = Ent{c.j, c.pre, si % S_BUCKET};
+            ent[boff[sj / S_BUCKET] + s2] = Ent{c.i, c.pre, sj % S_BUCKET};
+        }
     }
 }
 
 // (pre desc, partner asc): true if x ranks before y
 __device__ inline bool ranks_before(float px, uint32_t ix, float py, uint32_t iy) {
     return px > py || (px == py && ix < iy);
-}
-
-// Orders the LDS writes of a wave before its following LDS reads (the lanes
-// of one wave execute each LDS instruction together and in program order; the
-// fences keep the compiler from moving accesses across).
-__device__ inline void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Bitonic sort of sz (power of two) LDS entries by the whole block (BY_RANK:
@@ -1609,14 +1659,19 @@ __device__ bool wave_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t de
     }
 }
 
-// Appends (rid, deg, beg) to a row list: list[0] = count, records from
-// list[BIG_REC]; err bit `ovf` if the list is full.
+// Appends (rid, deg, beg) to a row list with its counter apart; err bit `ovf`
+// if the list is full.
 constexpr int BIG_REC = 4;  // uint32 words per row record: rid, deg, beg lo, beg hi
-__device__ inline void push_row(uint32_t* __restrict__ list, uint32_t cap, uint32_t rid, uint32_t deg, uint64_t beg,
+struct RowList {
+    uint32_t* rec;
+    uint32_t* cnt;
+    uint32_t cap;
+};
+__device__ inline void push_row(const RowList& L, uint32_t rid, uint32_t deg, uint64_t beg,
                                 unsigned int* __restrict__ err, unsigned int ovf) {
-    const uint32_t q = atomicAdd(&list[0], 1u);
-    if (q < cap) {
-        uint32_t* rec = list + BIG_REC * (1 + q);
+    const uint32_t q = atomicAdd(L.cnt, 1u);
+    if (q < L.cap) {
+        uint32_t* rec = L.rec + BIG_REC * q;
         rec[0] = rid;
         rec[1] = deg;
         rec[2] = (uint32_t)beg;
@@ -1633,10 +1688,10 @@ __device__ void block_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t d
                                  const float* __restrict__ tnf, const double* __restrict__ ls, float* key,
                                  uint32_t* id, double* zkey, int* s_z, uint32_t* s_cnt,
                                  uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg,
-                                 uint32_t* __restrict__ huge, uint32_t huge_cap, unsigned int* __restrict__ err,
+                                 const RowList& huge, unsigned int* __restrict__ err,
                                  unsigned long long* __restrict__ capped) {
     if (deg > SEL_CAP) {
-        if (threadIdx.x == 0) push_row(huge, huge_cap, rid, deg, beg, err, 1u);
+        if (threadIdx.x == 0) push_row(huge, rid, deg, beg, err, 8u);
         return;
     }
     const int sz = pow2_at_least(deg);
@@ -1664,7 +1719,7 @@ __device__ void block_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t d
         __syncthreads();
         const int z0 = s_z[0], z1 = s_z[1], zn = z1 - z0;
         if (zn > ZONE_CAP) {  // block-uniform: adj is still untouched
-            if (threadIdx.x == 0) push_row(huge, huge_cap, rid, deg, beg, err, 1u);
+            if (threadIdx.x == 0) push_row(huge, rid, deg, beg, err, 8u);
             __syncthreads();
             return;
         }
@@ -1718,12 +1773,12 @@ __device__ void block_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t d
 // offsets as ent), then select every row by one wave.  Output per contig row:
 // out_cnt (edges kept: partners above the row, sorted) and rbeg (where they
 // are in adj).  Rows the wave path declines go to a list for
-// k_bigrow_select: big[0] = count, then (row id, degree, begin) records.
+// k_bigrow_select ((row id, degree, begin) records).
 
 __global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
     const uint64_t* __restrict__ boff, const Ent* __restrict__ ent, Adj* __restrict__ adj, uint32_t n, uint32_t K,
     const uint32_t* __restrict__ perm, const float* __restrict__ tnf, const double* __restrict__ ls,
-    uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, uint32_t* __restrict__ big, uint32_t big_cap,
+    uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, const RowList big,
     unsigned int* __restrict__ err, unsigned long long* __restrict__ capped) {
     constexpr int PER = S_BUCKET / 64;
     constexpr int BATCH = 4;
@@ -1800,31 +1855,30 @@ __global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
         } else {
             done = wave_row_select(adj, beg, deg, rid, K, tnf, ls, wkey[wave], wid[wave], out_cnt, rbeg, capped, lane);
         }
-        if (!done && lane == 0) push_row(big, big_cap, rid, deg, beg, err, 4u);
+        if (!done && lane == 0) push_row(big, rid, deg, beg, err, 4u);
     }
 }
 
 // Rows the wave path declined (over W_CAP entries, or a tie zone wider than a
 // wave): one block per row, blocks striding over the list.  err bit 4: the
 // list overflowed its capacity.  Rows beyond the LDS capacities go on to the
-// `huge` list (err bit 1, bit 8 if that list overflowed).
+// `huge` list (err bit 8 if that list overflowed).
 __global__ __launch_bounds__(S_THREADS) void k_bigrow_select(
-    const uint32_t* __restrict__ big, uint32_t big_cap, Adj* __restrict__ adj, uint32_t K,
-    const float* __restrict__ tnf, const double* __restrict__ ls, uint32_t* __restrict__ out_cnt,
-    uint64_t* __restrict__ rbeg, uint32_t* __restrict__ huge, uint32_t huge_cap, unsigned int* __restrict__ err,
-    unsigned long long* __restrict__ capped) {
+    const RowList big, Adj* __restrict__ adj, uint32_t K, const float* __restrict__ tnf,
+    const double* __restrict__ ls, uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, const RowList huge,
+    unsigned int* __restrict__ err, unsigned long long* __restrict__ capped) {
     __shared__ float bkey[SEL_CAP];
     __shared__ uint32_t bid[SEL_CAP];
     __shared__ double zkey[ZONE_CAP];
     __shared__ int s_z[2];
     __shared__ uint32_t s_cnt;
-    const uint32_t nbig = big[0];
-    const uint32_t m = nbig < big_cap ? nbig : big_cap;
+    const uint32_t nbig = *big.cnt;
+    const uint32_t m = nbig < big.cap ? nbig : big.cap;
     for (uint32_t q = blockIdx.x; q < m; q += gridDim.x) {
-        const uint32_t* rec = big + BIG_REC * (1 + q);
+        const uint32_t* rec = big.rec + BIG_REC * q;
         const uint64_t beg = (uint64_t)rec[2] | ((uint64_t)rec[3] << 32);
         block_row_select(adj, beg, rec[1], rec[0], K, tnf, ls, bkey, bid, zkey, s_z, &s_cnt, out_cnt, rbeg, huge,
-                         huge_cap, err, capped);
+                         err, capped);
     }
 }
 
@@ -1875,7 +1929,7 @@ __global__ __launch_bounds__(HUGE_THREADS) void k_hugerow_select(
     uint32_t* __restrict__ sk32, uint32_t* __restrict__ sv, float* __restrict__ spre,
     uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, unsigned long long* __restrict__ capped) {
     __shared__ uint32_t s_cnt;
-    const uint32_t* rec = huge + BIG_REC * (1 + blockIdx.x);
+    const uint32_t* rec = huge + BIG_REC * blockIdx.x;
     const uint32_t rid = rec[0], deg = rec[1];
     const uint64_t beg = (uint64_t)rec[2] | ((uint64_t)rec[3] << 32);
     uint32_t sz = 1;
@@ -1923,9 +1977,12 @@ __global__ __launch_bounds__(HUGE_THREADS) void k_hugerow_select(
 }
 
 // Edges of row r (contig order) to their place eoff[r]; one wave per row.
+// *total = their number.
 __global__ void k_emit(const uint64_t* __restrict__ rbeg, const Adj* __restrict__ adj,
                        const uint32_t* __restrict__ out_cnt, const uint64_t* __restrict__ eoff, uint32_t n,
-                       uint32_t* __restrict__ from, uint32_t* __restrict__ to, float* __restrict__ s) {
+                       uint32_t* __restrict__ from, uint32_t* __restrict__ to, float* __restrict__ s,
+                       unsigned long long* __restrict__ total) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *total = eoff[n];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t row = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
     if (row >= n) return;
@@ -2141,35 +2198,14 @@ int exclusive_scan_u32_to_u64(mdet_ctx* ctx, const uint32_t* in, uint64_t* out, 
     return MDET_OK;
 }
 
-// Contig order of the MFMA prefilter (ascending composition key).
-int sort_by_composition(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, uint32_t** perm_out) {
-    float *key, *key_sorted;
-    uint32_t *idx, *perm;
-    MDET_TRY(ctx_buf(ctx, "sort.key", n, &key));
-    MDET_TRY(ctx_buf(ctx, "sort.key2", n, &key_sorted));
-    MDET_TRY(ctx_buf(ctx, "sort.idx", n, &idx));
-    MDET_TRY(ctx_buf(ctx, "sort.perm", n, &perm));
-    hipLaunchKernelGGL(k_sort_key, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, tnf_dev, n, key, idx);
-    MDET_HIP(hipGetLastError());
-    size_t tmp = 0;
-    MDET_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, key, key_sorted, idx, perm, (int)n, 0, 32, ctx->stream));
-    void* t;
-    MDET_TRY(ctx_buf(ctx, "cub.sorttmp", tmp, &t));
-    MDET_HIP(hipcub::DeviceRadixSort::SortPairs(t, tmp, key, key_sorted, idx, perm, (int)n, 0, 32, ctx->stream));
-    *perm_out = perm;
-    return MDET_OK;
-}
-
-// Prefilter items for the MFMA kernel: (row block, column begin, column end),
-// each row block's columns from its diagonal in segments of seg columns.
-// With one queue (row-block major) the survivor-heavy diagonal item of every
-// row block is one of ~n/seg items in flight; with per-XCD queues (column
-// start major within a queue of every 8th row block) the diagonal items still
-// come spread over time and XCDs, while an XCD's blocks share column ranges
-// in its L2: memory-side traffic 19.4 -> 3.5 GB and 10% faster at 200k
-// contigs.  (An earlier column-major order with one block per item and an
-// XCD-aware block map ran the diagonal items back to back on one XCD: 8%
-// slower.)
+// Scan items over the whole triangle: (row block of `rows`, column begin,
+// column end), each row block's columns from its diagonal in segments of seg
+// columns.  With one queue (row-block major) the survivor-heavy diagonal item
+// of every row block is one of ~n/seg items in flight; with per-XCD queues
+// (column start major within a queue of every 8th row block) the diagonal
+// items still come spread over time and XCDs, while an XCD's blocks share
+// column ranges in its L2: memory-side traffic 19.4 -> 3.5 GB and 10% faster
+// at 200k contigs in the full Gram over 256-row blocks.
 // Default column span by size: the power of two nearest n / 100 in [512,
 // 4096] (the autotuner's picks measured at 50k, 200k and 1M contigs were
 // 512, 2048 and 4096, with persistent blocks).
@@ -2183,9 +2219,10 @@ uint32_t seg_cols_for(uint32_t n) {
 // rb with rb % PF_QUEUES == q), each ordered by column start then row block,
 // so the blocks of one XCD work on neighbouring column ranges together;
 // qbounds[0..PF_QUEUES] delimit the lists.
-int build_items(mdet_ctx* ctx, uint32_t n_pad, uint32_t seg, uint32_t order, uint4** items_dev, uint32_t* nitems,
-                uint32_t** qbounds_dev) {
-    if (ctx->items_npad == n_pad && ctx->items_seg == seg && ctx->items_order == order && ctx->nitems) {
+int build_items(mdet_ctx* ctx, uint32_t n, uint32_t rows, uint32_t seg, uint32_t order, uint4** items_dev,
+                uint32_t* nitems, uint32_t** qbounds_dev) {
+    if (ctx->items_n == n && ctx->items_rows == rows && ctx->items_seg == seg && ctx->items_order == order &&
+        ctx->nitems) {
         auto it = ctx->bufs.find("pairs.items");
         auto iq = ctx->bufs.find("pairs.item_qb");
         if (it != ctx->bufs.end() && iq != ctx->bufs.end()) {
@@ -2197,10 +2234,10 @@ int build_items(mdet_ctx* ctx, uint32_t n_pad, uint32_t seg, uint32_t order, uin
     }
     std::vector<uint4> items;
     std::vector<uint32_t> qb(PF_QUEUES + 1, 0);
-    const uint32_t nrb = n_pad / M_ROWS;
+    const uint32_t nrb = (n + rows - 1) / rows;
     auto row_items = [&](uint32_t rb, std::vector<uint4>& v) {
-        for (uint32_t c = rb * M_ROWS; c < n_pad; c += seg)
-            v.push_back(make_uint4(rb * M_ROWS, rb * M_ROWS + M_ROWS, c, std::min<uint32_t>(c + seg, n_pad) | ITEM_TRI));
+        for (uint32_t c = rb * rows; c < n; c += seg)
+            v.push_back(make_uint4(rb * rows, std::min(rb * rows + rows, n), c, std::min<uint32_t>(c + seg, n) | ITEM_TRI));
     };
     if (order == 0) {
         for (uint32_t rb = 0; rb < nrb; ++rb) row_items(rb, items);
@@ -2216,6 +2253,7 @@ int build_items(mdet_ctx* ctx, uint32_t n_pad, uint32_t seg, uint32_t order, uin
         qb[PF_QUEUES] = (uint32_t)items.size();
     }
     *nitems = (uint32_t)items.size();
+    ctx->nitems = 0;  // not cached until the upload is queued
     MDET_TRY(ctx_buf(ctx, "pairs.items", items.size(), items_dev));
     MDET_TRY(ctx_buf(ctx, "pairs.item_qb", PF_QUEUES + 1, qbounds_dev));
     MDET_HIP(hipMemcpyAsync(*items_dev, items.data(), items.size() * sizeof(uint4), hipMemcpyHostToDevice,
@@ -2223,20 +2261,45 @@ int build_items(mdet_ctx* ctx, uint32_t n_pad, uint32_t seg, uint32_t order, uin
     MDET_HIP(hipMemcpyAsync(*qbounds_dev, qb.data(), qb.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
                             ctx->stream));
     MDET_HIP(hipStreamSynchronize(ctx->stream));
-    ctx->items_npad = n_pad;
+    ctx->items_n = n;
+    ctx->items_rows = rows;
     ctx->items_seg = seg;
     ctx->items_order = order;
     ctx->nitems = *nitems;
     return MDET_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-}  // extern "C"
-
-namespace {
+// Counters of one edge-list call (64-bit words of the zeroed block; the first
+// CTR_HOST are copied to the host together).
+enum : uint32_t {
+    CTR_MM = 0,      // k_prep_rows: log-size range, out-of-domain count
+    CTR_LIST = 3,    // listed tiles (everything from here on is cleared for a repeated pass)
+    CTR_CAND,        // candidate records
+    CTR_KEPT,        // kept candidates ...
+    CTR_ADJ,         // ... and the ones decided in FP64 (k_adjudicate: the word after CTR_KEPT)
+    CTR_AMB,         // tie-band list lengths, first pass and fallback
+    CTR_AMB2,
+    CTR_FULL,        // full rows of the fallback
+    CTR_FB_LIST,     // its listed tiles
+    CTR_SURV,        // tiles with survivors, first pass and fallback
+    CTR_FB_SURV,
+    CTR_ERR,         // select flags
+    CTR_CAPPED,      // capped rows
+    CTR_BIG,         // rows for the block-wide and the global-memory selection
+    CTR_HUGE,
+    CTR_EDGES,       // edges
+    CTR_HOST,
+    CTR_QUEUES = 24, // scan queues: PF_QUEUES counters PF_CTR_STRIDE 32-bit words apart
+    CTR_FB_QUEUE = CTR_QUEUES + PF_QUEUES * PF_CTR_STRIDE / 2,
+    CTR_WORDS = CTR_FB_QUEUE + 8,
+};
+static_assert(CTR_HOST <= CTR_QUEUES, "counter layout");
+constexpr int PREP_EVENT = 6;  // context event index marking the log-size range's copy
+// Exhaustive modes up to this many contigs skip the row order and the first
+// pass: every tile goes to the second one.
+constexpr uint32_t DIRECT_MAX = 6144;
+// Resident refinement blocks per CU at most (39 KiB of LDS each).
+constexpr uint32_t REFINE_PER_CU = 4;
 
 int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, uint32_t n, double cutoff,
                uint32_t max_edges, int precision, mdet_mlp* mlp, float radius2, uint32_t n_clusters,
@@ -2267,37 +2330,50 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
     Timer tm{ctx, 0};
     MDET_TRY(tm.record(0));
 
-    // -- prep rows
+    // -- counters and per-call arrays that start at zero, in one allocation:
+    // CTR_WORDS counters (64-bit), then kept endpoints per select bucket, the
+    // buckets' fill cursors, and the edges per row
+    const uint32_t nb = (n + S_BUCKET - 1) / S_BUCKET;
+    unsigned long long* ctr;
+    const size_t zero_words = 2 * (size_t)CTR_WORDS + (nb + 1) + nb + ((size_t)n + 1);
+    MDET_TRY(ctx_buf(ctx, "pairs.zero", (zero_words + 1) / 2, &ctr));
+    uint32_t* bcnt = reinterpret_cast<uint32_t*>(ctr + CTR_WORDS);
+    uint32_t* bcur = bcnt + nb + 1;
+    uint32_t* out_cnt = bcur + nb;
+    MDET_HIP(hipMemsetAsync(ctr, 0, zero_words * 4, ctx->stream));
+
+    // -- prep rows: the log sizes' range goes to the host, which finds the
+    // radius while the device orders the rows
     float* tvec;
-    unsigned long long* mm;
     MDET_TRY(ctx_buf(ctx, "pairs.tvec", n, &tvec));
-    MDET_TRY(ctx_buf(ctx, "pairs.mm", 8, &mm));
-    {
-        unsigned long long init[4] = {~0ull, 0ull, 0ull, 0ull};
-        void* st_host;
-        MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-        memcpy(st_host, init, sizeof init);
-        MDET_HIP(hipMemcpyAsync(mm, st_host, sizeof init, hipMemcpyHostToDevice, ctx->stream));
-    }
-    unsigned int* bad = reinterpret_cast<unsigned int*>(mm + 2);
-    hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, mm, bad);
+    hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, ctr + CTR_MM);
     MDET_HIP(hipGetLastError());
-    unsigned long long mmh[3];
-    {
-        void* st_host;
-        MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-        MDET_HIP(hipMemcpyAsync(st_host, mm, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));
-        MDET_HIP(hipStreamSynchronize(ctx->stream));
-        memcpy(mmh, st_host, sizeof mmh);
-    }
-    if ((unsigned int)mmh[2] != 0)
+    void* stage_host;
+    MDET_TRY(ctx_host_stage(ctx, 8 * CTR_HOST, &stage_host));
+    unsigned long long* host = static_cast<unsigned long long*>(stage_host);
+    hipEvent_t prep_done;
+    MDET_TRY(ctx_event(ctx, PREP_EVENT, &prep_done));
+    MDET_HIP(hipMemcpyAsync(host, ctr + CTR_MM, 3 * 8, hipMemcpyDeviceToHost, ctx->stream));
+    MDET_HIP(hipEventRecord(prep_done, ctx->stream));
+    // small inputs: every 32 x 32 tile of the triangle goes straight to the
+    // second pass, in contig order
+    const bool gram_all = precision != MDET_LEARNED;  // the exhaustive modes
+    const bool direct = gram_all && n <= DIRECT_MAX;
+    const bool cluster = precision == MDET_LEARNED && n_probe > 0;
+    ProjOrder order;
+    if (!direct && !cluster)
+        MDET_TRY(proj_order(ctx, tnf_dev, n,
+                            precision == MDET_BF16_REFINE ? PROJ_BF16 : precision == MDET_F16_REFINE ? PROJ_F16 : PROJ_F32,
+                            &order));
+    MDET_HIP(hipEventSynchronize(prep_done));
+    if (host[2] != 0)
         MDET_FAIL(MDET_E_RANGE,
                   "mdet_tnf_edges: %u log sizes outside [log10 1500, log10 500000] (contigs shorter than 1500 "
                   "are not allowed in the graph)",
-                  (unsigned int)mmh[2]);
+                  (unsigned int)host[2]);
     double xlo, xhi;
     {
-        long long a = (long long)mmh[0], b = (long long)mmh[1];
+        const unsigned long long a = ~host[0], b = host[1];
         memcpy(&xlo, &a, 8);
         memcpy(&xhi, &b, 8);
     }
@@ -2324,516 +2400,372 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
     mdet_edges result{0, nullptr, nullptr, nullptr};
 
     if (R > 0) {
-        // -- prefilter
-        const uint32_t n_pad = (n + M_ROWS - 1) / M_ROWS * M_ROWS;
-        unsigned long long *scnt, *soff, *sstat, *rc;
-        MDET_TRY(ctx_buf(ctx, "pairs.shard_cnt", (size_t)NSHARD * SHARD_STRIDE, &scnt));
-        MDET_TRY(ctx_buf(ctx, "pairs.shard_off", (size_t)NSHARD + 1, &soff));
-        MDET_TRY(ctx_buf(ctx, "pairs.stat", 8, &sstat));
-        rc = sstat + 4;  // [4] kept candidates [5] FP64-adjudicated [6] [7] tie-band list lengths
-        uint64_t shard_cap = std::max<uint64_t>(2048, ((uint64_t)n * 256) / NSHARD);
-        auto it_cap = ctx->bufs.find("pairs.sbuf");
-        if (it_cap != ctx->bufs.end())
-            shard_cap = std::max<uint64_t>(shard_cap, it_cap->second.bytes / sizeof(uint2) / NSHARD);
-        uint2 *sbuf = nullptr, *surv = nullptr;
-        uint32_t* perm = nullptr;  // sorted position -> contig id (MFMA modes)
-        uint64_t ns = 0;
-        // MFMA modes: chunked survivor output, listed item by item afterwards
-        const bool chunked = precision != MDET_EXACT_F32;
-        uint64_t chunk_cap = 64;
-        if (auto it = ctx->bufs.find("pairs.cmeta"); it != ctx->bufs.end())
-            chunk_cap = std::max<uint64_t>(chunk_cap, it->second.bytes / sizeof(uint2) / NSHARD);
-        ChunkOut co{};
-        uint32_t *ckey = nullptr, *cslot = nullptr;
-        uint32_t items_launched = 0;
-        const uint4* tile_items = nullptr;  // row-block items: survivor chunks sorted by tile
-        uint64_t nchunks = 0;
-        // a wave flushes once per item it has survivors in, plus once per
-        // M_STAGE survivors; sized for ~128 survivors per contig at first
         const mdet_ctx::Tune tune = ctx->tune[precision];
-        // persistent prefilter: the resident blocks (8 waves per CU) pull items
-        // from a counter, or with per-XCD queues (qbounds) each from its
-        // queue's counter (the grid then covers every queue: a multiple of
-        // PF_QUEUES blocks)
-        uint32_t* pf_ctr = nullptr;
-        uint32_t* qbounds = nullptr;
-        auto pf_grid = [&](uint32_t nitems, int waves) {
-            const uint32_t resident = (uint32_t)ctx->num_cus * (8 / waves);
-            if (!pf_ctr) return dim3(nitems);
-            if (qbounds) return dim3((std::max<uint32_t>(resident, PF_QUEUES) + PF_QUEUES - 1) / PF_QUEUES * PF_QUEUES);
-            return dim3(std::min<uint32_t>(nitems, resident));
-        };
-        auto chunk_out = [&](uint32_t nitems, int attempt) -> int {
-            if (tune.persistent) {
-                MDET_TRY(ctx_buf(ctx, "pairs.item_ctr", PF_QUEUES * PF_CTR_STRIDE, &pf_ctr));
-                MDET_HIP(hipMemsetAsync(pf_ctr, 0, PF_QUEUES * PF_CTR_STRIDE * 4, ctx->stream));
-            }
-            if (attempt == 0)
-                chunk_cap = std::max<uint64_t>(
-                    chunk_cap, ((uint64_t)nitems * 4 + (uint64_t)n * 128 / M_STAGE) / NSHARD * 5 / 4 + 16);
-            MDET_TRY(ctx_buf(ctx, "pairs.cbuf", (size_t)NSHARD * chunk_cap * M_STAGE, &co.buf));
-            MDET_TRY(ctx_buf(ctx, "pairs.cmeta", (size_t)NSHARD * chunk_cap, &co.meta));
-            MDET_TRY(ctx_buf(ctx, "pairs.ckey", (size_t)NSHARD * chunk_cap, &ckey));
-            MDET_TRY(ctx_buf(ctx, "pairs.cslot", (size_t)NSHARD * chunk_cap, &cslot));
-            co.cnt = scnt;
-            co.cap = chunk_cap;
-            items_launched = nitems;
-            return MDET_OK;
-        };
-        IvfIndex ivf;  // learned mode with probes
-        uint4 *frag = nullptr, *frag_a = nullptr;  // learned mode: the fragments (and where full rows go)
-        uint32_t frag_rows = 0;
-        // FP32 rows in the prefilter's order for refinement (MFMA modes)
-        float *tnfs = nullptr, *tvs = nullptr;
-        bool rows_sorted = false;
-        auto sort_rows = [&]() -> int {
-            if (rows_sorted) return MDET_OK;
-            MDET_TRY(ctx_buf(ctx, "pairs.tnfs", (size_t)n_pad * NT, &tnfs));
-            MDET_TRY(ctx_buf(ctx, "pairs.tvs", (size_t)n_pad, &tvs));
-            hipLaunchKernelGGL(k_sort_rows, dim3(n_pad / 4), dim3(256), 0, ctx->stream, tnf_dev, tvec, perm, n, n_pad,
-                               tnfs, tvs);
-            rows_sorted = true;
-            return MDET_OK;
-        };
-        // squared-distance bound of the BF16/FP16 Gram prefilter: |d~ - d| <=
-        // |a~ - a| + |b~ - b| <= 2u for unit rows (u = unit roundoff of the
-        // format), plus FP32 accumulation slack
-        auto gram_r2 = [&](bool bf) {
-            const double u = bf ? 1.0 / 256.0 : 1.0 / 2048.0;
-            const double Rm = R + 2.0 * u * 1.0001 + 2e-4;
-            return (float)(Rm * Rm) + 1e-4f;
-        };
-        for (int attempt = 0; attempt < 2; ++attempt) {
-            MDET_HIP(hipMemsetAsync(scnt, 0, (size_t)NSHARD * SHARD_STRIDE * 8, ctx->stream));
-            MDET_HIP(hipMemsetAsync(sstat, 0, 8 * 8, ctx->stream));
-            if (precision == MDET_EXACT_F32) {
-                MDET_TRY(ctx_buf(ctx, "pairs.sbuf", (size_t)NSHARD * shard_cap, &sbuf));
-                const SurvOut so{sbuf, scnt, (unsigned long long)shard_cap};
-                float* tnft;
-                MDET_TRY(ctx_buf(ctx, "pairs.tnft", (size_t)NT * n_pad, &tnft));
-                hipLaunchKernelGGL(k_prep_f32t, dim3(n_pad / 64), dim3(256), 0, ctx->stream, tnf_dev, n, n_pad, tnft);
-                if (attempt == 0) MDET_TRY(tm.record(1));
-                const uint32_t ntiles = n_pad / F_T;
-                const uint64_t ntri = (uint64_t)ntiles * (ntiles + 1) / 2;
+        const bool bf = precision != MDET_F16_REFINE;      // format of the Gram
+        const bool f32 = precision == MDET_EXACT_F32;
+        const bool tnf_gram = !(radius2 > 0.f);            // Gram of the TNF rows (else of embeddings)
+        // exact cover: the cluster pairs that can hold a pair within
+        // the radius R (TNF-space triangle bound) instead of probes;
+        // then no row can miss a partner and no row is completed
+        const bool exact_cover = cluster && tnf_gram && ctx->learned_exact_cover;
+        // rows per scan item, and the rows padded to whole blocks
+        const uint32_t item_rows = gram_all ? scan_rows(PROJ_RT) : ITEM_ROWS;
+        const uint32_t n_pad = (n + item_rows - 1) / item_rows * item_rows;
+        // distance below which the Gram must keep every pair, and the distance
+        // beyond which the second pass keeps none: the FP32 mode's own bound,
+        // or what the Gram adds to its radius: its slack (2 GRAM_SLACK (|x|^2 +
+        // 1) on the square for unit rows) here, and twice each row's rounding
+        // in the row's own margin
+        const float gram_r = (float)(R * (1.0 + 1e-6)) + 1e-5f;
+        const float f32_r2 = (float)(R * R * (1.0 + 1e-4)) + 1e-6f;
+        const float reach = std::sqrt(f32 ? f32_r2 : gram_r * gram_r + 4.4f * GRAM_SLACK) * (1.f + 1e-5f) + 1e-6f;
 
-                const float R2 = (float)(R * R * (1.0 + 1e-4)) + 1e-6f;
-                const unsigned grid = (unsigned)std::min<uint64_t>(ntri, 1u << 22);
-                hipLaunchKernelGGL(k_prefilter_f32, dim3(grid), dim3(256), 0, ctx->stream, tnft, n, n_pad, ntiles, ntri,
-                                   R2, so);
-            } else if (precision == MDET_LEARNED) {
-                // embedding rows (n x 32) in BF16, threshold = calibrated radius^2;
-                // with probes, only the pairs of probed cluster pairs (items of
-                // the cluster index), else every pair in composition order.
-                // radius2 == 0 with probes: the BF16 TNF Gram (as BF16_REFINE)
-                // decides within the probed cluster pairs instead of the
-                // embedding radius.
-                const bool tnf_gram = n_probe && radius2 == 0.f;
-                // exact cover: the cluster pairs that can hold a pair within
-                // the radius R (TNF-space triangle bound) instead of probes;
-                // then no row can miss a partner and no row is completed
-                const bool exact_cover = tnf_gram && ctx->learned_exact_cover;
-                float* emb;
-                MDET_TRY(ctx_buf(ctx, "learn.emb", (size_t)n * 32, &emb));
-                if (attempt == 0) {
-                    if (exact_cover)
-                        MDET_TRY(ivf_cover_space(ctx, tnf_dev, n, emb));
-                    else
-                        MDET_TRY(mdet_mlp_embed(mlp, tnf_dev, n, emb));
-                    if (n_probe) MDET_TRY(ivf_launch(ctx, emb, n, n_clusters, n_probe, exact_cover, &ivf));
-                }
-                // cluster items start column steps anywhere: room for one more
-                // block; with the TNF Gram also for the fallback's full rows,
-                // appended after the first n_frag
-                const uint32_t n_frag = n_probe ? n_pad + ITEM_ROWS : n_pad;
-                const uint32_t n_alloc = tnf_gram ? n_frag + n_pad : n_frag;
-                MDET_TRY(ctx_buf(ctx, "learn.frag", (size_t)n_alloc / 32 * (tnf_gram ? KS : KS_E) * 64, &frag));
-                MDET_TRY(ctx_buf(ctx, "learn.frag_a", (size_t)n_alloc / 32 * 64, &frag_a));
-                frag_rows = n_frag;
-                if (n_probe)
-                    perm = ivf.perm;
-                else
-                    MDET_TRY(sort_by_composition(ctx, tnf_dev, n, &perm));
-                if (tnf_gram)
-                    hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), dim3(n_frag / 4), dim3(256), 0, ctx->stream,
-                                       tnf_dev, perm, n, n_frag, gram_r2(true), frag, frag_a);
-                else
-                    hipLaunchKernelGGL((k_prep_lowp<true, 32, KS_E, true>), dim3(n_frag / 4), dim3(256), 0, ctx->stream,
-                                       emb, perm, n, n_frag, radius2, frag, frag_a);
-                if (n_probe && attempt == 0) {
-                    MDET_TRY(sort_rows());         // device work queued behind the index copies ...
-                    // the cover's radius: every pair the BF16 prefilter can keep
-                    // (|a~ - b~|^2 below its bound; |d - d~| <= 2u for unit rows)
-                    if (exact_cover)
-                        MDET_TRY(ivf_cover(ctx, frag, tnfs, n, std::sqrt((double)gram_r2(true)) + 2.0 / 256.0 + 1e-4,
-                                           &ivf));
-                    MDET_TRY(ivf_finish(ctx, &ivf));  // ... runs while the host builds the items
-                }
-                uint4* items = ivf.items_dev;
-                uint32_t nitems = ivf.nitems;
-                if (!n_probe)
-                    MDET_TRY(build_items(ctx, n_pad, tune.seg_cols ? tune.seg_cols : seg_cols_for(n), 0, &items,
-                                         &nitems, &qbounds));
-                qbounds = nullptr;  // one queue
-                MDET_TRY(chunk_out(nitems, attempt));
-                if (attempt == 0) MDET_TRY(tm.record(1));
-                if (nitems && tnf_gram)
-                    hipLaunchKernelGGL((k_prefilter_mfma<true, KS>), pf_grid(nitems, 4), dim3(256), 0, ctx->stream,
-                                       frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, co);
-                else if (nitems && n_probe)  // cluster items: at most ITEM_ROWS rows
-                    hipLaunchKernelGGL((k_prefilter_mfma<true, KS_E>), pf_grid(nitems, 4), dim3(256), 0,
-                                       ctx->stream, frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, co);
-                else if (nitems)  // row-block items of M_ROWS rows
-                    hipLaunchKernelGGL((k_prefilter_mfma<true, KS_E, M_GRAM_WAVES>), pf_grid(nitems, M_GRAM_WAVES),
-                                       dim3(64 * M_GRAM_WAVES), 0, ctx->stream, frag, frag_a, items, nitems, pf_ctr,
-                                       (const uint32_t*)nullptr, co);
-            } else {
-                const bool bf = precision == MDET_BF16_REFINE;
-                const float R2 = gram_r2(bf);
-                uint4 *frag, *frag_a8;
-                MDET_TRY(ctx_buf(ctx, "pairs.frag", (size_t)n_pad / 32 * KS * 64, &frag));
-                MDET_TRY(ctx_buf(ctx, "pairs.frag_a8", (size_t)n_pad / 32 * 64, &frag_a8));
-                MDET_TRY(sort_by_composition(ctx, tnf_dev, n, &perm));
-                if (bf)
-                    hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), dim3(n_pad / 4), dim3(256), 0, ctx->stream, tnf_dev,
-                                       perm, n, n_pad, R2, frag, frag_a8);
-                else
-                    hipLaunchKernelGGL((k_prep_lowp<false, NT, KS>), dim3(n_pad / 4), dim3(256), 0, ctx->stream,
-                                       tnf_dev, perm, n, n_pad, R2, frag, frag_a8);
-                uint4* items;
-                uint32_t nitems;
-                const uint32_t order = tune.persistent ? tune.item_order : 0u;
-                MDET_TRY(build_items(ctx, n_pad, tune.seg_cols ? tune.seg_cols : seg_cols_for(n), order, &items,
-                                     &nitems, &qbounds));
-                tile_items = n_pad <= (1u << 26) ? items : nullptr;  // the tile key fits 32 bits
-                if (!order) qbounds = nullptr;
-                MDET_TRY(chunk_out(nitems, attempt));
-                if (attempt == 0) MDET_TRY(tm.record(1));
-                if (bf)
-                    hipLaunchKernelGGL((k_prefilter_mfma<true, KS, M_GRAM_WAVES>), pf_grid(nitems, M_GRAM_WAVES),
-                                       dim3(64 * M_GRAM_WAVES), 0, ctx->stream, frag, frag_a8, items, nitems, pf_ctr,
-                                       (const uint32_t*)qbounds, co);
-                else
-                    hipLaunchKernelGGL((k_prefilter_mfma<false, KS, M_GRAM_WAVES>), pf_grid(nitems, M_GRAM_WAVES),
-                                       dim3(64 * M_GRAM_WAVES), 0, ctx->stream, frag, frag_a8, items, nitems, pf_ctr,
-                                       (const uint32_t*)qbounds, co);
-            }
-            MDET_HIP(hipGetLastError());
-            if (attempt == 0) MDET_TRY(tm.record(2));
-            const uint64_t cap_now = chunked ? chunk_cap : shard_cap;
-            hipLaunchKernelGGL(k_shard_scan, dim3(1), dim3(1024), 0, ctx->stream, scnt, (unsigned long long)cap_now,
-                               soff, sstat);
-            if (chunked)
-                hipLaunchKernelGGL(k_chunk_list, dim3(NSHARD), dim3(256), 0, ctx->stream, co.meta,
-                                   (unsigned long long)chunk_cap, soff, tile_items, ckey, cslot, sstat + 2);
-            unsigned long long st2[3];
-            {
-                void* st_host;
-                MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-                MDET_HIP(hipMemcpyAsync(st_host, sstat, 24, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipStreamSynchronize(ctx->stream));
-                memcpy(st2, st_host, 24);
-            }
-            // st2: [0] entries (chunks if chunked) kept, [1] largest raw shard count, [2] chunked survivors
-            if (st2[1] <= cap_now) {
-                ns = chunked ? st2[2] : st2[0];
-                nchunks = chunked ? st2[0] : 0;
-                break;
-            }
-            if (attempt == 1) MDET_FAIL(MDET_E_STATE, "mdet_tnf_edges: survivor count grew between passes");
-            if (chunked)
-                chunk_cap = st2[1] + st2[1] / 4 + 16;
-            else
-                shard_cap = st2[1] + st2[1] / 4 + 64;
+        // -- fragments of the Gram in the scan's row order
+        uint32_t* perm = order.perm;  // position -> contig (null: itself)
+        uint4 *frag = nullptr, *frag_a = nullptr, *pfrag = nullptr, *pfrag_a = nullptr;
+        uint4* items = nullptr;
+        uint32_t nitems = 0;
+        uint32_t* qbounds = nullptr;
+        IvfIndex ivf;
+        const int ks = tnf_gram ? KS : KS_E;
+        // cluster items start column steps anywhere: room for one more block;
+        // with the TNF Gram also for the fallback's full rows, appended after
+        // the first n_frag
+        const uint32_t n_frag = cluster ? n_pad + ITEM_ROWS : n_pad;
+        const uint32_t n_alloc = cluster && tnf_gram ? n_frag + n_pad : n_frag;
+        if (!f32) {
+            MDET_TRY(ctx_buf(ctx, gram_all ? "pairs.frag" : "learn.frag", (size_t)n_alloc / 32 * ks * 64, &frag));
+            MDET_TRY(ctx_buf(ctx, gram_all ? "pairs.frag_a" : "learn.frag_a", (size_t)n_alloc / 32 * 64, &frag_a));
         }
-        MDET_TRY(ctx_buf(ctx, "pairs.surv", std::max<uint64_t>(ns, 1), &surv));
-        if (chunked && nchunks) {
-            // chunks in item order (stable within an item), then their entries packed
-            if (nchunks > 0x7fffffffull) MDET_FAIL(MDET_E_RANGE, "mdet_tnf_edges: too many survivor chunks");
-            uint32_t *ckey2, *cslot2, *ccnt;
-            uint64_t* coff;
-            MDET_TRY(ctx_buf(ctx, "pairs.ckey2", nchunks, &ckey2));
-            MDET_TRY(ctx_buf(ctx, "pairs.cslot2", nchunks, &cslot2));
-            MDET_TRY(ctx_buf(ctx, "pairs.ccnt", nchunks + 1, &ccnt));  // the scan reads one past the end
-            MDET_TRY(ctx_buf(ctx, "pairs.coff", nchunks + 1, &coff));
-            // key bits: item indices, or the tile key (16 + bits of n_pad / 1024)
-            const uint64_t key_range = tile_items ? ((uint64_t)(n_pad >> 10) + 1) << 16 : (uint64_t)items_launched;
-            int end_bit = 1;
-            while (end_bit < 32 && (1ull << end_bit) < key_range) ++end_bit;
-            size_t tmp = 0;
-            MDET_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, ckey, ckey2, cslot, cslot2, (int)nchunks, 0,
-                                                        end_bit, ctx->stream));
-            void* t;
-            MDET_TRY(ctx_buf(ctx, "cub.sorttmp", tmp, &t));
-            MDET_HIP(hipcub::DeviceRadixSort::SortPairs(t, tmp, ckey, ckey2, cslot, cslot2, (int)nchunks, 0, end_bit,
-                                                        ctx->stream));
-            hipLaunchKernelGGL(k_chunk_counts, dim3((unsigned)((nchunks + 255) / 256)), dim3(256), 0, ctx->stream,
-                               co.meta, cslot2, (uint32_t)nchunks, ccnt);
-            MDET_TRY(exclusive_scan_u32_to_u64(ctx, ccnt, coff, (uint32_t)nchunks));
-            hipLaunchKernelGGL(k_chunk_compact, dim3((unsigned)((nchunks + 3) / 4)), dim3(256), 0, ctx->stream, co.buf,
-                               cslot2, ccnt, coff, (uint32_t)nchunks, surv);
-        } else if (!chunked) {
-            hipLaunchKernelGGL(k_compact, dim3(NSHARD), dim3(256), 0, ctx->stream, sbuf,
-                               (unsigned long long)shard_cap, soff, surv);
+        const uint32_t seg = tune.seg_cols ? tune.seg_cols : seg_cols_for(n);
+        const dim3 fgrid(n_frag / 32);
+        if (gram_all) {
+            if (!f32 && bf)
+                hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), fgrid, dim3(256), 0, ctx->stream, tnf_dev, perm, n,
+                                   gram_r, frag, frag_a);
+            else if (!f32)
+                hipLaunchKernelGGL((k_prep_lowp<false, NT, KS>), fgrid, dim3(256), 0, ctx->stream, tnf_dev, perm, n,
+                                   gram_r, frag, frag_a);
+            if (!direct) {
+                MDET_TRY(ctx_buf(ctx, "pairs.pfrag", (size_t)n_pad / 32 * PROJ_KS * 64, &pfrag));
+                MDET_TRY(ctx_buf(ctx, "pairs.pfrag_a", (size_t)n_pad / 32 * 64, &pfrag_a));
+                MDET_TRY(proj_frags(ctx, order, n, n_pad, reach, pfrag, pfrag_a));
+                const uint32_t ord = tune.persistent ? tune.item_order : 0u;
+                MDET_TRY(build_items(ctx, n, item_rows, seg, ord, &items, &nitems, &qbounds));
+                if (!ord) qbounds = nullptr;
+            }
+        } else {
+            // embedding rows (n x 32) in BF16, threshold = calibrated radius^2;
+            // with probes, only the pairs of probed cluster pairs (items of
+            // the cluster index), else every pair.  radius2 == 0 with probes:
+            // the BF16 TNF Gram (as BF16_REFINE) decides within the probed
+            // cluster pairs instead of the embedding radius.
+            float* emb;
+            MDET_TRY(ctx_buf(ctx, "learn.emb", (size_t)n * 32, &emb));
+            if (exact_cover)
+                MDET_TRY(ivf_cover_space(ctx, tnf_dev, n, emb));
+            else
+                MDET_TRY(mdet_mlp_embed(mlp, tnf_dev, n, emb));
+            if (cluster) {
+                MDET_TRY(ivf_launch(ctx, emb, n, n_clusters, n_probe, exact_cover, &ivf));
+                perm = ivf.perm;
+            }
+            if (tnf_gram)
+                hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), fgrid, dim3(256), 0, ctx->stream, tnf_dev, perm, n,
+                                   gram_r, frag, frag_a);
+            else
+                hipLaunchKernelGGL((k_prep_lowp<true, 32, KS_E, true>), fgrid, dim3(256), 0, ctx->stream, emb, perm, n,
+                                   std::sqrt(radius2), frag, frag_a);
+            if (exact_cover) {
+                // FP32 rows in cluster order for the cover's passes
+                float* tnfs;
+                MDET_TRY(ctx_buf(ctx, "pairs.tnfs", (size_t)n_pad * NT, &tnfs));
+                hipLaunchKernelGGL(k_sort_rows, dim3(n_pad / 4), dim3(256), 0, ctx->stream, tnf_dev, perm, n, n_pad,
+                                   tnfs);
+                // the cover's radius: every pair the BF16 Gram can keep (unit
+                // rows: the rounding of one row is at most u = 1/256)
+                MDET_TRY(ivf_cover(ctx, frag, tnfs, n, (double)reach + 4.0 / 256.0 * 1.0001, &ivf));
+            }
+            if (cluster) {
+                MDET_TRY(ivf_finish(ctx, &ivf));
+                items = ivf.items_dev;
+                nitems = ivf.nitems;
+            } else {
+                MDET_TRY(build_items(ctx, n, item_rows, seg, 0, &items, &nitems, &qbounds));
+            }
+            qbounds = nullptr;  // one queue
+        }
+        uint32_t* iperm = nullptr;
+        if (perm) {
+            MDET_TRY(ctx_buf(ctx, "sel.iperm", (size_t)n, &iperm));
+            hipLaunchKernelGGL(k_iperm, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, perm, n, iperm);
         }
         MDET_HIP(hipGetLastError());
-        st.survivors = ns;
-        st.pairs_evaluated = (precision == MDET_LEARNED && n_probe) ? ivf.pairs : st.pairs_total;
+        st.pairs_evaluated = cluster ? ivf.pairs : st.pairs_total;
 
-
-        // -- refine (in place: cand[k] belongs to surv[k]); counts the kept
-        // candidates' endpoints per select bucket
-        Cand* cand;
-        MDET_TRY(ctx_buf(ctx, "pairs.cand", std::max<uint64_t>(ns, 1), &cand));
-        const uint32_t nb = (n + S_BUCKET - 1) / S_BUCKET;
-        uint32_t* bcnt;
-        MDET_TRY(ctx_buf(ctx, "sel.bcnt", (size_t)nb + 1, &bcnt));
-        MDET_HIP(hipMemsetAsync(bcnt, 0, ((size_t)nb + 1) * 4, ctx->stream));
-        if (ns) {
-            const float* rows = tnf_dev;
-            const float* tv = tvec;
-            if (perm) {  // MFMA modes: survivors are sorted positions
-                MDET_TRY(sort_rows());
-                rows = tnfs;
-                tv = tvs;
+        // -- both passes over the pairs and the selection, again with larger
+        // buffers if a list did not fit (its counter says how much it needs)
+        const uint64_t ntiles = (n + 31) / 32;
+        uint64_t list_cap = std::min<uint64_t>(ntiles * (ntiles + 1) / 2, std::max<uint64_t>(1u << 16, 8ull * n));
+        uint64_t surv_cap = direct ? ntiles * (ntiles + 1) / 2 : std::max<uint64_t>(1u << 16, 2ull * n);
+        uint64_t cand_cap = 128ull * n + 65536, fb_cap = 0;
+        if (auto it = ctx->bufs.find("pairs.tiles"); it != ctx->bufs.end())
+            list_cap = std::max<uint64_t>(list_cap, it->second.bytes / sizeof(uint4));
+        if (auto it = ctx->bufs.find("pairs.stiles"); it != ctx->bufs.end())
+            surv_cap = std::max<uint64_t>(surv_cap, it->second.bytes / sizeof(uint4));
+        if (auto it = ctx->bufs.find("pairs.cand"); it != ctx->bufs.end())
+            cand_cap = std::max<uint64_t>(cand_cap, it->second.bytes / sizeof(Cand));
+        for (int attempt = 0;; ++attempt) {
+            if (attempt == 4) MDET_FAIL(MDET_E_STATE, "mdet_tnf_edges: survivor count grew between passes");
+            if (attempt) MDET_HIP(hipMemsetAsync(ctr + CTR_LIST, 0, (zero_words - 2 * CTR_LIST) * 4, ctx->stream));
+            uint4* list = nullptr;
+            Cand* cand;
+            uint64_t* amb;
+            MDET_TRY(ctx_buf(ctx, "pairs.cand", cand_cap, &cand));
+            MDET_TRY(ctx_buf(ctx, "pairs.amb", cand_cap, &amb));
+            if (!direct) MDET_TRY(ctx_buf(ctx, "pairs.tiles", list_cap, &list));
+            // -- first pass: the tiles
+            MDET_TRY(tm.record(1));
+            if (!direct && nitems) {
+                // persistent blocks: the resident ones pull items from a
+                // counter, or with per-XCD queues (qbounds) each from its
+                // queue's counter (the grid then covers every queue)
+                uint32_t* pf_ctr = tune.persistent ? reinterpret_cast<uint32_t*>(ctr + CTR_QUEUES) : nullptr;
+                const TileList tl{list, ctr + CTR_LIST, (unsigned long long)list_cap};
+                auto grid = [&](uint32_t per_cu) {
+                    const uint32_t resident = (uint32_t)ctx->num_cus * per_cu;
+                    if (!pf_ctr) return dim3(nitems);
+                    if (qbounds)
+                        return dim3((std::max<uint32_t>(resident, PF_QUEUES) + PF_QUEUES - 1) / PF_QUEUES * PF_QUEUES);
+                    return dim3(std::min<uint32_t>(nitems, resident));
+                };
+                const dim3 block(64 * SCAN_WAVES);
+                if (gram_all)
+                    hipLaunchKernelGGL((k_tile_scan<false, PROJ_KS, PROJ_RT, PROJ_CT, 4>), grid(4), block, 0,
+                                       ctx->stream, pfrag, pfrag_a, items, nitems, pf_ctr, (const uint32_t*)qbounds, tl);
+                else if (tnf_gram)
+                    hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>), grid(2), block, 0, ctx->stream,
+                                       frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, tl);
+                else
+                    hipLaunchKernelGGL((k_tile_scan<true, KS_E, GRAM_RT, GRAM_CT, 4>), grid(4), block, 0, ctx->stream,
+                                       frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, tl);
+                MDET_HIP(hipGetLastError());
             }
-            uint64_t blocks = std::min<uint64_t>((ns + 63) / 64, (uint64_t)ctx->num_cus * tune.refine_blocks);
-            blocks = (blocks + 7) / 8 * 8;
-            uint64_t* amb_list;
-            MDET_TRY(ctx_buf(ctx, "pairs.amb", ns, &amb_list));
-            hipLaunchKernelGGL(k_refine, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, surv, ns, perm, rows, tv, T,
-                               cand, rc, bcnt, amb_list, rc + 2);
-            hipLaunchKernelGGL(k_adjudicate, dim3(2 * ctx->num_cus), dim3(256), 0, ctx->stream, surv, perm, rows,
-                               logsize_dev, T, rule, cutoff, amb_list, rc + 2, cand, rc, bcnt);
-            MDET_HIP(hipGetLastError());
-        }
-        // -- learned mode with the cluster index and the TNF Gram: the exact
-        // fallback for full rows
-        uint64_t ns2 = 0;
-        Cand* cand2 = nullptr;
-        if (precision == MDET_LEARNED && n_probe && radius2 == 0.f && max_edges > 0 && ns && ctx->learned_fallback &&
-            !ivf.exact) {
-            // rows whose proposals fill all but max_edges / margin_div of the
-            // slots (a row that missed more partners than that and still
-            // exceeds max_edges in truth can keep a wrong edge)
-            const uint32_t need = max_edges - max_edges / ctx->learned_margin_div;
-            uint32_t *kept, *full_pos, *full_ids, *n_full_dev;
-            uint8_t* full;
-            MDET_TRY(ctx_buf(ctx, "fb.kept", (size_t)n, &kept));
-            MDET_TRY(ctx_buf(ctx, "fb.full", (size_t)n, &full));
-            MDET_TRY(ctx_buf(ctx, "fb.pos", (size_t)n, &full_pos));
-            MDET_TRY(ctx_buf(ctx, "fb.ids", (size_t)n, &full_ids));
-            MDET_TRY(ctx_buf(ctx, "fb.nfull", 4, &n_full_dev));
-            MDET_HIP(hipMemsetAsync(kept, 0, (size_t)n * 4, ctx->stream));
-            hipLaunchKernelGGL(k_row_kept, dim3((unsigned)std::min<uint64_t>((ns + 255) / 256, 8u * ctx->num_cus)),
-                               dim3(256), 0, ctx->stream, surv, cand, ns, kept);
-            hipLaunchKernelGGL(k_full_flags, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, kept, n, need, full);
-            hipcub::CountingInputIterator<uint32_t> pos_it(0);
-            size_t tmp = 0;
-            MDET_HIP(hipcub::DeviceSelect::Flagged(nullptr, tmp, pos_it, full, full_pos, n_full_dev, (int)n,
-                                                   ctx->stream));
-            void* t;
-            MDET_TRY(ctx_buf(ctx, "cub.selecttmp", tmp, &t));
-            MDET_HIP(hipcub::DeviceSelect::Flagged(t, tmp, pos_it, full, full_pos, n_full_dev, (int)n, ctx->stream));
-            uint32_t n_full = 0;
-            {
-                void* st_host;
-                MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-                MDET_HIP(hipMemcpyAsync(st_host, n_full_dev, 4, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipStreamSynchronize(ctx->stream));
-                memcpy(&n_full, st_host, 4);
-            }
-            st.fallback_rows = n_full;
-            if (n_full) {
-                // the full rows' fragments after the first frag_rows rows
-                hipLaunchKernelGGL(k_gather_ids, dim3((n_full + 255) / 256), dim3(256), 0, ctx->stream, full_pos, perm,
-                                   n_full, full_ids);
-                const uint32_t n_fpad = (n_full + ITEM_ROWS - 1) / ITEM_ROWS * ITEM_ROWS;
-                hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), dim3(n_fpad / 4), dim3(256), 0, ctx->stream, tnf_dev,
-                                   full_ids, n_full, n_fpad, gram_r2(true), frag + (size_t)frag_rows / 32 * KS * 64,
-                                   frag_a + (size_t)frag_rows / 32 * 64);
-                // items: 256 full rows x 4096 columns, taken by resident blocks
-                // in column-segment-major order, so that the blocks in flight
-                // share a segment's column fragments in L2 (the full rows'
-                // fragments are the small, reused side)
-                constexpr uint32_t FB_SEG = 4096;
-                uint32_t w = 0;
-                const uint32_t nseg = (n + FB_SEG - 1) / FB_SEG;
-                void* hi;
-                MDET_TRY(ctx_host_buf(ctx, "fb.h_items", (size_t)(n_fpad / ITEM_ROWS) * nseg * sizeof(uint4), &hi));
-                uint4* hitems = static_cast<uint4*>(hi);
-                for (uint32_t c0 = 0; c0 < n; c0 += FB_SEG)
-                    for (uint32_t r0 = 0; r0 < n_full; r0 += ITEM_ROWS)
-                        hitems[w++] = make_uint4(frag_rows + r0, frag_rows + std::min(r0 + ITEM_ROWS, n_full), c0,
-                                                 std::min(c0 + FB_SEG, n));
-                st.pairs_evaluated += (uint64_t)n_full * (n - 1);  // some counted in phase one too
-                uint4* fitems;
-                MDET_TRY(ctx_buf(ctx, "fb.items", (size_t)w, &fitems));
-                MDET_HIP(hipMemcpyAsync(fitems, hitems, (size_t)w * sizeof(uint4), hipMemcpyHostToDevice, ctx->stream));
-                uint32_t* pbits;
-                const uint64_t nbits = (uint64_t)ivf.k * ivf.k;
-                MDET_TRY(ctx_buf(ctx, "fb.pbits", (size_t)(nbits + 31) / 32, &pbits));
-                MDET_HIP(hipMemsetAsync(pbits, 0, (size_t)(nbits + 31) / 32 * 4, ctx->stream));
-                hipLaunchKernelGGL(k_probed_bits, dim3((unsigned)(((uint64_t)ivf.k * ivf.n_probe + 255) / 256)),
-                                   dim3(256), 0, ctx->stream, ivf.probes_dev, ivf.k, ivf.n_probe, pbits);
-                uint32_t* fctr;
-                MDET_TRY(ctx_buf(ctx, "fb.item_ctr", 16, &fctr));
-                unsigned long long *fscnt, *fsoff, *fstat;
-                MDET_TRY(ctx_buf(ctx, "fb.shard_cnt", (size_t)NSHARD * SHARD_STRIDE, &fscnt));
-                MDET_TRY(ctx_buf(ctx, "fb.shard_off", (size_t)NSHARD + 1, &fsoff));
-                MDET_TRY(ctx_buf(ctx, "fb.stat", 8, &fstat));
-                uint64_t fcap = std::max<uint64_t>(64, ((uint64_t)w * 4 + (uint64_t)n_full * 16 / M_STAGE) / NSHARD + 16);
-                if (auto it = ctx->bufs.find("fb.cmeta"); it != ctx->bufs.end())
-                    fcap = std::max<uint64_t>(fcap, it->second.bytes / sizeof(uint2) / NSHARD);
-                uint64_t ocap = std::max<uint64_t>(1u << 16, (uint64_t)n_full * 32);
-                if (auto it = ctx->bufs.find("fb.pairs"); it != ctx->bufs.end())
-                    ocap = std::max<uint64_t>(ocap, it->second.bytes / sizeof(uint2));
-                uint2* surv2 = nullptr;
-                for (int attempt = 0; attempt < 3; ++attempt) {
-                    ChunkOut fco{};
-                    MDET_TRY(ctx_buf(ctx, "fb.cbuf", (size_t)NSHARD * fcap * M_STAGE, &fco.buf));
-                    MDET_TRY(ctx_buf(ctx, "fb.cmeta", (size_t)NSHARD * fcap, &fco.meta));
-                    MDET_TRY(ctx_buf(ctx, "fb.pairs", ocap, &surv2));
-                    fco.cnt = fscnt;
-                    fco.cap = fcap;
-                    MDET_HIP(hipMemsetAsync(fscnt, 0, (size_t)NSHARD * SHARD_STRIDE * 8, ctx->stream));
-                    MDET_HIP(hipMemsetAsync(fstat, 0, 8 * 8, ctx->stream));
-                    MDET_HIP(hipMemsetAsync(fctr, 0, 64, ctx->stream));
-                    const uint32_t resident = (uint32_t)ctx->num_cus * 2;
-                    hipLaunchKernelGGL((k_prefilter_mfma<true, KS>), dim3(std::min(w, resident)), dim3(256), 0,
-                                       ctx->stream, frag, frag_a, fitems, w, fctr, (const uint32_t*)nullptr, fco);
-                    hipLaunchKernelGGL(k_shard_scan, dim3(1), dim3(1024), 0, ctx->stream, fscnt, (unsigned long long)fcap,
-                                       fsoff, fstat);
-                    hipLaunchKernelGGL(k_fb_collect, dim3(NSHARD), dim3(256), 0, ctx->stream, fco, full_pos, frag_rows,
-                                       full, ivf.cluster_dev, pbits, ivf.k, surv2, (uint64_t)ocap, fstat + 4);
-                    MDET_HIP(hipGetLastError());
-                    unsigned long long fh[5];
-                    void* st_host;
-                    MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-                    MDET_HIP(hipMemcpyAsync(st_host, fstat, 40, hipMemcpyDeviceToHost, ctx->stream));
-                    MDET_HIP(hipStreamSynchronize(ctx->stream));
-                    memcpy(fh, st_host, 40);
-                    // fh[1]: largest shard's chunk count, fh[0]: chunks, fh[4]: pairs collected
-                    const bool chunks_fit = fh[1] <= fcap, pairs_fit = fh[4] <= ocap;
-                    if (chunks_fit && pairs_fit) {
-                        ns2 = fh[4];
-                        st.fallback_chunks = fh[0];
-                        break;
-                    }
-                    if (attempt == 2) MDET_FAIL(MDET_E_STATE, "mdet_tnf_edges_learned: fallback output grew between passes");
-                    if (!chunks_fit) fcap = fh[1] + fh[1] / 4 + 16;
-                    if (chunks_fit && !pairs_fit) ocap = fh[4] + fh[4] / 8 + 64;
-                }
-                st.fallback_pairs = ns2;
-                if (ns2) {
-                    MDET_TRY(ctx_buf(ctx, "fb.cand", ns2, &cand2));
-                    uint64_t blocks = std::min<uint64_t>((ns2 + 63) / 64, (uint64_t)ctx->num_cus * tune.refine_blocks);
-                    blocks = (blocks + 7) / 8 * 8;
-                    uint64_t* amb2;
-                    MDET_TRY(ctx_buf(ctx, "fb.amb", ns2, &amb2));
-                    hipLaunchKernelGGL(k_refine, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, surv2, ns2, perm,
-                                       tnfs, tvs, T, cand2, rc, bcnt, amb2, rc + 3);
-                    hipLaunchKernelGGL(k_adjudicate, dim3(2 * ctx->num_cus), dim3(256), 0, ctx->stream, surv2, perm,
-                                       tnfs, logsize_dev, T, rule, cutoff, amb2, rc + 3, cand2, rc, bcnt);
-                    MDET_HIP(hipGetLastError());
-                }
-            }
-        }
-        MDET_TRY(tm.record(3));
-        // no host round trip here (outside the learned fallback): the select
-        // buffers are sized by the survivor count (a bound on the kept
-        // candidates), so the select stage queues behind k_refine; the kept
-        // and adjudicated counts are read with the select stage's flags
-        const uint64_t nc = ns + ns2;  // candidate records (kept ones flagged)
-        ctx->last_pairs = ns;
-        st.candidates = st.adjudicated = 0;
-
-        // -- select
-        uint32_t *bcur, *out_cnt, *iperm = nullptr;
-        uint64_t *boff, *eoff, *rbeg;
-        Ent* ent;
-        Adj* adj;
-        unsigned int* err;
-        unsigned long long* capped;
-        MDET_TRY(ctx_buf(ctx, "sel.bcur", (size_t)nb, &bcur));
-        MDET_TRY(ctx_buf(ctx, "sel.boff", (size_t)nb + 1, &boff));
-        MDET_TRY(ctx_buf(ctx, "sel.outcnt", (size_t)n + 1, &out_cnt));
-        MDET_TRY(ctx_buf(ctx, "sel.rbeg", (size_t)n, &rbeg));
-        MDET_TRY(ctx_buf(ctx, "sel.eoff", (size_t)n + 1, &eoff));
-        MDET_TRY(ctx_buf(ctx, "sel.ent", std::max<uint64_t>(2 * nc, 1), &ent));
-        MDET_TRY(ctx_buf(ctx, "sel.adj", std::max<uint64_t>(2 * nc, 1), &adj));
-        // err[0] flags, err[2..3] capped rows (u64)
-        MDET_TRY(ctx_buf(ctx, "sel.err", 8, &err));
-        capped = reinterpret_cast<unsigned long long*>(err + 2);
-        // rows for the block-wide path (big) and for the global-memory path (huge)
-        const uint32_t big_cap = std::min<uint32_t>(n, 1u << 20);
-        uint32_t *big, *huge;
-        MDET_TRY(ctx_buf(ctx, "sel.big", (size_t)BIG_REC * (big_cap + 1), &big));
-        MDET_TRY(ctx_buf(ctx, "sel.huge", (size_t)BIG_REC * (big_cap + 1), &huge));
-        MDET_HIP(hipMemsetAsync(big, 0, 4, ctx->stream));
-        MDET_HIP(hipMemsetAsync(huge, 0, 4, ctx->stream));
-        MDET_HIP(hipMemsetAsync(bcur, 0, (size_t)nb * 4, ctx->stream));
-        MDET_HIP(hipMemsetAsync(out_cnt, 0, ((size_t)n + 1) * 4, ctx->stream));
-        MDET_HIP(hipMemsetAsync(err, 0, 32, ctx->stream));
-        if (nc) {
-            if (perm) {
-                MDET_TRY(ctx_buf(ctx, "sel.iperm", (size_t)n, &iperm));
-                hipLaunchKernelGGL(k_iperm, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, perm, n, iperm);
-            }
-            // the fill's grid covers the pieces of its own list (see k_bucket_fill)
-            auto fill_blocks = [](uint64_t cnt) {
-                const uint64_t pieces = (cnt + 255) / 256;
-                return (unsigned)(pieces <= FILL_SPREAD ? pieces
-                                                        : (uint64_t)FILL_SPREAD * ((pieces + FILL_SPREAD - 1) / FILL_SPREAD));
+            MDET_TRY(tm.record(2));
+            // -- second pass: the tiles' pairs
+            SurvTiles sv{nullptr, nullptr, ctr + CTR_SURV, (unsigned long long)surv_cap, ctr + CTR_CAND};
+            MDET_TRY(ctx_buf(ctx, "pairs.stiles", surv_cap, &sv.buf));
+            MDET_TRY(ctx_buf(ctx, "pairs.smask", surv_cap * 64, &sv.mask));
+            const RowArgs rows{tnf_dev, tvec, perm, n, nullptr, 0};
+            // persistent blocks over the device's counts (a multiple of 8: one
+            // XCD each in turn), no more than a small input has tiles for
+            auto work_grid = [&](uint64_t per_cu, uint64_t most) {
+                return dim3((unsigned)((std::min<uint64_t>(ctx->num_cus * per_cu, most) + 7) / 8 * 8));
             };
-            MDET_TRY(exclusive_scan_u32_to_u64(ctx, bcnt, boff, nb));
-            hipLaunchKernelGGL(k_bucket_fill, dim3(fill_blocks(ns)), dim3(256), 0, ctx->stream, cand, ns, iperm, boff,
-                               bcur, ent);
-            if (ns2)
-                hipLaunchKernelGGL(k_bucket_fill, dim3(fill_blocks(ns2)), dim3(256), 0, ctx->stream, cand2, ns2, iperm,
-                                   boff, bcur, ent);
-            hipLaunchKernelGGL(k_bucket_select, dim3(nb), dim3(S_THREADS), 0, ctx->stream, boff, ent, adj, n, max_edges,
-                               perm, tnf_dev, logsize_dev, out_cnt, rbeg, big, big_cap, err, capped);
-            hipLaunchKernelGGL(k_bigrow_select, dim3(ctx->num_cus), dim3(S_THREADS), 0, ctx->stream, big, big_cap, adj,
-                               max_edges, tnf_dev, logsize_dev, out_cnt, rbeg, huge, big_cap, err, capped);
-            MDET_HIP(hipGetLastError());
-            MDET_TRY(exclusive_scan_u32_to_u64(ctx, out_cnt, eoff, n));
-            // one round trip: select flags and capped rows, kept and adjudicated
-            // candidates (k_refine's counters), edge count, list lengths
-            unsigned long long errh[4], rch[2];
-            uint64_t ne;
-            uint32_t nbig, nhuge;
-            {
-                void* st_host;
-                MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-                char* h = static_cast<char*>(st_host);
-                MDET_HIP(hipMemcpyAsync(h, err, 32, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipMemcpyAsync(h + 32, rc, 16, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipMemcpyAsync(h + 48, eoff + n, 8, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipMemcpyAsync(h + 56, big, 4, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipMemcpyAsync(h + 60, huge, 4, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipStreamSynchronize(ctx->stream));
-                memcpy(errh, h, 32);
-                memcpy(rch, h + 32, 16);
-                memcpy(&ne, h + 48, 8);
-                memcpy(&nbig, h + 56, 4);
-                memcpy(&nhuge, h + 60, 4);
+            const uint64_t most = direct ? ntiles * (ntiles + 1) / 2 : ~0ull;
+            const dim3 ggrid = work_grid(8, most / 8 + 1);
+            const dim3 rgrid = work_grid(std::min<uint32_t>(tune.refine_blocks, REFINE_PER_CU), most);
+            GramArgs ga{};
+            ga.frag = frag;
+            ga.frag_a = frag_a;
+            ga.items = direct ? nullptr : items;
+            ga.whole = make_uint4(0, n, 0, n | ITEM_TRI);
+            ga.list = list;
+            ga.n_list = ctr + CTR_LIST;
+            ga.list_cap = list_cap;
+            ga.ntiles = (uint32_t)ntiles;
+            ga.out = sv;
+            if (f32) {
+                const F32Args fa{rows, list, ctr + CTR_LIST, (unsigned long long)list_cap, (uint32_t)ntiles, f32_r2, sv};
+                hipLaunchKernelGGL(k_tile_f32, rgrid, dim3(256), 0, ctx->stream, fa);
+            } else if (!tnf_gram) {
+                hipLaunchKernelGGL((k_tile_gram<true, KS_E, false>), ggrid, dim3(256), 0, ctx->stream, ga);
+            } else if (bf) {
+                hipLaunchKernelGGL((k_tile_gram<true, KS, false>), ggrid, dim3(256), 0, ctx->stream, ga);
+            } else {
+                hipLaunchKernelGGL((k_tile_gram<false, KS, false>), ggrid, dim3(256), 0, ctx->stream, ga);
             }
-            st.candidates = rch[0];
-            st.adjudicated = rch[1];
-            if ((unsigned int)errh[0] & 4u)
+            RefineArgs ra{rows, sv, (float)T, cand, (unsigned long long)cand_cap, ctr + CTR_KEPT, bcnt, amb, ctr + CTR_AMB};
+            hipLaunchKernelGGL(k_tile_refine, rgrid, dim3(256), 0, ctx->stream, ra);
+            const dim3 agrid(2 * ctx->num_cus);
+            hipLaunchKernelGGL(k_adjudicate, agrid, dim3(256), 0, ctx->stream, tnf_dev, logsize_dev, iperm, T, rule,
+                               cutoff, amb, ctr + CTR_AMB, cand, ctr + CTR_KEPT, bcnt);
+            MDET_HIP(hipGetLastError());
+            // what a list needed, from the counters at host[]: true if the pass has to run again
+            auto too_small = [&]() {
+                bool again = false;
+                auto grow = [&](unsigned long long need, uint64_t& cap) {
+                    if (need > cap) cap = need + need / 4 + 64, again = true;
+                };
+                if (!direct) grow(host[CTR_LIST], list_cap);
+                grow(std::max(host[CTR_SURV], host[CTR_FB_SURV]), surv_cap);
+                grow(host[CTR_FB_LIST], fb_cap);
+                grow(host[CTR_CAND], cand_cap);
+                return again;
+            };
+            // -- learned mode with the cluster index and the TNF Gram: the exact
+            // fallback for full rows
+            uint64_t ns1 = 0;
+            const bool fallback = cluster && tnf_gram && max_edges > 0 && ctx->learned_fallback && !ivf.exact;
+            if (fallback) {
+                // rows whose proposals fill all but max_edges / margin_div of the
+                // slots (a row that missed more partners than that and still
+                // exceeds max_edges in truth can keep a wrong edge)
+                const uint32_t need = max_edges - max_edges / ctx->learned_margin_div;
+                uint32_t *kept, *full_pos, *full_ids;
+                uint8_t* full;
+                MDET_TRY(ctx_buf(ctx, "fb.kept", (size_t)n, &kept));
+                MDET_TRY(ctx_buf(ctx, "fb.full", (size_t)n, &full));
+                MDET_TRY(ctx_buf(ctx, "fb.pos", (size_t)n, &full_pos));
+                MDET_TRY(ctx_buf(ctx, "fb.ids", (size_t)n, &full_ids));
+                uint32_t* n_full_dev = reinterpret_cast<uint32_t*>(ctr + CTR_FULL);
+                MDET_HIP(hipMemsetAsync(kept, 0, (size_t)n * 4, ctx->stream));
+                hipLaunchKernelGGL(k_row_kept, dim3(8u * ctx->num_cus), dim3(256), 0, ctx->stream, cand, ctr + CTR_CAND,
+                                   (unsigned long long)cand_cap, iperm, kept);
+                hipLaunchKernelGGL(k_full_flags, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, kept, n, need, full);
+                hipcub::CountingInputIterator<uint32_t> pos_it(0);
+                size_t tmp = 0;
+                MDET_HIP(hipcub::DeviceSelect::Flagged(nullptr, tmp, pos_it, full, full_pos, n_full_dev, (int)n,
+                                                       ctx->stream));
+                void* t;
+                MDET_TRY(ctx_buf(ctx, "cub.selecttmp", tmp, &t));
+                MDET_HIP(hipcub::DeviceSelect::Flagged(t, tmp, pos_it, full, full_pos, n_full_dev, (int)n, ctx->stream));
+                MDET_HIP(hipMemcpyAsync(host, ctr, 8 * CTR_HOST, hipMemcpyDeviceToHost, ctx->stream));
+                MDET_HIP(hipStreamSynchronize(ctx->stream));
+                if (too_small()) continue;
+                ns1 = host[CTR_CAND];
+                const uint32_t n_full = ns1 ? (uint32_t)host[CTR_FULL] : 0;
+                st.fallback_rows = n_full;
+                if (n_full) {
+                    // the full rows' fragments after the first n_frag rows
+                    hipLaunchKernelGGL(k_gather_ids, dim3((n_full + 255) / 256), dim3(256), 0, ctx->stream, full_pos,
+                                       perm, n_full, full_ids);
+                    const uint32_t n_fpad = (n_full + ITEM_ROWS - 1) / ITEM_ROWS * ITEM_ROWS;
+                    hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), dim3(n_fpad / 32), dim3(256), 0, ctx->stream,
+                                       tnf_dev, full_ids, n_full, gram_r, frag + (size_t)n_frag / 32 * KS * 64,
+                                       frag_a + (size_t)n_frag / 32 * 64);
+                    // items: 256 full rows x 4096 columns, taken by resident blocks
+                    // in column-segment-major order, so that the blocks in flight
+                    // share a segment's column fragments in L2 (the full rows'
+                    // fragments are the small, reused side)
+                    constexpr uint32_t FB_SEG = 4096;
+                    uint32_t w = 0;
+                    const uint32_t nseg = (n + FB_SEG - 1) / FB_SEG;
+                    void* hi;
+                    MDET_TRY(ctx_host_buf(ctx, "fb.h_items", (size_t)(n_fpad / ITEM_ROWS) * nseg * sizeof(uint4), &hi));
+                    uint4* hitems = static_cast<uint4*>(hi);
+                    for (uint32_t c0 = 0; c0 < n; c0 += FB_SEG)
+                        for (uint32_t r0 = 0; r0 < n_full; r0 += ITEM_ROWS)
+                            hitems[w++] = make_uint4(n_frag + r0, n_frag + std::min(r0 + ITEM_ROWS, n_full), c0,
+                                                     std::min(c0 + FB_SEG, n));
+                    uint4* fitems;
+                    MDET_TRY(ctx_buf(ctx, "fb.items", (size_t)w, &fitems));
+                    MDET_HIP(hipMemcpyAsync(fitems, hitems, (size_t)w * sizeof(uint4), hipMemcpyHostToDevice,
+                                            ctx->stream));
+                    uint32_t* pbits;
+                    const uint64_t nbits = (uint64_t)ivf.k * ivf.k;
+                    MDET_TRY(ctx_buf(ctx, "fb.pbits", (size_t)(nbits + 31) / 32, &pbits));
+                    MDET_HIP(hipMemsetAsync(pbits, 0, (size_t)(nbits + 31) / 32 * 4, ctx->stream));
+                    hipLaunchKernelGGL(k_probed_bits, dim3((unsigned)(((uint64_t)ivf.k * ivf.n_probe + 255) / 256)),
+                                       dim3(256), 0, ctx->stream, ivf.probes_dev, ivf.k, ivf.n_probe, pbits);
+                    fb_cap = std::max<uint64_t>(fb_cap, std::max<uint64_t>(1u << 16, 64ull * n_full));
+                    if (auto it = ctx->bufs.find("fb.tiles"); it != ctx->bufs.end())
+                        fb_cap = std::max<uint64_t>(fb_cap, it->second.bytes / sizeof(uint4));
+                    uint4* flist;
+                    uint64_t* amb2;
+                    MDET_TRY(ctx_buf(ctx, "fb.tiles", fb_cap, &flist));
+                    MDET_TRY(ctx_buf(ctx, "fb.amb", cand_cap, &amb2));
+                    const TileList tl{flist, ctr + CTR_FB_LIST, (unsigned long long)fb_cap};
+                    hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>),
+                                       dim3(std::min<uint32_t>(w, (uint32_t)ctx->num_cus * 2)), dim3(64 * SCAN_WAVES),
+                                       0, ctx->stream, frag, frag_a, fitems, w,
+                                       reinterpret_cast<uint32_t*>(ctr + CTR_FB_QUEUE), (const uint32_t*)nullptr, tl);
+                    // its survivor tiles after the first phase's are worked off
+                    sv.cnt = ctr + CTR_FB_SURV;
+                    ga.items = fitems;
+                    ga.list = flist;
+                    ga.n_list = ctr + CTR_FB_LIST;
+                    ga.list_cap = fb_cap;
+                    ga.out = sv;
+                    ga.full_pos = full_pos;
+                    ga.full_base = n_frag;
+                    ga.full = full;
+                    ga.cl = ivf.cluster_dev;
+                    ga.bits = pbits;
+                    ga.k = ivf.k;
+                    ra.in = sv;
+                    ra.amb = amb2;
+                    ra.amb_cnt = ctr + CTR_AMB2;
+                    ra.rows.full_pos = full_pos;
+                    ra.rows.full_base = n_frag;
+                    hipLaunchKernelGGL((k_tile_gram<true, KS, true>), ggrid, dim3(256), 0, ctx->stream, ga);
+                    hipLaunchKernelGGL(k_tile_refine, rgrid, dim3(256), 0, ctx->stream, ra);
+                    hipLaunchKernelGGL(k_adjudicate, agrid, dim3(256), 0, ctx->stream, tnf_dev, logsize_dev, iperm, T,
+                                       rule, cutoff, amb2, ctr + CTR_AMB2, cand, ctr + CTR_KEPT, bcnt);
+                    MDET_HIP(hipGetLastError());
+                }
+            }
+            MDET_TRY(tm.record(3));
+
+            // -- select: no host round trip up to the edges; every buffer is
+            // sized by the candidates' capacity
+            uint64_t *boff, *eoff, *rbeg;
+            Ent* ent;
+            Adj* adj;
+            MDET_TRY(ctx_buf(ctx, "sel.boff", (size_t)nb + 1, &boff));
+            MDET_TRY(ctx_buf(ctx, "sel.rbeg", (size_t)n, &rbeg));
+            MDET_TRY(ctx_buf(ctx, "sel.eoff", (size_t)n + 1, &eoff));
+            MDET_TRY(ctx_buf(ctx, "sel.ent", 2 * cand_cap, &ent));
+            MDET_TRY(ctx_buf(ctx, "sel.adj", 2 * cand_cap, &adj));
+            unsigned int* err = reinterpret_cast<unsigned int*>(ctr + CTR_ERR);
+            unsigned long long* capped = ctr + CTR_CAPPED;
+            // rows for the block-wide path (big) and for the global-memory path (huge)
+            const uint32_t big_cap = std::min<uint32_t>(n, 1u << 20);
+            uint32_t *big_rec, *huge_rec;
+            MDET_TRY(ctx_buf(ctx, "sel.big", (size_t)BIG_REC * big_cap, &big_rec));
+            MDET_TRY(ctx_buf(ctx, "sel.huge", (size_t)BIG_REC * big_cap, &huge_rec));
+            const RowList big{big_rec, reinterpret_cast<uint32_t*>(ctr + CTR_BIG), big_cap};
+            const RowList huge{huge_rec, reinterpret_cast<uint32_t*>(ctr + CTR_HUGE), big_cap};
+            uint32_t *from, *to;
+            float* s;
+            MDET_TRY(ctx_buf(ctx, "out.from", cand_cap, &from));
+            MDET_TRY(ctx_buf(ctx, "out.to", cand_cap, &to));
+            MDET_TRY(ctx_buf(ctx, "out.s", cand_cap, &s));
+            MDET_TRY(exclusive_scan_u32_to_u64(ctx, bcnt, boff, nb));
+            const uint64_t pieces = (cand_cap + 255) / 256;
+            hipLaunchKernelGGL(k_bucket_fill, dim3((unsigned)std::min<uint64_t>(pieces, 16u * ctx->num_cus)), dim3(256),
+                               0, ctx->stream, cand, ctr + CTR_CAND, (unsigned long long)cand_cap, iperm, boff, bcur,
+                               ent);
+            hipLaunchKernelGGL(k_bucket_select, dim3(nb), dim3(S_THREADS), 0, ctx->stream, boff, ent, adj, n, max_edges,
+                               perm, tnf_dev, logsize_dev, out_cnt, rbeg, big, err, capped);
+            hipLaunchKernelGGL(k_bigrow_select, dim3(ctx->num_cus), dim3(S_THREADS), 0, ctx->stream, big, adj,
+                               max_edges, tnf_dev, logsize_dev, out_cnt, rbeg, huge, err, capped);
+            MDET_HIP(hipGetLastError());
+            auto emit = [&]() -> int {
+                MDET_TRY(exclusive_scan_u32_to_u64(ctx, out_cnt, eoff, n));
+                hipLaunchKernelGGL(k_emit, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, rbeg, adj, out_cnt, eoff, n,
+                                   from, to, s, ctr + CTR_EDGES);
+                MDET_HIP(hipGetLastError());
+                MDET_HIP(hipMemcpyAsync(host, ctr, 8 * CTR_HOST, hipMemcpyDeviceToHost, ctx->stream));
+                MDET_TRY(tm.record(4));
+                MDET_HIP(hipStreamSynchronize(ctx->stream));
+                return MDET_OK;
+            };
+            MDET_TRY(emit());
+            if (too_small()) continue;
+            if ((unsigned int)host[CTR_ERR] & 4u)
                 MDET_FAIL(MDET_E_CAPACITY, "mdet_tnf_edges: more than %u rows need the block-wide selection", big_cap);
-            if ((unsigned int)errh[0] & 8u)
+            if ((unsigned int)host[CTR_ERR] & 8u)
                 MDET_FAIL(MDET_E_CAPACITY, "mdet_tnf_edges: more than %u rows need the global-memory selection",
                           big_cap);
-            st.rows_block = std::min(nbig, big_cap);
-            st.rows_global = nhuge;
+            const uint32_t nhuge = (uint32_t)host[CTR_HUGE];
             if (nhuge) {
                 // rows beyond the LDS capacities: sort them in global scratch
                 uint32_t* rec_h;
                 MDET_TRY(ctx_host_buf(ctx, "sel.huge_h", (size_t)BIG_REC * 4 * nhuge, (void**)&rec_h));
                 uint64_t* soff_h;
                 MDET_TRY(ctx_host_buf(ctx, "sel.huge_off_h", (size_t)8 * nhuge, (void**)&soff_h));
-                MDET_HIP(hipMemcpyAsync(rec_h, huge + BIG_REC, (size_t)BIG_REC * 4 * nhuge, hipMemcpyDeviceToHost,
+                MDET_HIP(hipMemcpyAsync(rec_h, huge_rec, (size_t)BIG_REC * 4 * nhuge, hipMemcpyDeviceToHost,
                                         ctx->stream));
                 MDET_HIP(hipStreamSynchronize(ctx->stream));
                 uint64_t total = 0;
@@ -2853,37 +2785,31 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 MDET_TRY(ctx_buf(ctx, "sel.huge_pre", total, &spre));
                 MDET_TRY(ctx_buf(ctx, "sel.huge_off", nhuge, &soff));
                 MDET_HIP(hipMemcpyAsync(soff, soff_h, (size_t)8 * nhuge, hipMemcpyHostToDevice, ctx->stream));
-                hipLaunchKernelGGL(k_hugerow_select, dim3(nhuge), dim3(HUGE_THREADS), 0, ctx->stream, huge, soff, adj,
-                                   max_edges, tnf_dev, logsize_dev, sk64, sk32, sv, spre, out_cnt, rbeg, capped);
+                hipLaunchKernelGGL(k_hugerow_select, dim3(nhuge), dim3(HUGE_THREADS), 0, ctx->stream, huge_rec, soff,
+                                   adj, max_edges, tnf_dev, logsize_dev, sk64, sk32, sv, spre, out_cnt, rbeg, capped);
                 MDET_HIP(hipGetLastError());
-                MDET_TRY(exclusive_scan_u32_to_u64(ctx, out_cnt, eoff, n));
-                void* st_host;
-                MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-                char* h = static_cast<char*>(st_host);
-                MDET_HIP(hipMemcpyAsync(h, err, 32, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipMemcpyAsync(h + 48, eoff + n, 8, hipMemcpyDeviceToHost, ctx->stream));
-                MDET_HIP(hipStreamSynchronize(ctx->stream));
-                memcpy(errh, h, 32);
-                memcpy(&ne, h + 48, 8);
+                MDET_TRY(emit());
             }
-            st.rows_capped = errh[1];
-            uint32_t *from, *to;
-            float* s;
-            MDET_TRY(ctx_buf(ctx, "out.from", std::max<uint64_t>(ne, 1), &from));
-            MDET_TRY(ctx_buf(ctx, "out.to", std::max<uint64_t>(ne, 1), &to));
-            MDET_TRY(ctx_buf(ctx, "out.s", std::max<uint64_t>(ne, 1), &s));
-            hipLaunchKernelGGL(k_emit, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, rbeg, adj, out_cnt, eoff, n, from,
-                               to, s);
-            MDET_HIP(hipGetLastError());
-            result = mdet_edges{ne, from, to, s};
+            st.survivors = ns1 ? ns1 : host[CTR_CAND];
+            st.fallback_pairs = ns1 ? host[CTR_CAND] - ns1 : 0;
+            st.fallback_chunks = host[CTR_FB_LIST];
+            st.pairs_evaluated += st.fallback_rows * (uint64_t)(n - 1);  // some counted in phase one too
+            st.candidates = host[CTR_KEPT];
+            st.adjudicated = host[CTR_ADJ];
+            st.rows_block = std::min<uint64_t>((uint32_t)host[CTR_BIG], big_cap);
+            st.rows_global = nhuge;
+            st.rows_capped = host[CTR_CAPPED];
+            ctx->last_pairs = st.survivors;
+            result = mdet_edges{host[CTR_EDGES], from, to, s};
+            break;
         }
     } else {
         MDET_TRY(tm.record(1));
         MDET_TRY(tm.record(2));
         MDET_TRY(tm.record(3));
+        MDET_TRY(tm.record(4));
+        MDET_HIP(hipEventSynchronize(ctx->events[4]));
     }
-    MDET_TRY(tm.record(4));
-    MDET_HIP(hipEventSynchronize(ctx->events[4]));
     st.ms_prefilter = tm.ms(1, 2);
     st.ms_refine = tm.ms(2, 3);
     st.ms_select = tm.ms(3, 4);
@@ -2951,9 +2877,9 @@ int mdet_tune_set(mdet_ctx* ctx, int precision, const mdet_tune* in) {
     MDET_TRY(check_ctx(ctx));
     if (precision < MDET_EXACT_F32 || precision > MDET_LEARNED || !in)
         MDET_FAIL(MDET_E_INVALID, "mdet_tune_set: bad precision %d or null input", precision);
-    if (in->seg_cols != 0 && (in->seg_cols < M_ROWS || in->seg_cols > 65536 || in->seg_cols % M_ROWS))
+    if (in->seg_cols != 0 && (in->seg_cols < ITEM_ROWS || in->seg_cols > 65536 || in->seg_cols % ITEM_ROWS))
         MDET_FAIL(MDET_E_RANGE, "mdet_tune_set: seg_cols %u is neither 0 nor a multiple of %d in [%d, 65536]",
-                  in->seg_cols, M_ROWS, M_ROWS);
+                  in->seg_cols, (int)ITEM_ROWS, (int)ITEM_ROWS);
     if (in->persistent > 1) MDET_FAIL(MDET_E_RANGE, "mdet_tune_set: persistent must be 0 or 1");
     if (in->refine_blocks < 1 || in->refine_blocks > 64)
         MDET_FAIL(MDET_E_RANGE, "mdet_tune_set: refine_blocks %u outside [1, 64]", in->refine_blocks);
@@ -3100,15 +3026,8 @@ int mdet_tnf_rowmax(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_d
     MDET_TRY(ctx_buf(ctx, "rm.mm", 8, &mm));
     MDET_TRY(ctx_buf(ctx, "rm.m32", n_sample, &m32));
     MDET_TRY(ctx_buf(ctx, "rm.m64", n_sample, &m64));
-    {
-        unsigned long long init[4] = {~0ull, 0ull, 0ull, 0ull};
-        void* st_host;
-        MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-        memcpy(st_host, init, sizeof init);
-        MDET_HIP(hipMemcpyAsync(mm, st_host, sizeof init, hipMemcpyHostToDevice, ctx->stream));
-    }
-    hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, mm,
-                       reinterpret_cast<unsigned int*>(mm + 2));
+    MDET_HIP(hipMemsetAsync(mm, 0, 32, ctx->stream));
+    hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, mm);
     unsigned long long bad = 0;
     MDET_TRY(read_scalar(ctx, mm + 2, &bad));
     if ((unsigned int)bad != 0)
@@ -3159,16 +3078,9 @@ int mdet_tnf_preprob(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_
     unsigned long long* mm;
     MDET_TRY(ctx_buf(ctx, "pp.tvec", n, &tvec));
     MDET_TRY(ctx_buf(ctx, "pp.mm", 8, &mm));
-    {
-        // [0] min, [1] max log size bits, [2] out-of-domain count, [3] bad indices
-        unsigned long long init[4] = {~0ull, 0ull, 0ull, 0ull};
-        void* st_host;
-        MDET_TRY(ctx_host_stage(ctx, 64, &st_host));
-        memcpy(st_host, init, sizeof init);
-        MDET_HIP(hipMemcpyAsync(mm, st_host, sizeof init, hipMemcpyHostToDevice, ctx->stream));
-    }
-    hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, mm,
-                       reinterpret_cast<unsigned int*>(mm + 2));
+    // [0..1] log-size range, [2] out-of-domain count, [3] bad indices
+    MDET_HIP(hipMemsetAsync(mm, 0, 32, ctx->stream));
+    hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, mm);
     hipLaunchKernelGGL(k_preprob_pairs, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, ctx->stream, tnf_dev,
                        logsize_dev, tvec, n, pi_dev, pj_dev, np, pre32_dev, pre64_dev,
                        reinterpret_cast<unsigned int*>(mm + 3));
