@@ -144,7 +144,7 @@ __device__ inline float dist2_f32(const float* __restrict__ a, const float* __re
 // cuda/Cuda2.cu:192-241 compiled with fused multiply-add contraction:
 // float differences and squares accumulated in double, every "acc + c*m" of
 // the polynomials and "b + c*d" one fma, monomials as plain products.
-__device__ double model64(const float* __restrict__ a, const float* __restrict__ b, double r1, double r2) {
+__device__ inline double dist2_f64(const float* __restrict__ a, const float* __restrict__ b) {
 #pragma clang fp contract(off)
     double d = 0;
     for (int i = 0; i < NT; ++i) {
@@ -152,7 +152,13 @@ __device__ double model64(const float* __restrict__ a, const float* __restrict__
         float sq = diff * diff;
         d += (double)sq;
     }
-    d = sqrt(d);
+    return d;
+}
+
+// preProb from the squared distance.
+__device__ double model64_d2(double d2, double r1, double r2) {
+#pragma clang fp contract(off)
+    const double d = sqrt(d2);
     double lw[19];
     lw[0] = r1 < r2 ? r1 : r2;
     lw[1] = r1 < r2 ? r2 : r1;
@@ -193,6 +199,10 @@ __device__ double model64(const float* __restrict__ a, const float* __restrict__
         if (pre > MODEL_FLOOR_PREPROB) pre = MODEL_FLOOR_PREPROB;
     }
     return pre;
+}
+
+__device__ double model64(const float* __restrict__ a, const float* __restrict__ b, double r1, double r2) {
+    return model64_d2(dist2_f64(a, b), r1, r2);
 }
 
 // Order-preserving maps of floats and doubles to unsigned integers (for
@@ -379,12 +389,17 @@ __device__ inline uint4 pack8(const uint16_t* h) {
 // One block per 32-row tile: the rows (perm: position -> row; null: itself)
 // pass through LDS once, so reads and the 16-byte fragment writes are both
 // whole lines.
+// With err: no share, acc = -|a~ - b~|^2 / 2 of the pair, err[row] = e; rows
+// that hold a value that is not finite become padding with err = NaN, and a
+// finite row of squared norm above PLAIN_NORM2 sets *outside.
 constexpr float GRAM_SLACK = 5e-5f;
+constexpr float PLAIN_NORM2 = 1.05f;
 
 template <bool BF16, int D, int KSX, bool EMB = false>
 __global__ __launch_bounds__(256) void k_prep_lowp(const float* __restrict__ x, const uint32_t* __restrict__ perm,
                                                    uint32_t n, float R, uint4* __restrict__ frag,
-                                                   uint4* __restrict__ frag_a) {
+                                                   uint4* __restrict__ frag_a, float* __restrict__ err = nullptr,
+                                                   uint32_t* __restrict__ outside = nullptr) {
     static_assert(D + 6 <= 16 * KSX && D % 8 == 0, "no room for the threshold slots");
     constexpr int STR = D + 4;
     __shared__ __align__(16) float X[32][STR];
@@ -399,26 +414,36 @@ __global__ __launch_bounds__(256) void k_prep_lowp(const float* __restrict__ x, 
     __syncthreads();
     {  // eight lanes a row: squared norms of the rounded and the given values
         const uint32_t r = tid >> 3, s = tid & 7, pos = t * 32 + r;
-        float part = 0.f, norm2 = 0.f, err2 = 0.f;
+        float part = 0.f, norm2 = 0.f, err2 = 0.f, nonfinite = 0.f;
         for (uint32_t k = s; k < (uint32_t)D; k += 8) {
             const float v = X[r][k], back = from_low<BF16>(to_low<BF16>(v));
             part = fmaf(back, back, part);
             norm2 = fmaf(v, v, norm2);
             err2 = fmaf(v - back, v - back, err2);
+            nonfinite += v * 0.f;
         }
 #pragma unroll
         for (int off = 4; off >= 1; off >>= 1) {
             part += __shfl_xor(part, off, 64);
             norm2 += __shfl_xor(norm2, off, 64);
             err2 += __shfl_xor(err2, off, 64);
+            nonfinite += __shfl_xor(nonfinite, off, 64);
         }
+        const bool pad = pos >= n || (err && nonfinite != 0.f);
+        if (pad)
+            for (uint32_t k = s; k < (uint32_t)D; k += 8) X[r][k] = 0.f;
         if (s == 0) {
             // padding rows get a large finite h (the split of +inf would be NaN)
             const float big = BF16 ? 1e30f : 6.0e4f;
             const float u = BF16 ? 1.0f / 256.0f : 1.0f / 2048.0f;
-            const float half_r = 0.5f * R + (EMB ? u * 1.0001f * sqrtf(norm2) : 1.001f * sqrtf(err2) + 1e-6f);
-            const float share = 2.0f * half_r * half_r + (EMB ? 1e-5f : GRAM_SLACK) * (norm2 + 1.0f);
-            float rem = (pos < n) ? fmaf(0.5f, part, -0.5f * share) : big;
+            const float e = EMB ? u * 1.0001f * sqrtf(norm2) : 1.001f * sqrtf(err2) + 1e-6f, half_r = 0.5f * R + e;
+            const float share =
+                err ? 0.f : 2.0f * half_r * half_r + (EMB ? 1e-5f : GRAM_SLACK) * (norm2 + 1.0f);
+            float rem = pad ? big : fmaf(0.5f, part, -0.5f * share);
+            if (err) {
+                err[pos] = pad ? __builtin_nanf("") : e;
+                if (!pad && norm2 > PLAIN_NORM2) *outside = 1u;
+            }
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 const uint16_t p = to_low<BF16>(rem);
@@ -514,6 +539,71 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Squared distances of 64 pairs of rows in FP64, the sums in the order of
+// dist2_f64: one pair a lane (all 64 lanes call; i, j < n also where the result
+// is not used).  The rows pass through LDS 32 floats at a time, read eight lanes
+// a row: whole 128-byte pieces instead of one 4-byte word of 64 rows per load.
+// A row i that the pair before has too is loaded once.  4.1M edges of 47,111
+// contigs (2.2 GB of rows j from the last-level cache, 7.8 TB/s): 287 us; one
+// row a lane took 497 us, pieces of 16 floats (twice the waves, half lines)
+// 341 us.  lds: DIST_LDS floats of the wave's own.
+constexpr int DIST_STR = 36;  // floats between rows: 16 lanes' 16-byte reads cover all banks
+constexpr int DIST_LDS = 128 * DIST_STR;
+constexpr int DIST_WAVES = 2;
+
+__device__ inline double wave_dist2_f64(const float* __restrict__ tnf, uint32_t i, uint32_t j, float* lds) {
+#pragma clang fp contract(off)
+    const uint32_t lane = lane_id(), sub = lane & 7, r0 = lane >> 3;
+    const uint32_t before = (uint32_t)__shfl_up((int)i, 1, 64);  // by all lanes: an inactive one gives 0
+    const uint64_t first = __ballot(lane == 0 || i != before);
+    const uint32_t lead = 63 - __builtin_clzll(first & (~0ull >> (63 - lane)));
+    uint32_t id[16];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        id[m] = (uint32_t)__shfl((int)i, (int)(r0 + 8 * m), 64);
+        id[m + 8] = (uint32_t)__shfl((int)j, (int)(r0 + 8 * m), 64);
+    }
+    f32x4_t v[16];
+    auto load = [&](uint32_t k) {
+#pragma unroll
+        for (int m = 0; m < 16; ++m)
+            if (m >= 8 || (first >> (r0 + 8 * m) & 1))
+                v[m] = *reinterpret_cast<const f32x4_t*>(tnf + (size_t)id[m] * NT + k + 4 * sub);
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int m = 0; m < 16; ++m)
+            if (m >= 8 || (first >> (r0 + 8 * m) & 1))
+                *reinterpret_cast<f32x4_t*>(lds + (r0 + 8 * m) * DIST_STR + 4 * sub) = v[m];
+    };
+    load(0);
+    const f32x4_t* a = reinterpret_cast<const f32x4_t*>(lds + lead * DIST_STR);
+    const f32x4_t* b = reinterpret_cast<const f32x4_t*>(lds + (64 + lane) * DIST_STR);
+    double d = 0;
+    auto add = [&](int q) {
+        const f32x4_t diff = a[q] - b[q], sq = diff * diff;
+        d += (double)sq.x;
+        d += (double)sq.y;
+        d += (double)sq.z;
+        d += (double)sq.w;
+    };
+#pragma unroll 1
+    for (uint32_t c = 0; c < 4; ++c) {
+        store();
+        wave_sync();
+        if (c < 3 || sub < 2) load(32 * (c + 1));  // the last piece: 8 floats
+#pragma unroll
+        for (int q = 0; q < 8; ++q) add(q);
+        wave_sync();
+    }
+    if (sub < 2) store();
+    wave_sync();
+    add(0);
+    add(1);
+    wave_sync();
+    return d;
 }
 
 // Tile list: entries (row tile, column tile, item, 0); the counter keeps
@@ -1999,12 +2089,372 @@ __global__ void k_emit(const uint64_t* __restrict__ rbeg, const Adj* __restrict_
 // ------------------------------------------------------------- row max --
 // Sampled row maxima of preProb (get_tnf_max_prob_sample, cuda/Cuda2.cu:
 // 281-314): for each sampled position p < n_sample, the maximum over all
-// positions q != p of preProb(idx[p], idx[q]).  Block = 64 sampled rows x a
-// chunk of columns; both sides staged K-major in LDS, each thread owns a 4x4
-// block of pairs: FP32 squared distance, FP32 model, running row maximum.
-// Pass 1 (EXACT=false) finds the FP32 maximum m32 of each row; pass 2
-// (EXACT=true) re-evaluates in FP64 every pair with FP32 preProb >= m32 - 2*EPS
-// (the true maximum is among them) and keeps their FP64 maximum.
+// positions q != p of preProb(idx[p], idx[q]).
+//
+// On MFMA: preProb falls with the distance for any two sizes, so bounds of a
+// pair's distance give bounds of its preProb.  A first scan takes each sampled
+// row's largest lower bound, a second lists the pairs whose upper bound reaches
+// it, and only those are evaluated in FP64 (k_rm_exact).  Per 32 x 32 tile of
+// pairs a scan forms three kinds of MFMA products of FP16 fragments:
+//   -|a~ - b~|^2 / 2   the TNF Gram (9 k-steps); the distance itself differs by
+//             the two rows' rounding errors (measured per row) and the FP32
+//             accumulation (RM_D2)
+//   b, c      the model's two polynomials of the sizes, preProb = -(b + c d):
+//             with one size's variable folded into the coefficients each is a
+//             dot product of 8 coefficients with the other's Chebyshev values,
+//             as hi + lo FP16 pairs (2 k-steps; ~1e-6 of preProb, ~4e-4 where
+//             subnormal parts are lost: EPS_PRE covers both)
+// Positions are ordered by size, so which side of a tile is the smaller one
+// (the model's x) is known for the whole tile; tiles around the diagonal run
+// both ways under a per-pair condition, which leaves out q = p as well.
+// RM_BEST1 bounds by model 1 alone (it applies above ln 9, where nearly every
+// row's maximum lies); RM_BEST2 adds model 2 for blocks that hold a row without
+// a pair above ln 9.  Block = 4 waves, a 32-row tile of sampled positions each
+// (fragments in registers), over a segment of tiles of all positions, streamed
+// through LDS in two buffers.  Bound by the VALU (a square root, three multiply-
+// adds, an addition and half a minimum per pair: ~90 us at 20,011^2 pairs) and
+// the 13 MFMAs a tile (65 us) beside each other.  All of 20,011 maxima: 0.55 ms
+// (172 us RM_BEST1, 45 RM_BEST2, 199 RM_LIST); the direct form alone took 20.2 ms
+// (FP32 differences and the whole model of every pair on the VALU, twice).
+// One buffer array with halves by index: 207, 60 and 248 us.
+// A finite row above PLAIN_NORM2 or more near-ties than the list holds leave
+// everything to k_rowmax.
+constexpr float RM_D2 = 4e-5f;  // |computed - exact| of |a~ - b~|^2 up to PLAIN_NORM2 (144 terms, 2^-24 each)
+constexpr int RM_PKS = 2;       // k-steps of a polynomial's product
+constexpr int RM_CHUNKS = KS + 2 * RM_PKS;  // 1 KiB chunks of a tile in LDS: Gram, b, c
+constexpr uint32_t RM_STAGE = 64;
+enum : int { RM_BEST1, RM_BEST2, RM_LIST };
+
+// Sort key of each position: its size, and itself as the value.
+__global__ __launch_bounds__(256) void k_rm_keys(const float* __restrict__ tvec, const uint64_t* __restrict__ idx,
+                                                 uint32_t m, uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= m) return;
+    key[p] = f2ord(tvec[(uint32_t)idx[p]]);
+    val[p] = p;
+}
+
+// Per element s of the order: its contig, and rank[position] = s.
+__global__ __launch_bounds__(256) void k_rm_contigs(const uint64_t* __restrict__ idx, const uint32_t* __restrict__ order,
+                                                    uint32_t m, uint32_t* __restrict__ contig,
+                                                    uint32_t* __restrict__ rank) {
+    const uint32_t s = blockIdx.x * 256 + threadIdx.x;
+    if (s >= m) return;
+    const uint32_t p = order[s];
+    contig[s] = (uint32_t)idx[p];
+    if (rank) rank[p] = s;
+}
+
+__device__ inline uint4 rm_pack(const _Float16* x) {
+    uint16_t h[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) h[k] = __builtin_bit_cast(uint16_t, x[k]);
+    return pack8(h);
+}
+
+// All positions: the 8 folded coefficients of polynomial p (b1 c1 b2 c2) in
+// role v (0: the position's is the smaller size), in the slots hi (k = 0..7),
+// lo (8..15), hi (16..23), 0; and per tile the largest rounding error (NaN
+// ones, of padding, aside).  Eight threads a position.
+__global__ __launch_bounds__(256) void k_rm_poly(const float* __restrict__ tvec, const uint32_t* __restrict__ contig,
+                                                 const float* __restrict__ err, uint32_t m,
+                                                 uint4* __restrict__ pfrag, float* __restrict__ tile_err) {
+    const uint32_t s = blockIdx.x * 32 + (threadIdx.x >> 3), v = (threadIdx.x >> 2) & 1, p = threadIdx.x & 3;
+    const float x = s < m ? tvec[contig[s]] : 0.f;
+    float T[MODEL_CX];
+    T[0] = 1.f;
+    T[1] = x;
+#pragma unroll
+    for (int k = 2; k < MODEL_CX; ++k) T[k] = fmaf(2.f * x, T[k - 1], -T[k - 2]);
+    _Float16 hi[8], lo[8], zero[8] = {};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        float f = 0.f;
+        if (v == 0) {
+            if (k < MODEL_CY)
+#pragma unroll
+                for (int a = 0; a < MODEL_CX; ++a) f = fmaf(c_cheb[p][a][k], T[a], f);
+        } else {
+#pragma unroll
+            for (int b = 0; b < MODEL_CY; ++b) f = fmaf(c_cheb[p][k][b], T[b], f);
+        }
+        hi[k] = (_Float16)f;
+        lo[k] = (_Float16)(f - (float)hi[k]);
+    }
+    uint4* dst = pfrag + (((size_t)blockIdx.x * 2 + v) * 4 + p) * RM_PKS * 64 + (s & 31);
+    dst[0] = dst[64] = rm_pack(hi);
+    dst[32] = rm_pack(lo);
+    dst[96] = rm_pack(zero);
+    if (threadIdx.x < 64) {
+        float e = threadIdx.x < 32 ? err[blockIdx.x * 32 + threadIdx.x] : 0.f;
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1) e = fmaxf(e, __shfl_xor(e, off, 64));
+        if (threadIdx.x == 0) tile_err[blockIdx.x] = e > 0.f ? e : 0.f;
+    }
+}
+
+// Sampled positions: the Chebyshev values, slots hi, hi, lo, 0.
+__global__ __launch_bounds__(256) void k_rm_cheb(const float* __restrict__ tvec, const uint32_t* __restrict__ contig,
+                                                 uint32_t m, uint32_t tiles, uint4* __restrict__ tfrag) {
+    const uint32_t s = blockIdx.x * 256 + threadIdx.x;
+    if (s >= tiles * 32) return;
+    const float x = s < m ? tvec[contig[s]] : 0.f;
+    float T[8];
+    T[0] = 1.f;
+    T[1] = x;
+    _Float16 hi[8], lo[8], zero[8] = {};
+#pragma unroll
+    for (int k = 2; k < 8; ++k) T[k] = fmaf(2.f * x, T[k - 1], -T[k - 2]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        hi[k] = (_Float16)T[k];
+        lo[k] = (_Float16)(T[k] - (float)hi[k]);
+    }
+    uint4* dst = tfrag + (size_t)(s >> 5) * RM_PKS * 64 + (s & 31);
+    dst[0] = dst[32] = rm_pack(hi);
+    dst[64] = rm_pack(lo);
+    dst[96] = rm_pack(zero);
+}
+
+struct RmArgs {
+    // all positions by size
+    const uint4 *frag, *frag_a, *pfrag;
+    const float* tile_err;
+    const uint32_t* order;
+    uint32_t n, tiles, seg;  // seg: tiles a block
+    // sampled positions by size
+    const uint4 *cfrag, *tfrag;
+    const float* cerr;
+    const uint32_t *corder, *rank;  // rank: of a position among all
+    uint32_t ns, ctiles;
+    uint32_t* best;  // per sampled element: largest lower bound (f2ord; 0: none)
+    uint2* list;     // (sampled element, position)
+    unsigned long long* n_list;
+    uint32_t cap;
+    const uint32_t* outside;
+};
+
+template <int PASS>
+__global__ __launch_bounds__(256, 3) void k_rm_scan(const RmArgs A) {
+    __shared__ uint4 R0[RM_CHUNKS * 64], R1[RM_CHUNKS * 64];
+    __shared__ uint2 stage_all[PASS == RM_LIST ? 4 : 1][RM_STAGE];
+    if (*A.outside) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t ct = 4 * blockIdx.x + wave, r0 = blockIdx.y * A.seg, r1 = min(A.tiles, r0 + A.seg);
+    const bool active = ct < A.ctiles;
+    const uint32_t col = 32 * ct + (lane & 31);
+    const bool in = active && col < A.ns;
+    const float ej = in ? A.cerr[col] : 0.f;
+    const bool have = in && ej == ej;
+    const float best = have && PASS != RM_BEST1 ? ord2f(A.best[col]) : 0.f;  // NaN: none
+    const bool low = have && PASS != RM_BEST1 && !(best > FLOOR32);           // model 2 may decide
+    bool need2 = false;
+    if (PASS == RM_BEST2) {
+        if (!__syncthreads_or(low)) return;
+    } else if (PASS == RM_LIST) {
+        need2 = __any(low);
+    }
+    uint4 B[KS], Tc[RM_PKS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) B[k] = active ? A.cfrag[((size_t)ct * KS + k) * 64 + lane] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < RM_PKS; ++k)
+        Tc[k] = active ? A.tfrag[((size_t)ct * RM_PKS + k) * 64 + lane] : make_uint4(0, 0, 0, 0);
+    const uint32_t rj = in ? A.rank[A.corder[col]] : 0u;
+    // ranks are ascending along the sampled elements
+    const uint32_t b_lo = A.rank[A.corder[128 * blockIdx.x]];
+    const uint32_t b_hi = A.rank[A.corder[min(128 * blockIdx.x + 127, A.ns - 1)]];
+    // role of tile rt's positions against the block's: 0 smaller, 1 larger, 2 both
+    auto role = [&](uint32_t rt) { return 32 * rt + 31 < b_lo ? 0 : 32 * rt > b_hi ? 1 : 2; };
+    constexpr int P0 = PASS == RM_BEST2 ? 2 : 0;  // polynomials in LDS: b1 c1, or b2 c2
+    auto poly = [&](uint32_t rt, int v, int p) {
+        return A.pfrag + (((size_t)rt * 2 + v) * 4 + p) * RM_PKS * 64;
+    };
+    auto fill = [&](uint32_t rt, uint4* buf) {
+        const uint4* pf = poly(rt, role(rt) == 1, P0);
+#pragma unroll
+        for (int m = 0; m < (RM_CHUNKS + 3) / 4; ++m) {
+            const int c = 4 * m + wave;
+            if (c < RM_CHUNKS) {
+                const uint4* src = c < KS - 1    ? A.frag + ((size_t)rt * KS + c) * 64
+                                   : c == KS - 1 ? A.frag_a + (size_t)rt * 64
+                                                 : pf + (c - KS) * 64;
+                __builtin_amdgcn_global_load_lds((const void*)(src + lane),
+                                                 (__attribute__((address_space(3))) void*)(buf + 64 * c), 16, 0, 0);
+            }
+        }
+    };
+    // in terms of w = -preProb: its smallest upper bound, and the listing limits
+    // of model 1 and model 2 (where the maximum is known to be ln 9 at least, only
+    // pairs that may lie above it)
+    const float nfloor = -FLOOR32, inf = __builtin_inff();
+    float wbest = inf, lim1 = 0.f, lim2 = 0.f;
+    if (PASS == RM_LIST) {
+        lim1 = have ? (best > FLOOR32 ? 2.f * EPS_PRE - best : nfloor + EPS_PRE) : -inf;
+        lim2 = have && best < FLOOR32 ? 2.f * EPS_PRE - best : -inf;
+    }
+    uint2* stage = stage_all[PASS == RM_LIST ? wave : 0];
+    uint32_t nst = 0;
+    auto flush = [&]() {
+        unsigned long long k = 0;
+        if (lane == 0) k = atomicAdd(A.n_list, (unsigned long long)nst);
+        k = lane0_u64(k);
+        wave_sync();
+        if ((uint32_t)lane < nst && k + lane < A.cap) A.list[k + lane] = stage[lane];
+        wave_sync();
+        nst = 0;
+    };
+    // the segment's largest rounding error: one a tile would have to be loaded
+    // in the loop, and waited for behind the fill
+    float E = 0.f;
+    for (uint32_t rt = r0 + lane; rt < r1; rt += 64) E = fmaxf(E, A.tile_err[rt]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) E = fmaxf(E, __shfl_xor(E, off, 64));
+    E += ej;
+    auto step = [&](const uint32_t rt, const uint4* R, uint4* next) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (rt + 1 < r1) fill(rt + 1, next);
+        if (!active) return;
+        const int ro = role(rt);
+        f32x16_t acc = f32x16_t{}, pb = f32x16_t{}, pc = f32x16_t{};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) acc = mfma32<false>(R[k * 64 + lane], B[k], acc);
+#pragma unroll
+        for (int k = 0; k < RM_PKS; ++k) {
+            pb = mfma32<false>(R[(KS + k) * 64 + lane], Tc[k], pb);
+            pc = mfma32<false>(R[(KS + RM_PKS + k) * 64 + lane], Tc[k], pc);
+        }
+        const uint32_t i0 = 32 * rt + 4 * (lane >> 5);
+        auto d_least = [&](float a) {
+            return fmaxf(__builtin_amdgcn_sqrtf(fmaxf(fmaf(-2.f, a, -RM_D2), 0.f)) - E, 0.f);
+        };
+        if (PASS == RM_LIST && ro != 2 && !need2) {
+            // most tiles hold no pair to list: all 16 at the shortest distance first
+            float near = acc[0], least = inf;
+#pragma unroll
+            for (int r = 1; r < 16; ++r) near = fmaxf(near, acc[r]);
+            const float dn = d_least(near);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) least = fminf(least, fmaf(pc[r], dn, pb[r]));
+            if (!__any(least <= lim1)) return;
+        }
+        float d[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            d[r] = PASS == RM_LIST ? d_least(acc[r]) : __builtin_amdgcn_sqrtf(fmaf(-2.f, acc[r], RM_D2)) + E;
+        uint32_t bits = 0;  // RM_LIST: pairs to list among this lane's 16
+        auto take = [&](const f32x16_t& b, const f32x16_t& c, uint32_t use, float lim) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float w = fmaf(c[r], d[r], b[r]);
+                if (PASS == RM_LIST)
+                    bits |= (w <= lim ? 1u : 0u) << r & use;
+                else
+                    wbest = fminf(wbest, use >> r & 1u ? w : inf);
+            }
+        };
+        // positions of this lane's 16 on one side of its own (not itself)
+        auto side = [&](bool larger) {
+            uint32_t use = 0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t i = i0 + (r & 3) + 8 * (r >> 2);
+                use |= (i < A.n && (larger ? i > rj : i < rj) ? 1u : 0u) << r;
+            }
+            return use;
+        };
+        auto product = [&](int v, int p) {
+            const uint4* f = poly(rt, v, p);
+            f32x16_t x = f32x16_t{};
+#pragma unroll
+            for (int k = 0; k < RM_PKS; ++k) x = mfma32<false>(f[k * 64 + lane], Tc[k], x);
+            return x;
+        };
+        if (ro != 2) {
+            take(pb, pc, 0xffffu, lim1);
+            if (PASS == RM_LIST && need2) take(product(ro, 2), product(ro, 3), 0xffffu, lim2);
+        } else {
+            take(pb, pc, side(false), lim1);
+            take(product(1, P0), product(1, P0 + 1), side(true), lim1);
+            if (PASS == RM_LIST && need2) {
+                take(product(0, 2), product(0, 3), side(false), lim2);
+                take(product(1, 2), product(1, 3), side(true), lim2);
+            }
+        }
+        if (PASS == RM_LIST) {
+            if (!__any(bits != 0)) return;
+            const uint32_t cnt = (uint32_t)__popc(bits), incl = wave_incl_sum_dpp(cnt);
+            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            uint32_t o = incl - cnt, done = 0;
+            while (done < total) {
+                const uint32_t took = min(RM_STAGE - nst, total - done);
+                while (bits && o < done + took) {
+                    const int r = __builtin_ctz(bits);
+                    bits &= bits - 1;
+                    const uint32_t i = i0 + (r & 3) + 8 * (r >> 2);
+                    stage[nst + (o - done)] = make_uint2(col, i < A.n ? A.order[i] : A.corder[col]);
+                    ++o;
+                }
+                nst += took;
+                done += took;
+                if (nst == RM_STAGE) flush();
+            }
+        }
+    };
+    // two arrays by name: of one array's halves the compiler cannot tell the
+    // fill's from the one read, and waits for the fill before the reads
+    fill(r0, R0);
+    for (uint32_t rt = r0; rt < r1; rt += 2) {
+        step(rt, R0, R1);
+        if (rt + 1 < r1) step(rt + 1, R1, R0);
+    }
+    if (PASS == RM_LIST) {
+        if (nst) flush();
+    } else {
+        wbest = fminf(wbest, __shfl_xor(wbest, 32, 64));
+        if (have && lane < 32 && wbest < inf) {
+            // model 1's bound counts where it certainly applies; model 2's is clamped to ln 9
+            if (PASS == RM_BEST1) {
+                if (wbest < nfloor - EPS_PRE) atomicMax(&A.best[col], f2ord(-wbest));
+            } else if (low) {
+                atomicMax(&A.best[col], f2ord(-fmaxf(wbest + EPS_PRE, nfloor)));
+            }
+        }
+    }
+}
+
+// FP64 preProb of the listed pairs, into each sampled position's maximum; a
+// maximum known to be ln 9 at least starts there.
+__global__ __launch_bounds__(64 * DIST_WAVES) void k_rm_exact(const RmArgs A, const float* __restrict__ tnf,
+                                                              const double* __restrict__ ls,
+                                                              const uint64_t* __restrict__ idx,
+                                                              unsigned long long* __restrict__ m64) {
+    __shared__ __align__(16) float X[DIST_WAVES][DIST_LDS];
+    const unsigned long long m = *A.n_list;
+    if (*A.outside || m > A.cap) return;
+    const uint32_t g = blockIdx.x * (64 * DIST_WAVES) + threadIdx.x, step = gridDim.x * (64 * DIST_WAVES);
+    for (uint32_t c = g; c < A.ns; c += step)
+        if (A.best[c] && ord2f(A.best[c]) == FLOOR32) atomicMax(&m64[A.corder[c]], d2ord(MODEL_FLOOR_PREPROB));
+    for (uint32_t k0 = g & ~63u; k0 < (uint32_t)m; k0 += step) {
+        const uint32_t k = k0 + (threadIdx.x & 63);
+        const bool in = k < (uint32_t)m;
+        const uint2 e = in ? A.list[k] : make_uint2(0, 0);
+        const uint32_t p = in ? A.corder[e.x] : 0u, i = in ? (uint32_t)idx[p] : 0u, j = in ? (uint32_t)idx[e.y] : 0u;
+        const double d2 = wave_dist2_f64(tnf, i, j, X[threadIdx.x >> 6]);
+        if (!in || p == e.y) continue;
+        const double v = model64_d2(d2, ls[i], ls[j]);
+        if (v == v) atomicMax(&m64[p], d2ord(v));
+    }
+}
+
+// The direct form, for small inputs and the ones the bounds do not cover (with
+// outside: only then).  Block = 64 sampled rows x a chunk of columns; both
+// sides staged K-major in LDS, each thread owns a 4x4 block of pairs: FP32
+// squared distance, FP32 model, running row maximum.  Pass 1 (EXACT=false)
+// finds the FP32 maximum m32 of each row; pass 2 (EXACT=true) re-evaluates in
+// FP64 every pair with FP32 preProb >= m32 - 2*EPS (the true maximum is among
+// them) and keeps their FP64 maximum.
 constexpr int RM_ROWS = 64, RM_COLS = 64, RM_CHUNK = 4096;
 
 
@@ -2012,7 +2462,10 @@ template <bool EXACT>
 __global__ __launch_bounds__(256) void k_rowmax(const float* __restrict__ tnf, const double* __restrict__ ls,
                                                 const float* __restrict__ tvec, const uint64_t* __restrict__ idx,
                                                 uint32_t n, uint32_t n_sample, uint32_t* __restrict__ m32,
-                                                unsigned long long* __restrict__ m64) {
+                                                unsigned long long* __restrict__ m64,
+                                                const uint32_t* __restrict__ outside,
+                                                const unsigned long long* __restrict__ n_list, uint32_t cap) {
+    if (outside && !*outside && *n_list <= cap) return;
     __shared__ float As[NT][RM_ROWS + 1];
     __shared__ float Bs[NT][RM_COLS + 1];
     __shared__ uint32_t rid[RM_ROWS], cid[RM_COLS];
@@ -2984,6 +3437,86 @@ int autotune_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev
     return MDET_OK;
 }
 
+// Up to here k_rowmax alone (one step of columns a block); from n = 300 on it
+// took 4x and more of the scans' time.
+constexpr uint32_t RM_DIRECT_MAX = 64;
+constexpr uint32_t RM_LIST_PER_ROW = 32;  // list capacity (2-5 a row measured)
+
+// The MFMA row maxima (see k_rm_scan): m64 of every sampled position unless
+// *outside is set or the list (its length: *n_list) overflows.
+int rowmax_mfma(mdet_ctx* ctx, const float* tnf_dev, const double* ls, const float* tvec, const uint64_t* idx,
+                uint32_t n, uint32_t ns, uint32_t* best, unsigned long long* m64, unsigned long long* n_list,
+                RmArgs* out) {
+    const hipStream_t s = ctx->stream;
+    const uint32_t tiles = (n + 31) / 32, ctiles = (ns + 31) / 32, m2 = ns == n ? 0 : ns;  // a second order
+    uint32_t *key, *val, *order, *contig, *rank;
+    uint4 *frag, *frag_a, *pfrag, *tfrag;
+    float *err, *tile_err;
+    const size_t all = (size_t)tiles * 32 + (m2 ? (size_t)ctiles * 32 : 0);
+    MDET_TRY(ctx_buf(ctx, "rm.key", 2 * (size_t)n, &key));
+    MDET_TRY(ctx_buf(ctx, "rm.val", n, &val));
+    MDET_TRY(ctx_buf(ctx, "rm.order", all, &order));
+    MDET_TRY(ctx_buf(ctx, "rm.contig", all, &contig));
+    MDET_TRY(ctx_buf(ctx, "rm.rank", n, &rank));
+    MDET_TRY(ctx_buf(ctx, "rm.frag", all * 2 * KS, &frag));
+    MDET_TRY(ctx_buf(ctx, "rm.frag_a", all * 2, &frag_a));
+    MDET_TRY(ctx_buf(ctx, "rm.err", all, &err));
+    MDET_TRY(ctx_buf(ctx, "rm.pfrag", (size_t)tiles * 2 * 4 * RM_PKS * 64, &pfrag));
+    MDET_TRY(ctx_buf(ctx, "rm.tile_err", tiles, &tile_err));
+    MDET_TRY(ctx_buf(ctx, "rm.tfrag", (size_t)ctiles * RM_PKS * 64, &tfrag));
+    RmArgs A{};
+    A.cap = RM_LIST_PER_ROW * ns;
+    MDET_TRY(ctx_buf(ctx, "rm.list", (size_t)A.cap, &A.list));
+    A.n_list = n_list;
+    uint32_t* outside = reinterpret_cast<uint32_t*>(n_list + 1);
+    A.outside = outside;
+    A.best = best;
+    auto sorted = [&](uint32_t m, uint32_t off, uint32_t* rk) -> int {
+        const dim3 g((m + 255) / 256), b(256);
+        hipLaunchKernelGGL(k_rm_keys, g, b, 0, s, tvec, idx, m, key, val);
+        size_t tmp = 0;
+        MDET_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, key, key + n, val, order + off, (int)m, 0, 32, s));
+        void* t;
+        MDET_TRY(ctx_buf(ctx, "cub.tmp", tmp, &t));
+        MDET_HIP(hipcub::DeviceRadixSort::SortPairs(t, tmp, key, key + n, val, order + off, (int)m, 0, 32, s));
+        hipLaunchKernelGGL(k_rm_contigs, g, b, 0, s, idx, order + off, m, contig + off, rk);
+        hipLaunchKernelGGL((k_prep_lowp<false, NT, KS>), dim3((m + 31) / 32), b, 0, s, tnf_dev, contig + off, m, 0.f,
+                           frag + (size_t)off * 2 * KS, frag_a + (size_t)off * 2, err + off, outside);
+        return MDET_OK;
+    };
+    MDET_TRY(sorted(n, 0, rank));
+    const uint32_t off = m2 ? tiles * 32 : 0;
+    if (m2) MDET_TRY(sorted(ns, off, nullptr));
+    hipLaunchKernelGGL(k_rm_poly, dim3(tiles), dim3(256), 0, s, tvec, contig, err, n, pfrag, tile_err);
+    hipLaunchKernelGGL(k_rm_cheb, dim3((ctiles * 32 + 255) / 256), dim3(256), 0, s, tvec, contig + off, ns, ctiles,
+                       tfrag);
+    A.frag = frag;
+    A.frag_a = frag_a;
+    A.pfrag = pfrag;
+    A.tile_err = tile_err;
+    A.order = order;
+    A.n = n;
+    A.tiles = tiles;
+    A.cfrag = frag + (size_t)off * 2 * KS;
+    A.tfrag = tfrag;
+    A.cerr = err + off;
+    A.corder = order + off;
+    A.rank = rank;
+    A.ns = ns;
+    A.ctiles = ctiles;
+    // about 8 blocks a CU
+    const uint32_t gx = (ctiles + 3) / 4, gy = std::min(tiles, std::max(1u, (8 * (uint32_t)ctx->num_cus + gx - 1) / gx));
+    A.seg = (tiles + gy - 1) / gy;
+    const dim3 grid(gx, (tiles + A.seg - 1) / A.seg), block(256);
+    hipLaunchKernelGGL(k_rm_scan<RM_BEST1>, grid, block, 0, s, A);
+    hipLaunchKernelGGL(k_rm_scan<RM_BEST2>, grid, block, 0, s, A);
+    hipLaunchKernelGGL(k_rm_scan<RM_LIST>, grid, block, 0, s, A);
+    hipLaunchKernelGGL(k_rm_exact, dim3(4 * (uint32_t)ctx->num_cus), dim3(64 * DIST_WAVES), 0, s, A, tnf_dev, ls, idx, m64);
+    MDET_HIP(hipGetLastError());
+    *out = A;
+    return MDET_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -3020,25 +3553,33 @@ int mdet_tnf_rowmax(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_d
     MDET_TRY(ensure_model(ctx));
     float* tvec;
     unsigned long long* mm;
-    uint32_t* m32;
     unsigned long long* m64;
     MDET_TRY(ctx_buf(ctx, "rm.tvec", n, &tvec));
     MDET_TRY(ctx_buf(ctx, "rm.mm", 8, &mm));
-    MDET_TRY(ctx_buf(ctx, "rm.m32", n_sample, &m32));
-    MDET_TRY(ctx_buf(ctx, "rm.m64", n_sample, &m64));
-    MDET_HIP(hipMemsetAsync(mm, 0, 32, ctx->stream));
+    // m64, then m32 and the bounds (32 bits each)
+    MDET_TRY(ctx_buf(ctx, "rm.max", (size_t)2 * n_sample, &m64));
+    uint32_t* m32 = reinterpret_cast<uint32_t*>(m64 + n_sample);
+    // mm: [0..2] log-size range and out-of-domain count, [3] listed pairs, [4] rows outside the bounds
+    MDET_HIP(hipMemsetAsync(mm, 0, 64, ctx->stream));
     hipLaunchKernelGGL(k_prep_rows, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, logsize_dev, n, tvec, mm);
     unsigned long long bad = 0;
     MDET_TRY(read_scalar(ctx, mm + 2, &bad));
     if ((unsigned int)bad != 0)
         MDET_FAIL(MDET_E_RANGE, "mdet_tnf_rowmax: %u log sizes outside [log10 1500, log10 500000]", (unsigned int)bad);
-    MDET_HIP(hipMemsetAsync(m32, 0, (size_t)n_sample * 4, ctx->stream));
-    MDET_HIP(hipMemsetAsync(m64, 0, (size_t)n_sample * 8, ctx->stream));
+    MDET_HIP(hipMemsetAsync(m64, 0, (size_t)n_sample * 16, ctx->stream));
+    const uint32_t* outside = nullptr;
+    uint32_t cap = 0;
+    if (n > RM_DIRECT_MAX) {
+        RmArgs A;
+        MDET_TRY(rowmax_mfma(ctx, tnf_dev, logsize_dev, tvec, idx_dev, n, n_sample, m32 + n_sample, m64, mm + 3, &A));
+        outside = A.outside;
+        cap = A.cap;
+    }
     const dim3 grid((n_sample + RM_ROWS - 1) / RM_ROWS, (n + RM_CHUNK - 1) / RM_CHUNK);
     hipLaunchKernelGGL(k_rowmax<false>, grid, dim3(256), 0, ctx->stream, tnf_dev, logsize_dev, tvec, idx_dev, n,
-                       n_sample, m32, m64);
+                       n_sample, m32, m64, outside, mm + 3, cap);
     hipLaunchKernelGGL(k_rowmax<true>, grid, dim3(256), 0, ctx->stream, tnf_dev, logsize_dev, tvec, idx_dev, n,
-                       n_sample, m32, m64);
+                       n_sample, m32, m64, outside, mm + 3, cap);
     hipLaunchKernelGGL(k_rowmax_final, dim3((n_sample + 255) / 256), dim3(256), 0, ctx->stream, m64, n_sample,
                        max_out_dev);
     MDET_HIP(hipGetLastError());
