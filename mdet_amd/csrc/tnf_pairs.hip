@@ -2580,19 +2580,21 @@ __global__ void k_preprob_pairs(const float* __restrict__ tnf, const double* __r
 // FP64 similarity of listed pairs, 1 - 1/(1 + exp(preProb)) with preProb from
 // the FP64 tie-breaker: the value get_tnf_graph2 stores (cuda/Cuda2.cu:257-258).
 // Pairs with an index >= n are counted in *bad_idx and get NaN.
-__global__ void k_similarity64(const float* __restrict__ tnf, const double* __restrict__ ls, uint32_t n,
-                               const uint32_t* __restrict__ pi, const uint32_t* __restrict__ pj, uint64_t np,
-                               double* __restrict__ s64, unsigned int* __restrict__ bad_idx) {
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= np) return;
-    const uint32_t i = pi[k], j = pj[k];
-    if (i >= n || j >= n) {
+__global__ __launch_bounds__(64 * DIST_WAVES) void k_similarity64(
+    const float* __restrict__ tnf, const double* __restrict__ ls, uint32_t n, const uint32_t* __restrict__ pi,
+    const uint32_t* __restrict__ pj, uint64_t np, double* __restrict__ s64, unsigned int* __restrict__ bad_idx) {
+    __shared__ __align__(16) float X[DIST_WAVES][DIST_LDS];
+    const uint64_t k = (uint64_t)blockIdx.x * (64 * DIST_WAVES) + threadIdx.x;
+    const bool in = k < np;
+    const uint32_t i = in ? pi[k] : 0u, j = in ? pj[k] : 0u;
+    const bool ok = in && i < n && j < n;
+    if (in && !ok) {
         atomicAdd(bad_idx, 1u);
         s64[k] = __builtin_nan("");
-        return;
     }
-    const double pre = model64(tnf + (size_t)i * NT, tnf + (size_t)j * NT, ls[i], ls[j]);
-    s64[k] = 1. - 1. / (1. + exp(pre));
+    if (!__any(ok)) return;  // n may be 0
+    const double d2 = wave_dist2_f64(tnf, ok ? i : 0u, ok ? j : 0u, X[threadIdx.x >> 6]);
+    if (ok) s64[k] = 1. - 1. / (1. + exp(model64_d2(d2, ls[i], ls[j])));
 }
 
 }  // namespace
@@ -3595,7 +3597,8 @@ int mdet_tnf_similarity64(mdet_ctx* ctx, const float* tnf_dev, const double* log
     unsigned int* bad;
     MDET_TRY(ctx_buf(ctx, "s64.bad", 16, &bad));
     MDET_HIP(hipMemsetAsync(bad, 0, 16, ctx->stream));
-    hipLaunchKernelGGL(k_similarity64, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, ctx->stream, tnf_dev,
+    hipLaunchKernelGGL(k_similarity64, dim3((unsigned)((np + 64 * DIST_WAVES - 1) / (64 * DIST_WAVES))),
+                       dim3(64 * DIST_WAVES), 0, ctx->stream, tnf_dev,
                        logsize_dev, n, pi_dev, pj_dev, np, s64_dev, bad);
     MDET_HIP(hipGetLastError());
     unsigned int nbad = 0;

@@ -103,3 +103,20 @@ def test_rowmax_outside_the_bounds(ctx, case):
         t[:] = t[0]
         ls[:] = ls[0]
     _check(ctx, t, ls, np.random.default_rng(2).permutation(n), n)
+
+
+def test_similarity_runs_of_equal_rows(ctx):
+    # runs of one i of every length from the same lanes on, contig 0 among them
+    t, ls = _rows(ctx, 400, seed=11)
+    rng = np.random.default_rng(3)
+    pi = np.concatenate([[5], np.zeros(3, int), [7], np.repeat(rng.integers(0, 400, 300), rng.integers(1, 70, 300)),
+                         np.tile([9, 0], 64)])
+    pi = np.concatenate([pi, pi[::-1], [3]])
+    pj = rng.integers(0, 400, len(pi))
+    dt, dl = ctx.to_device(t), ctx.to_device(ls)
+    got = ctx.tnf_similarity64(dt, dl, 400, pi, pj)
+    _, pre = ctx.tnf_preprob(dt, dl, 400, pi, pj)
+    dt.free()
+    dl.free()
+    want = 1 - 1 / (1 + np.exp(pre))  # one thread a pair, the same order of the sums
+    assert np.max(np.abs(got - want)) <= 4e-16
