@@ -636,20 +636,21 @@ __device__ inline void tiles_flush(const TileList& o, const uint4* stage, uint32
 
 template <bool BF16, int KSX, int RT, int CT>
 __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const uint4* __restrict__ frag_a,
-                                          const uint4 it, const uint32_t item, uint4 (*Bl)[CT * KSX * 64],
-                                          uint4* stage, uint32_t& nstage, const TileList& out) {
+                                          const uint4 it, const uint32_t item, uint4* B0, uint4* B1,
+                                          const int wave, uint4* stage, uint32_t& nstage,
+                                          const TileList& out) {
     constexpr int CG = 4 / RT;  // column tiles a pass: 4 independent accumulator chains
     constexpr uint32_t STEP = 32 * CT;
     static_assert(CG >= 1 && CT % CG == 0, "whole passes");
     const uint32_t r_lo = it.x, r_hi = it.y, c_lo = it.z, c_hi = it.w & ~ITEM_TRI;
     const bool tri = (it.w & ITEM_TRI) != 0;
     const uint32_t c_begin = c_lo & ~31u;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63;
     const uint32_t row0 = (r_lo & ~31u) + wave * (32 * RT);  // this wave's rows
     // a wave with no row of the item still takes its share of the column loads
     const bool active = row0 < r_hi;
     const uint32_t t0 = row0 >> 5;
-    issue_btile<KSX, CT>(frag, c_begin, Bl[0], tid, wave);
+    issue_btile<KSX, CT>(frag, c_begin, B0, tid, wave);
     uint4 a[RT][KSX];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -661,25 +662,15 @@ __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const 
         a[rt][KSX - 1] = active ? frag_a[(size_t)t * 64 + lane] : make_uint4(0, 0, 0, 0);
     }
 
-    int buf = 0;
-    for (uint32_t c0 = c_begin; c0 < c_hi; c0 += STEP, buf ^= 1) {
+    auto step = [&](const uint32_t c0, const uint4* B, uint4* next) __attribute__((always_inline)) {
+        // The barrier keeps the fill of the other buffer after every wave's
+        // reads of it in the step before, and the wait and barrier of the next
+        // step keep the reads after every wave's fill.
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        // The next step's fill is issued after the first pass's B reads
-        // (below): the compiler cannot tell Bl[buf ^ 1] from Bl[buf] and waits
-        // for the fill before the next pass's first read, so the first pass's
-        // MFMA drain and maximum tree cover part of it, and the CU's other
-        // blocks the rest.  The barrier above keeps the fill after every
-        // wave's reads of that buffer in the previous step; the wait and
-        // barrier at the next step's top keep the next reads after every
-        // wave's fill.
-        const bool more = c0 + STEP < c_hi;
+        if (c0 + STEP < c_hi) issue_btile<KSX, CT>(frag, c0 + STEP, next, tid, wave);
         // steps wholly left of the wave's rows hold no pair i < j
-        if (!active || (tri && c0 + STEP <= row0)) {
-            if (more) issue_btile<KSX, CT>(frag, c0 + STEP, Bl[buf ^ 1], tid, wave);
-            continue;
-        }
-        const uint4* B = Bl[buf];
+        if (!active || (tri && c0 + STEP <= row0)) return;
 #pragma unroll KSX == 9 ? CT / CG : 1
         for (int p = 0; p < CT / CG; ++p) {
             f32x16_t acc[RT][CG];
@@ -700,7 +691,6 @@ __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const 
 #pragma unroll
                     for (int c = 0; c < CG; ++c) acc[rt][c] = mfma32<BF16>(a[rt][ks], b[c], acc[rt][c]);
             }
-            if (p == 0 && more) issue_btile<KSX, CT>(frag, c0 + STEP, Bl[buf ^ 1], tid, wave);
             // per-lane maxima of each 32 x 32 tile.  acc > 0.0f exactly when
             // its bits, read as a signed int, are > 0, so the maxima are
             // integer max3 trees (a NaN may list its tile, never a pair).
@@ -735,6 +725,13 @@ __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const 
                     if (++nstage == TILE_STAGE) tiles_flush(out, stage, nstage, lane);
                 }
         }
+    };
+    // two arrays by name: of one array's halves the compiler cannot tell the
+    // fill's from the one read, and waits for the fill before the next reads
+    // (1,000,000 contigs: 24.5 against 22.9 ms)
+    for (uint32_t c0 = c_begin; c0 < c_hi; c0 += 2 * STEP) {
+        step(c0, B0, B1);
+        if (c0 + STEP < c_hi) step(c0 + STEP, B1, B0);
     }
 }
 
@@ -753,9 +750,10 @@ __global__ __launch_bounds__(64 * SCAN_WAVES, WPE) void k_tile_scan(const uint4*
                                                                     uint32_t* __restrict__ item_ctr,
                                                                     const uint32_t* __restrict__ qbounds,
                                                                     TileList out) {
-    __shared__ uint4 Bl[2][CT * KSX * 64];
+    __shared__ uint4 B0[CT * KSX * 64], B1[CT * KSX * 64];
     __shared__ uint4 stage_all[SCAN_WAVES][TILE_STAGE];
     __shared__ uint32_t s_item;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     uint32_t item = blockIdx.x, q_end = nitems, q_base = 0;
     uint32_t* ctr = item_ctr;
     if (item_ctr) {
@@ -769,12 +767,12 @@ __global__ __launch_bounds__(64 * SCAN_WAVES, WPE) void k_tile_scan(const uint4*
         __syncthreads();
         item = s_item;
     }
-    uint4* stage = stage_all[threadIdx.x >> 6];
+    uint4* stage = stage_all[wave];
     uint32_t nstage = 0;
     while (item < q_end) {
-        scan_item<BF16, KSX, RT, CT>(frag, frag_a, items[item], item, Bl, stage, nstage, out);
+        scan_item<BF16, KSX, RT, CT>(frag, frag_a, items[item], item, B0, B1, wave, stage, nstage, out);
         if (!item_ctr) break;
-        __syncthreads();  // every wave is done with Bl and s_item
+        __syncthreads();  // every wave is done with the buffers and s_item
         if (threadIdx.x == 0) s_item = q_base + atomicAdd(ctr, 1u);
         __syncthreads();
         item = s_item;
