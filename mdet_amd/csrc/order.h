@@ -19,7 +19,7 @@ struct ProjOrder {
 };
 
 // Queues, without a host round trip: the directions, the projected rows, and
-// the order of the rows by a Morton key of their leading coordinates (rows of
+// the order of the rows by the nearest of a number of centres in them (rows of
 // one population end up close together; rows holding a NaN or an infinity
 // come last).
 // fmt: the format the caller rounds the rows to afterwards; each row's margin
