@@ -548,6 +548,32 @@ __global__ __launch_bounds__(256) void k_proj_frags(const float* __restrict__ y,
     if (last) frag_a[(size_t)t * 64 + l] = pack(a);
 }
 
+// Bounding boxes of the 32-row tiles in the projection, box[d * T + t] =
+// (lowest, highest) and the largest margin, for T tiles; tiles without a bounded
+// row get empty boxes, ones with a row too long for FP16 boundless ones.  A
+// thread per tile and coordinate: a row is one 128-byte read of 32 lanes.
+__global__ __launch_bounds__(256) void k_tile_boxes(const float* __restrict__ y, const uint32_t* __restrict__ perm,
+                                                    uint32_t n, uint32_t T, float2* __restrict__ box,
+                                                    float* __restrict__ margin) {
+    const uint32_t t = blockIdx.x * 8 + (threadIdx.x >> 5), d = threadIdx.x & 31;
+    if (t >= T) return;  // T is a multiple of 8
+    float lo = 3e38f, hi = -3e38f, mg = 0.f;
+#pragma unroll
+    for (uint32_t r = 0; r < 32; ++r) {
+        const uint32_t s = t * 32 + r;
+        float v = d == PW_KIND ? 1.f : 0.f;
+        if (s < n) v = y[(size_t)perm[s] * PROJ_W + d];
+        const float kind = __shfl(v, PW_KIND, 32);
+        if (kind != 1.f) {
+            lo = fminf(lo, kind == 2.f ? -3e38f : v);
+            hi = fmaxf(hi, kind == 2.f ? 3e38f : v);
+            mg = fmaxf(mg, kind == 2.f ? 0.f : v);
+        }
+    }
+    if (d < PROJ_D) box[(size_t)d * T + t] = make_float2(lo, hi);
+    if (d == PW_MARGIN) margin[t] = mg;
+}
+
 }  // namespace
 
 namespace mdet {
@@ -602,6 +628,12 @@ int proj_order(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, 
     void* t;
     MDET_TRY(ctx_buf(ctx, "cub.sorttmp", tmp, &t));
     MDET_HIP(hipcub::DeviceRadixSort::SortPairs(t, tmp, key, key2, idx, out->perm, (int)n, 0, KEY_BITS, s));
+    return MDET_OK;
+}
+
+int proj_boxes(mdet_ctx* ctx, const ProjOrder& o, uint32_t n, uint32_t T, float2* box, float* margin) {
+    hipLaunchKernelGGL(k_tile_boxes, dim3(T / 8), dim3(256), 0, ctx->stream, o.y, o.perm, n, T, box, margin);
+    MDET_HIP(hipGetLastError());
     return MDET_OK;
 }
 

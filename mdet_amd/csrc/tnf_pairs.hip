@@ -8,12 +8,13 @@
 //            for the Gram modes the TNF rows in BF16/FP16, K padded 136 -> 144,
 //            in MFMA fragment order.  R = max over the length range of the edge
 //            distance threshold.
-//   scan     (k_tile_scan) which 32 x 32 tiles of the upper triangle can hold a
-//            pair within R: MFMA products of the projected rows, a lower bound
-//            of every pair's distance, with the threshold folded into K; small
-//            inputs skip it and take every tile.
-//            LEARNED: the same kernel on the TNF rows over the pairs of cluster
-//            pairs chosen by the learned embeddings (tnf_ivf.hip).
+//   scan     (k_box_scan) which 32 x 32 tiles of the upper triangle can hold a
+//            pair within R: the gap of the tiles' boxes in the projection, then
+//            MFMA products of the projected rows, a lower bound of every pair's
+//            distance, with the threshold folded into K; small inputs skip it
+//            and take every tile.
+//            LEARNED (k_tile_scan): products of the TNF rows over the pairs of
+//            cluster pairs chosen by the learned embeddings (tnf_ivf.hip).
 //   select survivors of the listed tiles
 //              EXACT_F32   FP32 sum of squared differences of every pair
 //                          (k_tile_f32), d < R
@@ -47,6 +48,8 @@
 namespace {
 
 using mdet::ITEM_TRI;
+using mdet::PROJ_D;
+using mdet::PROJ_KS;
 constexpr int NT = 136;
 constexpr int KS = 9;    // MFMA k-steps of 16 for TNF rows (K padded to 144)
 constexpr int KS_E = 3;  // k-steps for 32-dimensional embeddings (K padded to 48)
@@ -481,17 +484,14 @@ __global__ __launch_bounds__(256) void k_prep_lowp(const float* __restrict__ x, 
 
 // ------------------------------------------------------------- tile scan --
 // The first pass over the pairs: which 32 x 32 tiles hold a pair within the
-// radius at all.  Block = 4 waves of RT row tiles each (held in registers for
+// radius at all.  The exhaustive modes take k_box_scan (below), the learned
+// filter k_tile_scan: block = 4 waves of RT row tiles each (held in registers for
 // the whole column sweep of an item); columns stream through LDS CT tiles a
 // step in fragment order, double buffered and filled by
 // global_load_lds_dwordx4 (no register staging).  With the threshold folded
 // into K the test of a pair is "acc > 0"; a tile with one goes to the list,
 // which the second pass works off.  Nothing else leaves the kernel, so its cost
 // is the MFMAs and the maximum tree.
-//   KSX = 2, RT = 4, CT = 8: the exhaustive modes, on the projected rows
-//     (order.h): a lower bound of the distance in 28 dimensions drops ~99% of
-//     the tiles.  Bound by the MFMAs (2 per tile, 64 cycles) and the maximum
-//     tree beside them.
 //   KSX = 9, RT = 2, CT = 4: cluster pairs and full rows of the learned
 //     filter, on the TNF rows themselves.
 //   KSX = 3, RT = 2, CT = 4: the embedding radius of the learned filter.
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void k_prep_lowp(const float* __restrict__ x, 
 // 8-wave blocks, s_setprio around the chains, two distinct LDS arrays.
 constexpr uint32_t SCAN_WAVES = 4;
 constexpr uint32_t scan_rows(int rt) { return 32u * rt * SCAN_WAVES; }  // rows per item of row blocks
-constexpr int PROJ_RT = 4, PROJ_CT = 8;
+constexpr int PROJ_RT = 4;  // row tiles a wave of the projected scan
 constexpr int GRAM_RT = 2, GRAM_CT = 4;
 static_assert(scan_rows(GRAM_RT) == mdet::ITEM_ROWS, "cluster items hold one block's rows");
 // Scan item: (r_lo, r_hi, c_lo, c_hi | ITEM_TRI) = pairs of row positions
@@ -778,6 +778,139 @@ __global__ __launch_bounds__(64 * SCAN_WAVES, WPE) void k_tile_scan(const uint4*
         item = s_item;
     }
     tiles_flush(out, stage, nstage, threadIdx.x & 63);
+}
+
+// The first pass of the exhaustive modes: the projected rows (order.h).  Before
+// a pair of tiles is multiplied, the gap of their bounding boxes decides whether
+// it can hold a close pair at all: a lane takes one column tile against the
+// wave's PROJ_RT row tiles (their boxes from scalar loads), 64 column tiles at a
+// time, and only the pairs left (8% at 50,000 contigs, 12% at 200,000, ~21% at
+// 1,000,000) go to MFMA: 2 products and a maximum tree.  Waves work on their own
+// (no barrier in the loop): the columns left differ too much for a block to
+// stage them together, so each wave reads its column fragments from L1/L2, the
+// next ones ahead.  Bound by the box test (~480 instructions per 256 tile pairs:
+// ~3 of 10.7 ms at 1,000,000 contigs) and by the products and trees of the pairs
+// left, a wave's 2 products waiting on each other: six waves a SIMD (four: 11.6
+// ms).  All pairs multiplied (row blocks of 512, columns staged in LDS): 23.5 ms
+// and 929 us at 200,000 contigs, against 311 us.
+struct BoxArgs {
+    const uint4 *frag, *frag_a;
+    uint32_t T;  // tiles per coordinate of box
+    float R;
+    const uint4* items;
+    uint32_t nitems;
+    uint32_t* item_ctr;
+    const uint32_t* qbounds;
+    TileList out;
+};
+
+__device__ __forceinline__ void box_item(const BoxArgs& A, const float2* __restrict__ box,
+                                         const float* __restrict__ margin, const uint4 it, const uint32_t item, const int wave,
+                                         const int lane, uint4* stage, uint32_t& nstage) {
+    const uint32_t r_hi = it.y, c_hi = it.w & ~ITEM_TRI;
+    const bool tri = (it.w & ITEM_TRI) != 0;
+    const uint32_t t0 = it.x / 32 + wave * PROJ_RT;  // items start at whole blocks
+    if (32 * t0 >= r_hi) return;
+    uint4 a[PROJ_RT][PROJ_KS];
+#pragma unroll
+    for (int rt = 0; rt < PROJ_RT; ++rt) {
+        const uint32_t t = min(t0 + rt, (r_hi - 1) >> 5);
+        a[rt][0] = A.frag[(size_t)t * PROJ_KS * 64 + lane];
+        a[rt][1] = A.frag_a[(size_t)t * 64 + lane];
+    }
+    float reach[PROJ_RT];
+#pragma unroll
+    for (int rt = 0; rt < PROJ_RT; ++rt) reach[rt] = A.R + margin[t0 + rt];
+    uint32_t cb = it.z / 32;
+    if (tri && cb < t0) cb += (t0 - cb) / 64 * 64;
+    for (; 32 * cb < c_hi; cb += 64) {
+        const uint32_t tc = cb + lane;
+        float s[PROJ_RT] = {};
+        {
+            const float2* bc = box + tc;
+            const float2* br = box + t0;
+#pragma unroll 4
+            for (int d = 0; d < PROJ_D; ++d) {
+                const float2 c = bc[(size_t)d * A.T];
+#pragma unroll
+                for (int rt = 0; rt < PROJ_RT; ++rt) {
+                    const float2 r = br[(size_t)d * A.T + rt];
+                    const float g = fmaxf(fmaxf(c.x - r.y, r.x - c.y), 0.f);
+                    s[rt] = fmaf(g, g, s[rt]);
+                }
+            }
+        }
+        const float mc = margin[tc];
+        uint64_t m[PROJ_RT], u = 0;
+#pragma unroll
+        for (int rt = 0; rt < PROJ_RT; ++rt) {
+            const float th = (reach[rt] + mc) * (1.f + 1e-5f);
+            m[rt] = __ballot(s[rt] < th * th && 32 * tc < c_hi && (!tri || tc >= t0 + rt) && 32 * (t0 + rt) < r_hi);
+            u |= m[rt];
+        }
+        if (!u) continue;
+        auto load = [&](uint64_t bits, uint4* b) {
+            const uint32_t c = cb + (uint32_t)__builtin_ctzll(bits);
+#pragma unroll
+            for (int ks = 0; ks < PROJ_KS; ++ks) b[ks] = A.frag[((size_t)c * PROJ_KS + ks) * 64 + lane];
+        };
+        uint4 next[PROJ_KS];
+        load(u, next);
+        while (u) {
+            const uint32_t c = (uint32_t)__builtin_ctzll(u);
+            uint4 b[PROJ_KS];
+#pragma unroll
+            for (int ks = 0; ks < PROJ_KS; ++ks) b[ks] = next[ks];
+            u &= u - 1;
+            if (u) load(u, next);
+#pragma unroll
+            for (int rt = 0; rt < PROJ_RT; ++rt) {
+                if (!(m[rt] >> c & 1)) continue;
+                f32x16_t v = f32x16_t{};
+#pragma unroll
+                for (int ks = 0; ks < PROJ_KS; ++ks) v = mfma32<false>(a[rt][ks], b[ks], v);
+                // acc > 0 exactly when its bits, read as a signed int, are > 0
+                int x[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) x[r] = __float_as_int(v[r]);
+                const int m0 = max(max(x[0], x[1]), x[2]), m1 = max(max(x[3], x[4]), x[5]);
+                const int m2 = max(max(x[6], x[7]), x[8]), m3 = max(max(x[9], x[10]), x[11]);
+                const int m4 = max(max(x[12], x[13]), x[14]);
+                if (!__any(max(max(max(m0, m1), m2), max(max(m3, m4), x[15])) > 0)) continue;
+                if (lane == 0) stage[nstage] = make_uint4(t0 + rt, cb + c, item, 0u);
+                if (++nstage == TILE_STAGE) tiles_flush(A.out, stage, nstage, lane);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(64 * SCAN_WAVES, 6) void k_box_scan(const BoxArgs A, const float2* __restrict__ box,
+                                                                 const float* __restrict__ margin) {
+    __shared__ uint4 stage_all[SCAN_WAVES][TILE_STAGE];
+    __shared__ uint32_t s_item;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint32_t item = blockIdx.x, q_end = A.nitems, q_base = 0;
+    uint32_t* ctr = A.item_ctr;
+    if (ctr && A.qbounds) {
+        const uint32_t q = blockIdx.x % PF_QUEUES;
+        q_base = A.qbounds[q];
+        q_end = A.qbounds[q + 1];
+        ctr += q * PF_CTR_STRIDE;
+    }
+    uint4* stage = stage_all[wave];
+    uint32_t nstage = 0;
+    for (;;) {
+        if (ctr) {
+            __syncthreads();  // every wave has read s_item
+            if (threadIdx.x == 0) s_item = q_base + atomicAdd(ctr, 1u);
+            __syncthreads();
+            item = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_item);
+        }
+        if (item >= q_end) break;
+        box_item(A, box, margin, A.items[item], item, wave, lane, stage, nstage);
+        if (!ctr) break;
+    }
+    tiles_flush(A.out, stage, nstage, lane);
 }
 
 // ------------------------------------------------------------ tile pairs --
@@ -2876,6 +3009,9 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
         // -- fragments of the Gram in the scan's row order
         uint32_t* perm = order.perm;  // position -> contig (null: itself)
         uint4 *frag = nullptr, *frag_a = nullptr, *pfrag = nullptr, *pfrag_a = nullptr;
+        float2* pbox = nullptr;
+        float* pbox_margin = nullptr;
+        const uint32_t box_tiles = (n_pad / 32 + 127) / 64 * 64;  // a whole step past the last tile
         uint4* items = nullptr;
         uint32_t nitems = 0;
         uint32_t* qbounds = nullptr;
@@ -2903,6 +3039,9 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 MDET_TRY(ctx_buf(ctx, "pairs.pfrag", (size_t)n_pad / 32 * PROJ_KS * 64, &pfrag));
                 MDET_TRY(ctx_buf(ctx, "pairs.pfrag_a", (size_t)n_pad / 32 * 64, &pfrag_a));
                 MDET_TRY(proj_frags(ctx, order, n, n_pad, reach, pfrag, pfrag_a));
+                MDET_TRY(ctx_buf(ctx, "pairs.pbox", (size_t)PROJ_D * box_tiles, &pbox));
+                MDET_TRY(ctx_buf(ctx, "pairs.pbox_m", (size_t)box_tiles, &pbox_margin));
+                MDET_TRY(proj_boxes(ctx, order, n, box_tiles, pbox, pbox_margin));
                 const uint32_t ord = tune.persistent ? tune.item_order : 0u;
                 MDET_TRY(build_items(ctx, n, item_rows, seg, ord, &items, &nitems, &qbounds));
                 if (!ord) qbounds = nullptr;
@@ -2994,8 +3133,9 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 };
                 const dim3 block(64 * SCAN_WAVES);
                 if (gram_all)
-                    hipLaunchKernelGGL((k_tile_scan<false, PROJ_KS, PROJ_RT, PROJ_CT, 4>), grid(4), block, 0,
-                                       ctx->stream, pfrag, pfrag_a, items, nitems, pf_ctr, (const uint32_t*)qbounds, tl);
+                    hipLaunchKernelGGL(k_box_scan, grid(6), block, 0, ctx->stream,
+                                       BoxArgs{pfrag, pfrag_a, box_tiles, reach, items, nitems, pf_ctr, qbounds, tl},
+                                       pbox, pbox_margin);
                 else if (tnf_gram)
                     hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>), grid(2), block, 0, ctx->stream,
                                        frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, tl);
