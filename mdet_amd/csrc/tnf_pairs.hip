@@ -150,10 +150,14 @@ __device__ inline float dist2_f32(const float* __restrict__ a, const float* __re
 __device__ inline double dist2_f64(const float* __restrict__ a, const float* __restrict__ b) {
 #pragma clang fp contract(off)
     double d = 0;
-    for (int i = 0; i < NT; ++i) {
-        float diff = a[i] - b[i];
-        float sq = diff * diff;
-        d += (double)sq;
+#pragma unroll 4
+    for (int q = 0; q < NT / 4; ++q) {
+        const f32x4_t diff = reinterpret_cast<const f32x4_t*>(a)[q] - reinterpret_cast<const f32x4_t*>(b)[q];
+        const f32x4_t sq = diff * diff;
+        d += (double)sq.x;
+        d += (double)sq.y;
+        d += (double)sq.z;
+        d += (double)sq.w;
     }
     return d;
 }
@@ -247,26 +251,27 @@ __device__ inline uint32_t wave_incl_sum_dpp(uint32_t x) {
 constexpr int S_BUCKET = 64;
 static_assert(S_BUCKET >= 64 && S_BUCKET % 64 == 0, "the row scan gives each lane S_BUCKET / 64 rows");
 
-// Adds, for each distinct key held by the active lanes, the number of lanes
-// holding it to counter[key] (one atomic by the lowest such lane) and returns
-// to every active lane old value + its rank among the lanes with its key.
-// All 64 lanes call; the loop runs once per distinct key.
-__device__ inline uint32_t wave_aggregated_add(uint32_t* counter, uint32_t key, bool active) {
-    uint32_t slot = 0;
+// The active lanes by key: each lane's leader (the lowest lane with its key),
+// rank among them and, in the leader, their number.  All 64 lanes call; the loop
+// runs once per distinct key and touches no memory, so that a caller's atomics
+// (one by each leader) go out together instead of one round trip per key.
+struct KeyGroup {
+    int leader;
+    uint32_t rank, count;
+};
+__device__ inline KeyGroup wave_key_groups(uint32_t key, bool active) {
+    KeyGroup g{-1, 0, 0};
     uint64_t pending = __ballot(active);
     const uint32_t lane = lane_id();
     while (pending) {
         const int leader = __ffsll((long long)pending) - 1;
-        const uint32_t k = __shfl(key, leader, 64);
-        const bool mine = active && key == k;
-        const uint64_t same = __ballot(mine);
-        uint32_t base = 0;
-        if ((int)lane == leader) base = atomicAdd(&counter[k], (uint32_t)__popcll(same));
-        base = __shfl(base, leader, 64);
-        if (mine) slot = base + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+        const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)key, leader);
+        const uint64_t same = __ballot(active && key == k);
+        if (active && key == k)
+            g = KeyGroup{leader, (uint32_t)__popcll(same & ((1ull << lane) - 1ull)), (uint32_t)__popcll(same)};
         pending &= ~same;
     }
-    return slot;
+    return g;
 }
 
 // The same without the slots: counter[key] += lanes holding key (no return
@@ -1620,11 +1625,21 @@ __global__ __launch_bounds__(256) void k_bucket_fill(const Cand* __restrict__ ca
                 sj = position_of(iperm, c.j);
             }
         }
-        const uint32_t s1 = wave_aggregated_add(bcur, si / S_BUCKET, act);
-        const uint32_t s2 = wave_aggregated_add(bcur, sj / S_BUCKET, act);
+        const KeyGroup g1 = wave_key_groups(si / S_BUCKET, act), g2 = wave_key_groups(sj / S_BUCKET, act);
+        const int lane = (int)lane_id();
+        uint32_t b1 = 0, b2 = 0;
+        uint64_t o1 = 0, o2 = 0;
         if (act) {
-            ent[boff[si / S_BUCKET] + s1] = Ent{c.j, c.pre, si % S_BUCKET};
-            ent[boff[sj / S_BUCKET] + s2] = Ent{c.i, c.pre, sj % S_BUCKET};
+            if (g1.leader == lane) b1 = atomicAdd(&bcur[si / S_BUCKET], g1.count);
+            if (g2.leader == lane) b2 = atomicAdd(&bcur[sj / S_BUCKET], g2.count);
+            o1 = boff[si / S_BUCKET];
+            o2 = boff[sj / S_BUCKET];
+        }
+        b1 = (uint32_t)__shfl((int)b1, g1.leader, 64);
+        b2 = (uint32_t)__shfl((int)b2, g2.leader, 64);
+        if (act) {
+            ent[o1 + b1 + g1.rank] = Ent{c.j, c.pre, si % S_BUCKET};
+            ent[o2 + b2 + g2.rank] = Ent{c.i, c.pre, sj % S_BUCKET};
         }
     }
 }
@@ -1665,18 +1680,46 @@ __device__ inline int pow2_at_least(uint32_t v) {
     return sz;
 }
 
-// Bitonic sort of 64 * E elements held in registers by one wave, element
-// t = e * 64 + lane in slot e of lane t % 64 (ascending by ranks_before if
-// BY_RANK, else by id; the ids of a row are distinct).  Strides below 64 are
-// exchanges between lanes (shuffles), strides of 64 and more swap slots
-// within a lane.
-template <int E, bool BY_RANK>
-__device__ inline bool elem_before(float ka, uint32_t ia, float kb, uint32_t ib) {
-    return BY_RANK ? ranks_before(ka, ia, kb, ib) : ia < ib;
+// x of lane (lane ^ J): DPP moves and lane swaps, no LDS round trip.
+template <int J>
+__device__ __forceinline__ uint32_t xor_lane(uint32_t x, int lane) {
+    const int v = (int)x;
+    if (J == 1) return (uint32_t)__builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);  // quad_perm 1 0 3 2
+    if (J == 2) return (uint32_t)__builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);  // quad_perm 2 3 0 1
+    if (J == 4) {  // mirror in 8 lanes, then in 4: 7 ^ 3
+        const int m = __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);
+        return (uint32_t)__builtin_amdgcn_mov_dpp(m, 0x1B, 0xF, 0xF, true);
+    }
+    if (J == 8) return (uint32_t)__builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);  // row_ror 8
+    if (J == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return lane & 16 ? r[0] : r[1];
+    }
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return lane & 32 ? r[0] : r[1];
 }
 
-template <int E, bool BY_RANK>
-__device__ __forceinline__ void wave_sort_regs(float (&key)[E], uint32_t (&id)[E], int lane) {
+template <int J, int E>
+__device__ __forceinline__ void wave_exchange(float (&key)[E], uint32_t (&id)[E], int k, int lane) {
+    const bool lower = (lane & J) == 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint32_t pi = xor_lane<J>(id[e], lane);
+        const float pk = __uint_as_float(xor_lane<J>(__float_as_uint(key[e]), lane));
+        const bool up = ((e * 64 + lane) & k) == 0;
+        if ((lower == up) != (id[e] < pi)) {
+            key[e] = pk;
+            id[e] = pi;
+        }
+    }
+}
+
+// Bitonic sort by id of 64 * E elements held in registers by one wave, element
+// t = e * 64 + lane in slot e of lane t % 64 (the ids of a row are distinct;
+// padding ids are equal).  Strides below 64 are exchanges between lanes, larger
+// ones swap slots within a lane.
+template <int E>
+__device__ __forceinline__ void wave_sort_ids(float (&key)[E], uint32_t (&id)[E], int lane) {
 #pragma unroll
     for (int k = 2; k <= 64 * E; k <<= 1)
 #pragma unroll
@@ -1688,7 +1731,7 @@ __device__ __forceinline__ void wave_sort_regs(float (&key)[E], uint32_t (&id)[E
                     if ((e & sj) == 0) {
                         const int e2 = e | sj;
                         const bool up = ((e * 64 + lane) & k) == 0;
-                        if (elem_before<E, BY_RANK>(key[e2], id[e2], key[e], id[e]) == up) {
+                        if ((id[e2] < id[e]) == up) {
                             const float tk = key[e];
                             key[e] = key[e2];
                             key[e2] = tk;
@@ -1697,19 +1740,18 @@ __device__ __forceinline__ void wave_sort_regs(float (&key)[E], uint32_t (&id)[E
                             id[e2] = ti;
                         }
                     }
+            } else if (j == 32) {
+                wave_exchange<32, E>(key, id, k, lane);
+            } else if (j == 16) {
+                wave_exchange<16, E>(key, id, k, lane);
+            } else if (j == 8) {
+                wave_exchange<8, E>(key, id, k, lane);
+            } else if (j == 4) {
+                wave_exchange<4, E>(key, id, k, lane);
+            } else if (j == 2) {
+                wave_exchange<2, E>(key, id, k, lane);
             } else {
-                const bool lower = (lane & j) == 0;
-#pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    const float pk = __shfl_xor(key[e], j, 64);
-                    const uint32_t pi = __shfl_xor(id[e], j, 64);
-                    const bool up = ((e * 64 + lane) & k) == 0;
-                    const bool mine_first = elem_before<E, BY_RANK>(key[e], id[e], pk, pi);
-                    if ((lower == up) != mine_first) {
-                        key[e] = pk;
-                        id[e] = pi;
-                    }
-                }
+                wave_exchange<1, E>(key, id, k, lane);
             }
         }
 }
@@ -1728,7 +1770,7 @@ __device__ void sort_ids_and_store(const float* key, const uint32_t* id, uint32_
         k[e] = in ? key[t] : 0.f;
         v[e] = in ? id[t] : 0xffffffffu;
     }
-    wave_sort_regs<E, false>(k, v, lane);
+    wave_sort_ids<E>(k, v, lane);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const uint32_t t = e * 64 + lane;
@@ -1736,120 +1778,133 @@ __device__ void sort_ids_and_store(const float* key, const uint32_t* id, uint32_
     }
 }
 
-// deg (<= 64 * E) entries of adj[beg..] in rank order (pre desc, partner
-// asc) into LDS key/id[0..64E), padded with (-inf, 0xffffffff) entries.
+// The K largest preProb of the row's deg (<= 64 * E, > K) entries at
+// adj[beg..), FP32 ties within 2 * EPS of the K-th re-ranked in FP64: the
+// partners above rid compacted into LDS key/id, their number returned; -1 if
+// the tie zone is wider than a wave.  Only the K-th largest key is needed, not
+// their order: it is found bit by bit, counting the keys not below a candidate
+// (~25 rounds of E compares; a bitonic sort by rank took 45 exchange rounds).
 template <int E>
-__device__ void rank_sort_to_lds(const Adj* __restrict__ adj, uint64_t beg, uint32_t deg, float* key, uint32_t* id,
-                                 int lane) {
-    float k[E];
-    uint32_t v[E];
+__device__ int top_of_row(const Adj* __restrict__ adj, uint64_t beg, uint32_t deg, uint32_t rid, uint32_t K,
+                          const float* __restrict__ tnf, const double* __restrict__ ls, float* key, uint32_t* id,
+                          int lane) {
+    uint32_t k[E], v[E], hi = 0, lo = 0xffffffffu;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const uint32_t t = e * 64 + lane;
         const bool in = t < deg;
         const Adj a = in ? adj[beg + t] : Adj{0xffffffffu, 0.f};
-        k[e] = in ? a.pre : -__builtin_inff();
-        v[e] = in ? a.partner : 0xffffffffu;
+        k[e] = in ? f2ord(a.pre) : 0u;
+        v[e] = a.partner;
+        hi = max(hi, k[e]);
+        lo = min(lo, in ? k[e] : 0xffffffffu);
     }
-    wave_sort_regs<E, true>(k, v, lane);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
+    }
+    // all keys share the bits above the highest one in which hi and lo differ
+    hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi);
+    lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
+    uint32_t kth = hi;
+    if (hi != lo) {
+        int bit = 31 - __builtin_clz(hi ^ lo);
+        kth = bit == 31 ? 0u : hi & ~((2u << bit) - 1u);
+        for (; bit >= 0; --bit) {
+            const uint32_t c = kth | (1u << bit);
+            uint32_t cnt = 0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) cnt += (uint32_t)__popcll(__ballot(k[e] >= c));
+            if (cnt >= K) kth = c;
+            if (cnt == K) break;  // c lies above every key left out
+        }
+        // the smallest key not below it (the last round may have ended above that key)
+        uint32_t least = 0xffffffffu;
+#pragma unroll
+        for (int e = 0; e < E; ++e) least = min(least, k[e] >= kth ? k[e] : 0xffffffffu);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) least = min(least, (uint32_t)__shfl_xor((int)least, off, 64));
+        kth = (uint32_t)__builtin_amdgcn_readfirstlane((int)least);
+    }
+    const float vk = ord2f(kth);
+    // entries above the zone are in; of the zone, the best by FP64
+    uint32_t above = 0, zn = 0, zp[E];
+    bool sel[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        key[e * 64 + lane] = k[e];
-        id[e * 64 + lane] = v[e];
+        const bool in = e * 64 + lane < deg;
+        const float x = ord2f(k[e]);
+        const bool zone = in && fabsf(x - vk) <= 2.f * EPS_PRE;
+        sel[e] = in && !zone && x > vk;
+        const uint64_t zm = __ballot(zone);
+        zp[e] = zone ? zn + (uint32_t)__popcll(zm & ((1ull << lane) - 1ull)) : 0xffffffffu;
+        zn += (uint32_t)__popcll(zm);
+        above += (uint32_t)__popcll(__ballot(sel[e]));
     }
+    if (zn > 64) return -1;
+    const uint32_t need = K - above;
+    if (need < zn) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (zp[e] != 0xffffffffu) id[zp[e]] = v[e];
+        wave_sync();
+        double zk = 0.0;
+        uint32_t zi = 0xffffffffu;
+        if (lane < (int)zn) {
+            zi = id[lane];
+            zk = model64(tnf + (size_t)rid * NT, tnf + (size_t)zi * NT, ls[rid], ls[zi]);
+        }
+        uint32_t rk = 0;
+        for (uint32_t u = 0; u < zn; ++u) {
+            const double zu = __shfl(zk, (int)u, 64);
+            const uint32_t iu = (uint32_t)__shfl((int)zi, (int)u, 64);
+            rk += (zu > zk || (zu == zk && iu < zi)) ? 1u : 0u;
+        }
+        const uint64_t won = __ballot(lane < (int)zn && rk < need);
+        wave_sync();
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (zp[e] != 0xffffffffu) sel[e] = won >> zp[e] & 1;
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) sel[e] = sel[e] || zp[e] != 0xffffffffu;
+    }
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const bool keep = sel[e] && v[e] > rid;
+        const uint64_t m = __ballot(keep);
+        if (keep) {
+            const uint32_t o = cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            key[o] = ord2f(k[e]);
+            id[o] = v[e];
+        }
+        cnt += (uint32_t)__popcll(m);
+    }
+    return (int)cnt;
 }
 
 // Row `rid` (contig id), deg entries at adj[beg..): by one wave.  Returns
 // false, touching nothing in global memory, if the row needs the block path
-// (FP32 tie zone at the cut wider than a wave).
+// (FP32 tie zone at the cut wider than a wave).  capped counts in LDS: one
+// atomic per row on the call's counter serialised the 50,000 capped rows of a
+// 50,000-contig input.
 __device__ bool wave_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t deg, uint32_t rid, uint32_t K,
                                 const float* __restrict__ tnf, const double* __restrict__ ls, float* key,
                                 uint32_t* id, uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg,
-                                unsigned long long* __restrict__ capped, int lane) {
-    const bool cap = K && deg > K;
-    if (cap) {
-        // rank order (pre desc, partner asc) in registers, then to LDS
-        if (deg <= 64)
-            rank_sort_to_lds<1>(adj, beg, deg, key, id, lane);
-        else if (deg <= 128)
-            rank_sort_to_lds<2>(adj, beg, deg, key, id, lane);
-        else if (deg <= 256)
-            rank_sort_to_lds<4>(adj, beg, deg, key, id, lane);
-        else
-            rank_sort_to_lds<8>(adj, beg, deg, key, id, lane);
-        wave_sync();
-        const float vk = key[K - 1];
-        // the FP32 keys within 2*EPS of the K-th form a contiguous range [z0, z1)
-        int z0 = (int)deg, z1 = 0;
-        for (int t0 = 0; t0 < (int)deg; t0 += 64) {
-            const int t = t0 + lane;
-            const uint64_t m = __ballot(t < (int)deg && fabsf(key[t] - vk) <= 2.f * EPS_PRE);
-            if (m) {
-                z0 = min(z0, t0 + __ffsll((long long)m) - 1);
-                z1 = max(z1, t0 + 64 - __clzll((long long)m));
-            }
-        }
-        const int zn = z1 - z0;
-        if (zn > 64) return false;
-        if (zn > 1) {
-            double zk = 0.0;
-            uint32_t myid = 0xffffffffu;
-            float mykey = 0.f;
-            if (lane < zn) {
-                myid = id[z0 + lane];
-                mykey = key[z0 + lane];
-                zk = model64(tnf + (size_t)rid * NT, tnf + (size_t)myid * NT, ls[rid], ls[myid]);
-            }
-            int rk = 0;
-            for (int u = 0; u < zn; ++u) {
-                const double zu = __shfl(zk, u, 64);
-                const uint32_t iu = __shfl(myid, u, 64);
-                rk += (zu > zk || (zu == zk && iu < myid)) ? 1 : 0;
-            }
-            wave_sync();
-            if (lane < zn) {
-                id[z0 + rk] = myid;
-                key[z0 + rk] = mykey;
-            }
-            wave_sync();
-        }
-        if (lane == 0) atomicAdd(capped, 1ull);
-        // keep the K selected partners above the row, compacted in place
-        // (a chunk's writes land below its reads and below the next
-        // chunk's), then sort them by id
-        uint32_t cnt = 0;
-        for (uint32_t t0 = 0; t0 < K; t0 += 64) {
-            const uint32_t t = t0 + lane;
-            const bool in = t < K;
-            const float kk = in ? key[t] : 0.f;
-            const uint32_t kv = in ? id[t] : 0xffffffffu;
-            const bool keep = in && kv > rid && kv != 0xffffffffu;
-            const uint64_t m = __ballot(keep);
-            if (keep) {
-                const uint32_t o = cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                key[o] = kk;
-                id[o] = kv;
-            }
-            cnt += (uint32_t)__popcll(m);
-        }
-        wave_sync();
-        if (cnt <= 64)
-            sort_ids_and_store<1>(key, id, cnt, adj, beg, lane);
-        else if (cnt <= 128)
-            sort_ids_and_store<2>(key, id, cnt, adj, beg, lane);
-        else if (cnt <= 256)
-            sort_ids_and_store<4>(key, id, cnt, adj, beg, lane);
-        else
-            sort_ids_and_store<8>(key, id, cnt, adj, beg, lane);
-        if (lane == 0) {
-            out_cnt[rid] = cnt;
-            rbeg[rid] = beg;
-        }
-        return true;
+                                uint32_t* capped, int lane) {
+    uint32_t cnt = 0;
+    if (K && deg > K) {
+        const int c = deg <= 64    ? top_of_row<1>(adj, beg, deg, rid, K, tnf, ls, key, id, lane)
+                      : deg <= 128 ? top_of_row<2>(adj, beg, deg, rid, K, tnf, ls, key, id, lane)
+                      : deg <= 256 ? top_of_row<4>(adj, beg, deg, rid, K, tnf, ls, key, id, lane)
+                                   : top_of_row<8>(adj, beg, deg, rid, K, tnf, ls, key, id, lane);
+        if (c < 0) return false;
+        cnt = (uint32_t)c;
+        if (lane == 0) atomicAdd(capped, 1u);
     } else {
-        // every candidate is selected: gather the partners above the row,
-        // then sort them by id in registers
-        uint32_t cnt = 0;
+        // every candidate is selected: gather the partners above the row
         for (uint32_t t0 = 0; t0 < deg; t0 += 64) {
             const uint32_t t = t0 + lane;
             Adj e{0, 0.f};
@@ -1863,21 +1918,22 @@ __device__ bool wave_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t de
             }
             cnt += (uint32_t)__popcll(m);
         }
-        wave_sync();
-        if (cnt <= 64)
-            sort_ids_and_store<1>(key, id, cnt, adj, beg, lane);
-        else if (cnt <= 128)
-            sort_ids_and_store<2>(key, id, cnt, adj, beg, lane);
-        else if (cnt <= 256)
-            sort_ids_and_store<4>(key, id, cnt, adj, beg, lane);
-        else
-            sort_ids_and_store<8>(key, id, cnt, adj, beg, lane);
-        if (lane == 0) {
-            out_cnt[rid] = cnt;
-            rbeg[rid] = beg;
-        }
-        return true;
     }
+    // sorted by id in registers
+    wave_sync();
+    if (cnt <= 64)
+        sort_ids_and_store<1>(key, id, cnt, adj, beg, lane);
+    else if (cnt <= 128)
+        sort_ids_and_store<2>(key, id, cnt, adj, beg, lane);
+    else if (cnt <= 256)
+        sort_ids_and_store<4>(key, id, cnt, adj, beg, lane);
+    else
+        sort_ids_and_store<8>(key, id, cnt, adj, beg, lane);
+    if (lane == 0) {
+        out_cnt[rid] = cnt;
+        rbeg[rid] = beg;
+    }
+    return true;
 }
 
 // Appends (rid, deg, beg) to a row list with its counter apart; err bit `ovf`
@@ -2003,7 +2059,7 @@ __global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
     unsigned int* __restrict__ err, unsigned long long* __restrict__ capped) {
     constexpr int PER = S_BUCKET / 64;
     constexpr int BATCH = 4;
-    __shared__ uint32_t hist[S_BUCKET], rstart[S_BUCKET], rcur[S_BUCKET];
+    __shared__ uint32_t hist[S_BUCKET], rstart[S_BUCKET], rcur[S_BUCKET], s_capped;
     __shared__ float wkey[S_WAVES][W_CAP];
     __shared__ uint32_t wid[S_WAVES][W_CAP];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -2012,6 +2068,7 @@ __global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
     const uint32_t row0 = b * S_BUCKET;
     const uint32_t rows = n - row0 < (uint32_t)S_BUCKET ? n - row0 : (uint32_t)S_BUCKET;
     for (int t = tid; t < S_BUCKET; t += S_THREADS) hist[t] = rcur[t] = 0;
+    if (tid == 0) s_capped = 0;
     __syncthreads();
     // row histogram; BATCH independent loads in flight per thread
     for (uint64_t e = e0 + tid; e < e1; e += BATCH * S_THREADS) {
@@ -2074,10 +2131,12 @@ __global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
         } else if (deg > (uint32_t)W_CAP) {
             done = false;
         } else {
-            done = wave_row_select(adj, beg, deg, rid, K, tnf, ls, wkey[wave], wid[wave], out_cnt, rbeg, capped, lane);
+            done = wave_row_select(adj, beg, deg, rid, K, tnf, ls, wkey[wave], wid[wave], out_cnt, rbeg, &s_capped, lane);
         }
         if (!done && lane == 0) push_row(big, rid, deg, beg, err, 4u);
     }
+    __syncthreads();
+    if (tid == 0 && s_capped) atomicAdd(capped, (unsigned long long)s_capped);
 }
 
 // Rows the wave path declined (over W_CAP entries, or a tie zone wider than a
