@@ -11,11 +11,15 @@
 // back-propagates through the three layers and applies Adam to the FP32
 // master weights, refreshing their BF16 copies that the forward pass reads.
 //
-// GEMMs are FP32-accumulate tiles on the VALU (64x64 per 256-thread block,
-// 4x4 per thread, K streamed through LDS): the network is 109,088 weights and
-// a training step is ~10^9 flops, so these kernels are launch-bound, not
-// compute-bound; the all-pairs embedding Gram that uses the network at
-// inference runs on MFMA (tnf_pairs.hip).
+// Three launches a batch: forward and backward of 16 rows a block with
+// everything between in LDS and registers (k_train_rows), the weight gradients
+// split by rows (k_weight_grad), and the sums over blocks and splits
+// (k_grad_sum).  All products are FP32 (v_mfma_f32_16x16x4, 32x32x2): the
+// network is 109,088 weights and a batch of 512 pairs 0.67 GFLOP, so launches
+// and latency are the cost: 30 + 10 + 4 us at 512 pairs, against 288 us in 21
+// launches of one product, activation or sum each (64 x 64 tiles on the VALU, 16
+// to 64 blocks a launch).  The all-pairs embedding Gram that uses the network
+// at inference is in tnf_pairs.hip.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -59,140 +63,266 @@ __device__ inline float gelu_grad(float x) {
     return cdf + x * pdf;
 }
 
-// C[M x N] (+)= op(A) * op(B); A is M x K (row-major, lda) or K x M if TA;
-// B is K x N (row-major, ldb) or N x K if TB.  Epilogue: + bias[n], store
-// pre-activation to Z (optional) and act(.) to C (GELU if gelu_out).
-// Split K: block z covers k in [z * kchunk, (z + 1) * kchunk) and writes to
-// C + z * zstride (partial products, summed by k_sum_partials).
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, int lda, const float* __restrict__ B,
-                                              int ldb, float* __restrict__ C, int ldc, float* __restrict__ Z, int M,
-                                              int N, int K, const float* __restrict__ bias, int gelu_out,
-                                              int accumulate, int kchunk, size_t zstride) {
-    __shared__ float As[16][64 + 1], Bs[16][64 + 1];
-    const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
-    C += blockIdx.z * zstride;
-    float acc[4][4] = {};
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-        for (int e = tid; e < 16 * 64; e += 256) {
-            const int kk = e >> 6, mm = e & 63;
-            const int m = m0 + mm, k = k0 + kk;
-            float va = 0.f, vb = 0.f;
-            if (m < M && k < ke) va = TA ? A[(size_t)k * lda + m] : A[(size_t)m * lda + k];
-            const int n = n0 + mm;
-            if (n < N && k < ke) vb = TB ? B[(size_t)n * ldb + k] : B[(size_t)k * ldb + n];
-            As[kk][mm] = va;
-            Bs[kk][mm] = vb;
-        }
-        __syncthreads();
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// ------------------------------------------------------------ training --
+// Rows 2b and 2b + 1 of a batch are pair b's two contigs; block = 16 rows, 16
+// waves of one 16-column tile each.  A product's k index runs as 16 s + 4 g + j
+// (s the step, g = lane / 16, j the element of the lane's 4): A comes as 16-byte
+// LDS reads (row strides of an odd number of 16-byte units), B either as 16
+// bytes of a weight's row (products with the transposed weights) or as one
+// float of each of 4 rows.  Bound by the MFMAs of one CU a block (~22,000 cycles
+// a SIMD, 9 us) and the latency of the weights from L2 before them.
+constexpr int TR_ROWS = 16, TR_WAVES = 16;
+constexpr int X_STR = D_IN + 4, H_STR = D_H + 4, E_STR = D_E + 4;
+constexpr int N_BIAS = 2 * D_H + D_E;  // b1, b2, b3
+
+// acc += A[16 x K] * W^T for the columns n0 .. n0 + 15 (W row-major, ldw).
+template <int K>
+__device__ inline f32x4_t mul_wt(const float* a, int stride, const float* __restrict__ W, int ldw, int lane) {
+    const int c = lane & 15, g = lane >> 4;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int FULL = K / 16;
+    static_assert(K % 8 == 0, "half steps");
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float a[4], b[4];
+    for (int s = 0; s < FULL; ++s) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(a + c * stride + 16 * s + 4 * g);
+        const f32x4_t w = *reinterpret_cast<const f32x4_t*>(W + (size_t)c * ldw + 16 * s + 4 * g);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], w[j], acc, 0, 0, 0);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty + 16 * i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx + 16 * j;
-            if (n >= N) continue;
-            float v = acc[i][j] + (bias ? bias[n] : 0.f);
-            if (accumulate) v += C[(size_t)m * ldc + n];
-            if (Z) Z[(size_t)m * ldc + n] = v;
-            C[(size_t)m * ldc + n] = gelu_out ? gelu(v) : v;
+    if (K % 16) {
+        f32x4_t x = {0.f, 0.f, 0.f, 0.f}, w = x;
+        if (g < 2) {
+            x = *reinterpret_cast<const f32x4_t*>(a + c * stride + 16 * FULL + 4 * g);
+            w = *reinterpret_cast<const f32x4_t*>(W + (size_t)c * ldw + 16 * FULL + 4 * g);
         }
-    }
-}
-
-// Standardised inputs: rows 2b and 2b+1 of X are pairs[b]'s two contigs.
-__global__ void k_gather_pairs(const float* __restrict__ tnf, const uint32_t* __restrict__ pi,
-                               const uint32_t* __restrict__ pj, uint32_t B, const float* __restrict__ mean,
-                               const float* __restrict__ istd, float* __restrict__ X) {
-    const uint32_t r = blockIdx.x, k = threadIdx.x;
-    if (r >= 2 * B || k >= D_IN) return;
-    const uint32_t c = (r & 1) ? pj[r >> 1] : pi[r >> 1];
-    float v = tnf[(size_t)c * D_IN + k];
-    if (v != v) v = 0.f;  // rows with no valid window
-    X[(size_t)r * D_IN + k] = (v - mean[k]) * istd[k];
-}
-
-__global__ void k_gather_rows(const float* __restrict__ tnf, uint32_t n, const float* __restrict__ mean,
-                              const float* __restrict__ istd, float* __restrict__ X) {
-    const uint32_t r = blockIdx.x, k = threadIdx.x;
-    if (r >= n || k >= D_IN) return;
-    float v = tnf[(size_t)r * D_IN + k];
-    if (v != v) v = 0.f;
-    X[(size_t)r * D_IN + k] = (v - mean[k]) * istd[k];
-}
-
-// Loss and dL/dE for each pair (one wave per pair, lanes = 32 embedding
-// dims, 2 pairs per 64-wide wave).  loss_sum gets the batch sum.
-__global__ void k_pair_loss(const float* __restrict__ E, const float* __restrict__ y, uint32_t B, float margin,
-                            float* __restrict__ dE, float* __restrict__ loss_sum) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t b = g >> 5, d = g & 31;
-    float diff = 0.f;
-    if (b < B) diff = E[(size_t)(2 * b) * D_E + d] - E[(size_t)(2 * b + 1) * D_E + d];
-    float D = diff * diff;
 #pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) D += __shfl_xor(D, off, 32);
-    if (b >= B) return;
-    const float lab = y[b];
-    const float l = lab * D + (1.f - lab) * fmaxf(margin - D, 0.f);
-    const float dldD = (lab + (1.f - lab) * (D < margin ? -1.f : 0.f)) / (float)B;
-    dE[(size_t)(2 * b) * D_E + d] = dldD * 2.f * diff;
-    dE[(size_t)(2 * b + 1) * D_E + d] = -dldD * 2.f * diff;
-    if (d == 0) atomicAdd(loss_sum, l / (float)B);
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], w[j], acc, 0, 0, 0);
+    }
+    return acc;
 }
 
-// dZ = dA * gelu'(Z)
-__global__ void k_gelu_back(const float* __restrict__ dA, const float* __restrict__ Z, float* __restrict__ dZ,
-                            uint64_t count) {
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < count) dZ[k] = dA[k] * gelu_grad(Z[k]);
+// A[16 x K] * W for 16 columns (W: first of them, row-major, ldw).
+template <int K>
+__device__ inline f32x4_t mul_w(const float* a, int stride, const float* __restrict__ W, int ldw, int lane) {
+    const int c = lane & 15, g = lane >> 4;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < K / 16; ++s) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(a + c * stride + 16 * s + 4 * g);
+        float w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = W[(size_t)(16 * s + 4 * g + j) * ldw + c];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], w[j], acc, 0, 0, 0);
+    }
+    return acc;
 }
 
-// db[n] = sum_m dZ[m][n]: 64 columns x 16 row slices per block, the slices
-// summed in a fixed order.
-constexpr int CS_SLICES = 16;
-__global__ __launch_bounds__(64 * CS_SLICES) void k_colsum(const float* __restrict__ dZ, int M, int N,
-                                                          float* __restrict__ db) {
-    __shared__ float part[CS_SLICES][64];
-    const int c = threadIdx.x & 63, sl = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + c;
-    float s = 0.f;
-    if (n < N)
-        for (int m = sl; m < M; m += CS_SLICES) s += dZ[(size_t)m * N + n];
-    part[sl][c] = s;
+// Sum over the block's 16 rows of a tile's column (lane % 16).
+__device__ inline float column_sum(const f32x4_t v) {
+    float s = (v[0] + v[1]) + (v[2] + v[3]);
+    s += __shfl_xor(s, 16, 64);
+    return s + __shfl_xor(s, 32, 64);
+}
+
+struct TrainArgs {
+    const float* tnf;
+    const uint32_t *pi, *pj;
+    const float* label;
+    uint32_t B;
+    float margin;
+    const float *mean, *istd;
+    const float* w;  // BF16-rounded weights and FP32 biases
+    float *X, *A1, *A2, *dE, *dZ2, *dZ1;  // rows for the weight gradients
+    float* bias;  // per block: N_BIAS sums over its rows, then its loss
+};
+
+__global__ __launch_bounds__(64 * TR_WAVES) void k_train_rows(const TrainArgs A) {
+    __shared__ __align__(16) float xs[TR_ROWS * X_STR], h1[TR_ROWS * H_STR], h2[TR_ROWS * H_STR], de[TR_ROWS * E_STR];
+    __shared__ float ep[8][TR_ROWS][D_E + 1], ls[TR_ROWS / 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, r4 = 4 * (lane >> 4);  // this lane's column and first row of a result tile
+    const uint32_t row0 = blockIdx.x * TR_ROWS, M = 2 * A.B;
+    for (int e = tid; e < TR_ROWS * D_IN; e += 64 * TR_WAVES) {
+        const uint32_t r = e / D_IN, k = e % D_IN, row = row0 + r;
+        float v = 0.f;
+        if (row < M) {
+            const uint32_t contig = (row & 1) ? A.pj[row >> 1] : A.pi[row >> 1];
+            v = A.tnf[(size_t)contig * D_IN + k];
+            if (v != v) v = 0.f;  // rows with no valid window
+            v = (v - A.mean[k]) * A.istd[k];
+            A.X[(size_t)row * D_IN + k] = v;
+        }
+        xs[r * X_STR + k] = v;
+    }
     __syncthreads();
-    if (sl == 0 && n < N) {
-        float t = 0.f;
+    const int n0 = 16 * wave, n = n0 + c;
+    // a tile to its rows in LDS and in memory
+    auto put = [&](const f32x4_t v, float* lds, float* out) {
 #pragma unroll
-        for (int q = 0; q < CS_SLICES; ++q) t += part[q][c];
-        db[n] = t;
+        for (int r = 0; r < 4; ++r) {
+            if (lds) lds[(r4 + r) * H_STR + n] = v[r];
+            if (row0 + r4 + r < M) out[(size_t)(row0 + r4 + r) * D_H + n] = v[r];
+        }
+    };
+    f32x4_t z1 = mul_wt<D_IN>(xs, X_STR, A.w + OFF_W1 + n0 * D_IN, D_IN, lane), z2, t;
+    const float b1 = A.w[OFF_B1 + n], b2 = A.w[OFF_B2 + n];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        z1[r] += b1;
+        t[r] = gelu(z1[r]);
     }
+    put(t, h1, A.A1);
+    __syncthreads();
+    z2 = mul_wt<D_H>(h1, H_STR, A.w + OFF_W2 + n0 * D_H, D_H, lane);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        z2[r] += b2;
+        t[r] = gelu(z2[r]);
+    }
+    put(t, h2, A.A2);
+    __syncthreads();
+    {  // the 32 embedding columns, K in 8 slices of 32
+        const int e0 = 16 * (wave & 1), s = wave >> 1;
+        t = mul_wt<32>(h2 + 32 * s, H_STR, A.w + OFF_W3 + e0 * D_H + 32 * s, D_H, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ep[s][r4 + r][e0 + c] = t[r];
+    }
+    __syncthreads();
+    if (tid < TR_ROWS / 2 * D_E) {  // a pair's dimension a thread
+        const int p = tid >> 5, d = tid & 31;
+        const uint32_t pair = row0 / 2 + p;
+        float e[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            e[i] = A.w[OFF_B3 + d];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) e[i] += ep[s][2 * p + i][d];
+        }
+        const float diff = pair < A.B ? e[0] - e[1] : 0.f;
+        float D = diff * diff;
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1) D += __shfl_xor(D, off, 32);
+        const float lab = pair < A.B ? A.label[pair] : 0.f;
+        const float l = lab * D + (1.f - lab) * fmaxf(A.margin - D, 0.f);
+        const float dldD = (lab + (1.f - lab) * (D < A.margin ? -1.f : 0.f)) / (float)A.B;
+        const float g = pair < A.B ? dldD * 2.f * diff : 0.f;
+        de[2 * p * E_STR + d] = g;
+        de[(2 * p + 1) * E_STR + d] = -g;
+        if (pair < A.B) {
+            A.dE[(size_t)2 * pair * D_E + d] = g;
+            A.dE[(size_t)(2 * pair + 1) * D_E + d] = -g;
+        }
+        if (d == 0) ls[p] = pair < A.B ? l / (float)A.B : 0.f;
+    }
+    __syncthreads();
+    float* bias = A.bias + (size_t)blockIdx.x * (N_BIAS + 1);
+    t = mul_w<D_E>(de, E_STR, A.w + OFF_W3 + n0, D_H, lane);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r] *= gelu_grad(z2[r]);
+    put(t, h1, A.dZ2);  // h1: every wave is past the second layer
+    float s = column_sum(t);
+    if (lane < 16) bias[D_H + n] = s;
+    if (tid < D_E) {
+        float v = 0.f;
+        for (int r = 0; r < TR_ROWS; ++r) v += de[r * E_STR + tid];
+        bias[2 * D_H + tid] = v;
+    }
+    if (tid == 64) {
+        float v = 0.f;
+        for (int p = 0; p < TR_ROWS / 2; ++p) v += ls[p];
+        bias[N_BIAS] = v;
+    }
+    __syncthreads();
+    t = mul_w<D_H>(h1, H_STR, A.w + OFF_W2 + n0, D_H, lane);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r] *= gelu_grad(z1[r]);
+    put(t, nullptr, A.dZ1);
+    s = column_sum(t);
+    if (lane < 16) bias[n] = s;
 }
 
-// out[i] = sum over z < S of part[z * count + i], in order
-__global__ void k_sum_partials(const float* __restrict__ part, int S, size_t count, float* __restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
+// dW = dZ^T A over the rows of a split, one 32 x 32 tile of one weight a wave
+// (two rows a product, both operands straight from memory: 128-byte reads).
+// part: [split][N_PARAMS], the weights' places.
+constexpr int WG_T1 = D_H / 32 * ((D_IN + 31) / 32), WG_T2 = D_H / 32 * (D_H / 32), WG_T3 = D_E / 32 * (D_H / 32);
+constexpr int WG_TILES = WG_T1 + WG_T2 + WG_T3;
+
+__global__ __launch_bounds__(64) void k_weight_grad(const float* __restrict__ X, const float* __restrict__ A1,
+                                                    const float* __restrict__ A2, const float* __restrict__ dE,
+                                                    const float* __restrict__ dZ2, const float* __restrict__ dZ1,
+                                                    uint32_t M, uint32_t per, float* __restrict__ part) {
+    const int lane = threadIdx.x, c = lane & 31, h = lane >> 5;
+    int t = blockIdx.x;
+    const float *dz, *a;
+    int rows, cols, off;
+    if (t < WG_T1) {
+        dz = dZ1, a = X, rows = D_H, cols = D_IN, off = OFF_W1;
+    } else if (t < WG_T1 + WG_T2) {
+        dz = dZ2, a = A1, rows = D_H, cols = D_H, off = OFF_W2, t -= WG_T1;
+    } else {
+        dz = dE, a = A2, rows = D_E, cols = D_H, off = OFF_W3, t -= WG_T1 + WG_T2;
+    }
+    const int n0 = 32 * (t % (rows / 32)), k0 = 32 * (t / (rows / 32)), k = k0 + c;
+    const uint32_t m0 = blockIdx.y * per, m1 = min(M, m0 + per);  // per is even, M is even
+    const bool in = k < cols;
+    const float* pz = dz + (size_t)m0 * rows + (size_t)h * rows + n0 + c;
+    const float* pa = a + (size_t)m0 * cols + (size_t)h * cols + (in ? k : 0);
+    f32x16_t acc = {};
+    constexpr int U = 8;
+    for (uint32_t m = m0; m < m1; m += 2 * U) {
+        float x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool ok = m + 2 * u < m1;
+            x[u] = ok ? pz[(size_t)2 * u * rows] : 0.f;
+            y[u] = ok && in ? pa[(size_t)2 * u * cols] : 0.f;
+        }
+        pz += (size_t)2 * U * rows;
+        pa += (size_t)2 * U * cols;
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u], y[u], acc, 0, 0, 0);
+    }
+    float* out = part + (size_t)blockIdx.y * N_PARAMS + off + k;
+    if (in)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) out[(size_t)(n0 + (r & 3) + 8 * (r >> 2) + 4 * h) * cols] = acc[r];
+}
+
+// g: the weights' partial sums over the splits, the biases' and the loss over
+// the row blocks, in order; a thread a weight, a wave a bias.
+__device__ inline bool is_bias(uint32_t k) {
+    return (k >= (uint32_t)OFF_B1 && k < (uint32_t)OFF_W2) || (k >= (uint32_t)OFF_B2 && k < (uint32_t)OFF_W3) ||
+           k >= (uint32_t)OFF_B3;
+}
+constexpr uint32_t GS_WEIGHTS = (N_PARAMS + 255) / 256, GS_BLOCKS = GS_WEIGHTS + (N_BIAS + 1 + 3) / 4;
+
+__global__ __launch_bounds__(256) void k_grad_sum(const float* __restrict__ part, uint32_t splits,
+                                                  const float* __restrict__ bias, uint32_t blocks,
+                                                  float* __restrict__ g, float* __restrict__ loss) {
+    if (blockIdx.x < GS_WEIGHTS) {
+        const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+        if (k >= (uint32_t)N_PARAMS || is_bias(k)) return;
+        float t = 0.f;
+#pragma unroll 8
+        for (uint32_t z = 0; z < splits; ++z) t += part[(size_t)z * N_PARAMS + k];
+        g[k] = t;
+        return;
+    }
+    const uint32_t b = (blockIdx.x - GS_WEIGHTS) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (b > (uint32_t)N_BIAS) return;
     float t = 0.f;
-    for (int z = 0; z < S; ++z) t += part[(size_t)z * count + i];
-    out[i] = t;
+    for (uint32_t z = lane; z < blocks; z += 64) t += bias[(size_t)z * (N_BIAS + 1) + b];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) t += __shfl_xor(t, off, 64);
+    if (lane) return;
+    if (b == (uint32_t)N_BIAS)
+        *loss = t;
+    else
+        g[b < (uint32_t)D_H ? OFF_B1 + b : b < (uint32_t)(2 * D_H) ? OFF_B2 + b - D_H : OFF_B3 + b - 2 * D_H] = t;
 }
 
 // Adam on the FP32 master copy; writes the BF16-rounded weights the forward
@@ -209,8 +339,7 @@ __global__ void k_adam(float* __restrict__ p, float* __restrict__ wq, const floa
     m2[k] = v;
     const float w = p[k] - lr * (a / c1) / (sqrtf(v / c2) + eps);
     p[k] = w;
-    const bool is_bias = (k >= OFF_B1 && k < OFF_W2) || (k >= OFF_B2 && k < OFF_W3) || k >= OFF_B3;
-    wq[k] = is_bias ? w : bf16_round(w);
+    wq[k] = is_bias(k) ? w : bf16_round(w);
 }
 
 // One parameter block [off, off + count): weights are rounded to BF16, biases
@@ -432,91 +561,39 @@ int mlp_alloc(mdet_mlp* m, size_t bytes, void** out) {
     return MDET_OK;
 }
 
-dim3 gemm_grid(int M, int N) { return dim3((N + 63) / 64, (M + 63) / 64); }
-
-// forward for M rows of X (standardised input); writes Z1,A1,Z2,A2,E
-int mlp_forward(mdet_mlp* m, const float* X, int M, float* Z1, float* A1, float* Z2, float* A2, float* E) {
-    hipStream_t s = m->ctx->stream;
-    const float* w = m->wq;
-    hipLaunchKernelGGL((k_gemm<false, true>), gemm_grid(M, D_H), dim3(256), 0, s, X, D_IN, w + OFF_W1, D_IN, A1, D_H,
-                       Z1, M, D_H, D_IN, w + OFF_B1, 1, 0, D_IN, (size_t)0);
-    hipLaunchKernelGGL((k_gemm<false, true>), gemm_grid(M, D_H), dim3(256), 0, s, A1, D_H, w + OFF_W2, D_H, A2, D_H, Z2,
-                       M, D_H, D_H, w + OFF_B2, 1, 0, D_H, (size_t)0);
-    hipLaunchKernelGGL((k_gemm<false, true>), gemm_grid(M, D_E), dim3(256), 0, s, A2, D_H, w + OFF_W3, D_H, E, D_E,
-                       (float*)nullptr, M, D_E, D_H, w + OFF_B3, 0, 0, D_H, (size_t)0);
-    MDET_HIP(hipGetLastError());
-    return MDET_OK;
-}
-
 struct Scratch {
-    float *X, *Z1, *A1, *Z2, *A2, *E, *dE, *dA2, *dZ2, *dA1, *dZ1, *loss, *part;
+    float* loss;
 };
 
-// Weight gradients sum over the batch's rows: split into at most WG_SPLITS
-// slices of at least WG_MIN_ROWS rows, one partial product each, summed in
-// slice order (deterministic for a given batch size).
-constexpr int WG_SPLITS = 32, WG_MIN_ROWS = 64;
-int wg_splits(int M) { return std::max(1, std::min(WG_SPLITS, M / WG_MIN_ROWS)); }
-
-int scratch(mdet_mlp* m, int M, Scratch* S) {
-    mdet_ctx* c = m->ctx;
-    MDET_TRY(ctx_buf(c, "mlp.X", (size_t)M * D_IN, &S->X));
-    MDET_TRY(ctx_buf(c, "mlp.Z1", (size_t)M * D_H, &S->Z1));
-    MDET_TRY(ctx_buf(c, "mlp.A1", (size_t)M * D_H, &S->A1));
-    MDET_TRY(ctx_buf(c, "mlp.Z2", (size_t)M * D_H, &S->Z2));
-    MDET_TRY(ctx_buf(c, "mlp.A2", (size_t)M * D_H, &S->A2));
-    MDET_TRY(ctx_buf(c, "mlp.E", (size_t)M * D_E, &S->E));
-    MDET_TRY(ctx_buf(c, "mlp.dE", (size_t)M * D_E, &S->dE));
-    MDET_TRY(ctx_buf(c, "mlp.dA2", (size_t)M * D_H, &S->dA2));
-    MDET_TRY(ctx_buf(c, "mlp.dZ2", (size_t)M * D_H, &S->dZ2));
-    MDET_TRY(ctx_buf(c, "mlp.dA1", (size_t)M * D_H, &S->dA1));
-    MDET_TRY(ctx_buf(c, "mlp.dZ1", (size_t)M * D_H, &S->dZ1));
-    MDET_TRY(ctx_buf(c, "mlp.loss", 4, &S->loss));
-    MDET_TRY(ctx_buf(c, "mlp.part", (size_t)wg_splits(M) * std::max(D_H * D_H, D_H * D_IN), &S->part));
-    return MDET_OK;
-}
+// The weight gradients' sums over the batch's rows: at most WG_SPLITS splits of
+// at least WG_MIN_ROWS rows (one partial product each, summed in order, so the
+// result depends on the batch size only); 128 rows a split put ~900 waves to
+// work at 512 pairs.
+constexpr uint32_t WG_SPLITS = 32, WG_MIN_ROWS = 128;
 
 // loss + gradient (into m->g) of one batch of pairs
 int mlp_grad(mdet_mlp* m, const float* tnf, const uint32_t* pi, const uint32_t* pj, const float* y, uint32_t B,
              float margin, Scratch* S) {
     hipStream_t s = m->ctx->stream;
-    const int M = 2 * (int)B;
-    MDET_TRY(scratch(m, M, S));
-    MDET_HIP(hipMemsetAsync(S->loss, 0, 4, s));
-    hipLaunchKernelGGL(k_gather_pairs, dim3(M), dim3(160), 0, s, tnf, pi, pj, B, m->norm, m->norm + D_IN, S->X);
-    MDET_TRY(mlp_forward(m, S->X, M, S->Z1, S->A1, S->Z2, S->A2, S->E));
-    hipLaunchKernelGGL(k_pair_loss, dim3((B * 32 + 255) / 256), dim3(256), 0, s, S->E, y, B, margin, S->dE, S->loss);
-    const float* w = m->wq;
-    float* g = m->g;
-    // dW[rows x cols] = dZ^T A over the batch's M rows, split by rows
-    const int nsplit = wg_splits(M);
-    const int kchunk = ((M + nsplit - 1) / nsplit + 15) / 16 * 16;
-    auto weight_grad = [&](const float* dZ, int rows, const float* A, int cols, float* dW) {
-        dim3 grid = gemm_grid(rows, cols);
-        grid.z = (unsigned)nsplit;
-        const size_t count = (size_t)rows * cols;
-        hipLaunchKernelGGL((k_gemm<true, false>), grid, dim3(256), 0, s, dZ, rows, A, cols, S->part, cols,
-                           (float*)nullptr, rows, cols, M, (const float*)nullptr, 0, 0, kchunk, count);
-        hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, S->part, nsplit,
-                           count, dW);
-    };
-    const dim3 cs_block(64 * CS_SLICES);
-    // layer 3: dW3 = dE^T A2, db3 = sum dE, dA2 = dE W3
-    weight_grad(S->dE, D_E, S->A2, D_H, g + OFF_W3);
-    hipLaunchKernelGGL(k_colsum, dim3((D_E + 63) / 64), cs_block, 0, s, S->dE, M, D_E, g + OFF_B3);
-    hipLaunchKernelGGL((k_gemm<false, false>), gemm_grid(M, D_H), dim3(256), 0, s, S->dE, D_E, w + OFF_W3, D_H, S->dA2,
-                       D_H, (float*)nullptr, M, D_H, D_E, (const float*)nullptr, 0, 0, D_E, (size_t)0);
-    const uint64_t cnt = (uint64_t)M * D_H;
-    hipLaunchKernelGGL(k_gelu_back, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, S->dA2, S->Z2, S->dZ2, cnt);
-    // layer 2
-    weight_grad(S->dZ2, D_H, S->A1, D_H, g + OFF_W2);
-    hipLaunchKernelGGL(k_colsum, dim3((D_H + 63) / 64), cs_block, 0, s, S->dZ2, M, D_H, g + OFF_B2);
-    hipLaunchKernelGGL((k_gemm<false, false>), gemm_grid(M, D_H), dim3(256), 0, s, S->dZ2, D_H, w + OFF_W2, D_H,
-                       S->dA1, D_H, (float*)nullptr, M, D_H, D_H, (const float*)nullptr, 0, 0, D_H, (size_t)0);
-    hipLaunchKernelGGL(k_gelu_back, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, S->dA1, S->Z1, S->dZ1, cnt);
-    // layer 1
-    weight_grad(S->dZ1, D_H, S->X, D_IN, g + OFF_W1);
-    hipLaunchKernelGGL(k_colsum, dim3((D_H + 63) / 64), cs_block, 0, s, S->dZ1, M, D_H, g + OFF_B1);
+    mdet_ctx* c = m->ctx;
+    const uint32_t M = 2 * B, blocks = (M + TR_ROWS - 1) / TR_ROWS;
+    const uint32_t want = std::max(1u, std::min(WG_SPLITS, M / WG_MIN_ROWS));
+    const uint32_t per = ((M + want - 1) / want + 1) / 2 * 2, splits = (M + per - 1) / per;
+    TrainArgs A{tnf, pi, pj, y, B, margin, m->norm, m->norm + D_IN, m->wq};
+    float* part;
+    MDET_TRY(ctx_buf(c, "mlp.X", (size_t)M * D_IN, &A.X));
+    MDET_TRY(ctx_buf(c, "mlp.A1", (size_t)M * D_H, &A.A1));
+    MDET_TRY(ctx_buf(c, "mlp.A2", (size_t)M * D_H, &A.A2));
+    MDET_TRY(ctx_buf(c, "mlp.dE", (size_t)M * D_E, &A.dE));
+    MDET_TRY(ctx_buf(c, "mlp.dZ2", (size_t)M * D_H, &A.dZ2));
+    MDET_TRY(ctx_buf(c, "mlp.dZ1", (size_t)M * D_H, &A.dZ1));
+    MDET_TRY(ctx_buf(c, "mlp.bias", (size_t)blocks * (N_BIAS + 1), &A.bias));
+    MDET_TRY(ctx_buf(c, "mlp.part", (size_t)splits * N_PARAMS, &part));
+    MDET_TRY(ctx_buf(c, "mlp.loss", 4, &S->loss));
+    hipLaunchKernelGGL(k_train_rows, dim3(blocks), dim3(64 * TR_WAVES), 0, s, A);
+    hipLaunchKernelGGL(k_weight_grad, dim3(WG_TILES, splits), dim3(64), 0, s, A.X, A.A1, A.A2, A.dE, A.dZ2, A.dZ1, M,
+                       per, part);
+    hipLaunchKernelGGL(k_grad_sum, dim3(GS_BLOCKS), dim3(256), 0, s, part, splits, A.bias, blocks, m->g, S->loss);
     MDET_HIP(hipGetLastError());
     return MDET_OK;
 }
