@@ -13,19 +13,17 @@
 //   * Thread t reads words 4t .. 4t+3 of the chunk with one 16-byte load
 //     (a wave's load covers 1 KB) and the word before them for the halo:
 //     64 window ends per lane, so the per-lane tests (contig boundaries, N)
-//     are paid once per 64 windows.  A wave whose lanes all lie inside one
-//     contig each, N-free, counts with constant increments; otherwise every
-//     window's segment (of two) and 0/1 increment come from per-lane masks,
-//     without branches, and lanes spanning three contigs (contigs under 64
-//     bases) count window by window.
-//   * Windows are binned by their raw 8-bit code into block-shared LDS
-//     histograms per contig segment of the chunk; the fold to the 136 canonical
-//     columns (code and reverse complement) happens once per segment at flush,
-//     so the per-base work is extract + mask test + one LDS add.
+//     are paid once per 64 windows, as bit masks.  Windows go two at a time
+//     where both count towards one contig, the rest one by one, and lanes
+//     spanning three contigs (contigs under 64 bases) window by window.
+//   * Windows are binned by their raw codes (10 bits a pair, 8 a window) into
+//     block-shared LDS histograms per contig segment of the chunk; the fold to
+//     the 136 canonical columns (code and reverse complement) happens once per
+//     segment at flush, so the per-pair work is extract + mask test + one LDS
+//     add.
 //   * N bases come as a sorted run list; a block whose chunk meets runs turns
-//     them into an LDS bitmap of the chunk once (one dword per thread pass,
-//     a binary search over the run ends), and a word's 19-bit N mask is then
-//     one two-dword read.  Contig boundaries of the pass sit in registers.
+//     them into an LDS bitmap of the chunk once, and a lane's N mask is then
+//     three dwords of it.  Contig boundaries of the pass sit in registers.
 #include <hipcub/hipcub.hpp>
 
 #include <mutex>
@@ -39,15 +37,16 @@ constexpr int CNT_THREADS = 256;
 constexpr int CNT_WORDS = 4;  // consecutive words per thread (64 window ends)
 constexpr uint64_t CNT_CHUNK = (uint64_t)CNT_THREADS * CNT_WORDS * 16;
 constexpr int CNT_MAXSEG = 4;  // contig segments histogrammed per pass
-// Each segment's histogram exists in CNT_COPIES copies, lane l adding into copy
-// l % CNT_COPIES: same-bin adds of one wave instruction (frequent: 64 windows
-// over 256 codes) spread over the copies, and the copy stride of 264 words
-// (8 banks apart) spreads them over the LDS banks.  4 segments x 4 copies keep
-// the block at 19 KB of LDS; more segments or copies per pass cost more in
-// zeroing, folding and occupancy than they save.
-constexpr int CNT_COPIES = 4, CNT_CSTRIDE = 264;
-// N runs of a chunk kept in LDS as chunk-relative int32 (more: read from global memory)
-constexpr int CNT_RUNS = 64;
+// LDS adds bound the counting, so two neighbouring windows (5 bases) are one add
+// into a histogram of 1,024 codes wherever both count towards one contig in
+// every lane of a wave; the others, at contig ends and N runs, go one by one
+// into a histogram of 256 codes.  The fold adds a 4-base code's windows up from
+// the 5-base codes that begin or end with it.  With the larger code space adds
+// of one wave instruction to one bin are rare, so one copy of it does; 4
+// segments keep the block at 23 KB of LDS.  2.65e9 windows: 622 us (LDS and VALU
+// about half busy each, the rest latency of the short blocks); one add
+// a window (four copies of 256 codes): 752 us.
+constexpr int CNT_PAIRS = 1024, CNT_SEGSZ = CNT_PAIRS + 256;  // words of a segment's histograms
 // dwords of the per-chunk N bitmap: positions -32 .. CNT_CHUNK + 31
 constexpr int CNT_NBM = (int)(CNT_CHUNK / 32) + 2;
 
@@ -128,14 +127,13 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
                                                               const uint64_t* __restrict__ base_off,
                                                               const longlong4* __restrict__ meta,
                                                               uint32_t* __restrict__ counts) {
-    constexpr int SEGSZ = CNT_COPIES * CNT_CSTRIDE;  // words of one segment's histograms
+    constexpr int SEGSZ = CNT_SEGSZ;
     __shared__ __align__(16) uint32_t hist[CNT_MAXSEG][SEGSZ];
     __shared__ uint32_t fold[CNT_MAXSEG][136];
     // positions relative to the chunk start, as int32, clamped to [-4,
     // length + 17]: every comparison with a window of the chunk keeps its
     // outcome, and the per-lane tests stay 32-bit
     __shared__ int32_t seg[CNT_MAXSEG + 1];
-    __shared__ int32_t run_s[CNT_RUNS], run_e[CNT_RUNS];
     // N bitmap of the chunk: bit b is position b - 32 (the halo before the
     // chunk included); built once per chunk with N runs
     __shared__ uint32_t nbm[CNT_NBM];
@@ -145,40 +143,12 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
     const uint64_t chunk_hi = min(chunk_lo + CNT_CHUNK, n_bases);
     const int32_t clen = (int32_t)(chunk_hi - chunk_lo);
     const longlong4 mt = meta[blockIdx.x];
-    const int64_t c_first = mt.x, c_last = mt.y;
-    const int64_t r_first = mt.z, r_last = mt.w;
-    auto rel = [&](uint64_t p) {
-        const int64_t d = (int64_t)p - (int64_t)chunk_lo;
-        return (int32_t)(d < -4 ? -4 : (d > clen + 17 ? clen + 17 : d));
-    };
-    const int nr = (int)(r_last - r_first);
-    const bool any_n = nr > 0;
-    if (any_n) {
-        const bool runs_lds = nr <= CNT_RUNS;
-        if (runs_lds && tid < nr) {
-            run_s[tid] = rel(runs[2 * (r_first + tid)]);
-            run_e[tid] = rel(runs[2 * (r_first + tid) + 1]);
-        }
-        __syncthreads();
-        // zero the bitmap, then each run ORs its bits into the dwords it
-        // covers (runs are disjoint; most cover one or two dwords)
-        for (int d = tid; d < CNT_NBM; d += CNT_THREADS) nbm[d] = 0u;
-        __syncthreads();
-        for (int r = tid; r < nr; r += CNT_THREADS) {
-            const int32_t rs = (runs_lds ? run_s[r] : rel(runs[2 * (r_first + r)])) + 32;
-            const int32_t re = (runs_lds ? run_e[r] : rel(runs[2 * (r_first + r) + 1])) + 32;
-            // bits [rs, re) of the bitmap; rel() keeps both in [28, clen + 49]
-            for (int32_t d = rs >> 5; d <= (re - 1) >> 5 && rs < re; ++d) {
-                const int32_t x0 = max(rs - 32 * d, 0), x1 = min(re - 32 * d, 32);
-                atomicOr(&nbm[d], (uint32_t)(((1ull << x1) - 1ull) & ~((1ull << x0) - 1ull)));
-            }
-        }
-        __syncthreads();
-    }
 
     // This lane's 64 window ends q0 .. q0 + 63: words 4 tid .. 4 tid + 3 of the
     // chunk (one 16-byte load where aligned and whole) and the word before
-    // them (the 3-base halo of the first windows).
+    // them (the 3-base halo of the first windows).  A block lives for a few
+    // microseconds, most of them waiting: these loads, then the runs' and the
+    // boundaries' go out before the histograms are cleared.
     const int32_t q0 = tid * 64;
     const uint64_t w0 = chunk_lo / 16;
     const uint64_t n_words = (n_bases + 15) / 16;
@@ -198,6 +168,48 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
         }
         if (w0 + i0 > 0) H = packed[w0 + i0 - 1];
     }
+    const int64_t c_first = mt.x, c_last = mt.y;
+    const int64_t r_first = mt.z, r_last = mt.w;
+    auto rel = [&](uint64_t p) {
+        const int64_t d = (int64_t)p - (int64_t)chunk_lo;
+        return (int32_t)(d < -4 ? -4 : (d > clen + 17 ? clen + 17 : d));
+    };
+    const int nr = (int)(r_last - r_first);
+    const bool any_n = nr > 0;
+    uint64_t rs0 = 0, re0 = 0, off0 = 0;
+    if (tid < nr) {
+        rs0 = runs[2 * (r_first + tid)];
+        re0 = runs[2 * (r_first + tid) + 1];
+    }
+    const int nseg0 = (int)min<int64_t>(CNT_MAXSEG, c_last - c_first + 1);
+    if (tid <= CNT_MAXSEG && tid <= nseg0) off0 = base_off[c_first + tid];
+    auto clear = [&](int nseg) {
+        for (int i = tid; i < nseg * SEGSZ / 4; i += CNT_THREADS)
+            reinterpret_cast<uint4*>(&hist[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
+        for (int i = tid; i < CNT_MAXSEG * 136; i += CNT_THREADS) (&fold[0][0])[i] = 0;
+    };
+    clear(nseg0);
+    // the N bitmap: each run ORs its bits into the dwords it covers (runs are
+    // disjoint; most cover one or two dwords)
+    if (any_n) {
+        for (int d = tid; d < CNT_NBM; d += CNT_THREADS) nbm[d] = 0u;
+        __syncthreads();
+        for (int r = tid; r < nr; r += CNT_THREADS) {
+            if (r != tid) {
+                rs0 = runs[2 * (r_first + r)];
+                re0 = runs[2 * (r_first + r) + 1];
+            }
+            const int32_t rs = rel(rs0) + 32, re = rel(re0) + 32;
+            // bits [rs, re) of the bitmap; rel() keeps both in [28, clen + 49]
+            for (int32_t d = rs >> 5; d <= (re - 1) >> 5 && rs < re; ++d) {
+                const int32_t x0 = max(rs - 32 * d, 0), x1 = min(re - 32 * d, 32);
+                atomicOr(&nbm[d], (uint32_t)(((1ull << x1) - 1ull) & ~((1ull << x0) - 1ull)));
+            }
+        }
+    }
+    // boundaries past the pass's last segment read as "never reached"
+    if (tid <= CNT_MAXSEG) seg[tid] = tid <= nseg0 ? rel(off0) : INT32_MAX;
+    __syncthreads();
     // window k's N test: bit k of nvalid (bases q0 + k - 3 .. q0 + k N-free)
     uint64_t nvalid = ~0ull;
     if (any_n) {
@@ -207,16 +219,15 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
         const uint64_t B = m2 >> 29;  // positions q0 + 61 .. q0 + 63
         nvalid = ~(A | (A >> 1) | (A >> 2) | (A >> 3) | (B << 61) | (B << 62) | (B << 63));
     }
-    uint32_t* const hcopy0 = &hist[0][0] + (tid % CNT_COPIES) * CNT_CSTRIDE;
 
     for (int64_t cs = c_first; cs <= c_last; cs += CNT_MAXSEG) {
         const int nseg = (int)min<int64_t>(CNT_MAXSEG, c_last - cs + 1);
-        // boundaries past the pass's last segment read as "never reached"
-        if (tid <= CNT_MAXSEG) seg[tid] = tid <= nseg ? rel(base_off[cs + tid]) : INT32_MAX;
-        for (int i = tid; i < nseg * SEGSZ / 4; i += CNT_THREADS)
-            reinterpret_cast<uint4*>(&hist[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
-        for (int i = tid; i < CNT_MAXSEG * 136; i += CNT_THREADS) (&fold[0][0])[i] = 0;
-        __syncthreads();
+        if (cs != c_first) {  // a chunk of more contigs: again for the next ones
+            __syncthreads();
+            if (tid <= CNT_MAXSEG) seg[tid] = tid <= nseg ? rel(base_off[cs + tid]) : INT32_MAX;
+            clear(nseg);
+            __syncthreads();
+        }
         int32_t sg[CNT_MAXSEG + 1];
 #pragma unroll
         for (int k = 0; k <= CNT_MAXSEG; ++k) sg[k] = seg[k];
@@ -251,25 +262,38 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
             V &= nvalid;
             S &= V;
         }
-        uint32_t* const h0 = hcopy0 + t * SEGSZ;
-        // 16 windows (one word) at a time: where every lane's 16 are all
-        // counted into one segment, constant increments; else each window's
-        // segment (t or t + 1) and 0/1 increment from the masks, no branches
+        uint32_t* const h0 = &hist[t][0];
+        // windows in pairs (bit 2k of P: both of a pair count, into one
+        // segment), 8 pairs of a word at a time, the increment 0 or 1 and, where
+        // a lane's word meets a contig's end, the segment (t or t + 1) from the
+        // masks; what is left, U, window by window
+        const uint64_t P = V & (V >> 1) & ~(S ^ (S >> 1)) & 0x5555555555555555ull;
+        uint64_t U = V & ~(P | (P << 1));
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             const uint64_t x = ((uint64_t)W[m] << 32) | (m ? W[m > 0 ? m - 1 : 0] : H);
-            const uint32_t v16 = (uint32_t)(V >> (16 * m)) & 0xFFFFu, s16 = (uint32_t)(S >> (16 * m)) & 0xFFFFu;
-            if (__all(v16 == 0xFFFFu && (s16 == 0u || s16 == 0xFFFFu))) {
+            const uint32_t p16 = (uint32_t)(P >> (16 * m)) & 0xFFFFu, s16 = (uint32_t)(S >> (16 * m)) & 0xFFFFu;
+            // (N bases are scattered: in nearly every word some lane has one)
+            if (__all(s16 == 0u || s16 == 0xFFFFu)) {
                 uint32_t* const h = s16 ? h0 + SEGSZ : h0;
 #pragma unroll
-                for (int k = 0; k < 16; ++k) atomicAdd(&h[(uint32_t)(x >> (26 + 2 * k)) & 0xFFu], 1u);
+                for (int k = 0; k < 16; k += 2)
+                    atomicAdd(&h[(uint32_t)(x >> (26 + 2 * k)) & 0x3FFu], (p16 >> k) & 1u);
             } else {
 #pragma unroll
-                for (int k = 0; k < 16; ++k) {
-                    const uint32_t code = (uint32_t)(x >> (26 + 2 * k)) & 0xFFu;
-                    atomicAdd(&h0[((s16 >> k) & 1u) * SEGSZ + code], (v16 >> k) & 1u);
-                }
+                for (int k = 0; k < 16; k += 2)
+                    atomicAdd(&h0[((s16 >> k) & 1u) * SEGSZ + ((uint32_t)(x >> (26 + 2 * k)) & 0x3FFu)],
+                              (p16 >> k) & 1u);
             }
+        }
+        for (; __any(U != 0); U &= U - 1) {
+            if (!U) continue;
+            const int k = __builtin_ctzll(U), m = k >> 4;
+            const uint32_t hi = m == 0 ? W[0] : m == 1 ? W[1] : m == 2 ? W[2] : W[3];
+            const uint32_t lo = m == 0 ? H : m == 1 ? W[0] : m == 2 ? W[1] : W[2];
+            const uint64_t x = ((uint64_t)hi << 32) | lo;
+            atomicAdd(&h0[(uint32_t)((S >> k) & 1u) * SEGSZ + CNT_PAIRS + ((uint32_t)(x >> (26 + 2 * (k & 15))) & 0xFFu)],
+                      1u);
         }
         if (general) {
 #pragma unroll
@@ -283,7 +307,7 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
                     for (int j = 1; j <= CNT_MAXSEG; ++j) u += sg[j] <= p ? 1 : 0;
                     const int32_t u_lo = seg[u < CNT_MAXSEG ? u : CNT_MAXSEG];
                     const bool ok = p < clen && u < nseg && p >= u_lo + 3 && ((nvalid >> (16 * m + k)) & 1ull);
-                    if (ok) atomicAdd(hcopy0 + u * SEGSZ + ((uint32_t)(x >> (26 + 2 * k)) & 0xFFu), 1u);
+                    if (ok) atomicAdd(&hist[u][CNT_PAIRS + ((uint32_t)(x >> (26 + 2 * k)) & 0xFFu)], 1u);
                 }
             }
         }
@@ -291,9 +315,10 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
         // fold raw codes into canonical columns, then one global add per
         // nonzero column (a contig may span several chunks)
         for (int s = 0; s < nseg; ++s) {
-            uint32_t v = 0;
+            const uint4 last = *reinterpret_cast<const uint4*>(&hist[s][4 * tid]);  // pairs whose second window it is
+            uint32_t v = hist[s][CNT_PAIRS + tid] + ((last.x + last.y) + (last.z + last.w));
 #pragma unroll
-            for (int c = 0; c < CNT_COPIES; ++c) v += hist[s][c * CNT_CSTRIDE + tid];
+            for (int c = 0; c < 4; ++c) v += hist[s][256 * c + tid];  // ... whose first
             if (v) atomicAdd(&fold[s][c_colmap[tid]], v);
         }
         __syncthreads();
@@ -302,7 +327,6 @@ __global__ __launch_bounds__(CNT_THREADS) void k_count_packed(const uint32_t* __
             uint32_t v = fold[s][col];
             if (v) atomicAdd(&counts[(uint64_t)(cs + s) * 136 + col], v);
         }
-        __syncthreads();
     }
 }
 
