@@ -29,7 +29,7 @@ using mdet::PROJ_KS;
 using mdet::PROJ_W;
 
 constexpr int NT = 136;
-constexpr uint32_t COV_SAMPLE = 2048, COV_SPLITS = 32;
+constexpr uint32_t COV_SAMPLE = 2048, COV_SPLITS = 64;
 
 // Words PROJ_D.. of a projected row.
 constexpr int PW_PART = 28;  // sum of squares of the FP16-rounded coordinates
@@ -107,6 +107,7 @@ __global__ __launch_bounds__(256) void k_cov_sum(const float* __restrict__ part,
     if (e >= NT * NT) return;
     const uint32_t i = e / NT, j = e % NT;
     float c = 0.f, mi = 0.f, mj = 0.f, cnt = 0.f;
+#pragma unroll 8
     for (uint32_t s = 0; s < COV_SPLITS; ++s) {
         c += part[(size_t)s * NT * NT + e];
         mi += msum[s * (NT + 1) + i];
@@ -118,81 +119,129 @@ __global__ __launch_bounds__(256) void k_cov_sum(const float* __restrict__ part,
     if (j == 0) mean[i] = mi * inv;
 }
 
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 // The directions, one block: V = W (random signs), twice V = orthonormal basis
 // of C V (Cholesky QR of the 28 columns, the second time repeated for
 // accuracy), columns ordered by their variance, then scaled so that the
-// largest row sum of |P^T P|, a bound of |P|^2, is below 1.  Bound by the
-// latency of one CU (three 136 x 136 x 32 products and 28-step
-// factorisations); everything stays in its LDS.
+// largest row sum of |P^T P|, a bound of |P|^2, is below 1.  Everything stays
+// in one CU's LDS; the products are FP32 MFMAs (v_mfma_f32_32x32x2, a wave per
+// 32 rows), the 28 x 28 factorisation and its inverse one wave's registers.
+// Bound by these serial chains: 54 us (116 us with scalar products and a
+// barrier per factorisation step).
 // basis: P as [4][136][8] (coordinate 7 g + j of group g at [g][k][j]); off:
 // P mean [28]; sig: standard deviation of each coordinate.
-constexpr int B_THREADS = 1024;
+constexpr int B_THREADS = 512, B_WAVES = B_THREADS / 64, B_TILES = (NT + 31) / 32;
+constexpr int B_STR = PROJ_W + 1;  // rows apart by an odd number of banks: columns are read too
 
-__device__ inline void basis_mul(const float (*C)[NT], const float (*V)[PROJ_W], float (*Y)[PROJ_W]) {
-    for (int t = threadIdx.x; t < NT * 8; t += B_THREADS) {
-        const int r = t >> 3, c = (t & 7) * 4;
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int k = 0; k < NT; ++k) {
-            const float x = C[r][k];
-            const float4 v = *reinterpret_cast<const float4*>(&V[k][c]);
-            a.x = fmaf(x, v.x, a.x);
-            a.y = fmaf(x, v.y, a.y);
-            a.z = fmaf(x, v.z, a.z);
-            a.w = fmaf(x, v.w, a.w);
+// Y[136 x 32] = A B: A(m, k) row m of 136, K even, B(k, n).
+template <int K, class FA, class FB>
+__device__ inline void basis_product(FA A, FB B, float (*Y)[B_STR]) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int c = lane & 31, h = lane >> 5;
+    if (wave < B_TILES) {
+        const int m = min(32 * wave + c, NT - 1);
+        f32x16_t acc = {};
+#pragma unroll 4
+        for (int k = 0; k < K; k += 2) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(A(m, k + h), B(k + h, c), acc, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = 32 * wave + (r & 3) + 8 * (r >> 2) + 4 * h;
+            if (row < NT) Y[row][c] = acc[r];
         }
-        *reinterpret_cast<float4*>(&Y[r][c]) = a;
     }
     __syncthreads();
+}
+
+// G = A^T B of two 136 x 32 matrices, the rows split over the waves.
+__device__ inline void basis_gram(const float (*A)[B_STR], const float (*B)[B_STR], float (*part)[PROJ_W][B_STR],
+                                  float (*G)[B_STR]) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int c = lane & 31, h = lane >> 5;
+    f32x16_t acc = {};
+    constexpr int PER = (NT / 2 + B_WAVES - 1) / B_WAVES;  // row pairs a wave
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int k = 2 * (wave * PER + q) + h;
+        const float x = k < NT ? A[k][c] : 0.f, y = k < NT ? B[k][c] : 0.f;
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][(r & 3) + 8 * (r >> 2) + 4 * h][c] = acc[r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < PROJ_W * PROJ_W; e += B_THREADS) {
+        float g = 0.f;
+#pragma unroll
+        for (int w = 0; w < B_WAVES; ++w) g += part[w][e / PROJ_W][e % PROJ_W];
+        G[e / PROJ_W][e % PROJ_W] = g;
+    }
+    __syncthreads();
+}
+
+__device__ inline float lane_value(float v, int lane) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
 }
 
 // V = orthonormal columns spanning Y's (Y may be V); columns whose remainder
-// vanishes become zero.
-__device__ inline void basis_orth(const float (*Y)[PROJ_W], float (*V)[PROJ_W], float (*G)[PROJ_W + 1]) {
-    const int i = threadIdx.x >> 5, j = threadIdx.x & 31;
-    float g = 0.f;
-    for (int k = 0; k < NT; ++k) g = fmaf(Y[k][i], Y[k][j], g);
-    G[i][j] = g;
-    __syncthreads();
-    float gmax = 0.f;
-    for (int k = 0; k < PROJ_D; ++k) gmax = fmaxf(gmax, G[k][k]);
-    __syncthreads();
-    for (int k = 0; k < PROJ_D; ++k) {  // right-looking Cholesky, L in the lower triangle
-        const float p = G[k][k];
-        const float r = p > 1e-7f * gmax ? 1.f / sqrtf(p) : 0.f;
-        const float lik = i > k ? G[i][k] * r : 0.f, ljk = j > k ? G[j][k] * r : 0.f;
-        __syncthreads();
-        if (j == k && i > k) G[i][k] = lik;
-        if (i == k && j == k) G[k][k] = r;  // the reciprocal of the diagonal
-        if (i > k && j > k && j <= i) G[i][j] -= lik * ljk;
-        __syncthreads();
-    }
-    for (int r = threadIdx.x; r < NT; r += B_THREADS) {  // v L^T = y, row by row
-        float v[PROJ_D];
+// vanishes become zero.  G = Y^T Y = L L^T, V = Y L^-T.
+__device__ inline void basis_orth(const float (*Y)[B_STR], float (*V)[B_STR], float (*part)[PROJ_W][B_STR],
+                                  float (*G)[B_STR], float (*T)[B_STR]) {
+    basis_gram(Y, Y, part, G);
+    if (threadIdx.x < 64) {
+        const int i = threadIdx.x & 31;
+        float g[PROJ_D], diag[PROJ_D];  // row i of G, of L as it comes; 1 / L[k][k] (0: dropped)
+        float gmax = 0.f;
 #pragma unroll
-        for (int c = 0; c < PROJ_D; ++c) {
-            float s = Y[r][c];
-#pragma unroll
-            for (int k = 0; k < c; ++k) s = fmaf(-v[k], G[c][k], s);
-            v[c] = s * G[c][c];
+        for (int k = 0; k < PROJ_D; ++k) {
+            g[k] = G[i][k];
+            gmax = fmaxf(gmax, G[k][k]);
         }
 #pragma unroll
-        for (int c = 0; c < PROJ_D; ++c) V[r][c] = v[c];
+        for (int k = 0; k < PROJ_D; ++k) {
+            const float p = lane_value(g[k], k);
+            diag[k] = p > 1e-7f * gmax ? __builtin_amdgcn_rsqf(p) : 0.f;
+            g[k] *= diag[k];
 #pragma unroll
-        for (int c = PROJ_D; c < PROJ_W; ++c) V[r][c] = 0.f;
+            for (int j = k + 1; j < PROJ_D; ++j) g[j] = fmaf(-g[k], lane_value(g[k], j), g[j]);
+        }
+        float x[PROJ_D];  // column i of L^-1
+#pragma unroll
+        for (int r = 0; r < PROJ_D; ++r) {
+            float s = r == i ? 1.f : 0.f;
+#pragma unroll
+            for (int k = 0; k < r; ++k) s = fmaf(-lane_value(g[k], r), x[k], s);
+            x[r] = s * diag[r];
+        }
+        if (threadIdx.x < 32)
+#pragma unroll
+            for (int r = 0; r < PROJ_W; ++r) T[i][r] = r < PROJ_D && i < PROJ_D ? x[r < PROJ_D ? r : 0] : 0.f;
     }
     __syncthreads();
+    // (a wave reads its own 32 rows before it writes them)
+    basis_product<PROJ_W>([&](int m, int k) { return Y[m][k]; }, [&](int k, int n) { return T[k][n]; }, V);
 }
 
-__global__ __launch_bounds__(B_THREADS) void k_basis(const float* __restrict__ Cg, const float* __restrict__ mean,
+__global__ __launch_bounds__(B_THREADS, 2) void k_basis(const float* __restrict__ Cg, const float* __restrict__ mean,
                                                      float* __restrict__ basis, float* __restrict__ off,
                                                      float* __restrict__ sig) {
     __shared__ __align__(16) float C[NT][NT];
-    __shared__ __align__(16) float V[NT][PROJ_W], Y[NT][PROJ_W];
-    __shared__ float G[PROJ_W][PROJ_W + 1];
-    __shared__ float var[PROJ_W], scale;
+    __shared__ float V[NT][B_STR], Y[NT][B_STR], part[B_WAVES][PROJ_W][B_STR];
+    __shared__ float G[PROJ_W][B_STR], T[PROJ_W][B_STR];
+    __shared__ float var[PROJ_W], rowsum[PROJ_W], pm[16][PROJ_W], scale;
     __shared__ int place[PROJ_W];
     const int tid = threadIdx.x;
-    for (int e = tid; e < NT * NT; e += B_THREADS) C[e / NT][e % NT] = Cg[e];
+    {  // all 16-byte loads of C at once
+        constexpr int LOADS = (NT * NT / 4 + B_THREADS - 1) / B_THREADS;
+        f32x4_t v[LOADS];
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q)
+            v[q] = reinterpret_cast<const f32x4_t*>(Cg)[min(tid + q * B_THREADS, NT * NT / 4 - 1)];
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q)
+            if (tid + q * B_THREADS < NT * NT / 4) reinterpret_cast<f32x4_t*>(&C[0][0])[tid + q * B_THREADS] = v[q];
+    }
     for (int e = tid; e < NT * PROJ_W; e += B_THREADS) {
         uint32_t h = (uint32_t)e * 0x9E3779B9u + 0x7F4A7C15u;
         h = (h ^ (h >> 16)) * 0x85EBCA6Bu;
@@ -200,43 +249,49 @@ __global__ __launch_bounds__(B_THREADS) void k_basis(const float* __restrict__ C
         V[e / PROJ_W][e % PROJ_W] = e % PROJ_W < PROJ_D ? ((h >> 31) ? 1.f : -1.f) : 0.f;
     }
     __syncthreads();
-    basis_mul(C, V, Y);
-    basis_orth(Y, V, G);
-    basis_mul(C, V, Y);
-    basis_orth(Y, V, G);
-    basis_orth(V, V, G);
-    basis_mul(C, V, Y);
+    // C is symmetric: row k, consecutive lanes
+    auto mul = [&]() {
+        basis_product<NT>([&](int m, int k) { return C[k][m]; }, [&](int k, int n) { return V[k][n]; }, Y);
+    };
+    // one loop: straight-line copies of the factorisation are instruction misses
+#pragma unroll 1
+    for (int pass = 0; pass < 4; ++pass) {
+        if (pass != 2) mul();
+        if (pass < 3) basis_orth(pass == 2 ? V : Y, V, part, G, T);
+    }
+    basis_gram(V, Y, part, T);  // variances on its diagonal
+    basis_gram(V, V, part, G);
     if (tid < PROJ_W) {
+        var[tid] = tid < PROJ_D ? fmaxf(T[tid][tid], 0.f) : -1.f;
         float s = 0.f;
-        for (int k = 0; k < NT; ++k) s = fmaf(V[k][tid], Y[k][tid], s);
-        var[tid] = tid < PROJ_D ? fmaxf(s, 0.f) : -1.f;
+#pragma unroll
+        for (int b = 0; b < PROJ_D; ++b) s += fabsf(G[tid][b]);
+        rowsum[tid] = s;
     }
-    const int i = tid >> 5, j = tid & 31;
-    float g = 0.f;
-    for (int k = 0; k < NT; ++k) g = fmaf(V[k][i], V[k][j], g);
-    G[i][j] = fabsf(g);
+    {  // P mean, unscaled: 16 slices of the rows
+        const int c = tid & 31, q = tid >> 5;
+        float s = 0.f;
+        for (int k = q; k < NT; k += 16) s = fmaf(V[k][c], mean[k], s);
+        pm[q][c] = s;
+    }
     __syncthreads();
-    if (tid < PROJ_D) {  // rank by variance, ties by index
-        int p = 0;
-        for (int c = 0; c < PROJ_D; ++c) p += (var[c] > var[tid] || (var[c] == var[tid] && c < tid)) ? 1 : 0;
-        place[tid] = p;
-    }
-    if (tid == 0) {
-        float m = 0.f;
-        bool ok = true;
-        for (int a = 0; a < PROJ_D; ++a) {
-            float s = 0.f;
-            for (int b = 0; b < PROJ_D; ++b) s += G[a][b];
-            ok = ok && finite_bits(s);
-            m = fmaxf(m, s);
-        }
-        for (int a = 0; a < PROJ_D; ++a) ok = ok && finite_bits(var[a]);
+    if (tid < 64) {
+        const int c = tid & 31;
+        float m = c < PROJ_D ? rowsum[c] : 0.f;
+        const bool fine = c >= PROJ_D || (finite_bits(m) && finite_bits(var[c]));
+        const bool ok = __all(fine);
+#pragma unroll
+        for (int o = 16; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
         // |P|^2 <= the largest row sum; a basis that did not come out finite is dropped (P = 0: no tile is)
-        scale = ok && m > 0.f ? 1.f / sqrtf(m * (1.f + 1e-5f)) : 0.f;
+        if (tid == 0) scale = ok && m > 0.f ? 1.f / sqrtf(m * (1.f + 1e-5f)) : 0.f;
+        if (tid < PROJ_D) {  // rank by variance, ties by index
+            int p = 0;
+#pragma unroll
+            for (int d = 0; d < PROJ_D; ++d)
+                p += (var[d] > var[tid] || (var[d] == var[tid] && d < tid)) ? 1 : 0;
+            place[tid] = ok ? p : tid;  // not a permutation otherwise
+        }
     }
-    __syncthreads();
-    if (!(scale > 0.f))  // place may not be a permutation
-        for (int e = tid; e < PROJ_D; e += B_THREADS) place[e] = e;
     __syncthreads();
     for (int e = tid; e < NT * PROJ_D; e += B_THREADS) {
         const int k = e / PROJ_D, c = e % PROJ_D, p = place[c];
@@ -245,9 +300,9 @@ __global__ __launch_bounds__(B_THREADS) void k_basis(const float* __restrict__ C
     for (int e = tid; e < 4 * NT; e += B_THREADS) basis[e * 8 + 7] = 0.f;
     if (tid < PROJ_D) {
         float s = 0.f;
-        if (scale > 0.f)
-            for (int k = 0; k < NT; ++k) s = fmaf(V[k][tid] * scale, mean[k], s);
-        off[place[tid]] = s;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) s += pm[q][tid];
+        off[place[tid]] = scale > 0.f ? s * scale : 0.f;
         sig[place[tid]] = scale > 0.f ? sqrtf(var[tid]) * scale : 0.f;
     }
 }
@@ -333,9 +388,6 @@ __global__ __launch_bounds__(256) void k_project(const float* __restrict__ tnf, 
 constexpr uint32_t CL_SAMPLE = 16384, CL_ROWS = 96, CL_MIN = 64, CL_MAX = 4096;
 constexpr int CL_SIGNS = 12;
 constexpr float CL_FIX = 16384.f;  // fixed point of the centres' sums (sums that do not depend on the order)
-
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 // Centres c [k][PROJ_W]: from the sample's rows (sums == null), or the means of
 // the rows assigned to them (a centre without rows stays); their MFMA fragments
@@ -558,16 +610,20 @@ __global__ __launch_bounds__(256) void k_tile_boxes(const float* __restrict__ y,
     const uint32_t t = blockIdx.x * 8 + (threadIdx.x >> 5), d = threadIdx.x & 31;
     if (t >= T) return;  // T is a multiple of 8
     float lo = 3e38f, hi = -3e38f, mg = 0.f;
+    // all loads of 16 rows go out at once: past the end the last row, left out
+    for (uint32_t r0 = 0; r0 < 32; r0 += 16) {
+        float v[16];
 #pragma unroll
-    for (uint32_t r = 0; r < 32; ++r) {
-        const uint32_t s = t * 32 + r;
-        float v = d == PW_KIND ? 1.f : 0.f;
-        if (s < n) v = y[(size_t)perm[s] * PROJ_W + d];
-        const float kind = __shfl(v, PW_KIND, 32);
-        if (kind != 1.f) {
-            lo = fminf(lo, kind == 2.f ? -3e38f : v);
-            hi = fmaxf(hi, kind == 2.f ? 3e38f : v);
-            mg = fmaxf(mg, kind == 2.f ? 0.f : v);
+        for (uint32_t r = 0; r < 16; ++r) v[r] = y[(size_t)perm[min(t * 32 + r0 + r, n - 1)] * PROJ_W + d];
+#pragma unroll
+        for (uint32_t r = 0; r < 16; ++r) {
+            const float word = __shfl(v[r], PW_KIND, 32);
+            const float kind = t * 32 + r0 + r < n ? word : 1.f;
+            if (kind != 1.f) {
+                lo = fminf(lo, kind == 2.f ? -3e38f : v[r]);
+                hi = fmaxf(hi, kind == 2.f ? 3e38f : v[r]);
+                mg = fmaxf(mg, kind == 2.f ? 0.f : v[r]);
+            }
         }
     }
     if (d < PROJ_D) box[(size_t)d * T + t] = make_float2(lo, hi);
@@ -603,7 +659,7 @@ int proj_order(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, 
                        (int)fmt);
     uint32_t k = CL_MIN;
     while (k < CL_MAX && k * CL_ROWS * 3 / 2 < n) k *= 2;
-    const uint32_t S = std::min({n, CL_SAMPLE, 8 * k});
+    const uint32_t S = std::min({n, CL_SAMPLE, 4 * k});
     uint32_t *ckey, *rank;
     float* cen;
     int* sums;
