@@ -32,9 +32,12 @@ int proj_order(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, 
 // of rows at distance R (plus both rows' margins) or less.  frag: n_pad / 32 x PROJ_KS x 64 entries;
 // frag_a: n_pad / 32 x 64 (the row-role form of the last k-step).
 int proj_frags(mdet_ctx* ctx, const ProjOrder& o, uint32_t n, uint32_t n_pad, float R, uint4* frag, uint4* frag_a);
-// Boxes of T tiles (a multiple of 8, those past n empty) in that order: box
-// [PROJ_D][T] (lowest, highest), margin [T].  Rows of two tiles within R of each
-// other project to within R + both margins.
-int proj_boxes(mdet_ctx* ctx, const ProjOrder& o, uint32_t n, uint32_t T, float2* box, float* margin);
+// Boxes of `tiles` 32-row tiles (those past n empty) in that order: box[d * T + t]
+// (lowest, highest), margin[t].  Rows of two tiles within R of each other project
+// to within R + both margins.
+int proj_boxes(mdet_ctx* ctx, const ProjOrder& o, uint32_t n, uint32_t tiles, uint32_t T, float2* box, float* margin);
+// The projected rows alone; proj_frags and proj_boxes then take any order of
+// any of the rows (perm, with n its length).
+int proj_rows(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, float** y);
 
 }  // namespace mdet

@@ -601,14 +601,14 @@ __global__ __launch_bounds__(256) void k_proj_frags(const float* __restrict__ y,
 }
 
 // Bounding boxes of the 32-row tiles in the projection, box[d * T + t] =
-// (lowest, highest) and the largest margin, for T tiles; tiles without a bounded
-// row get empty boxes, ones with a row too long for FP16 boundless ones.  A
+// (lowest, highest) and the largest margin, for `tiles` tiles; ones without a bounded
+// row get empty boxes, ones with a row too long for FP16 boundless boxes.  A
 // thread per tile and coordinate: a row is one 128-byte read of 32 lanes.
 __global__ __launch_bounds__(256) void k_tile_boxes(const float* __restrict__ y, const uint32_t* __restrict__ perm,
-                                                    uint32_t n, uint32_t T, float2* __restrict__ box,
-                                                    float* __restrict__ margin) {
+                                                    uint32_t n, uint32_t tiles, uint32_t T,
+                                                    float2* __restrict__ box, float* __restrict__ margin) {
     const uint32_t t = blockIdx.x * 8 + (threadIdx.x >> 5), d = threadIdx.x & 31;
-    if (t >= T) return;  // T is a multiple of 8
+    if (t >= tiles) return;  // the 32 lanes of a tile together
     float lo = 3e38f, hi = -3e38f, mg = 0.f;
     // all loads of 16 rows go out at once: past the end the last row, left out
     for (uint32_t r0 = 0; r0 < 32; r0 += 16) {
@@ -636,27 +636,43 @@ namespace mdet {
 
 static_assert(PROJ_D == 28 && PROJ_KS == 2 && PROJ_W == 32, "k_project's groups and k_proj_frags' slots");
 
-int proj_order(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, ProjOrder* out) {
+namespace {
+// proj_rows, with the deviations of the coordinates (device, context buffer).
+int project(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, float** y, float** sig) {
     hipStream_t s = ctx->stream;
-    float *part, *msum, *cov, *mean, *basis, *off, *sig;
-    uint32_t *key, *key2, *idx;
+    float *part, *msum, *cov, *mean, *basis;
     MDET_TRY(ctx_buf(ctx, "proj.part", (size_t)COV_SPLITS * NT * NT, &part));
     MDET_TRY(ctx_buf(ctx, "proj.msum", (size_t)COV_SPLITS * (NT + 1), &msum));
     MDET_TRY(ctx_buf(ctx, "proj.cov", (size_t)NT * NT, &cov));
     MDET_TRY(ctx_buf(ctx, "proj.vec", (size_t)NT + 2 * PROJ_W, &mean));  // mean, offsets, deviations
-    off = mean + NT;
-    sig = off + PROJ_W;
+    float* off = mean + NT;
+    *sig = off + PROJ_W;
     MDET_TRY(ctx_buf(ctx, "proj.basis", (size_t)4 * NT * 8, &basis));
-    MDET_TRY(ctx_buf(ctx, "proj.y", (size_t)n * PROJ_W, &out->y));
+    MDET_TRY(ctx_buf(ctx, "proj.y", (size_t)n * PROJ_W, y));
+    hipLaunchKernelGGL(k_cov_part, dim3(COV_SPLITS), dim3(320), 0, s, tnf_dev, n, std::min(n, COV_SAMPLE), part, msum);
+    hipLaunchKernelGGL(k_cov_sum, dim3((NT * NT + 255) / 256), dim3(256), 0, s, part, msum, cov, mean);
+    hipLaunchKernelGGL(k_basis, dim3(1), dim3(B_THREADS), 0, s, cov, mean, basis, off, *sig);
+    hipLaunchKernelGGL(k_project, dim3((n + PJ_ROWS - 1) / PJ_ROWS), dim3(256), 0, s, tnf_dev, n, basis, off, *y,
+                       (int)fmt);
+    MDET_HIP(hipGetLastError());
+    return MDET_OK;
+}
+}  // namespace
+
+int proj_rows(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, float** y) {
+    float* sig;
+    return project(ctx, tnf_dev, n, fmt, y, &sig);
+}
+
+int proj_order(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, ProjOrder* out) {
+    hipStream_t s = ctx->stream;
+    float* sig;
+    uint32_t *key, *key2, *idx;
+    MDET_TRY(project(ctx, tnf_dev, n, fmt, &out->y, &sig));
     MDET_TRY(ctx_buf(ctx, "proj.key", (size_t)n, &key));
     MDET_TRY(ctx_buf(ctx, "proj.key2", (size_t)n, &key2));
     MDET_TRY(ctx_buf(ctx, "proj.idx", (size_t)n, &idx));
     MDET_TRY(ctx_buf(ctx, "proj.perm", (size_t)n, &out->perm));
-    hipLaunchKernelGGL(k_cov_part, dim3(COV_SPLITS), dim3(320), 0, s, tnf_dev, n, std::min(n, COV_SAMPLE), part, msum);
-    hipLaunchKernelGGL(k_cov_sum, dim3((NT * NT + 255) / 256), dim3(256), 0, s, part, msum, cov, mean);
-    hipLaunchKernelGGL(k_basis, dim3(1), dim3(B_THREADS), 0, s, cov, mean, basis, off, sig);
-    hipLaunchKernelGGL(k_project, dim3((n + PJ_ROWS - 1) / PJ_ROWS), dim3(256), 0, s, tnf_dev, n, basis, off, out->y,
-                       (int)fmt);
     uint32_t k = CL_MIN;
     while (k < CL_MAX && k * CL_ROWS * 3 / 2 < n) k *= 2;
     const uint32_t S = std::min({n, CL_SAMPLE, 4 * k});
@@ -687,8 +703,10 @@ int proj_order(mdet_ctx* ctx, const float* tnf_dev, uint32_t n, ProjFormat fmt, 
     return MDET_OK;
 }
 
-int proj_boxes(mdet_ctx* ctx, const ProjOrder& o, uint32_t n, uint32_t T, float2* box, float* margin) {
-    hipLaunchKernelGGL(k_tile_boxes, dim3(T / 8), dim3(256), 0, ctx->stream, o.y, o.perm, n, T, box, margin);
+int proj_boxes(mdet_ctx* ctx, const ProjOrder& o, uint32_t n, uint32_t tiles, uint32_t T, float2* box,
+               float* margin) {
+    hipLaunchKernelGGL(k_tile_boxes, dim3((tiles + 7) / 8), dim3(256), 0, ctx->stream, o.y, o.perm, n, tiles, T, box,
+                       margin);
     MDET_HIP(hipGetLastError());
     return MDET_OK;
 }

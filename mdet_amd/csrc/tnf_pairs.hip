@@ -2943,6 +2943,9 @@ constexpr int PREP_EVENT = 6;  // context event index marking the log-size range
 // Exhaustive modes up to this many contigs skip the row order and the first
 // pass: every tile goes to the second one.
 constexpr uint32_t DIRECT_MAX = 6144;
+// Pairs of full rows and contigs from which on the learned filter's fallback
+// scans projected rows.
+constexpr uint64_t FB_PROJ_PAIRS = 1500000000;
 // Resident refinement blocks per CU at most (39 KiB of LDS each).
 constexpr uint32_t REFINE_PER_CU = 4;
 
@@ -3100,7 +3103,7 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 MDET_TRY(proj_frags(ctx, order, n, n_pad, reach, pfrag, pfrag_a));
                 MDET_TRY(ctx_buf(ctx, "pairs.pbox", (size_t)PROJ_D * box_tiles, &pbox));
                 MDET_TRY(ctx_buf(ctx, "pairs.pbox_m", (size_t)box_tiles, &pbox_margin));
-                MDET_TRY(proj_boxes(ctx, order, n, box_tiles, pbox, pbox_margin));
+                MDET_TRY(proj_boxes(ctx, order, n, box_tiles, box_tiles, pbox, pbox_margin));
                 const uint32_t ord = tune.persistent ? tune.item_order : 0u;
                 MDET_TRY(build_items(ctx, n, item_rows, seg, ord, &items, &nitems, &qbounds));
                 if (!ord) qbounds = nullptr;
@@ -3289,6 +3292,10 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 const uint32_t n_full = ns1 ? (uint32_t)host[CTR_FULL] : 0;
                 st.fallback_rows = n_full;
                 if (n_full) {
+                    // large fallbacks run the box scan on projected rows, as the
+                    // exhaustive modes do (the projection is ~200 us at 200,000
+                    // contigs, multiplying all tile pairs 0.14 us per 1e6 pairs)
+                    const bool projected = (uint64_t)n_full * n >= FB_PROJ_PAIRS;
                     // the full rows' fragments after the first n_frag rows
                     hipLaunchKernelGGL(k_gather_ids, dim3((n_full + 255) / 256), dim3(256), 0, ctx->stream, full_pos,
                                        perm, n_full, full_ids);
@@ -3296,7 +3303,7 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                     hipLaunchKernelGGL((k_prep_lowp<true, NT, KS>), dim3(n_fpad / 32), dim3(256), 0, ctx->stream,
                                        tnf_dev, full_ids, n_full, gram_r, frag + (size_t)n_frag / 32 * KS * 64,
                                        frag_a + (size_t)n_frag / 32 * 64);
-                    // items: 256 full rows x 4096 columns, taken by resident blocks
+                    // items: a block's full rows x 4096 columns, taken by resident blocks
                     // in column-segment-major order, so that the blocks in flight
                     // share a segment's column fragments in L2 (the full rows'
                     // fragments are the small, reused side)
@@ -3305,10 +3312,11 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                     const uint32_t nseg = (n + FB_SEG - 1) / FB_SEG;
                     void* hi;
                     MDET_TRY(ctx_host_buf(ctx, "fb.h_items", (size_t)(n_fpad / ITEM_ROWS) * nseg * sizeof(uint4), &hi));
+                    const uint32_t fb_rows = projected ? scan_rows(PROJ_RT) : ITEM_ROWS;
                     uint4* hitems = static_cast<uint4*>(hi);
                     for (uint32_t c0 = 0; c0 < n; c0 += FB_SEG)
-                        for (uint32_t r0 = 0; r0 < n_full; r0 += ITEM_ROWS)
-                            hitems[w++] = make_uint4(n_frag + r0, n_frag + std::min(r0 + ITEM_ROWS, n_full), c0,
+                        for (uint32_t r0 = 0; r0 < n_full; r0 += fb_rows)
+                            hitems[w++] = make_uint4(n_frag + r0, n_frag + std::min(r0 + fb_rows, n_full), c0,
                                                      std::min(c0 + FB_SEG, n));
                     uint4* fitems;
                     MDET_TRY(ctx_buf(ctx, "fb.items", (size_t)w, &fitems));
@@ -3328,10 +3336,32 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                     MDET_TRY(ctx_buf(ctx, "fb.tiles", fb_cap, &flist));
                     MDET_TRY(ctx_buf(ctx, "fb.amb", cand_cap, &amb2));
                     const TileList tl{flist, ctr + CTR_FB_LIST, (unsigned long long)fb_cap};
-                    hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>),
-                                       dim3(std::min<uint32_t>(w, (uint32_t)ctx->num_cus * 2)), dim3(64 * SCAN_WAVES),
-                                       0, ctx->stream, frag, frag_a, fitems, w,
-                                       reinterpret_cast<uint32_t*>(ctr + CTR_FB_QUEUE), (const uint32_t*)nullptr, tl);
+                    uint32_t* const fb_ctr = reinterpret_cast<uint32_t*>(ctr + CTR_FB_QUEUE);
+                    auto fb_grid = [&](uint32_t per_cu) {
+                        return dim3(std::min<uint32_t>(w, (uint32_t)ctx->num_cus * per_cu));
+                    };
+                    if (projected) {
+                        const uint32_t ct = n_frag / 32, ft = n_fpad / 32, T = (ct + ft + 127) / 64 * 64;
+                        ProjOrder all{perm, nullptr}, some{full_ids, nullptr};
+                        MDET_TRY(proj_rows(ctx, tnf_dev, n, PROJ_BF16, &all.y));
+                        some.y = all.y;
+                        MDET_TRY(ctx_buf(ctx, "pairs.pfrag", (size_t)(ct + ft) * PROJ_KS * 64, &pfrag));
+                        MDET_TRY(ctx_buf(ctx, "pairs.pfrag_a", (size_t)(ct + ft) * 64, &pfrag_a));
+                        MDET_TRY(ctx_buf(ctx, "pairs.pbox", (size_t)PROJ_D * T, &pbox));
+                        MDET_TRY(ctx_buf(ctx, "pairs.pbox_m", (size_t)T, &pbox_margin));
+                        MDET_TRY(proj_frags(ctx, all, n, n_frag, reach, pfrag, pfrag_a));
+                        MDET_TRY(proj_frags(ctx, some, n_full, n_fpad, reach, pfrag + (size_t)ct * PROJ_KS * 64,
+                                            pfrag_a + (size_t)ct * 64));
+                        MDET_TRY(proj_boxes(ctx, all, n, ct, T, pbox, pbox_margin));
+                        MDET_TRY(proj_boxes(ctx, some, n_full, T - ct, T, pbox + ct, pbox_margin + ct));
+                        hipLaunchKernelGGL(k_box_scan, fb_grid(6), dim3(64 * SCAN_WAVES), 0, ctx->stream,
+                                           BoxArgs{pfrag, pfrag_a, T, reach, fitems, w, fb_ctr, nullptr, tl}, pbox,
+                                           pbox_margin);
+                    } else {
+                        hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>), fb_grid(2),
+                                           dim3(64 * SCAN_WAVES), 0, ctx->stream, frag, frag_a, fitems, w, fb_ctr,
+                                           (const uint32_t*)nullptr, tl);
+                    }
                     // its survivor tiles after the first phase's are worked off
                     sv.cnt = ctr + CTR_FB_SURV;
                     ga.items = fitems;
