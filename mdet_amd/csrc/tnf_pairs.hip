@@ -814,8 +814,11 @@ __device__ __forceinline__ void box_item(const BoxArgs& A, const float2* __restr
                                          const int lane, uint4* stage, uint32_t& nstage) {
     const uint32_t r_hi = it.y, c_hi = it.w & ~ITEM_TRI;
     const bool tri = (it.w & ITEM_TRI) != 0;
-    const uint32_t t0 = it.x / 32 + wave * PROJ_RT;  // items start at whole blocks
-    if (32 * t0 >= r_hi) return;
+    // waves without rows of a short item take every 2nd or 4th step of columns
+    const uint32_t groups = (r_hi - (it.x & ~31u) + 32 * PROJ_RT - 1) / (32 * PROJ_RT);
+    const uint32_t split = groups == 1 ? 4 : groups == 2 ? 2 : 1, part = (uint32_t)wave / groups;
+    if (part >= split) return;
+    const uint32_t t0 = it.x / 32 + (uint32_t)wave % groups * PROJ_RT;
     uint4 a[PROJ_RT][PROJ_KS];
 #pragma unroll
     for (int rt = 0; rt < PROJ_RT; ++rt) {
@@ -828,7 +831,7 @@ __device__ __forceinline__ void box_item(const BoxArgs& A, const float2* __restr
     for (int rt = 0; rt < PROJ_RT; ++rt) reach[rt] = A.R + margin[t0 + rt];
     uint32_t cb = it.z / 32;
     if (tri && cb < t0) cb += (t0 - cb) / 64 * 64;
-    for (; 32 * cb < c_hi; cb += 64) {
+    for (cb += 64 * part; 32 * cb < c_hi; cb += 64 * split) {
         const uint32_t tc = cb + lane;
         float s[PROJ_RT] = {};
         {
@@ -2943,9 +2946,13 @@ constexpr int PREP_EVENT = 6;  // context event index marking the log-size range
 // Exhaustive modes up to this many contigs skip the row order and the first
 // pass: every tile goes to the second one.
 constexpr uint32_t DIRECT_MAX = 6144;
-// Pairs of full rows and contigs from which on the learned filter's fallback
-// scans projected rows.
-constexpr uint64_t FB_PROJ_PAIRS = 1500000000;
+// Pairs of full rows and contigs, and of the probed clusters, from which on the
+// learned filter scans projected rows as the exhaustive modes do: the projection
+// takes ~190 us at 200,000 contigs (110 of them at any size) and serves both;
+// multiplying all tile pairs takes 135 us per 1e9 pairs of full rows and 250 of
+// the ragged cluster pairs, the box scan 25 and 200.
+constexpr uint64_t PROBE_PROJ_PAIRS = 750000000;
+constexpr uint64_t PROJ_PAIRS = 1500000000;
 // Resident refinement blocks per CU at most (39 KiB of LDS each).
 constexpr uint32_t REFINE_PER_CU = 4;
 
@@ -3149,6 +3156,21 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             }
             qbounds = nullptr;  // one queue
         }
+        // projected rows in cluster order for the learned filter's scans (with
+        // room for the fallback's full rows behind them)
+        float* proj_y = nullptr;
+        const uint32_t proj_T = (n_alloc / 32 + 127) / 64 * 64;
+        auto project_clusters = [&]() -> int {
+            MDET_TRY(proj_rows(ctx, tnf_dev, n, PROJ_BF16, &proj_y));
+            MDET_TRY(ctx_buf(ctx, "pairs.pfrag", (size_t)n_alloc / 32 * PROJ_KS * 64, &pfrag));
+            MDET_TRY(ctx_buf(ctx, "pairs.pfrag_a", (size_t)n_alloc / 32 * 64, &pfrag_a));
+            MDET_TRY(ctx_buf(ctx, "pairs.pbox", (size_t)PROJ_D * proj_T, &pbox));
+            MDET_TRY(ctx_buf(ctx, "pairs.pbox_m", (size_t)proj_T, &pbox_margin));
+            const ProjOrder all{perm, proj_y};
+            MDET_TRY(proj_frags(ctx, all, n, n_frag, reach, pfrag, pfrag_a));
+            return proj_boxes(ctx, all, n, proj_T, proj_T, pbox, pbox_margin);
+        };
+        if (cluster && tnf_gram && !ivf.exact && ivf.pairs >= PROBE_PROJ_PAIRS) MDET_TRY(project_clusters());
         uint32_t* iperm = nullptr;
         if (perm) {
             MDET_TRY(ctx_buf(ctx, "sel.iperm", (size_t)n, &iperm));
@@ -3194,7 +3216,11 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                     return dim3(std::min<uint32_t>(nitems, resident));
                 };
                 const dim3 block(64 * SCAN_WAVES);
-                if (gram_all)
+                if (proj_y)
+                    hipLaunchKernelGGL(k_box_scan, grid(6), block, 0, ctx->stream,
+                                       BoxArgs{pfrag, pfrag_a, proj_T, reach, items, nitems, pf_ctr, nullptr, tl}, pbox,
+                                       pbox_margin);
+                else if (gram_all)
                     hipLaunchKernelGGL(k_box_scan, grid(6), block, 0, ctx->stream,
                                        BoxArgs{pfrag, pfrag_a, box_tiles, reach, items, nitems, pf_ctr, qbounds, tl},
                                        pbox, pbox_margin);
@@ -3292,10 +3318,7 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 const uint32_t n_full = ns1 ? (uint32_t)host[CTR_FULL] : 0;
                 st.fallback_rows = n_full;
                 if (n_full) {
-                    // large fallbacks run the box scan on projected rows, as the
-                    // exhaustive modes do (the projection is ~200 us at 200,000
-                    // contigs, multiplying all tile pairs 0.14 us per 1e6 pairs)
-                    const bool projected = (uint64_t)n_full * n >= FB_PROJ_PAIRS;
+                    const bool projected = proj_y || (uint64_t)n_full * n >= PROJ_PAIRS;
                     // the full rows' fragments after the first n_frag rows
                     hipLaunchKernelGGL(k_gather_ids, dim3((n_full + 255) / 256), dim3(256), 0, ctx->stream, full_pos,
                                        perm, n_full, full_ids);
@@ -3341,21 +3364,14 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                         return dim3(std::min<uint32_t>(w, (uint32_t)ctx->num_cus * per_cu));
                     };
                     if (projected) {
-                        const uint32_t ct = n_frag / 32, ft = n_fpad / 32, T = (ct + ft + 127) / 64 * 64;
-                        ProjOrder all{perm, nullptr}, some{full_ids, nullptr};
-                        MDET_TRY(proj_rows(ctx, tnf_dev, n, PROJ_BF16, &all.y));
-                        some.y = all.y;
-                        MDET_TRY(ctx_buf(ctx, "pairs.pfrag", (size_t)(ct + ft) * PROJ_KS * 64, &pfrag));
-                        MDET_TRY(ctx_buf(ctx, "pairs.pfrag_a", (size_t)(ct + ft) * 64, &pfrag_a));
-                        MDET_TRY(ctx_buf(ctx, "pairs.pbox", (size_t)PROJ_D * T, &pbox));
-                        MDET_TRY(ctx_buf(ctx, "pairs.pbox_m", (size_t)T, &pbox_margin));
-                        MDET_TRY(proj_frags(ctx, all, n, n_frag, reach, pfrag, pfrag_a));
+                        if (!proj_y) MDET_TRY(project_clusters());
+                        ProjOrder some{full_ids, proj_y};
+                        const uint32_t ct = n_frag / 32;
                         MDET_TRY(proj_frags(ctx, some, n_full, n_fpad, reach, pfrag + (size_t)ct * PROJ_KS * 64,
                                             pfrag_a + (size_t)ct * 64));
-                        MDET_TRY(proj_boxes(ctx, all, n, ct, T, pbox, pbox_margin));
-                        MDET_TRY(proj_boxes(ctx, some, n_full, T - ct, T, pbox + ct, pbox_margin + ct));
+                        MDET_TRY(proj_boxes(ctx, some, n_full, proj_T - ct, proj_T, pbox + ct, pbox_margin + ct));
                         hipLaunchKernelGGL(k_box_scan, fb_grid(6), dim3(64 * SCAN_WAVES), 0, ctx->stream,
-                                           BoxArgs{pfrag, pfrag_a, T, reach, fitems, w, fb_ctr, nullptr, tl}, pbox,
+                                           BoxArgs{pfrag, pfrag_a, proj_T, reach, fitems, w, fb_ctr, nullptr, tl}, pbox,
                                            pbox_margin);
                     } else {
                         hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>), fb_grid(2),
