@@ -1302,7 +1302,12 @@ struct RefineArgs {
 };
 
 // One block a tile: the rows in LDS, one survivor a thread: 68 16-byte LDS
-// reads, 136 differences, the FP32 Chebyshev model.  The next tile's rows are
+// reads, 136 differences, the FP32 Chebyshev model.  The model's four
+// polynomials of two sizes are folded per contig and tile into 7 coefficients
+// each (the smaller size's variable summed up), so a pair takes two dot products
+// of 7 (model_of_pair); evaluated in full it was 40% of the instructions, which
+// bound this kernel (88% of the issue slots): 527 -> 485 us at 200,000
+// contigs.  The next tile's rows are
 // in registers while this tile is worked off (its contigs known one tile
 // ahead), so the loads' latency is covered by this and the CU's other blocks.
 // Survivors become candidate records {i, j, preProb, flags} in place: there is
@@ -1313,8 +1318,45 @@ struct RefineArgs {
 // 200k contigs): 1.54 ms, and 0.3 ms to sort and pack the survivor list.
 constexpr uint32_t AMB_STAGE = 192;
 
-__global__ __launch_bounds__(256, 4) void k_tile_refine(const RefineArgs A) {
+// Per contig of the tile: 4 x 8 folded coefficients (b1 c1 b2 c2), then the
+// Chebyshev values T_0..T_6 of its size (an odd number of 16-byte units apart).
+constexpr int FOLD_STR = 11;
+
+// b + c d for the polynomials at F[0..1], F[2..3].
+__device__ inline float folded(const f32x4_t* F, f32x4_t t0, f32x4_t t1, float d) {
+    const f32x4_t b0 = F[0], b1 = F[1], c0 = F[2], c1 = F[3];
+    float b = b0.x, c = c0.x;
+    b = fmaf(b0.y, t0.y, b);
+    c = fmaf(c0.y, t0.y, c);
+    b = fmaf(b0.z, t0.z, b);
+    c = fmaf(c0.z, t0.z, c);
+    b = fmaf(b0.w, t0.w, b);
+    c = fmaf(c0.w, t0.w, c);
+    b = fmaf(b1.x, t1.x, b);
+    c = fmaf(c1.x, t1.x, c);
+    b = fmaf(b1.y, t1.y, b);
+    c = fmaf(c1.y, t1.y, c);
+    b = fmaf(b1.z, t1.z, b);
+    c = fmaf(c1.z, t1.z, c);
+    return fmaf(c, d, b);
+}
+
+// model32 from the folded coefficients of the pair's contigs (ta, tb: their sizes).
+__device__ inline Pre32 model_of_pair(float d, const f32x4_t* a, const f32x4_t* b, float ta, float tb) {
+    const f32x4_t* F = ta <= tb ? a : b;
+    const f32x4_t* T = (ta <= tb ? b : a) + 8;
+    const f32x4_t t0 = T[0], t1 = T[1];
+    Pre32 r;
+    r.pre1 = -folded(F, t0, t1, d);
+    r.pre = r.pre1;
+    if (r.pre1 <= FLOOR32) r.pre = fminf(-folded(F + 4, t0, t1, d), FLOOR32);
+    return r;
+}
+
+__global__ __launch_bounds__(256, 3) void k_tile_refine(const RefineArgs A) {
     __shared__ __align__(16) f32x4_t rows[64][TSTR];
+    __shared__ __align__(16) f32x4_t fold[64][FOLD_STR];
+    __shared__ __align__(16) f32x4_t cheb[4][MODEL_CX][2];  // coefficients by degree in the smaller size
     __shared__ uint16_t pl[1024];  // survivors of the tile: row << 5 | column
     __shared__ uint32_t id[2][64];
     __shared__ float tv[2][64];
@@ -1337,6 +1379,10 @@ __global__ __launch_bounds__(256, 4) void k_tile_refine(const RefineArgs A) {
     }
     if (wave == 1) bits = A.in.mask[e0 * 64 + lane];
     if (tid == 0) s_amb = 0;
+    if (tid < 4 * MODEL_CX * 8) {
+        const int k = tid & 7;
+        reinterpret_cast<float*>(cheb)[tid] = k < MODEL_CY ? c_cheb[tid >> 6][(tid >> 3) & 7][k < MODEL_CY ? k : 0] : 0.f;
+    }
     __syncthreads();
     TileRows pre;
     pre.load(A.rows.tnf, id[0][tid >> 2], tid);
@@ -1344,6 +1390,28 @@ __global__ __launch_bounds__(256, 4) void k_tile_refine(const RefineArgs A) {
     for (int buf = 0;; buf ^= 1) {
         // this tile's rows and survivor list to LDS, the next tile's contigs beside them
         pre.store(rows, tid);
+        {  // four threads a contig, a polynomial each
+            const uint32_t ct = tid >> 2, p = tid & 3;
+            const float t = tv[buf][ct];
+            float T[MODEL_CX];
+            T[0] = 1.f;
+            T[1] = t;
+#pragma unroll
+            for (int k = 2; k < MODEL_CX; ++k) T[k] = fmaf(2.f * t, T[k - 1], -T[k - 2]);
+            f32x4_t f0 = {0.f, 0.f, 0.f, 0.f}, f1 = f0;
+#pragma unroll
+            for (int k = 0; k < MODEL_CX; ++k) {
+                const f32x4_t c0 = cheb[p][k][0], c1 = cheb[p][k][1];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f0[e] = fmaf(c0[e], T[k], f0[e]);
+                    f1[e] = fmaf(c1[e], T[k], f1[e]);
+                }
+            }
+            fold[ct][2 * p] = f0;
+            fold[ct][2 * p + 1] = f1;
+            if (p < 2) fold[ct][8 + p] = f32x4_t{T[4 * p], T[4 * p + 1], T[4 * p + 2], T[4 * p + 3]};
+        }
         if (wave == 0) id[buf ^ 1][lane] = next_id;
         if (wave == 1) {
             const uint32_t pc = (uint32_t)__popc(bits);
@@ -1378,7 +1446,8 @@ __global__ __launch_bounds__(256, 4) void k_tile_refine(const RefineArgs A) {
             if (t < c) {
                 r = pl[t] >> 5;
                 const uint32_t col = 32 + (pl[t] & 31);
-                const Pre32 m = model32(sqrtf(tile_dist2(rows[r], rows[col])), tv[buf][r], tv[buf][col]);
+                const Pre32 m = model_of_pair(sqrtf(tile_dist2(rows[r], rows[col])), fold[r], fold[col], tv[buf][r],
+                                              tv[buf][col]);
                 const bool amb = fabsf(m.pre - A.T32) <= EPS_PRE || fabsf(m.pre1 - FLOOR32) <= EPS_PRE;
                 keep = !amb && m.pre > A.T32;  // a tie-band pair is kept (or not) by k_adjudicate
                 Cand cd;
@@ -2953,8 +3022,8 @@ constexpr uint32_t DIRECT_MAX = 6144;
 // the ragged cluster pairs, the box scan 25 and 200.
 constexpr uint64_t PROBE_PROJ_PAIRS = 750000000;
 constexpr uint64_t PROJ_PAIRS = 1500000000;
-// Resident refinement blocks per CU at most (39 KiB of LDS each).
-constexpr uint32_t REFINE_PER_CU = 4;
+// Resident refinement blocks per CU at most (52 KiB of LDS each).
+constexpr uint32_t REFINE_PER_CU = 3;
 
 int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, uint32_t n, double cutoff,
                uint32_t max_edges, int precision, mdet_mlp* mlp, float radius2, uint32_t n_clusters,
