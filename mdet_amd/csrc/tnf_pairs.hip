@@ -2923,12 +2923,13 @@ int exclusive_scan_u32_to_u64(mdet_ctx* ctx, const uint32_t* in, uint64_t* out, 
 // items still come spread over time and XCDs, while an XCD's blocks share
 // column ranges in its L2: memory-side traffic 19.4 -> 3.5 GB and 10% faster
 // at 200k contigs in the full Gram over 256-row blocks.
-// Default column span by size: the power of two nearest n / 100 in [512,
-// 4096] (the autotuner's picks measured at 50k, 200k and 1M contigs were
-// 512, 2048 and 4096, with persistent blocks).
+// Default column span by size: the power of two nearest n / 50 in [512, 16384].
+// Longer spans spare the box scan row fragments and boxes (43 -> 34 us at 50,000
+// contigs and 10.64 -> 10.49 ms at 1,000,000 against n / 100 and at most 4096);
+// short ones keep enough items for the blocks of small inputs.
 uint32_t seg_cols_for(uint32_t n) {
     uint32_t seg = 512;
-    while (seg < 4096 && (uint64_t)seg * 3 / 2 * 100 < n) seg *= 2;
+    while (seg < 16384 && (uint64_t)seg * 3 / 2 * 50 < n) seg *= 2;
     return seg;
 }
 
