@@ -407,11 +407,12 @@ int mdet_learned_set_exact_cover(mdet_ctx *ctx, int enabled);
 typedef struct mdet_tune {
     uint32_t seg_cols;      /* MFMA Gram modes: prefilter item column span, a
                              * multiple of 256 in [256, 65536], or 0 (default):
-                             * the power of two nearest n/100 in [512, 4096] */
+                             * the power of two nearest n/50 in [512, 16384] */
     uint32_t persistent;    /* MFMA modes: 0 one prefilter block per item, 1
                              * (default) resident blocks take items from a
                              * counter */
-    uint32_t refine_blocks; /* refinement blocks per CU, 1..64 (default 64) */
+    uint32_t refine_blocks; /* refinement blocks per CU, 1..64 (default 64;
+                             * no more than fit are launched) */
     uint32_t item_order;    /* Gram modes with persistent blocks: 0 one item
                              * queue, row-block major; 1 (default) one queue
                              * per XCD (row blocks rb % 8), column-start major */
