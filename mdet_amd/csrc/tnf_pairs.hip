@@ -3287,9 +3287,11 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 };
                 const dim3 block(64 * SCAN_WAVES);
                 if (proj_y)
-                    hipLaunchKernelGGL(k_box_scan, grid(6), block, 0, ctx->stream,
-                                       BoxArgs{pfrag, pfrag_a, proj_T, reach, items, nitems, pf_ctr, nullptr, tl}, pbox,
-                                       pbox_margin);
+                    // tens of thousands of small items: a block each (a returning
+                    // atomic an item on the one queue bound it, 300 us at 200,000)
+                    hipLaunchKernelGGL(k_box_scan, dim3(nitems), block, 0, ctx->stream,
+                                       BoxArgs{pfrag, pfrag_a, proj_T, reach, items, nitems, nullptr, nullptr, tl},
+                                       pbox, pbox_margin);
                 else if (gram_all)
                     hipLaunchKernelGGL(k_box_scan, grid(6), block, 0, ctx->stream,
                                        BoxArgs{pfrag, pfrag_a, box_tiles, reach, items, nitems, pf_ctr, qbounds, tl},
