@@ -1850,24 +1850,22 @@ __device__ void sort_ids_and_store(const float* key, const uint32_t* id, uint32_
     }
 }
 
-// The K largest preProb of the row's deg (<= 64 * E, > K) entries at
-// adj[beg..), FP32 ties within 2 * EPS of the K-th re-ranked in FP64: the
-// partners above rid compacted into LDS key/id, their number returned; -1 if
-// the tie zone is wider than a wave.  Only the K-th largest key is needed, not
+// The K largest preProb of the row's deg (<= 64 * E, > K) entries in LDS
+// key/id, FP32 ties within 2 * EPS of the K-th re-ranked in FP64: the partners
+// above rid compacted to the front of key/id, their number returned; -1, with
+// key/id as they were, if the tie zone is wider than a wave.  Only the K-th largest key is needed, not
 // their order: it is found bit by bit, counting the keys not below a candidate
 // (~25 rounds of E compares; a bitonic sort by rank took 45 exchange rounds).
 template <int E>
-__device__ int top_of_row(const Adj* __restrict__ adj, uint64_t beg, uint32_t deg, uint32_t rid, uint32_t K,
-                          const float* __restrict__ tnf, const double* __restrict__ ls, float* key, uint32_t* id,
-                          int lane) {
+__device__ int top_of_row(uint32_t deg, uint32_t rid, uint32_t K, const float* __restrict__ tnf,
+                          const double* __restrict__ ls, float* key, uint32_t* id, int lane) {
     uint32_t k[E], v[E], hi = 0, lo = 0xffffffffu;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const uint32_t t = e * 64 + lane;
         const bool in = t < deg;
-        const Adj a = in ? adj[beg + t] : Adj{0xffffffffu, 0.f};
-        k[e] = in ? f2ord(a.pre) : 0u;
-        v[e] = a.partner;
+        k[e] = in ? f2ord(key[t]) : 0u;
+        v[e] = in ? id[t] : 0xffffffffu;
         hi = max(hi, k[e]);
         lo = min(lo, in ? k[e] : 0xffffffffu);
     }
@@ -1917,6 +1915,7 @@ __device__ int top_of_row(const Adj* __restrict__ adj, uint64_t beg, uint32_t de
     if (zn > 64) return -1;
     const uint32_t need = K - above;
     if (need < zn) {
+        wave_sync();
 #pragma unroll
         for (int e = 0; e < E; ++e)
             if (zp[e] != 0xffffffffu) id[zp[e]] = v[e];
@@ -1942,6 +1941,7 @@ __device__ int top_of_row(const Adj* __restrict__ adj, uint64_t beg, uint32_t de
 #pragma unroll
         for (int e = 0; e < E; ++e) sel[e] = sel[e] || zp[e] != 0xffffffffu;
     }
+    wave_sync();  // the row is in registers by here; its entries in LDS are overwritten
     uint32_t cnt = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -1957,37 +1957,40 @@ __device__ int top_of_row(const Adj* __restrict__ adj, uint64_t beg, uint32_t de
     return (int)cnt;
 }
 
-// Row `rid` (contig id), deg entries at adj[beg..): by one wave.  Returns
-// false, touching nothing in global memory, if the row needs the block path
-// (FP32 tie zone at the cut wider than a wave).  capped counts in LDS: one
-// atomic per row on the call's counter serialised the 50,000 capped rows of a
-// 50,000-contig input.
+// Row `rid` (contig id), its deg entries in LDS key/id, which are overwritten:
+// the kept ones, by id, to adj[beg..), by one wave.  Returns false, with key/id
+// and adj as they were, if the row needs the block path (FP32 tie zone at the
+// cut wider than a wave).  capped counts in LDS: one atomic per row on the
+// call's counter serialised the 50,000 capped rows of a 50,000-contig input.
 __device__ bool wave_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t deg, uint32_t rid, uint32_t K,
                                 const float* __restrict__ tnf, const double* __restrict__ ls, float* key,
                                 uint32_t* id, uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg,
                                 uint32_t* capped, int lane) {
     uint32_t cnt = 0;
     if (K && deg > K) {
-        const int c = deg <= 64    ? top_of_row<1>(adj, beg, deg, rid, K, tnf, ls, key, id, lane)
-                      : deg <= 128 ? top_of_row<2>(adj, beg, deg, rid, K, tnf, ls, key, id, lane)
-                      : deg <= 256 ? top_of_row<4>(adj, beg, deg, rid, K, tnf, ls, key, id, lane)
-                                   : top_of_row<8>(adj, beg, deg, rid, K, tnf, ls, key, id, lane);
+        const int c = deg <= 64    ? top_of_row<1>(deg, rid, K, tnf, ls, key, id, lane)
+                      : deg <= 128 ? top_of_row<2>(deg, rid, K, tnf, ls, key, id, lane)
+                      : deg <= 256 ? top_of_row<4>(deg, rid, K, tnf, ls, key, id, lane)
+                                   : top_of_row<8>(deg, rid, K, tnf, ls, key, id, lane);
         if (c < 0) return false;
         cnt = (uint32_t)c;
         if (lane == 0) atomicAdd(capped, 1u);
     } else {
-        // every candidate is selected: gather the partners above the row
+        // every candidate is selected: gather the partners above the row.  An
+        // entry moves to its own place or before it, so those not read yet stay.
         for (uint32_t t0 = 0; t0 < deg; t0 += 64) {
             const uint32_t t = t0 + lane;
-            Adj e{0, 0.f};
-            if (t < deg) e = adj[beg + t];
-            const bool keep = t < deg && e.partner > rid;
+            const uint32_t p = t < deg ? id[t] : 0u;
+            const float x = t < deg ? key[t] : 0.f;
+            const bool keep = t < deg && p > rid;
             const uint64_t m = __ballot(keep);
+            wave_sync();
             if (keep) {
                 const uint32_t o = cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                key[o] = e.pre;
-                id[o] = e.partner;
+                key[o] = x;
+                id[o] = p;
             }
+            wave_sync();
             cnt += (uint32_t)__popcll(m);
         }
     }
@@ -2118,29 +2121,50 @@ __device__ void block_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t d
     __syncthreads();
 }
 
-// One block per bucket: group the bucket's entries by row into adj (same
-// offsets as ent), then select every row by one wave.  Output per contig row:
-// out_cnt (edges kept: partners above the row, sorted) and rbeg (where they
-// are in adj).  Rows the wave path declines go to a list for
-// k_bigrow_select ((row id, degree, begin) records).
+// One block per bucket: group the bucket's entries by row, then select every
+// row by one wave.  Output per contig row: out_cnt (edges kept: partners above
+// the row, sorted) and rbeg (where they are in adj, whose offsets are ent's).
+// Rows the wave path declines go to a list for k_bigrow_select ((row id,
+// degree, begin) records), their entries in adj.
+//
+// The rows are grouped in LDS, where each is selected in place, as far as
+// L_CAP entries go; only rows of more than W_CAP entries and those that end
+// beyond L_CAP are grouped in adj, the latter staged through LDS once the
+// rows in it are done.  Bound by vector instructions (the search of the K-th
+// key, the FP64 zone, the sort) and by the latency of the entries' two passes.
+// Grouped in adj, every row was written eight bytes here and there and read
+// back: 385 us at 200k contigs, 1289 at 1M, 194 at 50k in FP32; grouped in LDS
+// with two blocks a CU 350, 1111 and 201; with rows taken as waves become free
+// 321, 1001 and 172; with three blocks a CU 298, 880 and 152 (80 registers, at
+// the price of a few spills around the FP64 zone; four blocks: 307, 854 and
+// 162); with eight loads in flight instead of four 290, 873 and 149.  L_CAP is
+// what lets three blocks share a CU's 160 KB.  Taking the longest row first
+// gave nothing.
+constexpr uint32_t L_CAP = 6600;
+static_assert(S_WAVES * W_CAP <= (int)L_CAP, "staging of the rows grouped in adj");
 
-__global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
+// Whether a row of deg entries from slot `at` of its bucket is grouped in LDS.
+__device__ __forceinline__ bool in_lds(uint32_t at, uint32_t deg) {
+    return deg <= (uint32_t)W_CAP && at <= L_CAP - deg;
+}
+
+__global__ __launch_bounds__(S_THREADS, 6) void k_bucket_select(
     const uint64_t* __restrict__ boff, const Ent* __restrict__ ent, Adj* __restrict__ adj, uint32_t n, uint32_t K,
     const uint32_t* __restrict__ perm, const float* __restrict__ tnf, const double* __restrict__ ls,
     uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, const RowList big,
     unsigned int* __restrict__ err, unsigned long long* __restrict__ capped) {
     constexpr int PER = S_BUCKET / 64;
-    constexpr int BATCH = 4;
-    __shared__ uint32_t hist[S_BUCKET], rstart[S_BUCKET], rcur[S_BUCKET], s_capped;
-    __shared__ float wkey[S_WAVES][W_CAP];
-    __shared__ uint32_t wid[S_WAVES][W_CAP];
+    constexpr int BATCH = 8;
+    __shared__ uint32_t hist[S_BUCKET], rstart[S_BUCKET], rcur[S_BUCKET], s_next[2], s_capped;
+    __shared__ float lkey[L_CAP];
+    __shared__ uint32_t lid[L_CAP];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint32_t b = blockIdx.x;
     const uint64_t e0 = boff[b], e1 = boff[b + 1];
     const uint32_t row0 = b * S_BUCKET;
     const uint32_t rows = n - row0 < (uint32_t)S_BUCKET ? n - row0 : (uint32_t)S_BUCKET;
     for (int t = tid; t < S_BUCKET; t += S_THREADS) hist[t] = rcur[t] = 0;
-    if (tid == 0) s_capped = 0;
+    if (tid == 0) s_capped = s_next[0] = s_next[1] = 0;
     __syncthreads();
     // row histogram; BATCH independent loads in flight per thread
     for (uint64_t e = e0 + tid; e < e1; e += BATCH * S_THREADS) {
@@ -2184,28 +2208,58 @@ __global__ __launch_bounds__(S_THREADS, 4) void k_bucket_select(
 #pragma unroll
         for (int q = 0; q < BATCH; ++q)
             if (ok[q]) {
-                const uint32_t slot = atomicAdd(&rcur[x[q].lrow], 1u);
-                adj[e0 + rstart[x[q].lrow] + slot] = Adj{x[q].partner, x[q].pre};
+                const uint32_t lr = x[q].lrow, at = rstart[lr], deg = hist[lr];
+                const uint32_t slot = at + atomicAdd(&rcur[lr], 1u);
+                if (in_lds(at, deg)) {
+                    lid[slot] = x[q].partner;
+                    lkey[slot] = x[q].pre;
+                } else {
+                    adj[e0 + slot] = Adj{x[q].partner, x[q].pre};
+                }
             }
     }
     __syncthreads();
-    for (uint32_t r = wave; r < rows; r += S_WAVES) {
-        const uint32_t deg = hist[r];
-        const uint64_t beg = e0 + rstart[r];
-        const uint32_t pos = row0 + r;
-        const uint32_t rid = perm ? perm[pos] : pos;
-        bool done = true;
-        if (deg == 0) {
-            if (lane == 0) {
-                out_cnt[rid] = 0;
-                rbeg[rid] = beg;
-            }
-        } else if (deg > (uint32_t)W_CAP) {
-            done = false;
-        } else {
-            done = wave_row_select(adj, beg, deg, rid, K, tnf, ls, wkey[wave], wid[wave], out_cnt, rbeg, &s_capped, lane);
+    for (int pass = 0; pass < 2; ++pass) {  // the rows in LDS, then those staged through it
+        if (pass == 1) {
+            if (e1 - e0 <= L_CAP) break;
+            __syncthreads();
         }
-        if (!done && lane == 0) push_row(big, rid, deg, beg, err, 4u);
+        // rows are taken as waves become free: their degrees differ widely
+        for (;;) {
+            uint32_t r = lane == 0 ? atomicAdd(&s_next[pass], 1u) : 0u;
+            r = (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
+            if (r >= rows) break;
+            const uint32_t deg = hist[r], at = rstart[r];
+            const bool here = in_lds(at, deg), wide = deg > (uint32_t)W_CAP;
+            if (pass == 1 && (here || wide)) continue;
+            if (pass == 0 && !here && !wide) continue;
+            const uint64_t beg = e0 + at;
+            const uint32_t pos = row0 + r;
+            const uint32_t rid = perm ? perm[pos] : pos;
+            bool done = !wide;
+            if (deg == 0) {
+                if (lane == 0) {
+                    out_cnt[rid] = 0;
+                    rbeg[rid] = beg;
+                }
+            } else if (!wide) {
+                float* key = here ? lkey + at : lkey + wave * W_CAP;
+                uint32_t* id = here ? lid + at : lid + wave * W_CAP;
+                if (!here) {
+                    wave_sync();
+                    for (uint32_t t = lane; t < deg; t += 64) {
+                        const Adj a = adj[beg + t];
+                        key[t] = a.pre;
+                        id[t] = a.partner;
+                    }
+                    wave_sync();
+                }
+                done = wave_row_select(adj, beg, deg, rid, K, tnf, ls, key, id, out_cnt, rbeg, &s_capped, lane);
+                if (!done && here)
+                    for (uint32_t t = lane; t < deg; t += 64) adj[beg + t] = Adj{id[t], key[t]};
+            }
+            if (!done && lane == 0) push_row(big, rid, deg, beg, err, 4u);
+        }
     }
     __syncthreads();
     if (tid == 0 && s_capped) atomicAdd(capped, (unsigned long long)s_capped);
