@@ -43,6 +43,7 @@
 #include "ivf.h"
 #include "model_tables.h"
 #include "order.h"
+#include "pass_lists.h"
 #include "tnf_tables.h"
 
 namespace {
@@ -921,6 +922,39 @@ __global__ __launch_bounds__(64 * SCAN_WAVES, 6) void k_box_scan(const BoxArgs A
     tiles_flush(A.out, stage, nstage, lane);
 }
 
+// Counters of one edge-list call (64-bit words of the zeroed block; the first
+// CTR_HOST are copied to the host together).
+enum : uint32_t {
+    CTR_MM = 0,      // k_prep_rows: log-size range, out-of-domain count
+    CTR_LIST = 3,    // listed tiles (everything from here on is cleared for a repeated pass)
+    CTR_CAND,        // candidate records
+    CTR_KEPT,        // kept candidates ...
+    CTR_ADJ,         // ... and the ones decided in FP64 (k_adjudicate: the word after CTR_KEPT)
+    CTR_AMB,         // tie-band list lengths, first pass and fallback
+    CTR_AMB2,
+    CTR_FULL,        // full rows of the fallback
+    CTR_FB_LIST,     // its listed tiles
+    CTR_SURV,        // tiles with survivors, first pass and fallback
+    CTR_FB_SURV,
+    CTR_ERR,         // select flags
+    CTR_CAPPED,      // capped rows
+    CTR_BIG,         // rows for the block-wide and the global-memory selection
+    CTR_HUGE,
+    CTR_EDGES,       // edges
+    CTR_HOST,
+    CTR_QUEUES = 24, // scan queues: PF_QUEUES counters PF_CTR_STRIDE 32-bit words apart
+    CTR_FB_QUEUE = CTR_QUEUES + PF_QUEUES * PF_CTR_STRIDE / 2,
+    CTR_WORDS = CTR_FB_QUEUE + 8,
+};
+static_assert(CTR_HOST <= CTR_QUEUES, "counter layout");
+
+using mdet::PassCaps;
+using mdet::PassCounts;
+
+__host__ __device__ inline PassCounts pass_counts(const unsigned long long* ctr) {
+    return PassCounts{ctr[CTR_LIST], ctr[CTR_SURV], ctr[CTR_FB_LIST], ctr[CTR_FB_SURV], ctr[CTR_CAND]};
+}
+
 // ------------------------------------------------------------ tile pairs --
 // The second pass: the pairs of the listed tiles, decided in FP32.
 //   k_tile_gram    the low-precision Gram (9 k-steps, or 3 on embeddings) of
@@ -1539,6 +1573,20 @@ __global__ __launch_bounds__(256) void k_adjudicate(const float* __restrict__ tn
     }
 }
 
+// The candidate records as the passes left them, for the kernels that read them
+// before the host has seen the counters: their number, or none if one of the
+// lists was too small (the host then repeats the pass, and what these kernels
+// leave out is not used).
+struct Records {
+    const Cand* cand;
+    const unsigned long long* ctr;
+    PassCaps caps;
+};
+__device__ inline uint64_t records_to_read(const Records& r) {
+    const PassCounts n = pass_counts(r.ctr);
+    return mdet::records_written(n, r.caps) ? n.cand : 0ull;
+}
+
 // ------------------------------------------- learned mode: exact fallback --
 // The cluster index proposes pairs; a row whose proposals fill its max_edges
 // slots (a "full row") may have missed a better partner, which would leave a
@@ -1588,15 +1636,14 @@ __device__ inline void kept_count(uint32_t* __restrict__ h, uint32_t* __restrict
     }
 }
 
-__global__ __launch_bounds__(256) void k_row_kept(const Cand* __restrict__ cand,
-                                                  const unsigned long long* __restrict__ n_cand,
-                                                  unsigned long long cap, const uint32_t* __restrict__ iperm,
+__global__ __launch_bounds__(256) void k_row_kept(const Records rec, const uint32_t* __restrict__ iperm,
                                                   uint32_t* __restrict__ cnt) {
     __shared__ uint32_t hist[4][2][KEPT_SPAN];
     const uint32_t w = threadIdx.x >> 6, lane = lane_id();
     for (uint32_t s = lane; s < KEPT_SPAN; s += 64) hist[w][0][s] = hist[w][1][s] = 0u;
     __builtin_amdgcn_s_waitcnt(0);
-    const uint64_t nc = min(*n_cand, cap);
+    const Cand* __restrict__ cand = rec.cand;
+    const uint64_t nc = records_to_read(rec);
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u); base < nc; base += stride) {
         const uint64_t k = base + lane;
@@ -1675,12 +1722,11 @@ __global__ __launch_bounds__(256) void k_iperm(const uint32_t* __restrict__ perm
 // on the device.
 constexpr uint32_t FILL_SPREAD = 2048;
 
-__global__ __launch_bounds__(256) void k_bucket_fill(const Cand* __restrict__ cand,
-                                                     const unsigned long long* __restrict__ n_cand,
-                                                     unsigned long long cap, const uint32_t* __restrict__ iperm,
+__global__ __launch_bounds__(256) void k_bucket_fill(const Records rec, const uint32_t* __restrict__ iperm,
                                                      const uint64_t* __restrict__ boff, uint32_t* __restrict__ bcur,
                                                      Ent* __restrict__ ent) {
-    const uint64_t nc = min(*n_cand, cap);
+    const Cand* __restrict__ cand = rec.cand;
+    const uint64_t nc = records_to_read(rec);
     const uint64_t pieces = (nc + 255) / 256, per = (pieces + FILL_SPREAD - 1) / FILL_SPREAD;
     for (uint64_t b = blockIdx.x; b < per * FILL_SPREAD; b += gridDim.x) {
         const uint64_t piece = (b % FILL_SPREAD) * per + b / FILL_SPREAD;
@@ -2125,7 +2171,9 @@ __device__ void block_row_select(Adj* __restrict__ adj, uint64_t beg, uint32_t d
 // row by one wave.  Output per contig row: out_cnt (edges kept: partners above
 // the row, sorted) and rbeg (where they are in adj, whose offsets are ent's).
 // Rows the wave path declines go to a list for k_bigrow_select ((row id,
-// degree, begin) records), their entries in adj.
+// degree, begin) records), their entries in adj.  Without records to read (and
+// so without entries, whatever the bucket counts say) every row stays at no
+// edges, as the call cleared out_cnt.
 //
 // The rows are grouped in LDS, where each is selected in place, as far as
 // L_CAP entries go; only rows of more than W_CAP entries and those that end
@@ -2149,10 +2197,11 @@ __device__ __forceinline__ bool in_lds(uint32_t at, uint32_t deg) {
 }
 
 __global__ __launch_bounds__(S_THREADS, 6) void k_bucket_select(
-    const uint64_t* __restrict__ boff, const Ent* __restrict__ ent, Adj* __restrict__ adj, uint32_t n, uint32_t K,
-    const uint32_t* __restrict__ perm, const float* __restrict__ tnf, const double* __restrict__ ls,
-    uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, const RowList big,
+    const Records rec, const uint64_t* __restrict__ boff, const Ent* __restrict__ ent, Adj* __restrict__ adj,
+    uint32_t n, uint32_t K, const uint32_t* __restrict__ perm, const float* __restrict__ tnf,
+    const double* __restrict__ ls, uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, const RowList big,
     unsigned int* __restrict__ err, unsigned long long* __restrict__ capped) {
+    if (records_to_read(rec) == 0) return;
     constexpr int PER = S_BUCKET / 64;
     constexpr int BATCH = 8;
     __shared__ uint32_t hist[S_BUCKET], rstart[S_BUCKET], rcur[S_BUCKET], s_next[2], s_capped;
@@ -3063,31 +3112,6 @@ int build_items(mdet_ctx* ctx, uint32_t n, uint32_t rows, uint32_t seg, uint32_t
     return MDET_OK;
 }
 
-// Counters of one edge-list call (64-bit words of the zeroed block; the first
-// CTR_HOST are copied to the host together).
-enum : uint32_t {
-    CTR_MM = 0,      // k_prep_rows: log-size range, out-of-domain count
-    CTR_LIST = 3,    // listed tiles (everything from here on is cleared for a repeated pass)
-    CTR_CAND,        // candidate records
-    CTR_KEPT,        // kept candidates ...
-    CTR_ADJ,         // ... and the ones decided in FP64 (k_adjudicate: the word after CTR_KEPT)
-    CTR_AMB,         // tie-band list lengths, first pass and fallback
-    CTR_AMB2,
-    CTR_FULL,        // full rows of the fallback
-    CTR_FB_LIST,     // its listed tiles
-    CTR_SURV,        // tiles with survivors, first pass and fallback
-    CTR_FB_SURV,
-    CTR_ERR,         // select flags
-    CTR_CAPPED,      // capped rows
-    CTR_BIG,         // rows for the block-wide and the global-memory selection
-    CTR_HUGE,
-    CTR_EDGES,       // edges
-    CTR_HOST,
-    CTR_QUEUES = 24, // scan queues: PF_QUEUES counters PF_CTR_STRIDE 32-bit words apart
-    CTR_FB_QUEUE = CTR_QUEUES + PF_QUEUES * PF_CTR_STRIDE / 2,
-    CTR_WORDS = CTR_FB_QUEUE + 8,
-};
-static_assert(CTR_HOST <= CTR_QUEUES, "counter layout");
 constexpr int PREP_EVENT = 6;  // context event index marking the log-size range's copy
 // Exhaustive modes up to this many contigs skip the row order and the first
 // pass: every tile goes to the second one.
@@ -3328,24 +3352,25 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
         // -- both passes over the pairs and the selection, again with larger
         // buffers if a list did not fit (its counter says how much it needs)
         const uint64_t ntiles = (n + 31) / 32;
-        uint64_t list_cap = std::min<uint64_t>(ntiles * (ntiles + 1) / 2, std::max<uint64_t>(1u << 16, 8ull * n));
-        uint64_t surv_cap = direct ? ntiles * (ntiles + 1) / 2 : std::max<uint64_t>(1u << 16, 2ull * n);
-        uint64_t cand_cap = 128ull * n + 65536, fb_cap = 0;
+        PassCaps caps{};
+        caps.list = std::min<uint64_t>(ntiles * (ntiles + 1) / 2, std::max<uint64_t>(1u << 16, 8ull * n));
+        caps.surv = direct ? ntiles * (ntiles + 1) / 2 : std::max<uint64_t>(1u << 16, 2ull * n);
+        caps.cand = 128ull * n + 65536;
         if (auto it = ctx->bufs.find("pairs.tiles"); it != ctx->bufs.end())
-            list_cap = std::max<uint64_t>(list_cap, it->second.bytes / sizeof(uint4));
+            caps.list = std::max<uint64_t>(caps.list, it->second.bytes / sizeof(uint4));
         if (auto it = ctx->bufs.find("pairs.stiles"); it != ctx->bufs.end())
-            surv_cap = std::max<uint64_t>(surv_cap, it->second.bytes / sizeof(uint4));
+            caps.surv = std::max<uint64_t>(caps.surv, it->second.bytes / sizeof(uint4));
         if (auto it = ctx->bufs.find("pairs.cand"); it != ctx->bufs.end())
-            cand_cap = std::max<uint64_t>(cand_cap, it->second.bytes / sizeof(Cand));
+            caps.cand = std::max<uint64_t>(caps.cand, it->second.bytes / sizeof(Cand));
         for (int attempt = 0;; ++attempt) {
             if (attempt == 4) MDET_FAIL(MDET_E_STATE, "mdet_tnf_edges: survivor count grew between passes");
             if (attempt) MDET_HIP(hipMemsetAsync(ctr + CTR_LIST, 0, (zero_words - 2 * CTR_LIST) * 4, ctx->stream));
             uint4* list = nullptr;
             Cand* cand;
             uint64_t* amb;
-            MDET_TRY(ctx_buf(ctx, "pairs.cand", cand_cap, &cand));
-            MDET_TRY(ctx_buf(ctx, "pairs.amb", cand_cap, &amb));
-            if (!direct) MDET_TRY(ctx_buf(ctx, "pairs.tiles", list_cap, &list));
+            MDET_TRY(ctx_buf(ctx, "pairs.cand", caps.cand, &cand));
+            MDET_TRY(ctx_buf(ctx, "pairs.amb", caps.cand, &amb));
+            if (!direct) MDET_TRY(ctx_buf(ctx, "pairs.tiles", caps.list, &list));
             // -- first pass: the tiles
             MDET_TRY(tm.record(1));
             if (!direct && nitems) {
@@ -3353,7 +3378,7 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 // counter, or with per-XCD queues (qbounds) each from its
                 // queue's counter (the grid then covers every queue)
                 uint32_t* pf_ctr = tune.persistent ? reinterpret_cast<uint32_t*>(ctr + CTR_QUEUES) : nullptr;
-                const TileList tl{list, ctr + CTR_LIST, (unsigned long long)list_cap};
+                const TileList tl{list, ctr + CTR_LIST, (unsigned long long)caps.list};
                 auto grid = [&](uint32_t per_cu) {
                     const uint32_t resident = (uint32_t)ctx->num_cus * per_cu;
                     if (!pf_ctr) return dim3(nitems);
@@ -3382,9 +3407,9 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             }
             MDET_TRY(tm.record(2));
             // -- second pass: the tiles' pairs
-            SurvTiles sv{nullptr, nullptr, ctr + CTR_SURV, (unsigned long long)surv_cap, ctr + CTR_CAND};
-            MDET_TRY(ctx_buf(ctx, "pairs.stiles", surv_cap, &sv.buf));
-            MDET_TRY(ctx_buf(ctx, "pairs.smask", surv_cap * 64, &sv.mask));
+            SurvTiles sv{nullptr, nullptr, ctr + CTR_SURV, (unsigned long long)caps.surv, ctr + CTR_CAND};
+            MDET_TRY(ctx_buf(ctx, "pairs.stiles", caps.surv, &sv.buf));
+            MDET_TRY(ctx_buf(ctx, "pairs.smask", caps.surv * 64, &sv.mask));
             const RowArgs rows{tnf_dev, tvec, perm, n, nullptr, 0};
             // persistent blocks over the device's counts (a multiple of 8: one
             // XCD each in turn), no more than a small input has tiles for
@@ -3401,11 +3426,12 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             ga.whole = make_uint4(0, n, 0, n | ITEM_TRI);
             ga.list = list;
             ga.n_list = ctr + CTR_LIST;
-            ga.list_cap = list_cap;
+            ga.list_cap = caps.list;
             ga.ntiles = (uint32_t)ntiles;
             ga.out = sv;
             if (f32) {
-                const F32Args fa{rows, list, ctr + CTR_LIST, (unsigned long long)list_cap, (uint32_t)ntiles, f32_r2, sv};
+                const F32Args fa{rows, list, ctr + CTR_LIST, (unsigned long long)caps.list, (uint32_t)ntiles, f32_r2,
+                                 sv};
                 hipLaunchKernelGGL(k_tile_f32, rgrid, dim3(256), 0, ctx->stream, fa);
             } else if (!tnf_gram) {
                 hipLaunchKernelGGL((k_tile_gram<true, KS_E, false>), ggrid, dim3(256), 0, ctx->stream, ga);
@@ -3414,24 +3440,17 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             } else {
                 hipLaunchKernelGGL((k_tile_gram<false, KS, false>), ggrid, dim3(256), 0, ctx->stream, ga);
             }
-            RefineArgs ra{rows, sv, (float)T, cand, (unsigned long long)cand_cap, ctr + CTR_KEPT, bcnt, amb, ctr + CTR_AMB};
+            RefineArgs ra{rows, sv, (float)T, cand, (unsigned long long)caps.cand, ctr + CTR_KEPT, bcnt, amb,
+                          ctr + CTR_AMB};
             hipLaunchKernelGGL(k_tile_refine, rgrid, dim3(256), 0, ctx->stream, ra);
             const dim3 agrid(2 * ctx->num_cus);
             hipLaunchKernelGGL(k_adjudicate, agrid, dim3(256), 0, ctx->stream, tnf_dev, logsize_dev, iperm, T, rule,
                                cutoff, amb, ctr + CTR_AMB, cand, ctr + CTR_KEPT, bcnt);
             MDET_HIP(hipGetLastError());
-            // what a list needed, from the counters at host[]: true if the pass has to run again
-            auto too_small = [&]() {
-                bool again = false;
-                auto grow = [&](unsigned long long need, uint64_t& cap) {
-                    if (need > cap) cap = need + need / 4 + 64, again = true;
-                };
-                if (!direct) grow(host[CTR_LIST], list_cap);
-                grow(std::max(host[CTR_SURV], host[CTR_FB_SURV]), surv_cap);
-                grow(host[CTR_FB_LIST], fb_cap);
-                grow(host[CTR_CAND], cand_cap);
-                return again;
-            };
+            // what kernels may read of the candidates without the host, and
+            // whether the counters at host[] ask for another pass
+            const Records records{cand, ctr, caps};
+            auto too_small = [&]() { return mdet::grow_lists(pass_counts(host), caps); };
             // -- learned mode with the cluster index and the TNF Gram: the exact
             // fallback for full rows
             uint64_t ns1 = 0;
@@ -3449,8 +3468,8 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                 MDET_TRY(ctx_buf(ctx, "fb.ids", (size_t)n, &full_ids));
                 uint32_t* n_full_dev = reinterpret_cast<uint32_t*>(ctr + CTR_FULL);
                 MDET_HIP(hipMemsetAsync(kept, 0, (size_t)n * 4, ctx->stream));
-                hipLaunchKernelGGL(k_row_kept, dim3(8u * ctx->num_cus), dim3(256), 0, ctx->stream, cand, ctr + CTR_CAND,
-                                   (unsigned long long)cand_cap, iperm, kept);
+                hipLaunchKernelGGL(k_row_kept, dim3(8u * ctx->num_cus), dim3(256), 0, ctx->stream, records, iperm,
+                                   kept);
                 hipLaunchKernelGGL(k_full_flags, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, kept, n, need, full);
                 hipcub::CountingInputIterator<uint32_t> pos_it(0);
                 size_t tmp = 0;
@@ -3499,14 +3518,14 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                     MDET_HIP(hipMemsetAsync(pbits, 0, (size_t)(nbits + 31) / 32 * 4, ctx->stream));
                     hipLaunchKernelGGL(k_probed_bits, dim3((unsigned)(((uint64_t)ivf.k * ivf.n_probe + 255) / 256)),
                                        dim3(256), 0, ctx->stream, ivf.probes_dev, ivf.k, ivf.n_probe, pbits);
-                    fb_cap = std::max<uint64_t>(fb_cap, std::max<uint64_t>(1u << 16, 64ull * n_full));
+                    caps.fb_list = std::max<uint64_t>(caps.fb_list, std::max<uint64_t>(1u << 16, 64ull * n_full));
                     if (auto it = ctx->bufs.find("fb.tiles"); it != ctx->bufs.end())
-                        fb_cap = std::max<uint64_t>(fb_cap, it->second.bytes / sizeof(uint4));
+                        caps.fb_list = std::max<uint64_t>(caps.fb_list, it->second.bytes / sizeof(uint4));
                     uint4* flist;
                     uint64_t* amb2;
-                    MDET_TRY(ctx_buf(ctx, "fb.tiles", fb_cap, &flist));
-                    MDET_TRY(ctx_buf(ctx, "fb.amb", cand_cap, &amb2));
-                    const TileList tl{flist, ctr + CTR_FB_LIST, (unsigned long long)fb_cap};
+                    MDET_TRY(ctx_buf(ctx, "fb.tiles", caps.fb_list, &flist));
+                    MDET_TRY(ctx_buf(ctx, "fb.amb", caps.cand, &amb2));
+                    const TileList tl{flist, ctr + CTR_FB_LIST, (unsigned long long)caps.fb_list};
                     uint32_t* const fb_ctr = reinterpret_cast<uint32_t*>(ctr + CTR_FB_QUEUE);
                     auto fb_grid = [&](uint32_t per_cu) {
                         return dim3(std::min<uint32_t>(w, (uint32_t)ctx->num_cus * per_cu));
@@ -3531,7 +3550,7 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                     ga.items = fitems;
                     ga.list = flist;
                     ga.n_list = ctr + CTR_FB_LIST;
-                    ga.list_cap = fb_cap;
+                    ga.list_cap = caps.fb_list;
                     ga.out = sv;
                     ga.full_pos = full_pos;
                     ga.full_base = n_frag;
@@ -3561,8 +3580,8 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             MDET_TRY(ctx_buf(ctx, "sel.boff", (size_t)nb + 1, &boff));
             MDET_TRY(ctx_buf(ctx, "sel.rbeg", (size_t)n, &rbeg));
             MDET_TRY(ctx_buf(ctx, "sel.eoff", (size_t)n + 1, &eoff));
-            MDET_TRY(ctx_buf(ctx, "sel.ent", 2 * cand_cap, &ent));
-            MDET_TRY(ctx_buf(ctx, "sel.adj", 2 * cand_cap, &adj));
+            MDET_TRY(ctx_buf(ctx, "sel.ent", 2 * caps.cand, &ent));
+            MDET_TRY(ctx_buf(ctx, "sel.adj", 2 * caps.cand, &adj));
             unsigned int* err = reinterpret_cast<unsigned int*>(ctr + CTR_ERR);
             unsigned long long* capped = ctr + CTR_CAPPED;
             // rows for the block-wide path (big) and for the global-memory path (huge)
@@ -3574,16 +3593,15 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             const RowList huge{huge_rec, reinterpret_cast<uint32_t*>(ctr + CTR_HUGE), big_cap};
             uint32_t *from, *to;
             float* s;
-            MDET_TRY(ctx_buf(ctx, "out.from", cand_cap, &from));
-            MDET_TRY(ctx_buf(ctx, "out.to", cand_cap, &to));
-            MDET_TRY(ctx_buf(ctx, "out.s", cand_cap, &s));
+            MDET_TRY(ctx_buf(ctx, "out.from", caps.cand, &from));
+            MDET_TRY(ctx_buf(ctx, "out.to", caps.cand, &to));
+            MDET_TRY(ctx_buf(ctx, "out.s", caps.cand, &s));
             MDET_TRY(exclusive_scan_u32_to_u64(ctx, bcnt, boff, nb));
-            const uint64_t pieces = (cand_cap + 255) / 256;
+            const uint64_t pieces = (caps.cand + 255) / 256;
             hipLaunchKernelGGL(k_bucket_fill, dim3((unsigned)std::min<uint64_t>(pieces, 16u * ctx->num_cus)), dim3(256),
-                               0, ctx->stream, cand, ctr + CTR_CAND, (unsigned long long)cand_cap, iperm, boff, bcur,
-                               ent);
-            hipLaunchKernelGGL(k_bucket_select, dim3(nb), dim3(S_THREADS), 0, ctx->stream, boff, ent, adj, n, max_edges,
-                               perm, tnf_dev, logsize_dev, out_cnt, rbeg, big, err, capped);
+                               0, ctx->stream, records, iperm, boff, bcur, ent);
+            hipLaunchKernelGGL(k_bucket_select, dim3(nb), dim3(S_THREADS), 0, ctx->stream, records, boff, ent, adj, n,
+                               max_edges, perm, tnf_dev, logsize_dev, out_cnt, rbeg, big, err, capped);
             hipLaunchKernelGGL(k_bigrow_select, dim3(ctx->num_cus), dim3(S_THREADS), 0, ctx->stream, big, adj,
                                max_edges, tnf_dev, logsize_dev, out_cnt, rbeg, huge, err, capped);
             MDET_HIP(hipGetLastError());
