@@ -46,4 +46,10 @@ constexpr bool grow_lists(const PassCounts& n, PassCaps& cap) {
     return grown;
 }
 
+// Passes of one call at most.  A list's true length shows only in a pass in
+// which the list before it fits: listed tiles, then survivors and candidates,
+// then the full rows' listed tiles, then theirs (with all candidates), and the
+// pass after that holds everything.
+constexpr int PASS_MAX = 5;
+
 }  // namespace mdet

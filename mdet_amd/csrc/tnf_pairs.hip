@@ -3363,7 +3363,7 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
         if (auto it = ctx->bufs.find("pairs.cand"); it != ctx->bufs.end())
             caps.cand = std::max<uint64_t>(caps.cand, it->second.bytes / sizeof(Cand));
         for (int attempt = 0;; ++attempt) {
-            if (attempt == 4) MDET_FAIL(MDET_E_STATE, "mdet_tnf_edges: survivor count grew between passes");
+            if (attempt == mdet::PASS_MAX) MDET_FAIL(MDET_E_STATE, "mdet_tnf_edges: survivor count grew between passes");
             if (attempt) MDET_HIP(hipMemsetAsync(ctr + CTR_LIST, 0, (zero_words - 2 * CTR_LIST) * 4, ctx->stream));
             uint4* list = nullptr;
             Cand* cand;

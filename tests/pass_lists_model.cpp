@@ -1,7 +1,9 @@
 // Host model of the lists of an edge-list call (mdet_amd/csrc/pass_lists.h):
 // tiles reserve slots and records, the refinement writes the records of the
-// tiles that got a slot and fit, readers go by records_written.  Prints what
+// tiles that got a slot and fit, readers go by records_written; and passes are
+// repeated with grow_lists until everything fits.  Prints what
 // tests/test_pass_lists.py checks.
+#include <algorithm>
 #include <cstdio>
 #include <random>
 #include <vector>
@@ -10,9 +12,40 @@
 
 using namespace mdet;
 
+// One pass over an input whose lists would come out as `full` (cand: the first
+// pass's, fb_cand the full rows'), cut by what there is room for: entries past a
+// list's end are counted, but not worked on.
+static PassCounts pass(const PassCounts& full, uint64_t fb_cand, const PassCaps& cap, bool full_rows) {
+    auto share = [](uint64_t whole, uint64_t part, uint64_t of) {
+        return part >= of ? whole : (uint64_t)((double)whole * (double)part / (double)of);
+    };
+    PassCounts n{};
+    n.list = full.list;
+    n.surv = share(full.surv, cap.list, full.list);
+    n.cand = share(full.cand, cap.list, full.list);
+    PassCaps unused = cap;
+    if (!full_rows || grow_lists(n, unused)) return n;  // the host looks before the full rows
+    n.fb_list = full.fb_list;
+    n.fb_surv = share(full.fb_surv, cap.fb_list, full.fb_list);
+    n.cand += share(fb_cand, cap.fb_list, full.fb_list);
+    return n;
+}
+
 int main() {
     std::mt19937_64 rng(7);
     auto below = [&](uint64_t n) { return n ? rng() % n : 0; };
+    long failed[2] = {0, 0}, most[2] = {0, 0};
+    for (int trial = 0; trial < 40000; ++trial) {
+        auto length = [&] { return 1 + below(1ull << (1 + below(40))); };
+        const bool full_rows = trial & 1;
+        const PassCounts full{length(), length(), length(), length(), length()};
+        const uint64_t fb_cand = length();
+        PassCaps cap{length(), length(), length(), length()};
+        int passes = 1;
+        while (passes <= PASS_MAX && grow_lists(pass(full, fb_cand, cap, full_rows), cap)) ++passes;
+        failed[full_rows] += passes > PASS_MAX;
+        most[full_rows] = std::max<long>(most[full_rows], passes);
+    }
     long reads = 0, unwritten_read = 0, gaps = 0, refused_whole = 0;
     for (int trial = 0; trial < 20000; ++trial) {
         const uint64_t tiles = 1 + below(60);
@@ -45,6 +78,8 @@ int main() {
             refused_whole += whole;
         }
     }
+    std::printf("failed %ld failed_full_rows %ld most %ld most_full_rows %ld limit %d\n", failed[0], failed[1], most[0],
+                most[1], PASS_MAX);
     std::printf("reads %ld unwritten_read %ld gaps %ld refused_whole %ld\n", reads, unwritten_read, gaps, refused_whole);
     return 0;
 }

@@ -1,7 +1,8 @@
 """The lists of an edge-list call that the device fills before the host knows
 their lengths, on a host model built from the library's own rule
 (mdet_amd/csrc/pass_lists.h): whatever the capacities, no candidate record is
-read that no kernel wrote."""
+read that no kernel wrote, and the passes that a call may take are enough for
+every list to be sized from its own length."""
 import os
 import subprocess
 
@@ -21,7 +22,14 @@ def model(tmp_path_factory):
 
 
 def test_no_unwritten_record_is_read(model):
-    r = model[0]
+    r = model[1]
     assert r["gaps"] > 1000 and r["reads"] > 1000  # the sweep reaches both sides
     assert r["unwritten_read"] == 0
     assert r["refused_whole"] == 0  # and what is whole is read
+
+
+def test_every_list_is_sized_within_the_passes_of_a_call(model):
+    r = model[0]
+    assert r["failed"] == 0 and r["failed_full_rows"] == 0
+    # lists, survivors and candidates, then all fits; the full rows' lists come behind those
+    assert r["most"] == 3 and r["most_full_rows"] == r["limit"]
