@@ -422,16 +422,20 @@ typedef struct mdet_tune {
 int mdet_tune_get(mdet_ctx *ctx, int precision, mdet_tune *out);
 int mdet_tune_set(mdet_ctx *ctx, int precision, const mdet_tune *in);
 /* Times the candidate shapes on this input (each the median of reps calls of
- * mdet_tnf_edges; reps 1..15): prefilter column spans 512/1024/2048/4096 x
- * {per-item blocks, persistent blocks with item order 0 or 1} (for the Gram
- * modes; the exact mode has no prefilter shape) by the prefilter stage time,
- * then refine blocks per CU 8/16/32/64 by the refine stage time.  Keeps the fastest in ctx and returns
- * it (out may be NULL); the last call's edge list stays in ctx as after
- * mdet_tnf_edges.  ~(12 + 4) x reps + 1 edge-list calls. */
+ * mdet_tnf_edges; reps 1..15) by the prefilter stage time: column spans
+ * 512/1024/2048/4096, and longer ones up to the default where n makes that
+ * longer, x {per-item blocks, persistent blocks with item order 0 or 1} (for
+ * the Gram modes; EXACT_F32's shape is not tuned).  Keeps the fastest in ctx,
+ * the default unless another is more than 2% faster, and returns it (out may be
+ * NULL).  Small inputs (up to 6,144 contigs), which skip that stage, leave the
+ * shape as it is (ms_prefilter 0).  refine_blocks is set to its default (every
+ * value above what fits launches the same) and its stage timed there.  The last
+ * call's edge list stays in ctx as after mdet_tnf_edges.  ~13 x reps + 1
+ * edge-list calls, 19 x reps + 1 at 1,000,000 contigs. */
 int mdet_tnf_autotune(mdet_ctx *ctx, const float *tnf_dev, const double *logsize_dev, uint32_t n, double cutoff,
                       uint32_t max_edges, int precision, uint32_t reps, mdet_tune *out);
-/* The same for the learned mode (per-item or persistent prefilter blocks,
- * refine blocks per CU), with mdet_tnf_edges_learned's arguments. */
+/* The same for the learned mode (per-item or persistent prefilter blocks),
+ * with mdet_tnf_edges_learned's arguments. */
 int mdet_tnf_autotune_learned(mdet_ctx *ctx, mdet_mlp *mlp, const float *tnf_dev, const double *logsize_dev,
                               uint32_t n, double cutoff, uint32_t max_edges, float radius2, uint32_t n_clusters,
                               uint32_t n_probe, uint32_t reps, mdet_tune *out);

@@ -44,6 +44,7 @@
 #include "model_tables.h"
 #include "order.h"
 #include "pass_lists.h"
+#include "scan_spans.h"
 #include "tnf_tables.h"
 
 namespace {
@@ -3048,16 +3049,6 @@ int exclusive_scan_u32_to_u64(mdet_ctx* ctx, const uint32_t* in, uint64_t* out, 
 // items still come spread over time and XCDs, while an XCD's blocks share
 // column ranges in its L2: memory-side traffic 19.4 -> 3.5 GB and 10% faster
 // at 200k contigs in the full Gram over 256-row blocks.
-// Default column span by size: the power of two nearest n / 50 in [512, 16384].
-// Longer spans spare the box scan row fragments and boxes (43 -> 34 us at 50,000
-// contigs and 10.64 -> 10.49 ms at 1,000,000 against n / 100 and at most 4096);
-// short ones keep enough items for the blocks of small inputs.
-uint32_t seg_cols_for(uint32_t n) {
-    uint32_t seg = 512;
-    while (seg < 16384 && (uint64_t)seg * 3 / 2 * 50 < n) seg *= 2;
-    return seg;
-}
-
 // order 0: one list, row-block major.  order 1: PF_QUEUES lists (row blocks
 // rb with rb % PF_QUEUES == q), each ordered by column start then row block,
 // so the blocks of one XCD work on neighbouring column ranges together;
@@ -3762,13 +3753,16 @@ int mdet_tune_set(mdet_ctx* ctx, int precision, const mdet_tune* in) {
 
 namespace {
 
-// Times the launch shapes of the pair stage on this input and keeps the
-// fastest in ctx->tune[precision]: first the prefilter shape (item column
-// span for the Gram modes x {one block per item, persistent blocks with one
-// queue, persistent blocks with per-XCD queues}), by the median prefilter
-// stage time over reps calls, then the refine blocks per CU at that shape,
-// by the median refine stage time.  Every shape gives
-// the same edge list; the last call's list stays in ctx.
+// Times the launch shapes of the first pass on this input and keeps the
+// fastest in ctx->tune[precision]: item column span for the Gram modes x {one
+// block per item, persistent blocks with one queue, persistent blocks with
+// per-XCD queues}, by the median stage time over reps calls, the shape of an
+// untuned context first and kept unless another beats it (tuned_shape_wins).
+// Inputs that skip the pass leave the shape as it is: there is nothing to time,
+// and a larger input on the same context uses it.  The refinement launches the
+// blocks that fit (REFINE_PER_CU), one launch for all settings from there on:
+// it stays at the default and is timed at it.  Every shape gives the same edge
+// list; the last call's list stays in ctx.
 int autotune_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, uint32_t n, double cutoff,
                   uint32_t max_edges, int precision, mdet_mlp* mlp, float radius2, uint32_t n_clusters,
                   uint32_t n_probe, uint32_t reps, mdet_tune* out) {
@@ -3799,16 +3793,16 @@ int autotune_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev
         return rc;
     };
     if (int rc = call(); rc != MDET_OK) return fail(rc);  // first-call allocations at the current shape
-    // 1. prefilter shape
+    // 1. the first pass's shape
     struct Shape {
         uint32_t seg, pers, order;
     };
     std::vector<Shape> shapes;
     if (precision == MDET_BF16_REFINE || precision == MDET_F16_REFINE) {
-        for (uint32_t seg : {512u, 1024u, 2048u, 4096u})
-            for (const Shape sh : {Shape{seg, 0u, 0u}, Shape{seg, 1u, 0u}, Shape{seg, 1u, 1u}}) shapes.push_back(sh);
+        for (uint32_t seg : n > DIRECT_MAX ? tune_spans(n) : std::vector<uint32_t>())
+            for (const Shape sh : {Shape{seg, 1u, 1u}, Shape{seg, 1u, 0u}, Shape{seg, 0u, 0u}}) shapes.push_back(sh);
     } else if (precision == MDET_LEARNED) {
-        for (uint32_t pers : {0u, 1u}) shapes.push_back({t.seg_cols, pers, t.item_order});
+        for (uint32_t pers : {1u, 0u}) shapes.push_back({t.seg_cols, pers, t.item_order});
     }
     double best_pre = 0;
     if (!shapes.empty()) {
@@ -3820,7 +3814,7 @@ int autotune_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev
             t.item_order = sh.order;
             double ms;
             if (int rc = median_of(&mdet_pair_stats::ms_prefilter, &ms); rc != MDET_OK) return fail(rc);
-            if (ms < best_pre) {
+            if (tuned_shape_wins(ms, best_pre)) {
                 best_pre = ms;
                 best = sh;
             }
@@ -3829,19 +3823,10 @@ int autotune_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev
         t.persistent = best.pers;
         t.item_order = best.order;
     }
-    // 2. refine blocks per CU
-    double best_ref = 1e300;
-    uint32_t best_rb = t.refine_blocks;
-    for (uint32_t rb : {8u, 16u, 32u, 64u}) {
-        t.refine_blocks = rb;
-        double ms;
-        if (int rc = median_of(&mdet_pair_stats::ms_refine, &ms); rc != MDET_OK) return fail(rc);
-        if (ms < best_ref) {
-            best_ref = ms;
-            best_rb = rb;
-        }
-    }
-    t.refine_blocks = best_rb;
+    // 2. the refinement at that shape
+    t.refine_blocks = mdet_ctx::Tune().refine_blocks;
+    double best_ref;
+    if (int rc = median_of(&mdet_pair_stats::ms_refine, &best_ref); rc != MDET_OK) return fail(rc);
     t.ms_prefilter = best_pre;
     t.ms_refine = best_ref;
     if (out) *out = mdet_tune{t.seg_cols, t.persistent, t.refine_blocks, t.item_order, t.ms_prefilter, t.ms_refine};
