@@ -3107,6 +3107,12 @@ constexpr int PREP_EVENT = 6;  // context event index marking the log-size range
 // Exhaustive modes up to this many contigs skip the row order and the first
 // pass: every tile goes to the second one.
 constexpr uint32_t DIRECT_MAX = 6144;
+// Contigs above which the selection's buffers go by the counted candidates: 52
+// bytes each of 128 a contig are 7.5 KB a contig, more than half of a call's
+// memory (12.2 KB a contig; counted 7.8 with 86 survivors a contig and 4.8 with
+// hardly any), and the wait of ~20 us is nothing beside the 20 ms of such an
+// input.
+constexpr uint32_t COUNTED_SELECT = 1u << 20;
 // Pairs of full rows and contigs, and of the probed clusters, from which on the
 // learned filter scans projected rows as the exhaustive modes do: the projection
 // takes ~190 us at 200,000 contigs (110 of them at any size) and serves both;
@@ -3563,16 +3569,24 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             }
             MDET_TRY(tm.record(3));
 
-            // -- select: no host round trip up to the edges; every buffer is
-            // sized by the candidates' capacity
+            // -- select: no host round trip up to the edges, with every buffer
+            // sized by the candidates' capacity; large inputs wait for the
+            // counters and take what the kept candidates need
+            uint64_t sel_cap = caps.cand;
+            if (n > COUNTED_SELECT) {
+                MDET_HIP(hipMemcpyAsync(host, ctr, 8 * CTR_HOST, hipMemcpyDeviceToHost, ctx->stream));
+                MDET_HIP(hipStreamSynchronize(ctx->stream));
+                if (too_small()) continue;
+                sel_cap = std::max<uint64_t>(host[CTR_KEPT], 1);
+            }
             uint64_t *boff, *eoff, *rbeg;
             Ent* ent;
             Adj* adj;
             MDET_TRY(ctx_buf(ctx, "sel.boff", (size_t)nb + 1, &boff));
             MDET_TRY(ctx_buf(ctx, "sel.rbeg", (size_t)n, &rbeg));
             MDET_TRY(ctx_buf(ctx, "sel.eoff", (size_t)n + 1, &eoff));
-            MDET_TRY(ctx_buf(ctx, "sel.ent", 2 * caps.cand, &ent));
-            MDET_TRY(ctx_buf(ctx, "sel.adj", 2 * caps.cand, &adj));
+            MDET_TRY(ctx_buf(ctx, "sel.ent", 2 * sel_cap, &ent));
+            MDET_TRY(ctx_buf(ctx, "sel.adj", 2 * sel_cap, &adj));
             unsigned int* err = reinterpret_cast<unsigned int*>(ctr + CTR_ERR);
             unsigned long long* capped = ctr + CTR_CAPPED;
             // rows for the block-wide path (big) and for the global-memory path (huge)
@@ -3584,9 +3598,9 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
             const RowList huge{huge_rec, reinterpret_cast<uint32_t*>(ctr + CTR_HUGE), big_cap};
             uint32_t *from, *to;
             float* s;
-            MDET_TRY(ctx_buf(ctx, "out.from", caps.cand, &from));
-            MDET_TRY(ctx_buf(ctx, "out.to", caps.cand, &to));
-            MDET_TRY(ctx_buf(ctx, "out.s", caps.cand, &s));
+            MDET_TRY(ctx_buf(ctx, "out.from", sel_cap, &from));
+            MDET_TRY(ctx_buf(ctx, "out.to", sel_cap, &to));
+            MDET_TRY(ctx_buf(ctx, "out.s", sel_cap, &s));
             MDET_TRY(exclusive_scan_u32_to_u64(ctx, bcnt, boff, nb));
             const uint64_t pieces = (caps.cand + 255) / 256;
             hipLaunchKernelGGL(k_bucket_fill, dim3((unsigned)std::min<uint64_t>(pieces, 16u * ctx->num_cus)), dim3(256),
