@@ -502,9 +502,9 @@ __global__ __launch_bounds__(256) void k_prep_lowp(const float* __restrict__ x, 
 //   KSX = 9, RT = 2, CT = 4: cluster pairs and full rows of the learned
 //     filter, on the TNF rows themselves.
 //   KSX = 3, RT = 2, CT = 4: the embedding radius of the learned filter.
-// Measured and dropped in the full Gram form of this kernel (KSX = 9 over all
-// pairs): B reads ahead by hand, ping-pong accumulators (one wave per SIMD),
-// 8-wave blocks, s_setprio around the chains, two distinct LDS arrays.
+// Both in BF16.  Measured and dropped in the full Gram form of this kernel (KSX =
+// 9 over all pairs): B reads ahead by hand, ping-pong accumulators (one wave per
+// SIMD), 8-wave blocks, s_setprio around the chains.
 constexpr uint32_t SCAN_WAVES = 4;
 constexpr uint32_t scan_rows(int rt) { return 32u * rt * SCAN_WAVES; }  // rows per item of row blocks
 constexpr int PROJ_RT = 4;  // row tiles a wave of the projected scan
@@ -641,7 +641,7 @@ __device__ inline void tiles_flush(const TileList& o, const uint4* stage, uint32
     n = 0;
 }
 
-template <bool BF16, int KSX, int RT, int CT>
+template <int KSX, int RT, int CT>
 __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const uint4* __restrict__ frag_a,
                                           const uint4 it, const uint32_t item, uint4* B0, uint4* B1,
                                           const int wave, uint4* stage, uint32_t& nstage,
@@ -696,7 +696,7 @@ __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const 
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int c = 0; c < CG; ++c) acc[rt][c] = mfma32<BF16>(a[rt][ks], b[c], acc[rt][c]);
+                    for (int c = 0; c < CG; ++c) acc[rt][c] = mfma32<true>(a[rt][ks], b[c], acc[rt][c]);
             }
             // per-lane maxima of each 32 x 32 tile.  acc > 0.0f exactly when
             // its bits, read as a signed int, are > 0, so the maxima are
@@ -744,48 +744,39 @@ __device__ __forceinline__ void scan_item(const uint4* __restrict__ frag, const 
 
 // One block per item (item_ctr == nullptr: item = blockIdx.x), or persistent
 // blocks that take items from a counter until the items are handed out.
-// With qbounds (item_order 1), the items come in 8 queues [qbounds[q],
-// qbounds[q + 1]), one per XCD: block b serves queue b % 8 (the XCD
-// workgroups are dispatched to round-robin) from counter item_ctr[16 q].
-constexpr int PF_QUEUES = 8;
-constexpr int PF_CTR_STRIDE = 16;  // counters 64 bytes apart
-
-template <bool BF16, int KSX, int RT, int CT, int WPE>
+template <int KSX, int RT, int CT, int WPE>
 __global__ __launch_bounds__(64 * SCAN_WAVES, WPE) void k_tile_scan(const uint4* __restrict__ frag,
                                                                     const uint4* __restrict__ frag_a,
                                                                     const uint4* __restrict__ items, uint32_t nitems,
-                                                                    uint32_t* __restrict__ item_ctr,
-                                                                    const uint32_t* __restrict__ qbounds,
-                                                                    TileList out) {
+                                                                    uint32_t* __restrict__ item_ctr, TileList out) {
     __shared__ uint4 B0[CT * KSX * 64], B1[CT * KSX * 64];
     __shared__ uint4 stage_all[SCAN_WAVES][TILE_STAGE];
     __shared__ uint32_t s_item;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    uint32_t item = blockIdx.x, q_end = nitems, q_base = 0;
-    uint32_t* ctr = item_ctr;
+    uint32_t item = blockIdx.x;
     if (item_ctr) {
-        if (qbounds) {
-            const uint32_t q = blockIdx.x % PF_QUEUES;
-            q_base = qbounds[q];
-            q_end = qbounds[q + 1];
-            ctr = item_ctr + q * PF_CTR_STRIDE;
-        }
-        if (threadIdx.x == 0) s_item = q_base + atomicAdd(ctr, 1u);
+        if (threadIdx.x == 0) s_item = atomicAdd(item_ctr, 1u);
         __syncthreads();
         item = s_item;
     }
     uint4* stage = stage_all[wave];
     uint32_t nstage = 0;
-    while (item < q_end) {
-        scan_item<BF16, KSX, RT, CT>(frag, frag_a, items[item], item, B0, B1, wave, stage, nstage, out);
+    while (item < nitems) {
+        scan_item<KSX, RT, CT>(frag, frag_a, items[item], item, B0, B1, wave, stage, nstage, out);
         if (!item_ctr) break;
         __syncthreads();  // every wave is done with the buffers and s_item
-        if (threadIdx.x == 0) s_item = q_base + atomicAdd(ctr, 1u);
+        if (threadIdx.x == 0) s_item = atomicAdd(item_ctr, 1u);
         __syncthreads();
         item = s_item;
     }
     tiles_flush(out, stage, nstage, threadIdx.x & 63);
 }
+
+// Queues of k_box_scan with qbounds (item_order 1): the items come in 8 queues
+// [qbounds[q], qbounds[q + 1]), one per XCD: block b serves queue b % 8 (the XCD
+// workgroups are dispatched to round-robin) from counter item_ctr[16 q].
+constexpr int PF_QUEUES = 8;
+constexpr int PF_CTR_STRIDE = 16;  // counters 64 bytes apart
 
 // The first pass of the exhaustive modes: the projected rows (order.h).  Before
 // a pair of tiles is multiplied, the gap of their bounding boxes decides whether
@@ -3395,11 +3386,11 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                                        BoxArgs{pfrag, pfrag_a, box_tiles, reach, items, nitems, pf_ctr, qbounds, tl},
                                        pbox, pbox_margin);
                 else if (tnf_gram)
-                    hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>), grid(2), block, 0, ctx->stream,
-                                       frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, tl);
+                    hipLaunchKernelGGL((k_tile_scan<KS, GRAM_RT, GRAM_CT, 2>), grid(2), block, 0, ctx->stream, frag,
+                                       frag_a, items, nitems, pf_ctr, tl);
                 else
-                    hipLaunchKernelGGL((k_tile_scan<true, KS_E, GRAM_RT, GRAM_CT, 4>), grid(4), block, 0, ctx->stream,
-                                       frag, frag_a, items, nitems, pf_ctr, (const uint32_t*)nullptr, tl);
+                    hipLaunchKernelGGL((k_tile_scan<KS_E, GRAM_RT, GRAM_CT, 4>), grid(4), block, 0, ctx->stream, frag,
+                                       frag_a, items, nitems, pf_ctr, tl);
                 MDET_HIP(hipGetLastError());
             }
             MDET_TRY(tm.record(2));
@@ -3538,9 +3529,8 @@ int edges_impl(mdet_ctx* ctx, const float* tnf_dev, const double* logsize_dev, u
                                            BoxArgs{pfrag, pfrag_a, proj_T, reach, fitems, w, fb_ctr, nullptr, tl}, pbox,
                                            pbox_margin);
                     } else {
-                        hipLaunchKernelGGL((k_tile_scan<true, KS, GRAM_RT, GRAM_CT, 2>), fb_grid(2),
-                                           dim3(64 * SCAN_WAVES), 0, ctx->stream, frag, frag_a, fitems, w, fb_ctr,
-                                           (const uint32_t*)nullptr, tl);
+                        hipLaunchKernelGGL((k_tile_scan<KS, GRAM_RT, GRAM_CT, 2>), fb_grid(2), dim3(64 * SCAN_WAVES), 0,
+                                           ctx->stream, frag, frag_a, fitems, w, fb_ctr, tl);
                     }
                     // its survivor tiles after the first phase's are worked off
                     sv.cnt = ctr + CTR_FB_SURV;
