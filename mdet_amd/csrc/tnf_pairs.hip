@@ -2193,7 +2193,6 @@ __global__ __launch_bounds__(S_THREADS, 6) void k_bucket_select(
     uint32_t n, uint32_t K, const uint32_t* __restrict__ perm, const float* __restrict__ tnf,
     const double* __restrict__ ls, uint32_t* __restrict__ out_cnt, uint64_t* __restrict__ rbeg, const RowList big,
     unsigned int* __restrict__ err, unsigned long long* __restrict__ capped) {
-    if (records_to_read(rec) == 0) return;
     constexpr int PER = S_BUCKET / 64;
     constexpr int BATCH = 8;
     __shared__ uint32_t hist[S_BUCKET], rstart[S_BUCKET], rcur[S_BUCKET], s_next[2], s_capped;
@@ -2202,6 +2201,7 @@ __global__ __launch_bounds__(S_THREADS, 6) void k_bucket_select(
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint32_t b = blockIdx.x;
     const uint64_t e0 = boff[b], e1 = boff[b + 1];
+    if (records_to_read(rec) == 0) return;  // the counters' loads go out with the bucket's
     const uint32_t row0 = b * S_BUCKET;
     const uint32_t rows = n - row0 < (uint32_t)S_BUCKET ? n - row0 : (uint32_t)S_BUCKET;
     for (int t = tid; t < S_BUCKET; t += S_THREADS) hist[t] = rcur[t] = 0;
