@@ -209,7 +209,7 @@ typedef struct mdet_pair_stats {
     /* learned mode, cluster index with the TNF Gram (mdet_tnf_edges_learned):
      * the exact fallback for rows whose proposals fill max_edges */
     uint64_t fallback_rows;    /* full rows evaluated again against every column */
-    uint64_t fallback_chunks;  /* survivor chunks of that BF16 Gram pass */
+    uint64_t fallback_chunks;  /* 32 x 32 tiles of pairs that this pass's scan lists */
     uint64_t fallback_pairs;   /* its survivors outside the probed cluster pairs, refined */
 } mdet_pair_stats;
 

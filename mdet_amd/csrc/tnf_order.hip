@@ -13,9 +13,10 @@
 // decides how many tiles are dropped, never a result: the bound holds for any
 // P with norm <= 1, which k_basis enforces on what it computed.
 //
-// The rows are visited in the order of a Morton key of the 12 leading
-// coordinates (2 bits each): 0.4% of the 32 x 32 tiles then hold a pair within
-// the radius, against 13% in the order of GC content.
+// The rows are visited in the order of their nearest of up to 4,096 centres
+// ("row order" below): 0.14% of the 32 x 32 tiles then hold a pair within the
+// radius at 200,000 contigs, against 0.44% in the order of a Morton key of the
+// rows' leading coordinates and 13% in that of GC content.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -309,8 +310,11 @@ __global__ __launch_bounds__(B_THREADS, 2) void k_basis(const float* __restrict_
 
 // Projected rows, 64 rows a block: the rows pass through LDS
 // once (lane = row, odd stride), wave g forms coordinates 7 g .. 7 g + 6 with
-// the directions from scalar loads.  Bound by reading the rows (544 bytes in,
-// 128 out per row).
+// the directions from scalar loads.  100 us for 200,000 contigs, 1.3 TB/s of 544
+// bytes in and 128 out a row: bound by latency, not by that traffic.  45 KB of
+// LDS leave three blocks a CU, whose waves spend two thirds of their time
+// waiting for the rows and then for the directions; the vector units issue in
+// 40% of the cycles, LDS is busy in 15%.
 constexpr int PJ_ROWS = 64;
 
 __global__ __launch_bounds__(256) void k_project(const float* __restrict__ tnf, uint32_t n,

@@ -246,10 +246,10 @@ __device__ inline uint32_t wave_incl_sum_dpp(uint32_t x) {
 }
 
 // Rows of the select stage are grouped in buckets of S_BUCKET consecutive
-// positions of the scan's row order (a multiple of 64; at 200k contigs 64
-// rows selected 5-9% faster than 128 and 256 rows 28% slower: more, shorter
-// blocks balance better, for slightly more bucket counting in the refinement;
-// at 1M contigs the BF16 step's selection took 4.4 ms with 64 against 3.9).
+// positions of the scan's row order (a multiple of 64; measured while the rows
+// were grouped in memory: at 200k contigs 64 rows selected 5-9% faster than 128,
+// and 256 rows 28% slower, as more, shorter blocks balance better).  A bucket of
+// 64 rows is also what k_bucket_select's LDS holds.
 constexpr int S_BUCKET = 64;
 static_assert(S_BUCKET >= 64 && S_BUCKET % 64 == 0, "the row scan gives each lane S_BUCKET / 64 rows");
 
@@ -782,7 +782,7 @@ constexpr int PF_CTR_STRIDE = 16;  // counters 64 bytes apart
 // a pair of tiles is multiplied, the gap of their bounding boxes decides whether
 // it can hold a close pair at all: a lane takes one column tile against the
 // wave's PROJ_RT row tiles (their boxes from scalar loads), 64 column tiles at a
-// time, and only the pairs left (8% at 50,000 contigs, 12% at 200,000, ~21% at
+// time, and only the pairs left (10% at 50,000 contigs, 17% at 200,000, 30% at
 // 1,000,000) go to MFMA: 2 products and a maximum tree.  Waves work on their own
 // (no barrier in the loop): the columns left differ too much for a block to
 // stage them together, so each wave reads its column fragments from L1/L2, the
@@ -1333,8 +1333,9 @@ struct RefineArgs {
 // each (the smaller size's variable summed up), so a pair takes two dot products
 // of 7 (model_of_pair); evaluated in full it was 40% of the instructions, which
 // bound this kernel (88% of the issue slots): 527 -> 485 us at 200,000
-// contigs.  The next tile's rows are
-// in registers while this tile is worked off (its contigs known one tile
+// contigs.  Now LDS does, busy in 79% of the cycles (39% of that bank conflicts
+// of the survivors' rows) against 59% of the issue slots.  The next tile's rows
+// are in registers while this tile is worked off (its contigs known one tile
 // ahead), so the loads' latency is covered by this and the CU's other blocks.
 // Survivors become candidate records {i, j, preProb, flags} in place: there is
 // no survivor list to sort and pack, and a tile's kept pairs share one row and
