@@ -3097,7 +3097,11 @@ int build_items(mdet_ctx* ctx, uint32_t n, uint32_t rows, uint32_t seg, uint32_t
 
 constexpr int PREP_EVENT = 6;  // context event index marking the log-size range's copy
 // Exhaustive modes up to this many contigs skip the row order and the first
-// pass: every tile goes to the second one.
+// pass: every tile goes to the second one.  What that costs goes with the square
+// of the contigs, the order's ~190 us do not; BF16, us direct / ordered at 100,
+// 200 and 300 contigs a genome: 6,300 contigs 392 / 359, 487 / 438, 587 / 526;
+// 8,000 491 / 369, 607 / 445, 694 / 535.  Only inputs with next to no pair in
+// range would take a later line (8,000 contigs of 4,000 genomes 210 / 312).
 constexpr uint32_t DIRECT_MAX = 6144;
 // Contigs above which the selection's buffers go by the counted candidates: 52
 // bytes each of 128 a contig are 7.5 KB a contig, more than half of a call's
